@@ -333,13 +333,20 @@ __global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, CoderParams p,
 // The kernel is bound by instruction issue and latency, so a code costs a handful of vector
 // instructions: the bit window is two words {hi, lo} read with one funnel shift (`alignbit`, the
 // next code starting q bits above lo's lowest bit); codewords reach a lane through an LDS copy of
-// the R + 4 words from the 16-byte boundary at or below its next word, loaded at the start of
-// every round with 16-byte loads and one wait (a round takes at most one word per code), so
-// refilling the bit window is a branch-free select; the round is unrolled, its symbols collect in
-// registers at fixed positions; and the zero-count sums run only in the instance for the zero
-// counts of RLE items.
-// Symbols per round R: 16 for the long sequences' workgroups, 8 for the short ones' waves (which
-// then hold less LDS: the copy is R + 4 words, >= R + 3 since it starts up to 3 words early).
+// WW words from the 16-byte boundary at or below its next word, so refilling the bit window is a
+// branch-free select; the round is unrolled, its symbols collect in registers at fixed positions;
+// and the zero-count sums run only in the instance for the zero counts of RLE items.
+// A round of R codes of at most l bits takes at most (R l + 31) / 32 + 1 words, so the copy
+// is loaded again only before a round that some lane of the wave might not finish from it (its
+// 16-byte loads and their wait; a 64-symbol block of 5-bit codes is 10 words: one or two loads where
+// a load before every round was eight dependent ones).  The first load is issued beside the lookup
+// table's, before the barrier.  The word after the window is read ahead, and the copy lies so that a
+// lane stays in its own bank.
+// A code longer than the lookup table used to cost a wave a walk over the lengths in LDS and a
+// load of its symbol, each waited for (some lane of a wave meets one at most steps).
+// Measured on MI355X, the two launches (long + short): 2048 mixed bricks 1.33 + 0.17 -> 1.22 + 0.14
+// ms, one 128^3 brick 32 + 27 -> 27 + 21 us.  A copy of R + 8 words (fewer loads) took 1.30 ms, of
+// R + 12 1.37 ms: the LDS costs more waves than the loads cost time.
 template <uint32_t R>
 constexpr uint32_t win_words() { return R + 4; }
 // row of a lane's run-path symbols in LDS: an odd number of words, so lanes writing the same
@@ -354,13 +361,14 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
                                                        const uint32_t* scratch, const DecItem* items, RleChunks rc) {
     constexpr uint32_t kDecRound = R;
     constexpr uint32_t kWinWords = win_words<R>();
-    static_assert(R % 8 == 0 && kWinWords % 4 == 0, "16-byte stores and copies");
+    // a copy starts up to 3 words early and has to hold a round's R words and the one read ahead
+    static_assert(R % 8 == 0 && kWinWords % 4 == 0 && kWinWords >= R + 4, "16-byte stores and copies");
     constexpr uint32_t RW = run_row_words<S, R>();
     constexpr uint32_t NW = kDecRound * sizeof(S) / 4;  // words of a round's symbols
     __shared__ uint32_t lut[1 << kLut];
     __shared__ int tab[96];
     __shared__ S run_all[W][64 * RW * 4 / sizeof(S)];
-    __shared__ __align__(16) uint32_t win_all[W][64 * kWinWords];
+    __shared__ uint32_t win_all[W][64 * kWinWords];
     // the workgroups of one sequence (consecutive in the list) on one XCD: its tables leave HBM once
     const uint32_t wv = xcd_order(blockIdx.x, gridDim.x);
     const uint32_t sq = wave_seq[wv];
@@ -379,33 +387,24 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     auto symbol_at = [&](int idx) -> uint32_t { return (idx >= 0 && (uint32_t)idx < nsym) ? gsyms[idx] : 0u; };
     // lookup table: 2^lb entries, indexed by the next lb bits (lb = min(longest code, kLut))
     const uint32_t lb = s.nlen < kLut ? s.nlen : kLut;
-    if (multi) {
-        // all of the thread's table loads in flight at once, then the LDS stores
+    // all of the thread's table loads in flight at once; the LDS stores follow the window's loads
+    constexpr int kPer = (1 << kLut) / (64 * W), kTabPer = (96 + 64 * W - 1) / (64 * W);
+    const uint32_t nl = multi ? 1u << lb : 0u;
+    uint32_t lv[kPer];
+    int tv[kTabPer];
+    {
         const uint32_t* glut = scratch + s.lut_off;
-        constexpr int kPer = (1 << kLut) / (64 * W);
-        const uint32_t nl = 1u << lb;
-        uint32_t lv[kPer];
 #pragma unroll
         for (int k = 0; k < kPer; k++) lv[k] = (uint32_t)(t + 64 * W * k) < nl ? glut[t + 64 * W * k] : 0u;
-        int tv[(96 + 64 * W - 1) / (64 * W)];
 #pragma unroll
-        for (int k = 0; k < (96 + 64 * W - 1) / (64 * W); k++) tv[k] = t + 64 * W * k < 96 ? s.tab[t + 64 * W * k] : 0;
-#pragma unroll
-        for (int k = 0; k < kPer; k++)
-            if ((uint32_t)(t + 64 * W * k) < nl) lut[t + 64 * W * k] = lv[k];
-#pragma unroll
-        for (int k = 0; k < (96 + 64 * W - 1) / (64 * W); k++)
-            if (t + 64 * W * k < 96) tab[t + 64 * W * k] = tv[k];
+        for (int k = 0; k < kTabPer; k++) tv[k] = multi && t + 64 * W * k < 96 ? s.tab[t + 64 * W * k] : 0;
     }
-    __syncthreads();
     const uint32_t fb = fb0 + 64u * (uint32_t)wave;
-    if (fb >= nblk) return;  // no block for this wave
     S* run_row = &run_all[wave][lane * RW * 4 / sizeof(S)];
     // the run row and the codeword copy are also accessed as words / 16-byte vectors
     typedef uint32_t __attribute__((may_alias)) u32a;
     typedef uint32_t u32x4a __attribute__((ext_vector_type(4), may_alias));
-    uint32_t* win = &win_all[wave][lane * kWinWords];
-    const uint32_t single = nsym >= 1 ? symbol_at(0) : 0u;
+    uint32_t* win = &win_all[wave][lane];  // the copy's word k at win[64 k]: a lane's own bank
     const uint32_t b = fb + lane;
     const bool valid = b < nblk;
     // the zero counts of an RLE item also give the zero-run expansion its chunk spans: the sum of
@@ -417,8 +416,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     const uint64_t avail = s.nwords - s.words_off;  // readable words from the codeword start
     auto word = [&](uint32_t i) -> uint32_t { return i < avail ? words[i] : 0u; };
     // window {hi, lo} (the next code: alignbit(hi, lo, q), 32 + q bits unread, q in [0, 31] after a
-    // refill), word nxt next; the LDS copy holds words [w0, w0 + kWinWords) of the block's stream
-    uint32_t hi = 0, lo = 0, nxt = 0;
+    // refill), then word nxt, read ahead into nx; the LDS copy holds words [w0, w0 + kWinWords) of
+    // the block's stream
+    uint32_t hi = 0, lo = 0, nx = 0, nxt = 0;
     int q = 0, w0 = 0;
     if (valid && multi) {
         const uint32_t pos = b == 0 ? 0u : scratch[s.boff_off + b];
@@ -451,33 +451,74 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
 #pragma unroll
                 for (uint32_t k = 0; k < kWinWords / 4; k++) v[k] = g4[k];
 #pragma unroll
-                for (uint32_t k = 0; k < kWinWords / 4; k++) reinterpret_cast<u32x4a*>(win)[k] = v[k];
+                for (uint32_t k = 0; k < kWinWords; k++) win[64 * k] = v[k / 4][k % 4];
             }
         } else if (valid && multi) {
 #pragma unroll
             for (uint32_t k = 0; k < kWinWords; k++) {
                 const int i = w0 + (int)k;
-                win[k] = (i >= 0 && (uint64_t)i < avail) ? words[i] : 0u;
+                win[64 * k] = (i >= 0 && (uint64_t)i < avail) ? words[i] : 0u;
             }
         }
+        if (valid && multi) nx = win[64 * (nxt - (uint32_t)w0)];
     };
+    load_window();
+#pragma unroll
+    for (int k = 0; k < kPer; k++)
+        if ((uint32_t)(t + 64 * W * k) < nl) lut[t + 64 * W * k] = lv[k];
+#pragma unroll
+    for (int k = 0; k < kTabPer; k++)
+        if (multi && t + 64 * W * k < 96) tab[t + 64 * W * k] = tv[k];
+    __syncthreads();
+    if (fb >= nblk) return;  // no block for this wave
+    const uint32_t single = nsym >= 1 ? symbol_at(0) : 0u;
+    // words a round may take, at most R (mlen <= 31); the copy serves a round when it holds as many
+    // from nxt on and the one read ahead (an entry no code of a broken table reaches takes kLut + 1 bits)
+    const uint32_t round_words = min((kDecRound * max(s.nlen, kLut + 1) + 31) / 32 + 1, kDecRound);
     auto refill = [&]() {
-        const uint32_t w = win[nxt - (uint32_t)w0];
         const bool need = q < 0;
         hi = need ? lo : hi;
-        lo = need ? w : lo;
+        lo = need ? nx : lo;
         nxt += need ? 1u : 0u;
+        nx = win[64 * (nxt - (uint32_t)w0)];  // on its way beside the code's table lookup
         q &= 31;
     };
     const uint32_t sh = 32 - lb;
     const uint32_t mlen = s.nlen;
-    // a code longer than the lookup table: the per-length first/min codes; (len << 24) | symbol
+    // A code longer than the lookup table: its length is the first l whose last code, extended with
+    // ones to 32 bits, is not below the next 32 bits, and its symbol is number (code - first code +
+    // first index) of the symbol table.  Lane l - 1 holds length l's bound (an unused length has the
+    // one before it) and the step of the index offset from l to l + 1, read by lane number, so the
+    // lookup is a few vector instructions a length and touches no memory.
+    const bool used = multi && lane < (int)mlen && lane < 32 && tab[64 + (lane & 31)] >= 0;
+    uint32_t len0 = kLut + 1;  // the first used length past the lookup table (the last length if none)
+    uint32_t bound = 0;
+    int off = 0, off_step = 0;
+    if (multi && mlen > kLut) {
+        const uint64_t m = __ballot(used) >> kLut;
+        len0 = m ? min(kLut + (uint32_t)__ffsll((unsigned long long)m), mlen) : mlen;
+        const uint64_t end = used ? (uint64_t)((uint32_t)tab[64 + (lane & 31)] + 1u) << (31 - (lane & 31)) : 1ull;
+        bound = lane + 1 >= (int)len0 ? (uint32_t)min(end - 1, (uint64_t)0xFFFFFFFFu) : 0u;
+        bound = dpp::incl_scan<uint32_t>(bound, 0u, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+        const int o = lane < 32 ? tab[lane] - tab[32 + lane] : 0;
+        off_step = __shfl_down(o, 1) - o;
+        off = __builtin_amdgcn_readlane(o, (int)len0 - 1);
+    }
+    // kLong | (length << 24) | index into the symbol table (all ones: none)
+    constexpr uint32_t kLong = 0x80000000u;
     auto slow = [&](uint32_t pk) -> uint32_t {
-        uint32_t len = kLut + 1;
-        while (len < mlen && (int)(pk >> (32 - len)) > tab[64 + len - 1]) len++;
-        const int cw = (int)(pk >> (32 - len));
-        return (len << 24) | symbol_at(tab[len - 1] + cw - tab[32 + len - 1]);
+        uint32_t len = len0;
+        int idx = off;
+        for (uint32_t l = len0; l < mlen; l++) {
+            const bool past = pk > (uint32_t)__builtin_amdgcn_readlane((int)bound, (int)l - 1);
+            if (!__any(past)) break;  // (bounds do not fall, so no lane passes a later one)
+            len += past ? 1u : 0u;
+            idx += past ? __builtin_amdgcn_readlane(off_step, (int)l - 1) : 0;
+        }
+        idx += (int)(pk >> (32 - len));
+        return kLong | (len << 24) | (((uint32_t)idx < nsym ? (uint32_t)idx : 0xFFFFFFu) & 0xFFFFFFu);
     };
+    auto long_symbol = [&](uint32_t e) { return symbol_at((int)(e & 0xFFFFFFu)); };
     // one codeword of length 1 (then it is "0" and every other codeword starts with a 1): a run of
     // k zero bits is k copies of its symbol, taken at once (the zero-count sequences, where a zero
     // count is nearly every pair, decode a few steps per round instead of kDecRound)
@@ -515,7 +556,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
             for (uint32_t i = 0; i < kDecRound; i++) put(v, i, single);
             if constexpr (Z) zs += (single + 1) * vlen;
         } else {
-            load_window();
+            if (!__all(nxt - (uint32_t)w0 + round_words < kWinWords)) load_window();
             if (run0) {
                 // positions taken at a lane's own pace: its LDS row, prefilled with the run symbol
                 const uint32_t fill = sizeof(S) == 2 ? (sym0 & 0xFFFFu) * 0x10001u : sym0;
@@ -529,24 +570,43 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
                     uint32_t e = lut[pk >> sh];
                     if (!run && e == 0u) e = slow(pk);
                     const uint32_t k = min(pk ? (uint32_t)__clz(pk) : 32u, kDecRound - i);
-                    const uint32_t sym = e & 0xFFFFFFu;
+                    const uint32_t sym = !run && (e & kLong) ? long_symbol(e) : e & 0xFFFFFFu;
                     if (!run) run_row[i] = (S)sym;
                     if constexpr (Z)
                         zs += run ? (sym0 + 1) * (min(i + k, vlen) - min(i, vlen)) : (i < vlen ? sym + 1 : 0u);
-                    q -= (int)(run ? k : (e >> 24));
+                    q -= (int)(run ? k : ((e >> 24) & 31u));
                     i += run ? k : 1u;
                 }
 #pragma unroll
                 for (uint32_t k = 0; k < NW; k++) v[k] = reinterpret_cast<const u32a*>(run_row)[k];
             } else {
+                // the symbols of long codes are read after the round, all at once: only the lengths
+                // are on the way to the next code
+                uint32_t es[kDecRound], any = 0;
 #pragma unroll
                 for (uint32_t i = 0; i < kDecRound; i++) {
                     refill();
                     const uint32_t pk = __builtin_amdgcn_alignbit(hi, lo, (uint32_t)q);
                     uint32_t e = lut[pk >> sh];
                     if (e == 0u) e = slow(pk);
-                    q -= (int)(e >> 24);
-                    const uint32_t sym = e & 0xFFFFFFu;
+                    q -= (int)((e >> 24) & 31u);
+                    es[i] = e;
+                    any |= e;
+                }
+                if (__any((int)any < 0)) {
+                    uint32_t ls[kDecRound];
+#pragma unroll
+                    for (uint32_t i = 0; i < kDecRound; i++) {
+                        const uint32_t k = es[i] & 0xFFFFFFu;
+                        ls[i] = gsyms[(es[i] & kLong) && k < nsym ? k : 0u];  // (a table holds a symbol: multi)
+                        ls[i] = k < nsym ? ls[i] : 0u;
+                    }
+#pragma unroll
+                    for (uint32_t i = 0; i < kDecRound; i++) es[i] = (es[i] & kLong) ? ls[i] : es[i];
+                }
+#pragma unroll
+                for (uint32_t i = 0; i < kDecRound; i++) {
+                    const uint32_t sym = es[i] & 0xFFFFFFu;
                     put(v, i, sym);
                     if constexpr (Z) zs += i < vlen ? sym + 1 : 0u;
                 }
@@ -578,13 +638,14 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
         }
         return zs;
     };
+    // (lanes without a block stay out: their words are not theirs to read)
     if (zsum) {
-        uint32_t zs = rounds(std::true_type{});
+        uint32_t zs = valid ? rounds(std::true_type{}) : 0u;
         const uint32_t bpc = kRleChunk / cbs;
         for (uint32_t o = 1; o < bpc; o <<= 1) zs += (uint32_t)__shfl_xor((int)zs, (int)o);
         const uint32_t c = b / bpc;
         if ((lane & (bpc - 1)) == 0 && c < (zit.n + kRleChunk - 1) / kRleChunk) rc.sums[rc.item_first[s.item] + c] = zs;
-    } else {
+    } else if (valid) {
         (void)rounds(std::false_type{});
     }
 }
