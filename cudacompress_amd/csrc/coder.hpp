@@ -5,9 +5,10 @@
 // Encode.cpp:208-471, :649-790); a call has one item per input stream; an item yields one coded
 // sequence (Huffman only) or two (zero-run RLE: symbols, then zero counts).  Everything from the
 // symbol streams to the final bitstream stays in device memory:
-//   stats   one workgroup per item: zero-run RLE computed on the fly, histograms in LDS
+//   stats   one workgroup per item (or segment of a long one): zero-run RLE computed on the fly,
+//           histograms in LDS
 //   design  one wave per coded sequence: the table design of huff_design.hpp
-//   pack    one workgroup per item: RLE recomputed, codewords packed through an LDS window
+//   pack    one workgroup per item or segment: RLE recomputed, codewords packed through an LDS window
 //   layout  one workgroup: word offset of every section (sizes from the tables and bit counts)
 //   gather  one workgroup per coded sequence: table header, bit count, codewords, offsets
 // Intermediate data (histograms, tables, codewords, block offsets) live in a scratch arena
@@ -37,6 +38,34 @@ struct CodeItem {
     uint32_t rl;         // 1: zero-run RLE + two coded sequences
     uint32_t seq;        // index of the first coded sequence
     uint32_t call;       // coder call
+};
+
+// Work of one workgroup of the streaming passes: chunks [chunk0, chunk0 + nchunk) of an item.  Most
+// items are one unit (split == kWholeItem).  An item that would keep one workgroup busy after the
+// rest of the chip ran dry is split into nseg units, number seg of which owns the segment state
+// slot0 + seg; `split` numbers the split items.
+constexpr uint32_t kWholeItem = 0xFFFFFFFFu;
+struct CodeUnit {
+    uint32_t item, chunk0, nchunk, split;
+    uint32_t seg, nseg, slot0, pad;
+};
+struct SegState {            // one segment of a split item
+    uint64_t last_nz1;       // position of the segment's last nonzero + 1 (0: none)
+    uint64_t bits_s, bits_z; // codeword bits of its symbols and zero counts
+    uint32_t pairs, pad;
+    uint32_t first_s, last_s, first_z, last_z;  // its parts of the output words it shares with its neighbours
+};
+// Words per split item: arrival counters, the largest symbol, the wide flag; then its histograms.
+constexpr uint32_t kSplitHead = 16, kSplitWords = kSplitHead + kStatBins + 256;
+// The units of a job: nunits of them, of which the nsplit_units listed in split_list are segments of
+// nsplit split items.
+struct CodeUnits {
+    const CodeUnit* units;
+    uint32_t nunits;
+    const uint32_t* split_list;
+    uint32_t nsplit_units, nsplit;
+    SegState* segs;
+    uint32_t* split_state;  // nsplit * kSplitWords
 };
 
 enum CodeErr : uint32_t {
@@ -179,16 +208,14 @@ struct ConcatGroup {
 // Copies the jobs' bitstreams back to back into dst (capacity dst_cap words), in group order.
 void coder_concat(const ConcatGroup* d_groups, uint32_t ngroups, uint32_t* dst, uint64_t dst_cap, uint64_t bytes,
                   hipStream_t st);
-// d_classes: kDesignListBase + kDesignLists * nseq words of work lists.  d_item_order: workgroup
-// k of the stats and pack passes (one per item, each a serial loop over its chunks) serves item
-// d_item_order[k] (null: item k); largest items first, so the longest loops start first.
+// d_classes: kDesignListBase + kDesignLists * nseq words of work lists.  units: what the workgroups
+// of the stats and pack passes serve (each a serial loop over its chunks), the longest first.
 void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uint32_t nseq, const CoderParams& p,
                   int symSize, uint32_t* scratch, uint64_t scratch_cap, CoderState* d_state, uint32_t* d_classes,
                   CallOut* d_calls,
                   uint32_t ncalls, const uint32_t* d_call_first_item, uint32_t* d_out, uint64_t out_cap,
                   uint64_t total_symbols, hipStream_t st, const SideStreams* side,
-                  const LayoutLink* link = nullptr, const uint32_t* design_grid = nullptr, uint32_t lane_k = 0,
-                  const uint32_t* d_item_order = nullptr);
+                  const LayoutLink* link, const uint32_t* design_grid, uint32_t lane_k, const CodeUnits& units);
 // wave_seq: for every block-decoder workgroup the coded sequence it serves; wave_first: that
 // workgroup's first block.  The first nlong entries are workgroups of kDecGroupBlocks blocks of
 // the long sequences (dec_long of the block-count bound: RLE sequences have at most n pairs), the

@@ -299,6 +299,86 @@ __global__ void k_coder_init(CoderState* st, uint32_t* classes) {
     }
 }
 
+// ---- split items -------------------------------------------------------------------------------
+// One workgroup walks an item's chunks in order, a few microseconds each (two barriers, a scan, LDS
+// atomics), so an item of hundreds of chunks coded beside few others leaves the chip idle: three
+// streams of 700,001 symbols took 669 us in the stats pass and 1056 us in the pack on three of 256
+// CUs.  The host splits such items (CodeUnit); what runs through a stream from its start is supplied
+// per segment: the last nonzero before it by k_seg_last, the pairs by the stats pass and the codeword
+// bits by k_seg_bits.  Segments meet only between launches: an arrival counter instead of
+// k_code_stats_finish, with the fences it needs, took longer than that launch (the three streams: 56
+// us against 14 + 15 in the stats, 43 against 10 in k_seg_bits).  The three streams now take 3 + 14 +
+// 15 us in the stats and 10 + 23 + 6 in the pack, 64 mixed bricks 113 -> 66 and 164 -> 78 us.
+// The last nonzero of every segment of a zero-run item, searched from its end (one wave); the waves
+// also clear the split items' shared state.
+template <class S>
+__global__ __launch_bounds__(64) void k_seg_last(const CodeItem* items, CodeUnits U) {
+    const CodeUnit u = U.units[U.split_list[blockIdx.x]];
+    const CodeItem it = items[u.item];
+    const S* in = static_cast<const S*>(it.in);
+    const uint64_t lo = (uint64_t)u.chunk0 * kChunk;
+    const uint64_t hi = min((uint64_t)it.n, lo + (uint64_t)u.nchunk * kChunk);
+    const uint32_t words = U.nsplit * kSplitWords;
+    for (uint32_t i = blockIdx.x * 64 + threadIdx.x; i < words; i += gridDim.x * 64) U.split_state[i] = 0;
+    uint64_t last1 = 0;
+    if (it.rl) {
+        constexpr uint64_t kStep = 64 * kPerThread;
+        // steps from the segment's last one down (lo is a multiple of the step)
+        for (uint64_t base = lo + (hi - 1 - lo) / kStep * kStep;; base -= kStep) {
+            const uint64_t p0 = base + threadIdx.x * kPerThread;
+            uint32_t v[kPerThread];
+            load8(in, p0, (uint32_t)hi, v);
+            const long long l = thread_last_nz(v, p0, (uint32_t)hi);
+            const uint64_t m = __ballot(l >= 0);
+            if (m) {
+                const int src = 63 - __clzll(m);
+                last1 = base + (uint64_t)__builtin_amdgcn_readlane((int)(l - (long long)base), src) + 1;
+                break;
+            }
+            if (base == lo) break;
+        }
+    }
+    if (threadIdx.x == 0) U.segs[u.slot0 + u.seg].last_nz1 = last1;
+}
+
+// Largest last_nz1 of slots [lo, hi), for every thread of a wave.
+__device__ __forceinline__ uint64_t seg_max_last(const SegState* segs, uint32_t lo, uint32_t hi) {
+    long long m = -1;
+    for (uint32_t i = lo + (threadIdx.x & 63); i < hi; i += 64) {
+        const long long l = (long long)segs[i].last_nz1;
+        m = l > m ? l : m;
+    }
+    m = (long long)dpp::last_lane64((uint64_t)wave_incl_max_i64(m));
+    return m > 0 ? (uint64_t)m : 0ull;
+}
+
+// Pairs and bits of the segments before slot hi of an item whose slots start at lo.
+__device__ __forceinline__ SegState seg_before(const SegState* segs, uint32_t lo, uint32_t hi) {
+    uint64_t s = 0, z = 0, p = 0;
+    for (uint32_t i = lo + (threadIdx.x & 63); i < hi; i += 64) {
+        s += segs[i].bits_s;
+        z += segs[i].bits_z;
+        p += segs[i].pairs;
+    }
+    SegState r{};
+    r.bits_s = wave_sum_u64(s);
+    r.bits_z = wave_sum_u64(z);
+    r.pairs = (uint32_t)wave_sum_u64(p);
+    return r;
+}
+
+// Counts this workgroup in at *counter after everything it wrote; true for the last of n, whose
+// reads then see what the others wrote.  Every thread calls.
+__device__ __forceinline__ bool last_arrival(uint32_t* counter, uint32_t n, uint32_t* sh) {
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) *sh = atomicAdd(counter, 1u);
+    __syncthreads();
+    const bool last = *sh == n - 1;
+    if (last) __threadfence();
+    return last;
+}
+
 // Words of a histogram of nb bins in the arena and, when the table may be designed one per thread
 // (k < kLaneMaxK + 1 used symbols), its leaf list after it: (symbol, count) pairs in symbol order
 // from the next 4-word boundary.
@@ -322,93 +402,14 @@ __device__ void write_leaves(const uint32_t* h, uint32_t nb, uint2* out, uint64_
     }
 }
 
-// Pass A: pair counts, histograms (LDS), maxima; tables of the LDS class get their histogram
-// copied to the arena (with the leaf list of small tables); streams with symbols >= kStatBins are
-// marked wide and get a zeroed global histogram for k_code_stats_wide.
-template <class S>
-__global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* items, SeqInfo* seqs, CoderParams p,
-                                                              uint32_t* scratch, uint64_t cap, CoderState* st,
-                                                              const uint32_t* order) {
-    __shared__ uint32_t hs[kStatBins];
-    __shared__ uint32_t hz[256];
-    __shared__ int shl[2][4];  // alternate chunks: one barrier per chunk
-    __shared__ uint32_t shu[4];
-    __shared__ uint64_t sh_off[2];
-    __shared__ uint64_t shq[4];
-    const uint32_t ii = order ? order[blockIdx.x] : blockIdx.x;
-    const CodeItem it = items[ii];
-    const S* in = static_cast<const S*>(it.in);
+// The sequence records of an item from its histograms (pairs M, largest symbol vmax, wide: symbols
+// past the LDS histogram, carry: the last nonzero): maxima, distinct counts, the histograms' copies in
+// the arena with the leaf lists of small tables.  Every thread of the workgroup calls.
+__device__ void stats_finish(const CodeItem& it, uint32_t ii, uint32_t M, uint32_t vmax, uint32_t wide, long long carry,
+                             const uint32_t* hs, const uint32_t* hz, SeqInfo* seqs, const CoderParams& p,
+                             uint32_t* scratch, uint64_t cap, CoderState* st, uint32_t* shu, uint64_t* sh_off,
+                             uint64_t* shq) {
     const bool rl = it.rl != 0;
-    const uint32_t n = it.n;
-    for (uint32_t i = threadIdx.x; i < kStatBins; i += kCoderThreads) hs[i] = 0;
-    for (uint32_t i = threadIdx.x; i < 256; i += kCoderThreads) hz[i] = 0;
-    __syncthreads();
-    long long carry = -1;
-    uint32_t cnt = 0, vmax = 0, wide = 0;
-    // histogram updates are coalesced per thread: runs of one symbol and all zero counts of zero
-    // are counted in registers (zero runs dominate the zero-count histogram)
-    uint32_t run_sym = 0xFFFFFFFFu, run_len = 0, zc0 = 0;
-    auto flush_run = [&]() {
-        if (run_len) {
-            if (run_sym < kStatBins) atomicAdd(&hs[run_sym], run_len);
-            else wide = 1;
-        }
-    };
-    const uint32_t t8 = threadIdx.x * kPerThread;
-    uint32_t vn[kPerThread];
-    load8(in, (uint64_t)t8, n, vn);
-    uint32_t par = 0;
-    for (uint64_t base = 0; base < n; base += kChunk, par ^= 1) {
-        uint32_t v[kPerThread];
-#pragma unroll
-        for (int j = 0; j < (int)kPerThread; j++) v[j] = vn[j];
-        if (base + kChunk < n) load8(in, base + kChunk + t8, n, vn);  // next step's symbols in flight
-        const uint32_t nvalid = chunk_nvalid(base, n, t8);
-        int wl;
-        const int ex = wave_excl_last(thread_last_nz_rel(v, t8, nvalid), wl);
-        if ((threadIdx.x & 63) == 0) shl[par][threadIdx.x >> 6] = wl;
-        __syncthreads();
-        int prel, ctot;
-        wg_last_combine(ex, shl[par], prel, ctot);
-        uint32_t zc[kPerThread];
-        const uint32_t emit = thread_flags_rel(v, nvalid, rl, thread_g0(prel, t8, chunk_gc(base, carry)),
-                                               chunk_lim(base, (long long)n) - (int)t8, zc);
-#pragma unroll
-        for (int j = 0; j < (int)kPerThread; j++) {
-            if (!((emit >> j) & 1u)) continue;
-            const uint32_t s = v[j], z = zc[j];
-            cnt++;
-            vmax = max(vmax, s);
-            if (s == run_sym) {
-                run_len++;
-            } else {
-                flush_run();
-                run_sym = s;
-                run_len = 1;
-            }
-            if (rl) {
-                if (z == 0) zc0++;
-                else atomicAdd(&hz[z], 1u);
-            }
-        }
-        if (ctot >= 0) carry = (long long)base + ctot;
-    }
-    flush_run();
-    zc0 = wave_sum(zc0);
-    if (rl && (threadIdx.x & 63) == 0 && zc0) atomicAdd(&hz[0], zc0);
-    uint32_t M = wg_sum_u32(cnt, shu);
-    wide = wg_max_u32(wide, shu);
-    vmax = wg_max_u32(vmax, shu);
-    if (rl) {  // fillers of the trailing run are not emitted
-        const uint64_t r = (uint64_t)((long long)n - 1 - carry);
-        const uint32_t f = (uint32_t)(r / 256);
-        if (threadIdx.x == 0 && f) {
-            hs[0] -= f;
-            hz[255] -= f;
-        }
-        M -= f;
-        __syncthreads();
-    }
     // maxima and distinct counts from the histograms
     uint32_t smax_l = 0, ks = 0, zmax_l = 0, kz = 0;
     if (!wide) {
@@ -477,14 +478,150 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* it
     }
 }
 
+// Pass A: pair counts, histograms (LDS), maxima; tables of the LDS class get their histogram
+// copied to the arena (with the leaf list of small tables); streams with symbols >= kStatBins are
+// marked wide and get a zeroed global histogram for k_code_stats_wide.
+template <class S>
+__global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* items, SeqInfo* seqs, CoderParams p,
+                                                              uint32_t* scratch, uint64_t cap, CoderState* st,
+                                                              CodeUnits U) {
+    __shared__ uint32_t hs[kStatBins];
+    __shared__ uint32_t hz[256];
+    __shared__ int shl[2][4];  // alternate chunks: one barrier per chunk
+    __shared__ uint32_t shu[4];
+    __shared__ uint64_t sh_off[2];
+    __shared__ uint64_t shq[4];
+    const CodeUnit u = U.units[blockIdx.x];
+    const uint32_t ii = u.item;
+    const bool split = u.split != kWholeItem;
+    const CodeItem it = items[ii];
+    const S* in = static_cast<const S*>(it.in);
+    const bool rl = it.rl != 0;
+    const uint32_t n = it.n;
+    const uint64_t base0 = (uint64_t)u.chunk0 * kChunk;
+    const uint64_t end = split ? min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk) : (uint64_t)n;
+    for (uint32_t i = threadIdx.x; i < kStatBins; i += kCoderThreads) hs[i] = 0;
+    for (uint32_t i = threadIdx.x; i < 256; i += kCoderThreads) hz[i] = 0;
+    __syncthreads();
+    long long carry = -1, limit = (long long)n;
+    if (split) {  // the last nonzero before the segment, and the stream's (no filler follows that one)
+        carry = (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.seg) - 1;
+        limit = (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.nseg) - 1;
+    }
+    uint32_t cnt = 0, vmax = 0, wide = 0;
+    // histogram updates are coalesced per thread: runs of one symbol and all zero counts of zero
+    // are counted in registers (zero runs dominate the zero-count histogram)
+    uint32_t run_sym = 0xFFFFFFFFu, run_len = 0, zc0 = 0;
+    auto flush_run = [&]() {
+        if (run_len) {
+            if (run_sym < kStatBins) atomicAdd(&hs[run_sym], run_len);
+            else wide = 1;
+        }
+    };
+    const uint32_t t8 = threadIdx.x * kPerThread;
+    uint32_t vn[kPerThread];
+    load8(in, base0 + t8, n, vn);
+    uint32_t par = 0;
+    for (uint64_t base = base0; base < end; base += kChunk, par ^= 1) {
+        uint32_t v[kPerThread];
+#pragma unroll
+        for (int j = 0; j < (int)kPerThread; j++) v[j] = vn[j];
+        if (base + kChunk < end) load8(in, base + kChunk + t8, n, vn);  // next step's symbols in flight
+        const uint32_t nvalid = chunk_nvalid(base, n, t8);
+        int wl;
+        const int ex = wave_excl_last(thread_last_nz_rel(v, t8, nvalid), wl);
+        if ((threadIdx.x & 63) == 0) shl[par][threadIdx.x >> 6] = wl;
+        __syncthreads();
+        int prel, ctot;
+        wg_last_combine(ex, shl[par], prel, ctot);
+        uint32_t zc[kPerThread];
+        const uint32_t emit = thread_flags_rel(v, nvalid, rl, thread_g0(prel, t8, chunk_gc(base, carry)),
+                                               chunk_lim(base, limit) - (int)t8, zc);
+#pragma unroll
+        for (int j = 0; j < (int)kPerThread; j++) {
+            if (!((emit >> j) & 1u)) continue;
+            const uint32_t s = v[j], z = zc[j];
+            cnt++;
+            vmax = max(vmax, s);
+            if (s == run_sym) {
+                run_len++;
+            } else {
+                flush_run();
+                run_sym = s;
+                run_len = 1;
+            }
+            if (rl) {
+                if (z == 0) zc0++;
+                else atomicAdd(&hz[z], 1u);
+            }
+        }
+        if (ctot >= 0) carry = (long long)base + ctot;
+    }
+    flush_run();
+    zc0 = wave_sum(zc0);
+    if (rl && (threadIdx.x & 63) == 0 && zc0) atomicAdd(&hz[0], zc0);
+    uint32_t M = wg_sum_u32(cnt, shu);
+    wide = wg_max_u32(wide, shu);
+    vmax = wg_max_u32(vmax, shu);
+    if (split) {
+        // the segments' histograms add up in global memory, k_code_stats_finish goes on with the sums
+        uint32_t* sp = U.split_state + (size_t)u.split * kSplitWords;
+        for (uint32_t i = threadIdx.x; i < kStatBins; i += kCoderThreads)
+            if (hs[i]) atomicAdd(&sp[kSplitHead + i], hs[i]);
+        if (rl && hz[threadIdx.x]) atomicAdd(&sp[kSplitHead + kStatBins + threadIdx.x], hz[threadIdx.x]);
+        if (threadIdx.x == 0) {
+            U.segs[u.slot0 + u.seg].pairs = M;
+            atomicMax(&sp[2], vmax);
+            if (wide) atomicOr(&sp[3], 1u);
+        }
+        return;
+    }
+    if (rl) {  // fillers of the trailing run are not emitted
+        const uint64_t r = (uint64_t)((long long)n - 1 - carry);
+        const uint32_t f = (uint32_t)(r / 256);
+        if (threadIdx.x == 0 && f) {
+            hs[0] -= f;
+            hz[255] -= f;
+        }
+        M -= f;
+        __syncthreads();
+    }
+    stats_finish(it, ii, M, vmax, wide, carry, hs, hz, seqs, p, scratch, cap, st, shu, sh_off, shq);
+}
+
+// The items split over several workgroups, from the segments' sums (one workgroup per item).
+__global__ __launch_bounds__(kCoderThreads) void k_code_stats_finish(const CodeItem* items, SeqInfo* seqs,
+                                                                     CoderParams p, uint32_t* scratch, uint64_t cap,
+                                                                     CoderState* st, CodeUnits U) {
+    __shared__ uint32_t hs[kStatBins];
+    __shared__ uint32_t hz[256];
+    __shared__ uint32_t shu[4];
+    __shared__ uint64_t sh_off[2];
+    __shared__ uint64_t shq[4];
+    const CodeUnit u = U.units[U.split_list[blockIdx.x]];
+    if (u.seg) return;
+    const CodeItem it = items[u.item];
+    const uint32_t* sp = U.split_state + (size_t)u.split * kSplitWords;
+    for (uint32_t i = threadIdx.x; i < kStatBins; i += kCoderThreads) hs[i] = sp[kSplitHead + i];
+    hz[threadIdx.x] = it.rl ? sp[kSplitHead + kStatBins + threadIdx.x] : 0u;
+    uint32_t m = 0;
+    for (uint32_t i = threadIdx.x; i < u.nseg; i += kCoderThreads) m += U.segs[u.slot0 + i].pairs;
+    const long long last = (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.nseg) - 1;
+    __syncthreads();
+    m = wg_sum_u32(m, shu);
+    stats_finish(it, u.item, m, sp[2], sp[3], last, hs, hz, seqs, p, scratch, cap, st, shu, sh_off, shq);
+}
+
 // Pass A for streams with symbols >= kStatBins: histogram with global atomics, then the pad
 // quirk (Symbol16, GPU dialect, max symbol 65535, odd count: src/cudaCompress/Histogram.cu:90-105).
 template <class S>
 __global__ __launch_bounds__(kCoderThreads) void k_code_stats_wide(const CodeItem* items, SeqInfo* seqs,
-                                                                   CoderParams p, uint32_t* scratch) {
+                                                                   CoderParams p, uint32_t* scratch, CodeUnits U) {
     __shared__ long long shl[4];
     __shared__ uint32_t shu[4];
-    const CodeItem it = items[blockIdx.x];
+    const CodeUnit u = U.units[blockIdx.x];
+    const bool split = u.split != kWholeItem;
+    const CodeItem it = items[u.item];
     SeqInfo* ss = &seqs[it.seq];
     if (!ss->wide || ss->err) return;
     const S* in = static_cast<const S*>(it.in);
@@ -492,8 +629,10 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats_wide(const CodeIte
     const uint32_t n = it.n;
     uint32_t* h = scratch + ss->hist_off;
     const long long last_nz = (long long)ss->last_nz1 - 1;
-    long long carry = -1;
-    for (uint64_t base = 0; base < n; base += kChunk) {
+    const uint64_t base0 = (uint64_t)u.chunk0 * kChunk;
+    const uint64_t end = split ? min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk) : (uint64_t)n;
+    long long carry = split ? (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.seg) - 1 : -1;
+    for (uint64_t base = base0; base < end; base += kChunk) {
         const uint64_t p0 = base + (uint64_t)threadIdx.x * kPerThread;
         uint32_t v[kPerThread];
         load8(in, p0, n, v);
@@ -505,6 +644,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats_wide(const CodeIte
         carry = chunk_max > carry ? chunk_max : carry;
     }
     __syncthreads();
+    if (split && !last_arrival(U.split_state + (size_t)u.split * kSplitWords + 1, u.nseg, &shu[0])) return;
     const uint32_t nb = ss->smax + 1;
     const uint32_t quirk = (p.dialect == CC_DIALECT_GPU && sizeof(S) == 2 && ss->smax == 65535u && (ss->count & 1u)) ? 1u : 0u;
     uint32_t k = 0;
@@ -932,6 +1072,142 @@ __device__ uint32_t header_word(const SeqInfo& s, const uint32_t* cpl, const Cod
     return out;
 }
 
+// Code lengths of a table to LDS, each thread's loads issued four entries at a time.
+__device__ __forceinline__ void stage_lengths(const uint32_t* len, uint32_t nb, unsigned char* dl) {
+    for (uint32_t i0 = threadIdx.x; i0 < nb; i0 += 4 * kCoderThreads) {
+        uint32_t l[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) l[k] = i0 + k * kCoderThreads < nb ? len[i0 + k * kCoderThreads] : 0u;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (i0 + k * kCoderThreads < nb) dl[i0 + k * kCoderThreads] = (unsigned char)l[k];
+    }
+}
+
+// Codeword bits of every segment of the split items.
+template <class S>
+__global__ __launch_bounds__(kCoderThreads) void k_seg_bits(const CodeItem* items, const SeqInfo* seqs, CoderParams p,
+                                                            const uint32_t* scratch, const CoderState* st,
+                                                            uint64_t out_cap, CodeUnits U) {
+    __shared__ unsigned char lsh[kStatBins];
+    __shared__ unsigned char lz[256];
+    __shared__ int shl[2][4];
+    __shared__ uint64_t shq[4];
+    if (st->out_base + st->out_words > out_cap) return;
+    const CodeUnit u = U.units[U.split_list[blockIdx.x]];
+    const CodeItem it = items[u.item];
+    const bool rl = it.rl != 0;
+    const SeqInfo& ss = seqs[it.seq];
+    const SeqInfo& sz = seqs[it.seq + (rl ? 1 : 0)];
+    if (ss.err || sz.err || ss.count == 0) return;
+    const S* in = static_cast<const S*>(it.in);
+    const uint32_t n = it.n;
+    const bool sglob = ss.smax >= kStatBins;
+    const uint32_t* glen = scratch + ss.code_off + ss.smax + 1;
+    if (!sglob) stage_lengths(glen, ss.smax + 1, lsh);
+    if (rl) stage_lengths(scratch + sz.code_off + sz.smax + 1, sz.smax + 1, lz);
+    const bool single = ss.nlen == 0, zsingle = !rl || sz.nlen == 0;
+    const uint64_t base0 = (uint64_t)u.chunk0 * kChunk;
+    const uint64_t end = min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk);
+    long long carry = (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.seg) - 1;
+    const long long limit = rl ? (long long)ss.last_nz1 - 1 : (long long)n;
+    const uint32_t t8 = threadIdx.x * kPerThread;
+    uint64_t bs = 0, bz = 0;
+    uint32_t vn[kPerThread], par = 0;
+    load8(in, base0 + t8, n, vn);
+    __syncthreads();
+    for (uint64_t base = base0; base < end; base += kChunk, par ^= 1) {
+        uint32_t v[kPerThread];
+#pragma unroll
+        for (int j = 0; j < (int)kPerThread; j++) v[j] = vn[j];
+        if (base + kChunk < end) load8(in, base + kChunk + t8, n, vn);
+        const uint32_t nvalid = chunk_nvalid(base, n, t8);
+        int wl;
+        const int ex = wave_excl_last(thread_last_nz_rel(v, t8, nvalid), wl);
+        if ((threadIdx.x & 63) == 0) shl[par][threadIdx.x >> 6] = wl;
+        __syncthreads();
+        int prel, ctot;
+        wg_last_combine(ex, shl[par], prel, ctot);
+        uint32_t zc[kPerThread];
+        const uint32_t emit = thread_flags_rel(v, nvalid, rl, thread_g0(prel, t8, chunk_gc(base, carry)),
+                                               chunk_lim(base, limit) - (int)t8, zc);
+#pragma unroll
+        for (int j = 0; j < (int)kPerThread; j++) {
+            const bool e = (emit >> j) & 1u;
+            if (e && !single) bs += sglob ? glen[v[j]] : (uint32_t)lsh[v[j]];
+            if (e && !zsingle) bz += lz[zc[j]];
+        }
+        if (ctot >= 0) carry = (long long)base + ctot;
+    }
+    bs = block_sum_u64<kCoderThreads>(bs, shq);
+    bz = block_sum_u64<kCoderThreads>(bz, shq);
+    if (threadIdx.x == 0) {
+        U.segs[u.slot0 + u.seg].bits_s = bs;
+        U.segs[u.slot0 + u.seg].bits_z = bz;
+    }
+}
+
+// packInc16 increments of blocks [2 w0, 2 w1) of a coded sequence, from the absolute offsets
+__device__ __forceinline__ void write_increments(const uint32_t* bo, uint32_t nblk, uint32_t w0, uint32_t w1,
+                                                 uint32_t* o) {
+    for (uint32_t w = w0 + threadIdx.x; w < w1; w += kCoderThreads) {
+        const uint32_t b0 = 2 * w, b1 = 2 * w + 1;
+        const uint32_t i0 = b0 == 0 ? bo[0] : bo[b0] - bo[b0 - 1];
+        const uint32_t i1 = b1 < nblk ? bo[b1] - bo[b1 - 1] : 0u;
+        o[w] = (i0 & 0xFFFFu) | (i1 << 16);
+    }
+}
+// The output word in which segment `seg` of a split sequence ends, put together from its parts by the
+// segment that holds the word's first bit: that one's last part, the whole of the segments that lie
+// inside the word, and the first part of the one that goes on past it.  begin: bits before `seg`.
+template <class Bits, class First, class Last>
+__device__ void border_word(const SegState* segs, uint32_t seg, uint32_t nseg, uint64_t begin, uint32_t* w, Bits bits,
+                            First first, Last last) {
+    const uint64_t end = begin + bits(segs[seg]);
+    const uint64_t wi = end >> 5;
+    if ((end & 31) == 0 || begin > wi * 32) return;  // no part of a word left over, or not its first bit
+    if (end == begin) return;
+    uint32_t v = last(segs[seg]);
+    uint64_t at = end;
+    for (uint32_t g = seg + 1; g < nseg && (at >> 5) == wi && (at & 31); g++) {
+        const SegState& s = segs[g];
+        const uint64_t e = at + bits(s);
+        if (e != at) v |= (e >> 5) == wi ? last(s) : first(s);
+        at = e;
+    }
+    w[wi] = v;
+}
+
+// After the packs of the split items: the words that segments share, and the packInc16 increments, a
+// share of the blocks per segment.
+__global__ __launch_bounds__(kCoderThreads) void k_seg_increments(const CodeItem* items, const SeqInfo* seqs,
+                                                                  CoderParams p, const uint32_t* scratch,
+                                                                  const CoderState* st, uint32_t* out,
+                                                                  uint64_t out_cap, CodeUnits U) {
+    if (st->out_base + st->out_words > out_cap) return;
+    const CodeUnit u = U.units[U.split_list[blockIdx.x]];
+    const CodeItem it = items[u.item];
+    if (seqs[it.seq].err || (it.rl && seqs[it.seq + 1].err)) return;
+    const SegState* segs = U.segs + u.slot0;
+    const SegState before = seg_before(segs, 0, u.seg);
+    if (threadIdx.x == 0 && seqs[it.seq].count) {
+        auto words = [&](const SeqInfo& s) { return out + s.out_off + (table_bits(s, p) + 31) / 32 + 1; };
+        border_word(segs, u.seg, u.nseg, before.bits_s, words(seqs[it.seq]), [](const SegState& s) { return s.bits_s; },
+                    [](const SegState& s) { return s.first_s; }, [](const SegState& s) { return s.last_s; });
+        if (it.rl)
+            border_word(segs, u.seg, u.nseg, before.bits_z, words(seqs[it.seq + 1]),
+                        [](const SegState& s) { return s.bits_z; }, [](const SegState& s) { return s.first_z; },
+                        [](const SegState& s) { return s.last_z; });
+    }
+    for (uint32_t q = 0; q < (it.rl ? 2u : 1u); q++) {
+        const SeqInfo& s = seqs[it.seq + q];
+        const uint32_t nblk = (s.count + p.cbs - 1) / p.cbs, nw = (nblk + 1) / 2;
+        uint32_t* o = out + s.out_off + (table_bits(s, p) + 31) / 32 + 1 + (s.bits + 31) / 32;
+        write_increments(scratch + s.boff_off, nblk, (uint32_t)((uint64_t)nw * u.seg / u.nseg),
+                         (uint32_t)((uint64_t)nw * (u.seg + 1) / u.nseg), o);
+    }
+}
+
 // Pass B: pairs recomputed, codewords packed into an LDS window and flushed as whole words
 // straight to their place in the output section (laid out by k_layout_* from the designed bit
 // counts): each workgroup also writes its item's zero-run count, table headers and bit counts, and
@@ -940,7 +1216,7 @@ __device__ uint32_t header_word(const SeqInfo& s, const uint32_t* cpl, const Cod
 template <class S>
 __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* items, SeqInfo* seqs, CoderParams p,
                                                              uint32_t* scratch, const CoderState* st, uint32_t* out,
-                                                             uint64_t out_cap, const uint32_t* order) {
+                                                             uint64_t out_cap, CodeUnits U) {
     __shared__ uint32_t cs[kStatBins];
     __shared__ unsigned char lsh[kStatBins];
     __shared__ uint32_t cz[256];
@@ -949,7 +1225,9 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
     __shared__ int shl[4];
     __shared__ uint64_t shq[4];
     if (st->out_base + st->out_words > out_cap) return;  // the host reports the short output
-    const CodeItem it = items[order ? order[blockIdx.x] : blockIdx.x];
+    const CodeUnit u = U.units[blockIdx.x];
+    const bool split = u.split != kWholeItem;
+    const CodeItem it = items[u.item];
     const SeqInfo ss = seqs[it.seq];
     const bool rl = it.rl != 0;
     if (ss.err || (rl && seqs[it.seq + 1].err)) return;
@@ -957,7 +1235,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
     const uint32_t M = ss.count;
     // section heads: [M] (RLE items), then per sequence its table header and bit count
     const uint32_t tws = (uint32_t)((table_bits(ss, p) + 31) / 32), twz = (uint32_t)((table_bits(sz, p) + 31) / 32);
-    {
+    if (!split || u.seg == 0) {
         const uint32_t* syms_s = scratch + ss.syms_off;
         uint32_t* hs = out + ss.out_off;
         // the header from the global record: a local record whose address is taken lives in
@@ -1024,13 +1302,22 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
         // One barrier per chunk besides the one before the flush: the exclusive last nonzeros of
         // the next chunk (zero-run lengths) ride on this chunk's pair/bit-count scan, so the
         // symbols run two chunks ahead (v: this chunk, vn: the next, vnn: in flight).
+        const uint64_t base0 = (uint64_t)u.chunk0 * kChunk;
+        const uint64_t end = split ? min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk) : (uint64_t)n;
+        const SegState seg = split ? seg_before(U.segs, u.slot0, u.slot0 + u.seg) : SegState{};
+        const long long carry0 = split ? (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.seg) - 1 : -1;
+        SegState* own = split ? U.segs + u.slot0 + u.seg : nullptr;
+        // a segment's parts of its first word, unless it starts on a word boundary, and of its last go
+        // to its record (k_seg_increments)
+        const uint64_t shared_s = split && (seg.bits_s & 31) ? seg.bits_s >> 5 : ~0ull;
+        const uint64_t shared_z = split && (seg.bits_z & 31) ? seg.bits_z >> 5 : ~0ull;
         uint32_t v[kPerThread], vn[kPerThread];
-        load8(in, (uint64_t)t8, n, v);
-        load8(in, (uint64_t)t8 + kChunk, n, vn);
+        load8(in, base0 + t8, n, v);
+        load8(in, base0 + t8 + kChunk, n, vn);
         int prel, ctot;  // this chunk: the exclusive chunk-relative last nonzero, the chunk's last
         {
             int wl;
-            const int ex = wave_excl_last(thread_last_nz_rel(v, t8, chunk_nvalid(0, n, t8)), wl);
+            const int ex = wave_excl_last(thread_last_nz_rel(v, t8, chunk_nvalid(base0, n, t8)), wl);
             if (lane == 0) shl[wv] = wl;
             __syncthreads();
             wg_last_combine(ex, shl, prel, ctot);
@@ -1040,11 +1327,11 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
         // symbols >= kStatBins)
         auto chunks = [&](auto sg) {
             constexpr bool SG = decltype(sg)::value;
-            long long carry = -1;  // last nonzero before this chunk
-            uint64_t pairs = 0, cbits_s = 0, cbits_z = 0;
-            for (uint64_t base = 0; base < n && pairs < M; base += kChunk) {
+            long long carry = carry0;  // last nonzero before this chunk
+            uint64_t pairs = seg.pairs, cbits_s = seg.bits_s, cbits_z = seg.bits_z;
+            for (uint64_t base = base0; base < end && pairs < M; base += kChunk) {
                 uint32_t vnn[kPerThread];
-                if (base + 2 * kChunk < n) load8(in, base + 2 * kChunk + t8, n, vnn);
+                if (base + 2 * kChunk < end) load8(in, base + 2 * kChunk + t8, n, vnn);
                 const uint32_t nvalid = chunk_nvalid(base, n, t8);
                 // this thread's pairs; code lengths looked up once for both the scan and the packing
                 uint32_t zc[kPerThread], ls[kPerThread], lzs[kPerThread];
@@ -1069,7 +1356,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
                 }
                 const uint32_t np = __popc(emit);
                 // pair/bit-count scan, and the next chunk's last nonzeros, over one barrier
-                const bool more = base + kChunk < n;
+                const bool more = base + kChunk < end;
                 int wl;
                 const int exn =
                     wave_excl_last(more ? thread_last_nz_rel(vn, t8, chunk_nvalid(base + kChunk, n, t8)) : -1, wl);
@@ -1166,13 +1453,15 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
                 const uint32_t full_s = (uint32_t)((nend_s >> 5) - wbs), full_z = (uint32_t)((nend_z >> 5) - wbz);
                 for (uint32_t i = threadIdx.x; i < full_s; i += kCoderThreads) {
                     const uint32_t r = (uint32_t)(wbs + i) & WM;
-                    if (wbs + i < nws) ws[wbs + i] = win[0][r];
+                    if (wbs + i == shared_s) own->first_s = win[0][r];
+                    else if (wbs + i < nws) ws[wbs + i] = win[0][r];
                     win[0][r] = 0;
                 }
                 if (rl)
                     for (uint32_t i = threadIdx.x; i < full_z; i += kCoderThreads) {
                         const uint32_t r = (uint32_t)(wbz + i) & WM;
-                        if (wbz + i < nwz) wz[wbz + i] = win[1][r];
+                        if (wbz + i == shared_z) own->first_z = win[1][r];
+                        else if (wbz + i < nwz) wz[wbz + i] = win[1][r];
                         win[1][r] = 0;
                     }
                 cbits_s = nend_s;
@@ -1186,7 +1475,10 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
                     vn[j] = vnn[j];
                 }
             }
-            if (threadIdx.x == 0) {  // the partial last words (their ORs precede the last barrier)
+            if (threadIdx.x == 0 && split) {
+                own->last_s = win[0][(uint32_t)(cbits_s >> 5) & WM];
+                own->last_z = win[1][(uint32_t)(cbits_z >> 5) & WM];
+            } else if (threadIdx.x == 0) {  // the partial last words (their ORs precede the last barrier)
                 if ((cbits_s & 31) && (cbits_s >> 5) < nws) ws[cbits_s >> 5] = win[0][(uint32_t)(cbits_s >> 5) & WM];
                 if (rl && (cbits_z & 31) && (cbits_z >> 5) < nwz)
                     wz[cbits_z >> 5] = win[1][(uint32_t)(cbits_z >> 5) & WM];
@@ -1195,20 +1487,15 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
         if (sglob) chunks(std::true_type{});
         else chunks(std::false_type{});
     }
+    if (split) return;  // k_seg_increments
     // coding-block offsets as packInc16 increments, from the absolute offsets the pairs recorded
     __threadfence_block();
     __syncthreads();
     for (int q = 0; q < (rl ? 2 : 1); q++) {
         const SeqInfo& s = q ? sz : ss;
-        const uint32_t* bo = q ? bz : bs;
         uint32_t* o = out + s.out_off + (q ? twz : tws) + 1 + (q ? nwz : nws);
         const uint32_t nblk = (s.count + cbs - 1) / cbs;
-        for (uint32_t w = threadIdx.x; w < (nblk + 1) / 2; w += kCoderThreads) {
-            const uint32_t b0 = 2 * w, b1 = 2 * w + 1;
-            const uint32_t i0 = b0 == 0 ? bo[0] : bo[b0] - bo[b0 - 1];
-            const uint32_t i1 = b1 < nblk ? bo[b1] - bo[b1 - 1] : 0u;
-            o[w] = (i0 & 0xFFFFu) | (i1 << 16);
-        }
+        write_increments(q ? bz : bs, nblk, 0, (nblk + 1) / 2, o);
     }
 }
 
@@ -1330,27 +1617,33 @@ void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uin
                   CallOut* d_calls,
                   uint32_t ncalls, const uint32_t* d_call_first_item, uint32_t* d_out, uint64_t out_cap,
                   uint64_t total_symbols, hipStream_t st, const SideStreams* side, const LayoutLink* link,
-                  const uint32_t* design_grid, uint32_t lane_k, const uint32_t* d_item_order) {
+                  const uint32_t* design_grid, uint32_t lane_k, const CodeUnits& U) {
     CCA_REQUIRE(symSize == 2 || symSize == 4, CC_ERR_INVALID_ARG, "symbol size must be 2 or 4");
     uint64_t* item_off = reinterpret_cast<uint64_t*>(scratch + scratch_cap);  // caller reserves the tail
     CCA_LAUNCH("coder_init", 32, k_coder_init, dim3(1), dim3(64), 0, st, d_state, d_classes);
     CCA_LAUNCH_CHECK();
     if (nitems == 0) return;
     const uint64_t inb = total_symbols * symSize;
-    if (symSize == 2) {
-        CCA_LAUNCH("code_stats", inb, k_code_stats<uint16_t>, dim3(nitems), dim3(kCoderThreads), 0, st, d_items, d_seqs,
-                   p, scratch, scratch_cap, d_state, d_item_order);
+    auto stats = [&](auto sym) {
+        using S = decltype(sym);
+        if (U.nsplit_units) {
+            CCA_LAUNCH("code_seg_last", 0, k_seg_last<S>, dim3(U.nsplit_units), dim3(64), 0, st, d_items, U);
+            CCA_LAUNCH_CHECK();
+        }
+        CCA_LAUNCH("code_stats", inb, k_code_stats<S>, dim3(U.nunits), dim3(kCoderThreads), 0, st, d_items, d_seqs, p,
+                   scratch, scratch_cap, d_state, U);
         CCA_LAUNCH_CHECK();
-        CCA_LAUNCH("code_stats_wide", 0, k_code_stats_wide<uint16_t>, dim3(nitems), dim3(kCoderThreads), 0, st,
-                   d_items, d_seqs, p, scratch);
-    } else {
-        CCA_LAUNCH("code_stats", inb, k_code_stats<uint32_t>, dim3(nitems), dim3(kCoderThreads), 0, st, d_items, d_seqs,
-                   p, scratch, scratch_cap, d_state, d_item_order);
+        if (U.nsplit_units) {
+            CCA_LAUNCH("code_stats_finish", 0, k_code_stats_finish, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st,
+                       d_items, d_seqs, p, scratch, scratch_cap, d_state, U);
+            CCA_LAUNCH_CHECK();
+        }
+        CCA_LAUNCH("code_stats_wide", 0, k_code_stats_wide<S>, dim3(U.nunits), dim3(kCoderThreads), 0, st, d_items,
+                   d_seqs, p, scratch, U);
         CCA_LAUNCH_CHECK();
-        CCA_LAUNCH("code_stats_wide", 0, k_code_stats_wide<uint32_t>, dim3(nitems), dim3(kCoderThreads), 0, st,
-                   d_items, d_seqs, p, scratch);
-    }
-    CCA_LAUNCH_CHECK();
+    };
+    if (symSize == 2) stats(uint16_t{});
+    else stats(uint32_t{});
     // Design classes by distinct-symbol count (small LDS footprints keep many tables resident):
     // the sequences are sorted into per-class lists, and each class runs over its list only, the
     // classes concurrently on side streams, the largest tables' classes launched first.
@@ -1414,13 +1707,24 @@ void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uin
                    d_seqs, d_calls, ncalls, d_call_first_item, item_off, out_cap);
     CCA_LAUNCH_CHECK();
     if (link && link->signal) CCA_HIP(hipEventRecord(link->signal, st));
-    if (symSize == 2)
-        CCA_LAUNCH("code_pack", inb, k_code_pack<uint16_t>, dim3(nitems), dim3(kCoderThreads), 0, st, d_items, d_seqs,
-                   p, scratch, d_state, d_out, out_cap, d_item_order);
-    else
-        CCA_LAUNCH("code_pack", inb, k_code_pack<uint32_t>, dim3(nitems), dim3(kCoderThreads), 0, st, d_items, d_seqs,
-                   p, scratch, d_state, d_out, out_cap, d_item_order);
-    CCA_LAUNCH_CHECK();
+    auto pack = [&](auto sym) {
+        using S = decltype(sym);
+        if (U.nsplit_units) {
+            CCA_LAUNCH("code_seg_bits", 0, k_seg_bits<S>, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st, d_items,
+                       d_seqs, p, scratch, d_state, out_cap, U);
+            CCA_LAUNCH_CHECK();
+        }
+        CCA_LAUNCH("code_pack", inb, k_code_pack<S>, dim3(U.nunits), dim3(kCoderThreads), 0, st, d_items, d_seqs, p,
+                   scratch, d_state, d_out, out_cap, U);
+        CCA_LAUNCH_CHECK();
+        if (U.nsplit_units) {
+            CCA_LAUNCH("code_seg_increments", 0, k_seg_increments, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st,
+                       d_items, d_seqs, p, scratch, d_state, d_out, out_cap, U);
+            CCA_LAUNCH_CHECK();
+        }
+    };
+    if (symSize == 2) pack(uint16_t{});
+    else pack(uint32_t{});
 }
 
 }  // namespace cca

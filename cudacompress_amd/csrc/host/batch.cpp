@@ -23,6 +23,20 @@ uint64_t arena_estimate(const std::vector<ItemSpec>& items, uint32_t log2, uint3
     return words;
 }
 
+// Units of the streaming passes.  One workgroup takes about 3 us a chunk, and the chip runs some
+// thousand of these workgroups at once, so a job of T chunks is split to kUnitsTarget units when its
+// longest item alone would outlast the rest (kMinUnitChunks chunks or more each: a unit costs a few
+// microseconds of tables and histogram besides its chunks).  A batch of thousands of items has
+// T / kUnitsTarget above its longest item and is not split (2048 mixed bricks: 300,000 chunks, items
+// of at most 128).
+constexpr uint64_t kUnitsTarget = 1024;
+constexpr uint32_t kMinUnitChunks = 2;
+uint32_t unit_chunks(const std::vector<ItemSpec>& items) {
+    uint64_t total = 0;
+    for (const ItemSpec& it : items) total += div_up(it.n, kChunk);
+    return (uint32_t)std::max<uint64_t>(kMinUnitChunks, (total + kUnitsTarget - 1) / kUnitsTarget);
+}
+
 // Side streams of a coder context (created on first use, on the current device).
 const SideStreams* side_streams(DeviceCoder& D, SideStreams& out) {
     if (!D.fork) {
@@ -59,11 +73,22 @@ void encode_prepare(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>&
                     EncodeJob& job, hipStream_t st) {
     check_symbols(I, symSize);
     const uint32_t nitems = (uint32_t)items.size();
-    const size_t o_first = align_up(sizeof(CodeItem) * std::max<uint32_t>(nitems, 1), 256);
-    const size_t stage_bytes = o_first + sizeof(uint32_t) * (ncalls + 1 + nitems);
+    const uint32_t per_unit = unit_chunks(items);
+    auto segments = [&](const ItemSpec& it) { return std::max(1u, div_up(div_up(it.n, kChunk), per_unit)); };
+    uint32_t nunits = 0, nsplit = 0, nslots = 0;
+    for (const ItemSpec& it : items) {
+        const uint32_t k = segments(it);
+        nunits += k;
+        nsplit += k > 1 ? 1 : 0;
+        nslots += k > 1 ? k : 0;
+    }
+    job.o_first = align_up(sizeof(CodeItem) * nitems, 256);
+    job.o_units = align_up(job.o_first + sizeof(uint32_t) * (ncalls + 1), 256);
+    job.o_split = job.o_units + sizeof(CodeUnit) * nunits;
+    const size_t stage_bytes = job.o_split + sizeof(uint32_t) * nslots;
     unsigned char* h = (unsigned char*)D.h_stage.get(stage_bytes);
     CodeItem* hi = (CodeItem*)h;
-    uint32_t* hf = (uint32_t*)(h + o_first);
+    uint32_t* hf = (uint32_t*)(h + job.o_first);
     uint32_t seq = 0, call = 0;
     uint64_t total_syms = 0;
     hf[0] = 0;
@@ -77,10 +102,31 @@ void encode_prepare(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>&
         total_syms += it.n;
     }
     while (call < ncalls) hf[++call] = nitems;
-    // the stats and pack passes take the items largest first (their serial chunk loops start first)
-    uint32_t* ho = hf + ncalls + 1;
-    for (uint32_t i = 0; i < nitems; i++) ho[i] = i;
-    std::stable_sort(ho, ho + nitems, [&](uint32_t a, uint32_t b) { return items[a].n > items[b].n; });
+    CodeUnit* hu = (CodeUnit*)(h + job.o_units);
+    uint32_t* hs = (uint32_t*)(h + job.o_split);
+    uint32_t nu = 0, slot = 0, split = 0;
+    for (uint32_t i = 0; i < nitems; i++) {
+        const uint32_t nc = div_up(items[i].n, kChunk), k = segments(items[i]);
+        if (k == 1) {
+            hu[nu++] = CodeUnit{i, 0, nc, kWholeItem, 0, 1, 0, 0};
+            continue;
+        }
+        for (uint32_t g = 0; g < k; g++) {
+            const uint32_t c0 = (uint32_t)((uint64_t)nc * g / k), c1 = (uint32_t)((uint64_t)nc * (g + 1) / k);
+            hu[nu++] = CodeUnit{i, c0, c1 - c0, split, g, k, slot, 0};
+        }
+        slot += k;
+        split++;
+    }
+    // the streaming passes take the units longest first (their serial chunk loops start first)
+    std::stable_sort(hu, hu + nunits, [&](const CodeUnit& a, const CodeUnit& b) {
+        return a.nchunk != b.nchunk ? a.nchunk > b.nchunk : items[a.item].n > items[b.item].n;
+    });
+    for (uint32_t k = 0, q = 0; k < nunits; k++)
+        if (hu[k].split != kWholeItem) hs[q++] = k;
+    job.nunits = nunits;
+    job.nsplit_units = nslots;
+    job.nsplit = nsplit;
     job.nitems = nitems;
     job.nseq = seq;
     job.ncalls = ncalls;
@@ -89,15 +135,14 @@ void encode_prepare(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>&
     job.p = params_of(I);
     for (int c = 0; c < 4; c++) job.design_grid[c] = I->tuning.designGrid[c];
     job.lane_k = I->tuning.laneDesignK;
-    D.d_items.as<CodeItem>(std::max<uint32_t>(nitems, 1));
-    D.d_call_first.as<uint32_t>(ncalls + 1 + std::max<uint32_t>(nitems, 1));
+    D.d_items.get(stage_bytes);
+    D.d_split.get(sizeof(SegState) * nslots + 4ull * kSplitWords * nsplit);
     D.d_seqs.as<SeqInfo>(std::max<uint32_t>(job.nseq, 1));
     D.d_state.as<CoderState>(1);
     D.d_classes.as<uint32_t>(kDesignListBase + (uint64_t)kDesignLists * std::max<uint32_t>(job.nseq, 1));
     D.d_calls.as<CallOut>(std::max<uint32_t>(ncalls, 1));
     D.h_result.get(sizeof(CoderState) + sizeof(CallOut) * std::max<uint32_t>(ncalls, 1));
-    CCA_HIP(hipMemcpyAsync(D.d_items.p, hi, sizeof(CodeItem) * nitems, hipMemcpyHostToDevice, st));
-    CCA_HIP(hipMemcpyAsync(D.d_call_first.p, hf, sizeof(uint32_t) * (ncalls + 1 + nitems), hipMemcpyHostToDevice, st));
+    CCA_HIP(hipMemcpyAsync(D.d_items.p, h, stage_bytes, hipMemcpyHostToDevice, st));
     encode_reserve(D, job, std::max<uint64_t>(D.scratch_cap, arena_estimate(items, I->log2, I->cbs)));
     SideStreams ss;
     side_streams(D, ss);
@@ -114,12 +159,15 @@ void encode_reserve(DeviceCoder& D, EncodeJob& job, uint64_t words) {
 void encode_launch(DeviceCoder& D, const EncodeJob& job, uint32_t* d_out, uint64_t out_cap, hipStream_t st,
                    const LayoutLink* link) {
     SideStreams ss;
-    coder_encode((const CodeItem*)D.d_items.p, job.nitems, (SeqInfo*)D.d_seqs.p, job.nseq, job.p, job.symSize,
+    const unsigned char* d = (const unsigned char*)D.d_items.p;
+    const CodeUnits units{(const CodeUnit*)(d + job.o_units), job.nunits, (const uint32_t*)(d + job.o_split),
+                          job.nsplit_units, job.nsplit, (SegState*)D.d_split.p,
+                          (uint32_t*)((unsigned char*)D.d_split.p + sizeof(SegState) * job.nsplit_units)};
+    coder_encode((const CodeItem*)d, job.nitems, (SeqInfo*)D.d_seqs.p, job.nseq, job.p, job.symSize,
                  (uint32_t*)D.d_scratch.p, job.scratch_cap, (CoderState*)D.d_state.p, (uint32_t*)D.d_classes.p,
                  (CallOut*)D.d_calls.p,
-                 job.ncalls, (const uint32_t*)D.d_call_first.p, d_out, out_cap, job.total_syms, st,
-                 side_streams(D, ss), link, job.design_grid, job.lane_k,
-                 (const uint32_t*)D.d_call_first.p + job.ncalls + 1);
+                 job.ncalls, (const uint32_t*)(d + job.o_first), d_out, out_cap, job.total_syms, st,
+                 side_streams(D, ss), link, job.design_grid, job.lane_k, units);
 }
 
 CoderState encode_finish(DeviceCoder& D, const EncodeJob& job, std::vector<CallOut>* results, hipStream_t st) {
