@@ -405,7 +405,7 @@ __device__ void write_leaves(const uint32_t* h, uint32_t nb, uint2* out, uint64_
 // The sequence records of an item from its histograms (pairs M, largest symbol vmax, wide: symbols
 // past the LDS histogram, carry: the last nonzero): maxima, distinct counts, the histograms' copies in
 // the arena with the leaf lists of small tables.  Every thread of the workgroup calls.
-__device__ void stats_finish(const CodeItem& it, uint32_t ii, uint32_t M, uint32_t vmax, uint32_t wide, long long carry,
+__device__ __forceinline__ void stats_finish(const CodeItem& it, uint32_t ii, uint32_t M, uint32_t vmax, uint32_t wide, long long carry,
                              const uint32_t* hs, const uint32_t* hz, SeqInfo* seqs, const CoderParams& p,
                              uint32_t* scratch, uint64_t cap, CoderState* st, uint32_t* shu, uint64_t* sh_off,
                              uint64_t* shq) {
@@ -481,7 +481,7 @@ __device__ void stats_finish(const CodeItem& it, uint32_t ii, uint32_t M, uint32
 // Pass A: pair counts, histograms (LDS), maxima; tables of the LDS class get their histogram
 // copied to the arena (with the leaf list of small tables); streams with symbols >= kStatBins are
 // marked wide and get a zeroed global histogram for k_code_stats_wide.
-template <class S>
+template <class S, bool Split>  // Split: the job has split items (the checks cost the pack 4 %)
 __global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* items, SeqInfo* seqs, CoderParams p,
                                                               uint32_t* scratch, uint64_t cap, CoderState* st,
                                                               CodeUnits U) {
@@ -493,12 +493,12 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* it
     __shared__ uint64_t shq[4];
     const CodeUnit u = U.units[blockIdx.x];
     const uint32_t ii = u.item;
-    const bool split = u.split != kWholeItem;
+    const bool split = Split && u.split != kWholeItem;
     const CodeItem it = items[ii];
     const S* in = static_cast<const S*>(it.in);
     const bool rl = it.rl != 0;
     const uint32_t n = it.n;
-    const uint64_t base0 = (uint64_t)u.chunk0 * kChunk;
+    const uint64_t base0 = split ? (uint64_t)u.chunk0 * kChunk : 0;
     const uint64_t end = split ? min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk) : (uint64_t)n;
     for (uint32_t i = threadIdx.x; i < kStatBins; i += kCoderThreads) hs[i] = 0;
     for (uint32_t i = threadIdx.x; i < 256; i += kCoderThreads) hz[i] = 0;
@@ -1213,7 +1213,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_seg_increments(const CodeItem
 // counts): each workgroup also writes its item's zero-run count, table headers and bit counts, and
 // after the pairs its packInc16 coding-block offsets (src/cudaCompress/PackInc.cu:210-220).  The
 // absolute bit offset of every coding block is kept in the arena for the increments.
-template <class S>
+template <class S, bool Split>
 __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* items, SeqInfo* seqs, CoderParams p,
                                                              uint32_t* scratch, const CoderState* st, uint32_t* out,
                                                              uint64_t out_cap, CodeUnits U) {
@@ -1226,7 +1226,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
     __shared__ uint64_t shq[4];
     if (st->out_base + st->out_words > out_cap) return;  // the host reports the short output
     const CodeUnit u = U.units[blockIdx.x];
-    const bool split = u.split != kWholeItem;
+    const bool split = Split && u.split != kWholeItem;
     const CodeItem it = items[u.item];
     const SeqInfo ss = seqs[it.seq];
     const bool rl = it.rl != 0;
@@ -1302,7 +1302,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
         // One barrier per chunk besides the one before the flush: the exclusive last nonzeros of
         // the next chunk (zero-run lengths) ride on this chunk's pair/bit-count scan, so the
         // symbols run two chunks ahead (v: this chunk, vn: the next, vnn: in flight).
-        const uint64_t base0 = (uint64_t)u.chunk0 * kChunk;
+        const uint64_t base0 = split ? (uint64_t)u.chunk0 * kChunk : 0;
         const uint64_t end = split ? min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk) : (uint64_t)n;
         const SegState seg = split ? seg_before(U.segs, u.slot0, u.slot0 + u.seg) : SegState{};
         const long long carry0 = split ? (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.seg) - 1 : -1;
@@ -1630,8 +1630,8 @@ void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uin
             CCA_LAUNCH("code_seg_last", 0, k_seg_last<S>, dim3(U.nsplit_units), dim3(64), 0, st, d_items, U);
             CCA_LAUNCH_CHECK();
         }
-        CCA_LAUNCH("code_stats", inb, k_code_stats<S>, dim3(U.nunits), dim3(kCoderThreads), 0, st, d_items, d_seqs, p,
-                   scratch, scratch_cap, d_state, U);
+        CCA_LAUNCH("code_stats", inb, (U.nsplit ? k_code_stats<S, true> : k_code_stats<S, false>), dim3(U.nunits),
+                   dim3(kCoderThreads), 0, st, d_items, d_seqs, p, scratch, scratch_cap, d_state, U);
         CCA_LAUNCH_CHECK();
         if (U.nsplit_units) {
             CCA_LAUNCH("code_stats_finish", 0, k_code_stats_finish, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st,
@@ -1714,8 +1714,8 @@ void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uin
                        d_seqs, p, scratch, d_state, out_cap, U);
             CCA_LAUNCH_CHECK();
         }
-        CCA_LAUNCH("code_pack", inb, k_code_pack<S>, dim3(U.nunits), dim3(kCoderThreads), 0, st, d_items, d_seqs, p,
-                   scratch, d_state, d_out, out_cap, U);
+        CCA_LAUNCH("code_pack", inb, (U.nsplit ? k_code_pack<S, true> : k_code_pack<S, false>), dim3(U.nunits),
+                   dim3(kCoderThreads), 0, st, d_items, d_seqs, p, scratch, d_state, d_out, out_cap, U);
         CCA_LAUNCH_CHECK();
         if (U.nsplit_units) {
             CCA_LAUNCH("code_seg_increments", 0, k_seg_increments, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st,
