@@ -353,10 +353,11 @@ CCA_HD void design_table(Ex& ex, const uint32_t* hist, uint32_t nbins, int diale
         if (dialect == kDialectGpu) {
             ex.heap_make(w.heap, K);
         } else {
-            for (int i = 1; i < K; i++) ex.heap_push(w.heap, i, w.heap[i], HeapEntry{0u, 0u});
+            for (int i = 1; i < K; i++) ex.heap_build_push(w.heap, i, w.heap[i]);
         }
         int size = K, next = K;
         ex.barrier();
+        ex.heap_begin(w.heap, K);  // what the executor keeps beside the heap while merging
         HeapEntry top = w.heap[0];  // the executor's pop and push return the new top
         while (size > 1) {
             const HeapEntry a = top;
@@ -684,6 +685,8 @@ struct SerialEx {
     CCA_HD int lanes() const { return 1; }
     CCA_HD void barrier() const {}
     CCA_HD void heap_make(HeapEntry* h, int len) const { make_heap(h, len, QueueLess()); }
+    CCA_HD void heap_build_push(HeapEntry* h, int pos, HeapEntry v) const { push_heap_at(h, pos, 0, v, QueueLess()); }
+    CCA_HD void heap_begin(const HeapEntry*, int) const {}
     // pop / push return the new top (h[0])
     CCA_HD HeapEntry heap_pop(HeapEntry* h, int len) const {
         pop_heap(h, len, QueueLess());
@@ -728,6 +731,7 @@ struct SerialEx {
 struct PathEx : SerialEx {
     mutable int path[96];
     CCA_HD void heap_make(HeapEntry* h, int len) const { make_by_levels(h, len); }
+    CCA_HD void heap_build_push(HeapEntry* h, int pos, HeapEntry v) const { push_by_chain(h, pos, v); }
     CCA_HD HeapEntry heap_pop(HeapEntry* h, int len) const {
         pop_by_path(h, len, path);
         return h[0];
