@@ -210,6 +210,15 @@ void coder_concat(const ConcatGroup* d_groups, uint32_t ngroups, uint32_t* dst, 
                   hipStream_t st);
 // d_classes: kDesignListBase + kDesignLists * nseq words of work lists.  units: what the workgroups
 // of the stats and pack passes serve (each a serial loop over its chunks), the longest first.
+// The streaming passes alone, for tables designed elsewhere: stats leaves every sequence's record and
+// histogram (d_state: the arena in use); pack wants records with their table, offsets and section
+// filled in, and d_state with out_base and out_words.
+void coder_stats(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, const CoderParams& p, int symSize,
+                 uint32_t* scratch, uint64_t scratch_cap, CoderState* d_state, uint32_t* d_classes,
+                 uint64_t total_symbols, const CodeUnits& units, hipStream_t st);
+void coder_pack(const CodeItem* d_items, SeqInfo* d_seqs, const CoderParams& p, int symSize, uint32_t* scratch,
+                const CoderState* d_state, uint32_t* d_out, uint64_t out_cap, uint64_t total_symbols,
+                const CodeUnits& units, hipStream_t st);
 void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uint32_t nseq, const CoderParams& p,
                   int symSize, uint32_t* scratch, uint64_t scratch_cap, CoderState* d_state, uint32_t* d_classes,
                   CallOut* d_calls,
@@ -235,6 +244,14 @@ void coder_decode(const DecCall* d_calls, uint32_t ncalls, const DecItem* d_item
                   CoderState* d_state, DecCallOut* d_out, const uint32_t* d_wave_seq, const uint32_t* d_wave_first,
                   uint32_t nwaves, uint32_t nlong, uint64_t total_symbols, const RleChunks& rc,
                   hipStream_t st);
+// The same stages for sequences parsed on the host (records with the positions, counts, outputs and
+// arena ranges filled in): tables and block decode, then the zero-run expansion.
+void coder_decode_parsed(DecSeq* d_seqs, uint32_t nseq, const CoderParams& p, int symSize, uint32_t* scratch,
+                         CoderState* d_state, const DecItem* d_items, const uint32_t* d_wave_seq,
+                         const uint32_t* d_wave_first, uint32_t nwaves, uint32_t nlong, uint64_t total_symbols,
+                         const RleChunks& rc, hipStream_t st);
+void coder_decode_expand(const DecItem* d_items, uint32_t nitems, DecSeq* d_seqs, int symSize, const RleChunks& rc,
+                         CoderState* d_state, uint64_t total_symbols, hipStream_t st);
 // Resident decode index: parse + tables of every call once (RLE sequences get no decode buffer),
 // per-call results in d_out.  scratch then holds the tables and block offsets for bound decodes.
 void coder_decode_index(const DecCall* d_calls, uint32_t ncalls, const DecItem* d_items, DecSeq* d_seqs, uint32_t nseq,

@@ -1760,14 +1760,10 @@ void coder_concat(const ConcatGroup* d_groups, uint32_t ngroups, uint32_t* dst, 
     CCA_LAUNCH_CHECK();
 }
 
-void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uint32_t nseq, const CoderParams& p,
-                  int symSize, uint32_t* scratch, uint64_t scratch_cap, CoderState* d_state, uint32_t* d_classes,
-                  CallOut* d_calls,
-                  uint32_t ncalls, const uint32_t* d_call_first_item, uint32_t* d_out, uint64_t out_cap,
-                  uint64_t total_symbols, hipStream_t st, const SideStreams* side, const LayoutLink* link,
-                  const uint32_t* design_grid, uint32_t lane_k, const CodeUnits& U) {
+void coder_stats(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, const CoderParams& p, int symSize,
+                 uint32_t* scratch, uint64_t scratch_cap, CoderState* d_state, uint32_t* d_classes,
+                 uint64_t total_symbols, const CodeUnits& U, hipStream_t st) {
     CCA_REQUIRE(symSize == 2 || symSize == 4, CC_ERR_INVALID_ARG, "symbol size must be 2 or 4");
-    uint64_t* item_off = reinterpret_cast<uint64_t*>(scratch + scratch_cap);  // caller reserves the tail
     CCA_LAUNCH("coder_init", 32, k_coder_init, dim3(1), dim3(64), 0, st, d_state, d_classes);
     CCA_LAUNCH_CHECK();
     if (nitems == 0) return;
@@ -1792,6 +1788,41 @@ void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uin
     };
     if (symSize == 2) stats(uint16_t{});
     else stats(uint32_t{});
+}
+
+void coder_pack(const CodeItem* d_items, SeqInfo* d_seqs, const CoderParams& p, int symSize, uint32_t* scratch,
+                const CoderState* d_state, uint32_t* d_out, uint64_t out_cap, uint64_t total_symbols,
+                const CodeUnits& U, hipStream_t st) {
+    const uint64_t inb = total_symbols * symSize;
+    auto pack = [&](auto sym) {
+        using S = decltype(sym);
+        if (U.nsplit_units) {
+            CCA_LAUNCH("code_seg_bits", 0, k_seg_bits<S>, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st, d_items,
+                       d_seqs, p, scratch, d_state, out_cap, U);
+            CCA_LAUNCH_CHECK();
+        }
+        CCA_LAUNCH("code_pack", inb, (U.nsplit ? k_code_pack<S, true> : k_code_pack<S, false>), dim3(U.nunits),
+                   dim3(kCoderThreads), 0, st, d_items, d_seqs, p, scratch, d_state, d_out, out_cap, U);
+        CCA_LAUNCH_CHECK();
+        if (U.nsplit_units) {
+            CCA_LAUNCH("code_seg_increments", 0, k_seg_increments, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st,
+                       d_items, d_seqs, p, scratch, d_state, d_out, out_cap, U);
+            CCA_LAUNCH_CHECK();
+        }
+    };
+    if (symSize == 2) pack(uint16_t{});
+    else pack(uint32_t{});
+}
+
+void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uint32_t nseq, const CoderParams& p,
+                  int symSize, uint32_t* scratch, uint64_t scratch_cap, CoderState* d_state, uint32_t* d_classes,
+                  CallOut* d_calls,
+                  uint32_t ncalls, const uint32_t* d_call_first_item, uint32_t* d_out, uint64_t out_cap,
+                  uint64_t total_symbols, hipStream_t st, const SideStreams* side, const LayoutLink* link,
+                  const uint32_t* design_grid, uint32_t lane_k, const CodeUnits& U) {
+    uint64_t* item_off = reinterpret_cast<uint64_t*>(scratch + scratch_cap);  // caller reserves the tail
+    coder_stats(d_items, nitems, d_seqs, p, symSize, scratch, scratch_cap, d_state, d_classes, total_symbols, U, st);
+    if (nitems == 0) return;
     // Design classes by distinct-symbol count (small LDS footprints keep many tables resident):
     // the sequences are sorted into per-class lists, and each class runs over its list only, the
     // classes concurrently on side streams, the largest tables' classes launched first.
@@ -1855,24 +1886,7 @@ void coder_encode(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, uin
                    d_seqs, d_calls, ncalls, d_call_first_item, item_off, out_cap);
     CCA_LAUNCH_CHECK();
     if (link && link->signal) CCA_HIP(hipEventRecord(link->signal, st));
-    auto pack = [&](auto sym) {
-        using S = decltype(sym);
-        if (U.nsplit_units) {
-            CCA_LAUNCH("code_seg_bits", 0, k_seg_bits<S>, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st, d_items,
-                       d_seqs, p, scratch, d_state, out_cap, U);
-            CCA_LAUNCH_CHECK();
-        }
-        CCA_LAUNCH("code_pack", inb, (U.nsplit ? k_code_pack<S, true> : k_code_pack<S, false>), dim3(U.nunits),
-                   dim3(kCoderThreads), 0, st, d_items, d_seqs, p, scratch, d_state, d_out, out_cap, U);
-        CCA_LAUNCH_CHECK();
-        if (U.nsplit_units) {
-            CCA_LAUNCH("code_seg_increments", 0, k_seg_increments, dim3(U.nsplit_units), dim3(kCoderThreads), 0, st,
-                       d_items, d_seqs, p, scratch, d_state, d_out, out_cap, U);
-            CCA_LAUNCH_CHECK();
-        }
-    };
-    if (symSize == 2) pack(uint16_t{});
-    else pack(uint32_t{});
+    coder_pack(d_items, d_seqs, p, symSize, scratch, d_state, d_out, out_cap, total_symbols, U, st);
 }
 
 }  // namespace cca

@@ -644,7 +644,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
         const uint32_t bpc = kRleChunk / cbs;
         for (uint32_t o = 1; o < bpc; o <<= 1) zs += (uint32_t)__shfl_xor((int)zs, (int)o);
         const uint32_t c = b / bpc;
-        if ((lane & (bpc - 1)) == 0 && c < (zit.n + kRleChunk - 1) / kRleChunk) rc.sums[rc.item_first[s.item] + c] = zs;
+        if ((lane & (bpc - 1)) == 0 && c < (count + kRleChunk - 1) / kRleChunk) rc.sums[rc.item_first[s.item] + c] = zs;
     } else if (valid) {
         (void)rounds(std::false_type{});
     }
@@ -926,6 +926,26 @@ void launch_blocks_rle(const DecItem* d_items, uint32_t nitems, DecSeq* d_seqs, 
     launch_rle<S>(d_items, nitems, d_seqs, rc, d_state, outb, st);
 }
 }  // namespace
+
+void coder_decode_parsed(DecSeq* d_seqs, uint32_t nseq, const CoderParams& p, int symSize, uint32_t* scratch,
+                         CoderState* d_state, const DecItem* d_items, const uint32_t* d_wave_seq,
+                         const uint32_t* d_wave_first, uint32_t nwaves, uint32_t nlong, uint64_t total_symbols,
+                         const RleChunks& rc, hipStream_t st) {
+    if (nseq == 0) return;
+    CCA_LAUNCH("dec_tables", 0, k_dec_tables, dim3(nseq), dim3(256), 0, st, d_seqs, p, scratch, d_state);
+    CCA_LAUNCH_CHECK();
+    const uint64_t outb = total_symbols * symSize;
+    if (symSize == 2)
+        launch_blocks<uint16_t>(d_seqs, d_wave_seq, d_wave_first, nwaves, nlong, p, scratch, d_items, rc, outb, st);
+    else
+        launch_blocks<uint32_t>(d_seqs, d_wave_seq, d_wave_first, nwaves, nlong, p, scratch, d_items, rc, outb, st);
+}
+
+void coder_decode_expand(const DecItem* d_items, uint32_t nitems, DecSeq* d_seqs, int symSize, const RleChunks& rc,
+                         CoderState* d_state, uint64_t total_symbols, hipStream_t st) {
+    if (symSize == 2) launch_rle<uint16_t>(d_items, nitems, d_seqs, rc, d_state, total_symbols * symSize, st);
+    else launch_rle<uint32_t>(d_items, nitems, d_seqs, rc, d_state, total_symbols * symSize, st);
+}
 
 void coder_decode_index(const DecCall* d_calls, uint32_t ncalls, const DecItem* d_items, DecSeq* d_seqs, uint32_t nseq,
                         const CoderParams& p, int symSize, uint32_t* scratch, uint64_t scratch_cap, CoderState* d_state,

@@ -34,6 +34,60 @@ __global__ __launch_bounds__(256) void k_unsymbolize(int16_t* __restrict__ data,
     if (!i.ok) return;
     data[i.x + (size_t)i.y * row + (size_t)i.z * slice] = (int16_t)unsymbolize_u(sym[i.x + (size_t)i.y * sx + (size_t)i.z * sx * sy]);
 }
+// One level's octants at once (kernels.hpp): a thread takes V consecutive x of one half of a row, so a
+// wave reads and writes whole lines of one band.  Bound by memory; one launch instead of one per band,
+// of 2-3 us each, and a copy of the lowpass band.
+struct LevelBands {
+    uint16_t* hp;
+    uint64_t stride;
+    uint16_t* low_sym;
+    int16_t* low;
+    uint32_t hx, hy, hz;  // half sizes (hz 1, octants 4..7 absent in 2D)
+    uint32_t row;
+    uint64_t slice;
+};
+template <int V>
+struct alignas(2 * V) Shorts {
+    uint16_t v[V];
+};
+template <int V, bool Forward>
+__global__ __launch_bounds__(256) void k_level_bands(LevelBands L, int16_t* __restrict__ data) {
+    const uint32_t per_half = L.hx / V;
+    const uint32_t q = blockIdx.x * 64 + (threadIdx.x & 63);
+    const uint32_t y = blockIdx.y * 4 + (threadIdx.x >> 6), z = blockIdx.z;
+    if (q >= 2 * per_half || y >= 2 * L.hy) return;
+    const uint32_t bx = q >= per_half, by = y >= L.hy, bz = z >= L.hz;
+    const uint32_t b = bx + 2 * by + 4 * bz, x = (q - bx * per_half) * V;
+    if (b == 0 && !L.low_sym && !L.low) return;
+    const uint64_t in_band = x + (uint64_t)L.hx * ((y - by * L.hy) + (uint64_t)L.hy * (z - bz * L.hz));
+    int16_t* d = data + (x + bx * L.hx) + (uint64_t)y * L.row + z * L.slice;
+    const bool raw = b == 0 && !L.low_sym;
+    uint16_t* s = b ? L.hp + (b - 1) * L.stride + in_band
+                    : (raw ? reinterpret_cast<uint16_t*>(L.low) : L.low_sym) + in_band;
+    Shorts<V> v = *reinterpret_cast<const Shorts<V>*>(Forward ? reinterpret_cast<const uint16_t*>(d) : s);
+    if (!raw) {
+#pragma unroll
+        for (int i = 0; i < V; i++)
+            v.v[i] = Forward ? (uint16_t)symbolize_i((int16_t)v.v[i]) : (uint16_t)(int16_t)unsymbolize_u(v.v[i]);
+    }
+    *reinterpret_cast<Shorts<V>*>(Forward ? s : reinterpret_cast<uint16_t*>(d)) = v;
+}
+template <bool Forward>
+void launch_level_bands(const LevelBands& L, int16_t* data, bool is3d, hipStream_t st) {
+    const uint32_t ly = 2 * L.hy, lz = is3d ? 2 * L.hz : 1;
+    // four at a time where every row of the level and of the bands starts on 8 bytes
+    const bool four = L.hx % 4 == 0 && L.row % 4 == 0 && L.slice % 4 == 0 && L.stride % 4 == 0 &&
+                      ((reinterpret_cast<uintptr_t>(data) | reinterpret_cast<uintptr_t>(L.hp) |
+                        reinterpret_cast<uintptr_t>(L.low_sym) | reinterpret_cast<uintptr_t>(L.low)) & 7) == 0;
+    const uint64_t bytes = 4ull * 2 * L.hx * ly * lz;
+    const char* name = Forward ? "symbolize_level" : "unsymbolize_level";
+    const dim3 grid(div_up(2 * L.hx / (four ? 4 : 1), 64), div_up(ly, 4), lz);
+    if (four)
+        CCA_LAUNCH(name, bytes, (k_level_bands<4, Forward>), grid, dim3(256), 0, st, L, data);
+    else
+        CCA_LAUNCH(name, bytes, (k_level_bands<1, Forward>), grid, dim3(256), 0, st, L, data);
+    CCA_LAUNCH_CHECK();
+}
 template <typename S>
 __global__ __launch_bounds__(256) void k_quantize(S* __restrict__ sym, float* __restrict__ data, float step, float inv,
                                                   uint32_t sx, uint32_t sy, uint32_t sz, uint32_t row, uint32_t slice,
@@ -180,6 +234,19 @@ void max_abs(const float* data, uint32_t n, float* out, hipStream_t st) {
     uint32_t blocks = std::min<uint32_t>(div_up(n, 256 * 8), 2048u);
     CCA_LAUNCH("max_abs", (uint64_t)n * 4, k_max_abs, dim3(blocks), dim3(256), 0, st, data, n, (uint32_t*)out);
     CCA_LAUNCH_CHECK();
+}
+
+void symbolize_level(uint16_t* hp, uint64_t band_stride, uint16_t* low_sym, int16_t* low, const int16_t* data,
+                     uint32_t lx, uint32_t ly, uint32_t lz, uint32_t row, uint64_t slice, hipStream_t st) {
+    const LevelBands L{hp, band_stride, low_sym, low, lx / 2, ly / 2, lz > 1 ? lz / 2 : 1, row, slice};
+    launch_level_bands<true>(L, const_cast<int16_t*>(data), lz > 1, st);
+}
+void unsymbolize_level(int16_t* data, const uint16_t* hp, uint64_t band_stride, const uint16_t* low_sym,
+                       const int16_t* low, uint32_t lx, uint32_t ly, uint32_t lz, uint32_t row, uint64_t slice,
+                       hipStream_t st) {
+    const LevelBands L{const_cast<uint16_t*>(hp), band_stride, const_cast<uint16_t*>(low_sym), const_cast<int16_t*>(low),
+                       lx / 2, ly / 2, lz > 1 ? lz / 2 : 1, row, slice};
+    launch_level_bands<false>(L, data, lz > 1, st);
 }
 
 }  // namespace cca

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "../hip/huff_design.hpp"
 #include "huffman_table.hpp"
 
 namespace cca {
@@ -69,8 +70,8 @@ void check_symbols(const cc_instance* I, int symSize) {
 }
 
 // ------------------------------------------------------------------------------------- encode
-void encode_prepare(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>& items, uint32_t ncalls, int symSize,
-                    EncodeJob& job, hipStream_t st) {
+void encode_upload(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>& items, uint32_t ncalls, int symSize,
+                   EncodeJob& job, hipStream_t st) {
     check_symbols(I, symSize);
     const uint32_t nitems = (uint32_t)items.size();
     const uint32_t per_unit = unit_chunks(items);
@@ -137,12 +138,40 @@ void encode_prepare(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>&
     job.lane_k = I->tuning.laneDesignK;
     D.d_items.get(stage_bytes);
     D.d_split.get(sizeof(SegState) * nslots + 4ull * kSplitWords * nsplit);
+    D.d_classes.as<uint32_t>(kDesignListBase + (uint64_t)kDesignLists * std::max<uint32_t>(job.nseq, 1));
+    CCA_HIP(hipMemcpyAsync(D.d_items.p, h, stage_bytes, hipMemcpyHostToDevice, st));
+}
+
+namespace {
+CodeUnits units_of(const DeviceCoder& D, const EncodeJob& job) {
+    const unsigned char* d = (const unsigned char*)D.d_items.p;
+    return CodeUnits{(const CodeUnit*)(d + job.o_units), job.nunits, (const uint32_t*)(d + job.o_split),
+                     job.nsplit_units, job.nsplit, (SegState*)D.d_split.p,
+                     (uint32_t*)((unsigned char*)D.d_split.p + sizeof(SegState) * job.nsplit_units)};
+}
+}  // namespace
+
+void encode_stats(DeviceCoder& D, const EncodeJob& job, SeqInfo* d_seqs, uint32_t* scratch, uint64_t cap,
+                  CoderState* d_state, hipStream_t st) {
+    coder_stats((const CodeItem*)D.d_items.p, job.nitems, d_seqs, job.p, job.symSize, scratch, cap, d_state,
+                (uint32_t*)D.d_classes.p, job.total_syms, units_of(D, job), st);
+}
+
+void encode_pack(DeviceCoder& D, const EncodeJob& job, SeqInfo* d_seqs, uint32_t* scratch, const CoderState* d_state,
+                 uint32_t* d_out, uint64_t out_cap, hipStream_t st) {
+    coder_pack((const CodeItem*)D.d_items.p, d_seqs, job.p, job.symSize, scratch, d_state, d_out, out_cap,
+               job.total_syms, units_of(D, job), st);
+}
+
+uint32_t design_leaf_words() { return 2 * design::kLaneMaxK + 8; }
+
+void encode_prepare(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>& items, uint32_t ncalls, int symSize,
+                    EncodeJob& job, hipStream_t st) {
+    encode_upload(I, D, items, ncalls, symSize, job, st);
     D.d_seqs.as<SeqInfo>(std::max<uint32_t>(job.nseq, 1));
     D.d_state.as<CoderState>(1);
-    D.d_classes.as<uint32_t>(kDesignListBase + (uint64_t)kDesignLists * std::max<uint32_t>(job.nseq, 1));
     D.d_calls.as<CallOut>(std::max<uint32_t>(ncalls, 1));
     D.h_result.get(sizeof(CoderState) + sizeof(CallOut) * std::max<uint32_t>(ncalls, 1));
-    CCA_HIP(hipMemcpyAsync(D.d_items.p, h, stage_bytes, hipMemcpyHostToDevice, st));
     encode_reserve(D, job, std::max<uint64_t>(D.scratch_cap, arena_estimate(items, I->log2, I->cbs)));
     SideStreams ss;
     side_streams(D, ss);
@@ -160,14 +189,11 @@ void encode_launch(DeviceCoder& D, const EncodeJob& job, uint32_t* d_out, uint64
                    const LayoutLink* link) {
     SideStreams ss;
     const unsigned char* d = (const unsigned char*)D.d_items.p;
-    const CodeUnits units{(const CodeUnit*)(d + job.o_units), job.nunits, (const uint32_t*)(d + job.o_split),
-                          job.nsplit_units, job.nsplit, (SegState*)D.d_split.p,
-                          (uint32_t*)((unsigned char*)D.d_split.p + sizeof(SegState) * job.nsplit_units)};
     coder_encode((const CodeItem*)d, job.nitems, (SeqInfo*)D.d_seqs.p, job.nseq, job.p, job.symSize,
                  (uint32_t*)D.d_scratch.p, job.scratch_cap, (CoderState*)D.d_state.p, (uint32_t*)D.d_classes.p,
                  (CallOut*)D.d_calls.p,
                  job.ncalls, (const uint32_t*)(d + job.o_first), d_out, out_cap, job.total_syms, st,
-                 side_streams(D, ss), link, job.design_grid, job.lane_k, units);
+                 side_streams(D, ss), link, job.design_grid, job.lane_k, units_of(D, job));
 }
 
 CoderState encode_finish(DeviceCoder& D, const EncodeJob& job, std::vector<CallOut>* results, hipStream_t st) {
@@ -217,10 +243,7 @@ uint64_t device_encode(cc_instance* I, const std::vector<CoderCall>& calls, cons
 }
 
 // ------------------------------------------------------------------------------------- decode
-namespace {
-// Block-decoder entries of sequence `seq` of at most nblk blocks: workgroups of kDecGroupBlocks
-// blocks at wl (long sequences), one wave at ws (short ones).
-void add_entries(uint32_t seq, uint32_t nblk, uint32_t* hws, uint32_t* hwf, uint32_t& wl, uint32_t& ws) {
+void add_block_entries(uint32_t seq, uint32_t nblk, uint32_t* hws, uint32_t* hwf, uint32_t& wl, uint32_t& ws) {
     if (dec_long(nblk)) {
         for (uint32_t b = 0; b < nblk; b += kDecGroupBlocks) {
             hws[wl] = seq;
@@ -234,6 +257,7 @@ void add_entries(uint32_t seq, uint32_t nblk, uint32_t* hws, uint32_t* hwf, uint
     }
 }
 
+namespace {
 // first[i]: the first zero-run expansion chunk of item i (nitems + 1 entries); returns the total.
 uint32_t chunk_table(const std::vector<ItemSpec>& items, uint32_t* first) {
     uint64_t k = 0;
@@ -289,7 +313,7 @@ void decode_prepare(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>&
         hi[i] = DecItem{it.ptr, it.n, it.rl ? 1u : 0u, seq, it.call};
         const uint32_t nblk = div_up(it.n, cbs);
         for (uint32_t q = 0; q < (it.rl ? 2u : 1u); q++)
-            add_entries(seq + q, nblk, hws, hwf, wl, ws);
+            add_block_entries(seq + q, nblk, hws, hwf, wl, ws);
         seq += it.rl ? 2 : 1;
     }
     job.nitems = nitems;
@@ -447,7 +471,7 @@ void decode_prepare_bound(cc_instance* I, DeviceCoder& D, const DecodeIndex& X, 
             }
             hb[seq + q] = DecBind{X.call_first_seq[index_calls[it.call]] + local, i, off};
             local++;
-            add_entries(seq + q, nblk, hws, hwf, wl, ws);
+            add_block_entries(seq + q, nblk, hws, hwf, wl, ws);
         }
         seq += it.rl ? 2 : 1;
     }

@@ -41,6 +41,15 @@ struct EncodeJob {
     uint32_t design_grid[4] = {4096, 2048, 1536, 768};  // resident workgroups per design class
     uint32_t lane_k = 0;  // tables of at most this many symbols are designed one per thread (0: none)
 };
+// Uploads the items and units of an encode (the part of encode_prepare that the passes alone need).
+void encode_upload(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>& items, uint32_t ncalls, int symSize,
+                   EncodeJob& job, hipStream_t st);
+void encode_stats(DeviceCoder& D, const EncodeJob& job, SeqInfo* d_seqs, uint32_t* scratch, uint64_t cap,
+                  CoderState* d_state, hipStream_t st);
+void encode_pack(DeviceCoder& D, const EncodeJob& job, SeqInfo* d_seqs, uint32_t* scratch, const CoderState* d_state,
+                 uint32_t* d_out, uint64_t out_cap, hipStream_t st);
+// Arena words of a small table's leaf list, which the stats pass writes after its histogram.
+uint32_t design_leaf_words();
 void encode_prepare(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>& items, uint32_t ncalls, int symSize,
                     EncodeJob& job, hipStream_t st);
 // Sizes the arena to at least `words` (allocates: not during graph capture).
@@ -48,6 +57,10 @@ void encode_reserve(DeviceCoder& D, EncodeJob& job, uint64_t words);
 void encode_launch(DeviceCoder& D, const EncodeJob& job, uint32_t* d_out, uint64_t out_cap, hipStream_t st,
                    const LayoutLink* link = nullptr);
 CoderState encode_finish(DeviceCoder& D, const EncodeJob& job, std::vector<CallOut>* results, hipStream_t st);
+
+// Block-decoder entries of sequence `seq` of (at most) nblk blocks: workgroups of kDecGroupBlocks blocks
+// at wl (long sequences), one wave at ws (short ones).
+void add_block_entries(uint32_t seq, uint32_t nblk, uint32_t* hws, uint32_t* hwf, uint32_t& wl, uint32_t& ws);
 
 struct DecodeJob {
     uint32_t nitems = 0, nseq = 0, ncalls = 0, nwaves = 0, nlong = 0;

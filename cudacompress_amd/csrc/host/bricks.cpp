@@ -159,6 +159,17 @@ cc_status status_of_encode(uint32_t e) {
 
 }  // namespace
 
+std::vector<ItemSpec> bricks_transforms_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, hipStream_t st) {
+    check_bricks(job.bricks.data(), (uint32_t)job.bricks.size(), job.L);
+    make_layout(job);
+    float* work = ctx.d_bwork.as<float>(std::max<uint64_t>(job.work_floats, 64));
+    unsigned char* sym = (unsigned char*)ctx.d_bsym.get(std::max<uint64_t>(job.sym_elems, 64) * job.symSize);
+    upload_levels(ctx, job, work, sym, I->tuning, st);
+    return brick_items(job, sym);
+}
+
+bool bricks_serve(uint64_t volume_elems, uint32_t levels) { return volume_elems < (1ull << 31) && levels <= 10; }
+
 void bricks_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, bool enc, bool dec,
                     const std::vector<CallWords>* calls, hipStream_t st) {
     const uint32_t n = (uint32_t)job.bricks.size();
@@ -167,11 +178,7 @@ void bricks_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, bool enc, bool
         CCA_REQUIRE(!enc || job.bricks[i].src, CC_ERR_INVALID_ARG, "null brick source");
         CCA_REQUIRE(!dec || job.bricks[i].dst, CC_ERR_INVALID_ARG, "null brick destination");
     }
-    make_layout(job);
-    float* work = ctx.d_bwork.as<float>(std::max<uint64_t>(job.work_floats, 64));
-    unsigned char* sym = (unsigned char*)ctx.d_bsym.get(std::max<uint64_t>(job.sym_elems, 64) * job.symSize);
-    upload_levels(ctx, job, work, sym, I->tuning, st);
-    const std::vector<ItemSpec> items = brick_items(job, sym);
+    const std::vector<ItemSpec> items = bricks_transforms_prepare(I, ctx, job, st);
     if (enc) encode_prepare(I, ctx.coder, items, n, job.symSize, job.ej, st);
     if (dec) {
         if (calls) {
@@ -191,11 +198,8 @@ void bricks_prepare_bound(cc_instance* I, BrickCtx& ctx, BrickJob& job, const De
     check_bricks(job.bricks.data(), n, job.L);
     for (uint32_t i = 0; i < n; i++)
         CCA_REQUIRE(job.bricks[i].dst, CC_ERR_INVALID_ARG, "null brick destination");
-    make_layout(job);
-    float* work = ctx.d_bwork.as<float>(std::max<uint64_t>(job.work_floats, 64));
-    unsigned char* sym = (unsigned char*)ctx.d_bsym.get(std::max<uint64_t>(job.sym_elems, 64) * job.symSize);
-    upload_levels(ctx, job, work, sym, I->tuning, st);
-    decode_prepare_bound(I, ctx.coder, X, brick_items(job, sym), index_calls, job.symSize, job.bj, st);
+    decode_prepare_bound(I, ctx.coder, X, bricks_transforms_prepare(I, ctx, job, st), index_calls, job.symSize, job.bj,
+                         st);
     job.index = &X;
 }
 
@@ -221,8 +225,14 @@ void bricks_encode_launch(BrickCtx& ctx, const BrickJob& job, hipStream_t st, co
     encode_launch(ctx.coder, job.ej, job.d_out, job.out_cap, st, link);
 }
 
-void bricks_decode_launch(BrickCtx& ctx, const BrickJob& job, hipStream_t st, bool from_encode) {
+void bricks_inverse_launch(const BrickJob& job, hipStream_t st) {
     const uint32_t n = (uint32_t)job.bricks.size();
+    for (int l = (int)job.L - 1; l >= 0; l--)
+        bricks_inverse_level(job.d_levels + (size_t)l * n, job.d_tiles + (size_t)l * 4 * (n + 1), n,
+                             &job.tiles_total[4 * l], job.symSize, job.level_elems[l], st);
+}
+
+void bricks_decode_launch(BrickCtx& ctx, const BrickJob& job, hipStream_t st, bool from_encode) {
     if (job.index) {
         decode_launch_bound(ctx.coder, *job.index, job.bj, st);
     } else {
@@ -231,9 +241,7 @@ void bricks_decode_launch(BrickCtx& ctx, const BrickJob& job, hipStream_t st, bo
                                      st);
         decode_launch(ctx.coder, job.dj, st);
     }
-    for (int l = (int)job.L - 1; l >= 0; l--)
-        bricks_inverse_level(job.d_levels + (size_t)l * n, job.d_tiles + (size_t)l * 4 * (n + 1), n,
-                             &job.tiles_total[4 * l], job.symSize, job.level_elems[l], st);
+    bricks_inverse_launch(job, st);
 }
 
 bool bricks_encode_results(const BrickJob& job, const std::vector<CallOut>& res, uint64_t total, uint64_t* offsets,

@@ -32,6 +32,11 @@ struct BrickJob {
     uint64_t out_cap = 0;
 };
 
+// The transforms of a job alone: layout, buffers and level tables; returns the bricks' symbol streams
+// in bitstream order (lowpass, then 7 bands a level from the coarsest), one call per brick.
+std::vector<ItemSpec> bricks_transforms_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, hipStream_t st);
+// whether a volume of so many elements and levels can be a brick
+bool bricks_serve(uint64_t volume_elems, uint32_t levels);
 // decode calls: one bitstream per brick, or when `calls` is null the device results of the
 // encode staged in the same context
 void bricks_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, bool enc, bool dec,
@@ -46,6 +51,8 @@ void bricks_index_build(cc_instance* I, DecodeIndex& X, const std::vector<cc_bri
 bool bricks_decode_results(const BrickJob& job, const std::vector<DecCallOut>& res, uint32_t* status);
 // forward transform and quantization of every brick (the first part of bricks_encode_launch)
 void bricks_forward_launch(const BrickJob& job, hipStream_t st);
+// every level's synthesis from the symbols (the last part of bricks_decode_launch)
+void bricks_inverse_launch(const BrickJob& job, hipStream_t st);
 void bricks_encode_launch(BrickCtx& ctx, const BrickJob& job, hipStream_t st, const LayoutLink* link = nullptr);
 void bricks_decode_launch(BrickCtx& ctx, const BrickJob& job, hipStream_t st, bool from_encode);
 

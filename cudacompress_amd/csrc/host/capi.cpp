@@ -56,7 +56,7 @@ cc_status encode_entry(cc_instance* inst, bool rl, int symbolSize, const void* c
     return guarded_for(inst, [&] {
         CCA_REQUIRE(inst && outWords && outSegBegin && outSegBits, CC_ERR_INVALID_ARG, "null argument");
         cca::encode_streams(inst, rl, symbolSize, streams, ns, n, startBits);
-        *outWords = inst->out_words.data();
+        *outWords = inst->out_words;
         *outSegBegin = inst->seg_begin.data();
         *outSegBits = inst->seg_bits.data();
     });
@@ -122,8 +122,6 @@ cc_status cc_create_instance(int device, uint32_t streamCountMax, uint32_t elemC
             const uint64_t symSize = I->log2 > 16 ? 4 : 2;
             const uint64_t per = (uint64_t)streamCountMax * cca::align_up(std::max<uint32_t>(elemCountPerStreamMax, 1), 64) * symSize;
             if (per > 0) {
-                I->d_rle_sym.get(per);
-                I->d_rle_zc.get(per);
                 I->d_dec_sym.get(per);
                 I->d_dec_zc.get(per);
             }
@@ -658,8 +656,8 @@ cc_status cc_compress_volume_float(cc_instance* inst, const float* d_image, uint
         CCA_REQUIRE(inst && outWords && outBits, CC_ERR_INVALID_ARG, "null argument");
         cca::compress_volume_float(inst, d_image, sizeX, sizeY, sizeZ, numLevels, quantStepLevel0,
                                    doRLEOnlyOnLvl0 != 0, symbolSize);
-        *outWords = inst->vol_bits.data();
-        *outBits = 32ull * inst->vol_bits.size();
+        *outWords = inst->out_words;
+        *outBits = 32ull * inst->out_count;
     });
 }
 cc_status cc_decompress_volume_float(cc_instance* inst, float* d_image, uint32_t sizeX, uint32_t sizeY, uint32_t sizeZ,
@@ -678,8 +676,8 @@ cc_status cc_compress_volume_float_quant_first(cc_instance* inst, const float* d
         CCA_REQUIRE(inst && d_image && outWords && outBits, CC_ERR_INVALID_ARG, "null argument");
         cca::compress_volume_float_quant_first(inst, d_image, sizeX, sizeY, sizeZ, numLevels, quantizationStep,
                                                doRLEOnlyOnLvl0 != 0);
-        *outWords = inst->vol_bits.data();
-        *outBits = 32ull * inst->vol_bits.size();
+        *outWords = inst->out_words;
+        *outBits = 32ull * inst->out_count;
     });
 }
 cc_status cc_decompress_volume_float_quant_first(cc_instance* inst, float* d_image, uint32_t sizeX, uint32_t sizeY,
@@ -725,8 +723,8 @@ cc_status cc_compress_volume_lossless(cc_instance* inst, const int16_t* d_image,
     return guarded_for(inst, [&] {
         CCA_REQUIRE(inst && outWords && outBits, CC_ERR_INVALID_ARG, "null argument");
         cca::compress_volume_lossless(inst, d_image, sizeX, sizeY, sizeZ, numLevels);
-        *outWords = inst->vol_bits.data();
-        *outBits = 32ull * inst->vol_bits.size();
+        *outWords = inst->out_words;
+        *outBits = 32ull * inst->out_count;
     });
 }
 cc_status cc_decompress_volume_lossless(cc_instance* inst, int16_t* d_image, uint32_t sizeX, uint32_t sizeY,

@@ -1,17 +1,19 @@
-// Host orchestration of the entropy coder: the equivalent of src/cudaCompress/Encode.cpp:208-917.
+// Host orchestration of the entropy coder: the equivalent of src/cudaCompress/Encode.cpp:208-917, for
+// bitstreams in host memory.  The streaming passes are the device coder's (hip/coder.hip,
+// hip/decoder.hip); the tables are designed here, where a merge costs some 50 ns instead of the 600 ns
+// of a wave's serial chain, so a call of a few tables ends sooner.
 //
-// Encode (per call, all streams batched into each launch):
-//   1. zero-run RLE (rl) or per-stream max (huff)        -> sync #1: pair counts, maxima
-//   2. histograms of every coded stream                   -> sync #2: histograms
-//   3. table design on the host (libstdc++ heap/sort, as the reference), exact bit counts from
-//      histogram x length, encode tables uploaded once
-//   4. Huffman block lengths, offsets scan, pack; codewords and offsets downloaded -> sync #3
-//   5. bitstream layout (Encode.cpp:402-463 rl, :751-782 huff) written on the host.
-// The reference does >= streams + 6 host synchronisations per encodeRLHuff; this does 3.
+// Encode, for all streams of a volume at once:
+//   1. upload of the stream list; the stats pass (zero-run pairs, histograms)     -> sync #1: histograms
+//   2. table design on the host (libstdc++ heap/sort, as the reference), exact bit counts from
+//      histogram x length, the layout of every section (Encode.cpp:402-463 rl, :751-782 huff)
+//   3. one upload (tables and sequence records); the pack writes the sections in place -> sync #2: words
+// The reference does >= streams + 6 host synchronisations per encodeRLHuff, per level of a volume.
 //
-// Decode parses every header on the host (tables, bit counts, offsets -- as Encode.cpp:522-621),
-// stages tables, codewords and absolute offsets in one pinned buffer, uploads it with a single
-// copy and decodes all coded streams in one launch; RLE decode writes every output element.
+// Decode walks the sections' heads on the host (counts, sizes, as Encode.cpp:522-621; the symbol
+// lists and codewords are left to the device), stages the sequence records and the bitstream in one
+// pinned buffer, uploads it with a single copy and enqueues the table build, the block decode and the
+// zero-run expansion.
 #include "codec.hpp"
 
 #include <algorithm>
@@ -19,40 +21,39 @@
 #include <cstring>
 #include <thread>
 
-#include "../kernels.hpp"
+#include "batch.hpp"
 #include "bitio.hpp"
 #include "huffman_table.hpp"
 
 namespace cca {
 namespace {
 
-constexpr uint32_t kPackSyms = 2048;
-
+// f(i) for i < n, on up to 16 threads when the work (in microseconds) repays starting them.
 template <class F>
-void parallel_for(size_t n, size_t work_hint, F f) {
-    unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    size_t nt = std::min<size_t>({(size_t)hw, n, (size_t)16});
-    if (nt <= 1 || work_hint < (1u << 16)) {
+void parallel_for(size_t n, double work_us, F f) {
+    const size_t hw = std::max(1u, std::thread::hardware_concurrency());
+    const size_t nt = std::min<size_t>({hw, n, (size_t)16, (size_t)(work_us / 75.0) + 1});
+    if (nt <= 1) {
         for (size_t i = 0; i < n; i++) f(i);
         return;
     }
     std::vector<std::thread> th;
     std::atomic<size_t> next{0};
-    for (size_t t = 0; t < nt; t++)
-        th.emplace_back([&]() {
-            for (size_t i = next++; i < n; i = next++) f(i);
-        });
+    auto work = [&]() {
+        for (size_t i = next++; i < n; i = next++) f(i);
+    };
+    for (size_t t = 1; t < nt; t++) th.emplace_back(work);
+    work();
     for (auto& x : th) x.join();
 }
 
-struct Staging {  // bump allocator over a pinned host buffer mirrored by a device buffer
-    unsigned char* h;
-    unsigned char* d;
+// Bump allocator over a pinned host buffer mirrored by a device buffer.
+struct Staging {
     size_t off = 0;
     template <class T>
     size_t push(size_t count) {
         off = align_up(off, 256);
-        size_t o = off;
+        const size_t o = off;
         off += count * sizeof(T);
         return o;
     }
@@ -60,408 +61,352 @@ struct Staging {  // bump allocator over a pinned host buffer mirrored by a devi
 
 }  // namespace
 
-void encode_streams(cc_instance* I, bool rl, int symSize, const void* const* streams, uint32_t ns, uint32_t n,
-                    const uint32_t* startBits) {
+void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& streams, uint32_t ncalls,
+                  bool last_call_first) {
     DeviceGuard guard(I->device);
     hipStream_t st = I->stream;
-    const bool longSymbols = I->log2 > 16;
-    CCA_REQUIRE(symSize == (longSymbols ? 4 : 2), CC_ERR_INVALID_ARG,
-                "symbol size does not match the instance (log2HuffmanDistinctSymbolCountMax > 16 uses Symbol32)");
-    CCA_REQUIRE(I->dialect == CC_DIALECT_GPU || symSize == 2, CC_ERR_INVALID_ARG, "the CPU dialect is Symbol16 only");
-    CCA_REQUIRE(ns == 0 || streams != nullptr, CC_ERR_INVALID_ARG, "null stream array");
-    for (uint32_t i = 0; i < ns; i++) CCA_REQUIRE(streams[i] != nullptr || n == 0, CC_ERR_INVALID_ARG, "null stream");
-    if (startBits)
-        for (uint32_t i = 0; i < ns; i++) CCA_REQUIRE(startBits[i] < 32, CC_ERR_INVALID_ARG, "start bit offset >= 32");
+    check_symbols(I, symSize);
+    const uint32_t ns = (uint32_t)streams.size();
+    std::vector<ItemSpec> items(ns);
+    for (uint32_t i = 0; i < ns; i++) {
+        const EncodeStream& s = streams[i];
+        CCA_REQUIRE(s.in != nullptr || s.n == 0, CC_ERR_INVALID_ARG, "null stream");
+        CCA_REQUIRE(s.start_bit < 32, CC_ERR_INVALID_ARG, "start bit offset >= 32");
+        items[i] = ItemSpec{const_cast<void*>(s.in), s.n, s.rl, s.call};
+    }
     const uint32_t cbs = I->cbs;
     const HeaderFormat fmt = header_format(I->dialect, I->log2);
-    I->out_words.clear();
+    I->out_words = nullptr;
+    I->out_count = 0;
     I->seg_begin.assign(ns, 0);
     I->seg_bits.assign(ns, 0);
     if (ns == 0) return;
-    SectionTimer call(I, 1), stage(I, 2);
-    call(rl ? "Encode RLHuff" : "Encode Huff");
+    SectionTimer stage(I, 2);
 
-    // ---- 1. RLE / maxima --------------------------------------------------------------------
-    stage(rl ? "Encode: Run Length" : "Encode: Maxima");
-    const uint64_t cap = align_up(std::max<uint32_t>(n, 1), 64);
-    const uint32_t tiles_per = rl ? div_up(n, kRleTile) : 0;
-    const uint32_t ntiles = tiles_per * ns;
-    {
-        Staging s{(unsigned char*)I->h_up.get(0), nullptr};
-        size_t o_desc = s.push<RleStream>(ns);
-        size_t o_map = s.push<uint32_t>(ntiles);
-        unsigned char* h = (unsigned char*)I->h_up.get(s.off);
-        unsigned char* d = (unsigned char*)I->d_desc.get(s.off);
-        RleStream* hd = (RleStream*)(h + o_desc);
-        uint32_t* hm = (uint32_t*)(h + o_map);
-        unsigned char* dsym = rl ? (unsigned char*)I->d_rle_sym.get(cap * ns * symSize) : nullptr;
-        unsigned char* dzc = rl ? (unsigned char*)I->d_rle_zc.get(cap * ns * symSize) : nullptr;
-        for (uint32_t i = 0; i < ns; i++) {
-            hd[i].in = streams[i];
-            hd[i].out_sym = rl ? dsym + cap * i * symSize : nullptr;
-            hd[i].out_zc = rl ? dzc + cap * i * symSize : nullptr;
-            hd[i].n = n;
-            hd[i].tile_base = i * tiles_per;
-            for (uint32_t t = 0; t < tiles_per; t++) hm[i * tiles_per + t] = i;
-        }
-        CCA_HIP(hipMemcpyAsync(d, h, s.off, hipMemcpyHostToDevice, st));
-        RleResult* dres = I->d_results.as<RleResult>(ns);
-        if (rl) {
-            RleTile* dt = I->d_tiles.as<RleTile>(std::max<uint32_t>(ntiles, 1));
-            rle_encode((const RleStream*)(d + o_desc), ns, dt, ntiles, (const uint32_t*)(d + o_map), dres, symSize,
-                       (uint64_t)n * ns, st);
-        } else {
-            stream_max((const RleStream*)(d + o_desc), ns, n, dres, symSize, st);
-        }
-        CCA_HIP(hipMemcpyAsync(I->h_down.get(sizeof(RleResult) * ns), dres, sizeof(RleResult) * ns,
-                               hipMemcpyDeviceToHost, st));
-        CCA_HIP(hipStreamSynchronize(st));
-    }
-    std::vector<RleResult> res((RleResult*)I->h_down.p, (RleResult*)I->h_down.p + ns);
-
-    // ---- 2. histograms ----------------------------------------------------------------------
+    // ---- 1. pairs and histograms --------------------------------------------------------------
     stage("Encode: Histograms");
-    const uint32_t nt = rl ? 2 * ns : ns;
-    struct Coded {
-        const void* data;
-        uint32_t count, smax;
-        uint32_t quirk;
-        uint64_t hist_off;
-    };
-    std::vector<Coded> coded(nt);
-    uint32_t callmax_sym = 0, callmax_zc = 0;
-    uint64_t hist_total = 0;
-    for (uint32_t i = 0; i < ns; i++) {
-        const RleResult& r = res[i];
-        if (rl) {
-            const unsigned char* dsym = (const unsigned char*)I->d_rle_sym.p + cap * i * symSize;
-            const unsigned char* dzc = (const unsigned char*)I->d_rle_zc.p + cap * i * symSize;
-            coded[2 * i] = Coded{dsym, r.m, r.m ? r.sym_max : 0u, 0, 0};
-            coded[2 * i + 1] = Coded{dzc, r.m, r.m ? r.zc_max : 0u, 0, 0};
-            callmax_sym = std::max(callmax_sym, coded[2 * i].smax);
-            callmax_zc = std::max(callmax_zc, coded[2 * i + 1].smax);
-        } else {
-            coded[i] = Coded{streams[i], n, r.sym_max, 0, 0};
-            callmax_sym = std::max(callmax_sym, r.sym_max);
-        }
-    }
-    if (fmt.dialect == CC_DIALECT_GPU) {
-        // HuffmanTable.cu:409-419 (checked per design call: symbols, then zero counts)
-        CCA_REQUIRE((uint64_t)callmax_sym + 1 <= (1ull << I->log2), CC_ERR_SYMBOL_OVERFLOW,
-                    "symbol exceeds 2^log2HuffmanDistinctSymbolCountMax");
-        CCA_REQUIRE((uint64_t)callmax_zc + 1 <= (1ull << I->log2), CC_ERR_SYMBOL_OVERFLOW,
-                    "zero count exceeds 2^log2HuffmanDistinctSymbolCountMax");
-    }
-    for (uint32_t j = 0; j < nt; j++) {
-        Coded& c = coded[j];
-        const bool is_sym = !rl || (j % 2 == 0);
-        // Symbol16 streams are padded with 0xFFFF to a multiple of 8 before the histogram
-        // (Histogram.cu:90-96, Encode.cpp:260-264); when the design call has 65536 bins the
-        // 32-bit-word histogram pass counts one pad in bin 65535 for an odd symbol count.
-        c.quirk = (fmt.dialect == CC_DIALECT_GPU && symSize == 2 && is_sym && c.smax == 65535u && (c.count & 1u)) ? 1u : 0u;
-        c.hist_off = hist_total;
-        hist_total += align_up((uint64_t)c.smax + 1, 64);
-    }
-    {
-        uint32_t* dh = I->d_hist.as<uint32_t>(hist_total);
-        CCA_HIP(hipMemsetAsync(dh, 0, hist_total * 4, st));
-        Staging s{nullptr, nullptr};
-        size_t o_desc = s.push<HistStream>(nt);
-        HistStream* hd = (HistStream*)((unsigned char*)I->h_up.get(s.off) + o_desc);
-        for (uint32_t j = 0; j < nt; j++)
-            hd[j] = HistStream{coded[j].data, coded[j].count, coded[j].smax + 1, dh + coded[j].hist_off, coded[j].quirk};
-        unsigned char* d = (unsigned char*)I->d_desc.get(s.off);
-        CCA_HIP(hipMemcpyAsync(d, I->h_up.p, s.off, hipMemcpyHostToDevice, st));
-        histogram((const HistStream*)(d + o_desc), hd, nt, symSize, st);
-        CCA_HIP(hipMemcpyAsync(I->h_hist.get(hist_total * 4), dh, hist_total * 4, hipMemcpyDeviceToHost, st));
+    DeviceCoder& D = I->coder;
+    EncodeJob job;
+    encode_upload(I, D, items, ncalls, symSize, job, st);
+    const uint32_t nseq = job.nseq;
+    // one device buffer: the coder's state, the sequence records, the arena
+    const size_t o_seq = align_up(sizeof(CoderState), 64), o_arena = align_up(o_seq + sizeof(SeqInfo) * nseq, 256);
+    uint64_t cap = std::max<uint64_t>(I->enc_arena, 1024 + (uint64_t)nseq * (kStatBins + 2 * design_leaf_words()));
+    unsigned char *d, *h;
+    for (int attempt = 0;; attempt++) {
+        d = (unsigned char*)I->d_enc.get(o_arena + 4 * cap);
+        encode_stats(D, job, (SeqInfo*)(d + o_seq), (uint32_t*)(d + o_arena), cap, (CoderState*)d, st);
+        // the state, the records and as much of the arena as the last call used come down together
+        const uint64_t first = std::min(cap, std::max<uint64_t>(I->enc_down, 4096));
+        h = (unsigned char*)I->h_down.get(o_arena + 4 * cap);
+        CCA_HIP(hipMemcpyAsync(h, d, o_arena + 4 * first, hipMemcpyDeviceToHost, st));
         CCA_HIP(hipStreamSynchronize(st));
+        const CoderState s = *(const CoderState*)h;
+        if (s.err == kErrScratch && attempt < 4) {
+            cap = std::max<uint64_t>(2 * cap, s.scratch_used + s.scratch_used / 4);
+            continue;
+        }
+        CCA_REQUIRE(s.err == kErrNone, CC_ERR_OUT_OF_MEMORY, "coder arena exhausted");
+        const uint64_t used = std::min<uint64_t>(s.scratch_used, cap);
+        if (used > first) {
+            CCA_HIP(hipMemcpyAsync(h + o_arena + 4 * first, d + o_arena + 4 * first, 4 * (used - first),
+                                   hipMemcpyDeviceToHost, st));
+            CCA_HIP(hipStreamSynchronize(st));
+        }
+        I->enc_arena = cap;
+        I->enc_down = std::min<uint64_t>(align_up(used, 4096), 1u << 18);
+        break;
     }
-    const uint32_t* hh = (const uint32_t*)I->h_hist.p;
+    std::vector<SeqInfo> seqs((const SeqInfo*)(h + o_seq), (const SeqInfo*)(h + o_seq) + nseq);
+    const uint32_t* arena = (const uint32_t*)(h + o_arena);
 
-    // ---- 3. table design ----------------------------------------------------------------------
+    // ---- 2. table design and layout -------------------------------------------------------------
     stage("Encode: Design Huffman Tables");
-    std::vector<EncTable> tables(nt);
-    std::vector<cc_status> rcs(nt, CC_OK);
-    std::vector<uint64_t> bits(nt, 0);
-    uint64_t design_work = 0;
-    for (auto& c : coded) design_work += c.smax + 1;
-    parallel_for(nt, design_work, [&](size_t j) {
-        rcs[j] = design_table(fmt.dialect, hh + coded[j].hist_off, coded[j].smax, tables[j]);
+    std::vector<EncTable> tables(nseq);
+    std::vector<cc_status> rcs(nseq, CC_OK);
+    std::vector<uint64_t> bits(nseq, 0);
+    double work_us = 0;
+    for (const SeqInfo& s : seqs) work_us += s.err ? 0.0 : 0.08 * s.nsym + 0.002 * s.smax;
+    parallel_for(nseq, work_us, [&](size_t j) {
+        const SeqInfo& s = seqs[j];
+        if (s.err) return;
+        const uint32_t* hist = arena + s.hist_off;
+        rcs[j] = design_table(fmt.dialect, hist, s.smax, tables[j]);
         if (rcs[j] != CC_OK) return;
         uint64_t b = 0;
-        const uint32_t* h = hh + coded[j].hist_off;
-        for (uint32_t s = 0; s <= coded[j].smax; s++)
-            if (h[s]) b += (uint64_t)h[s] * tables[j].len[s];
-        if (coded[j].quirk) b -= tables[j].len[65535];  // the counted pad is not encoded
+        for (uint32_t k : tables[j].symbols) b += (uint64_t)hist[k] * tables[j].len[k];
+        if (s.quirk) b -= tables[j].len[65535];  // the counted pad is not encoded
         bits[j] = b;
     });
-    for (uint32_t j = 0; j < nt; j++) {
-        CCA_REQUIRE(rcs[j] == CC_OK, rcs[j], "Huffman codeword longer than 31 bits");
-        if (fmt.dialect == CC_DIALECT_CPU)
-            CCA_REQUIRE(tables[j].symbols.size() < (1u << 14), CC_ERR_SYMBOL_OVERFLOW,
-                        "more than 16383 distinct symbols cannot be described in the CPU dialect header");
-        CCA_REQUIRE(bits[j] < (1ull << 32), CC_ERR_INVALID_ARG, "coded stream exceeds 2^32 bits");
+    // first sequence of every stream, and of every call (streams come grouped by call)
+    std::vector<uint32_t> first_seq(ns), call_first(ncalls + 1, nseq);
+    for (uint32_t i = 0, k = 0; i < ns; i++) {
+        first_seq[i] = k;
+        k += streams[i].rl ? 2 : 1;
     }
-
-    // ---- 4. Huffman encode ------------------------------------------------------------------
-    stage("Encode: Huffman Encode");
-    std::vector<uint64_t> tab_off(nt), word_off(nt), offs_off(nt);
-    std::vector<uint32_t> nblk(nt), nchk(nt);
-    uint64_t tab_total = 0, word_total = 0, offs_total = 0;
-    uint32_t nblocks = 0, nchunks = 0;
-    for (uint32_t j = 0; j < nt; j++) {
-        tab_off[j] = tab_total;
-        tab_total += 2 * align_up((uint64_t)coded[j].smax + 1, 64);
-        word_off[j] = word_total;
-        word_total += align_up((bits[j] + 31) / 32 + 2, 64);
-        nblk[j] = div_up(coded[j].count, cbs);
-        nchk[j] = div_up(coded[j].count, kPackSyms);
-        offs_off[j] = offs_total;
-        offs_total += align_up(std::max<uint32_t>(nblk[j], 1), 64);
-        nblocks += nblk[j];
-        nchunks += nchk[j];
+    for (uint32_t i = ns, c = ncalls; c-- > 0;) {
+        call_first[c] = call_first[c + 1];
+        while (i > 0 && streams[i - 1].call == c) call_first[c] = first_seq[--i];
     }
-    uint32_t* dtab = I->d_tables.as<uint32_t>(tab_total);
-    uint32_t* dwords = I->d_words.as<uint32_t>(word_total);
-    uint32_t* doffs = I->d_offsets.as<uint32_t>(offs_total);
-    uint32_t* dbb = I->d_block_bits.as<uint32_t>(std::max<uint32_t>(nblocks, 1));
-    uint32_t* dsb = I->d_stream_bits.as<uint32_t>(nt);
-    {
-        Staging s{nullptr, nullptr};
-        size_t o_tab = s.push<uint32_t>(tab_total);
-        size_t o_desc = s.push<HuffEncStream>(nt);
-        size_t o_bmap = s.push<uint32_t>(nblocks);
-        size_t o_cmap = s.push<uint32_t>(nchunks);
-        unsigned char* h = (unsigned char*)I->h_up.get(s.off);
-        unsigned char* d = (unsigned char*)I->d_desc.get(s.off - o_desc);
-        uint32_t* htab = (uint32_t*)(h + o_tab);
-        HuffEncStream* hd = (HuffEncStream*)(h + o_desc);
-        uint32_t* hb = (uint32_t*)(h + o_bmap);
-        uint32_t* hc = (uint32_t*)(h + o_cmap);
-        uint32_t bb = 0, cb = 0;
-        for (uint32_t j = 0; j < nt; j++) {
-            const uint32_t nb = coded[j].smax + 1;
-            memcpy(htab + tab_off[j], tables[j].code.data(), 4ull * nb);
-            memcpy(htab + tab_off[j] + align_up(nb, 64), tables[j].len.data(), 4ull * nb);
-            hd[j] = HuffEncStream{coded[j].data, dtab + tab_off[j], dtab + tab_off[j] + align_up(nb, 64),
-                                  dwords + word_off[j], doffs + offs_off[j], coded[j].count, bb, cb, 0};
-            for (uint32_t b = 0; b < nblk[j]; b++) hb[bb + b] = j;
-            for (uint32_t c = 0; c < nchk[j]; c++) hc[cb + c] = j;
-            bb += nblk[j];
-            cb += nchk[j];
+    for (uint32_t q = 0; q < ncalls; q++) {
+        const uint32_t c = last_call_first ? ncalls - 1 - q : q;
+        const uint32_t j0 = call_first[c], j1 = call_first[c + 1];
+        // HuffmanTable.cu:409-419 (checked per design call)
+        for (uint32_t j = j0; j < j1; j++)
+            CCA_REQUIRE(seqs[j].err != kErrOverflow, CC_ERR_SYMBOL_OVERFLOW,
+                        "symbol exceeds 2^log2HuffmanDistinctSymbolCountMax");
+        for (uint32_t j = j0; j < j1; j++) {
+            CCA_REQUIRE(rcs[j] == CC_OK, rcs[j], "Huffman codeword longer than 31 bits");
+            if (fmt.dialect == CC_DIALECT_CPU)
+                CCA_REQUIRE(tables[j].symbols.size() < (1u << 14), CC_ERR_SYMBOL_OVERFLOW,
+                            "more than 16383 distinct symbols cannot be described in the CPU dialect header");
+            CCA_REQUIRE(bits[j] < (1ull << 32), CC_ERR_INVALID_ARG, "coded stream exceeds 2^32 bits");
         }
-        CCA_HIP(hipMemcpyAsync(dtab, h + o_tab, 4 * tab_total, hipMemcpyHostToDevice, st));
-        CCA_HIP(hipMemcpyAsync(d, h + o_desc, s.off - o_desc, hipMemcpyHostToDevice, st));
-        const HuffEncStream* dd = (const HuffEncStream*)d;
-        uint64_t total_bits = 0;
-        for (uint32_t j = 0; j < nt; j++) total_bits += bits[j];
-        huffman_encode(dd, hd, nt, cbs, symSize, dbb, nblocks, (const uint32_t*)(d + (o_bmap - o_desc)), dsb,
-                       (const uint32_t*)(d + (o_cmap - o_desc)), nchunks, total_bits, st);
-        // download codewords and offsets (exact sizes are known from the histograms)
-        uint64_t down_words = 0;
-        for (uint32_t j = 0; j < nt; j++) down_words += (bits[j] + 31) / 32 + nblk[j];
-        uint32_t* hw = I->h_words.as<uint32_t>(std::max<uint64_t>(down_words, 1));
-        uint64_t o = 0;
-        for (uint32_t j = 0; j < nt; j++) {
-            uint64_t nw = (bits[j] + 31) / 32;
-            if (nw) CCA_HIP(hipMemcpyAsync(hw + o, dwords + word_off[j], 4 * nw, hipMemcpyDeviceToHost, st));
-            o += nw;
-            if (nblk[j]) CCA_HIP(hipMemcpyAsync(hw + o, doffs + offs_off[j], 4ull * nblk[j], hipMemcpyDeviceToHost, st));
-            o += nblk[j];
-        }
-        CCA_HIP(hipStreamSynchronize(st));
     }
-
-    // ---- 5. bitstream layout ------------------------------------------------------------------
-    stage("Encode: Bitstream Layout");
-    const uint32_t* hw = (const uint32_t*)I->h_words.p;
-    std::vector<uint16_t> inc;
-    BitWriter w(I->out_words);
-    uint64_t o = 0;
-    auto put_coded = [&](uint32_t j) {
-        write_table(fmt, tables[j], w);
-        const uint32_t nb32 = (uint32_t)bits[j];
-        w.aligned_u32(&nb32, 1);
-        const uint64_t nw = (bits[j] + 31) / 32;
-        w.aligned_u32(hw + o, nw);
-        o += nw;
-        // offsets as 16-bit increments (packInc16CPU, PackInc.cu:210-220)
-        const uint32_t* off = hw + o;
-        inc.resize(nblk[j]);
-        uint32_t prev = 0;
-        for (uint32_t b = 0; b < nblk[j]; b++) {
-            inc[b] = (uint16_t)(off[b] - prev);
-            prev = off[b];
-        }
-        w.aligned_u16(inc.data(), nblk[j]);
-        o += nblk[j];
-    };
+    // sections in stream order; the arena: every table (code, len by symbol, symbols in codeword order),
+    // then the coding-block offsets, which the pack fills
+    uint64_t pos = 0, tab = 0;
     for (uint32_t i = 0; i < ns; i++) {
-        const uint64_t begin = I->out_words.size();
-        I->seg_begin[i] = begin;
-        w.set_pos(begin * 32 + (startBits ? startBits[i] : 0u));
-        if (rl) {
-            const uint32_t m = res[i].m;
-            w.aligned_u32(&m, 1);
-            put_coded(2 * i);
-            put_coded(2 * i + 1);
-        } else {
-            put_coded(i);
+        const EncodeStream& s = streams[i];
+        I->seg_begin[i] = pos;
+        if (s.rl) pos += 1 + (s.start_bit ? 1 : 0);  // the pair count, from a word boundary on
+        for (uint32_t q = 0; q < (s.rl ? 2u : 1u); q++) {
+            const uint32_t j = first_seq[i] + q;
+            SeqInfo& r = seqs[j];
+            const EncTable& t = tables[j];
+            const uint64_t tb = table_bits(fmt, t), tw = (tb + 31) / 32;
+            const uint64_t nblk = div_up(r.count, cbs);
+            // a header that starts inside a word may reach one word further
+            if (!s.rl) pos += (tb + s.start_bit + 31) / 32 - tw;
+            r.out_off = pos;
+            pos += tw + 1 + (bits[j] + 31) / 32 + (nblk + 1) / 2;
+            r.nlen = (uint32_t)t.count_per_length.size();
+            r.nsym = (uint32_t)t.symbols.size();
+            r.bits = bits[j];
+            for (uint32_t l = 0; l < 32; l++) r.cpl[l] = l < r.nlen ? t.count_per_length[l] : 0u;
+            r.code_off = tab;
+            r.syms_off = tab + 2ull * (r.smax + 1);
+            tab = align_up(r.syms_off + std::max<uint32_t>(r.nsym, 1), 16);
         }
-        w.align32();
-        I->seg_bits[i] = w.pos() - begin * 32;
+        I->seg_bits[i] = (pos - I->seg_begin[i]) * 32;
     }
+    const uint64_t total = pos;
+    uint64_t arena_words = tab;
+    for (SeqInfo& r : seqs) {
+        r.boff_off = arena_words;
+        arena_words += align_up(std::max<uint32_t>(div_up(r.count, cbs), 1), 16);
+    }
+
+    // ---- 3. codewords ----------------------------------------------------------------------------
+    stage("Encode: Huffman Encode");
+    if (arena_words > cap) {  // (nothing in the arena is needed any more)
+        I->enc_arena = arena_words;
+        d = (unsigned char*)I->d_enc.get(o_arena + 4 * arena_words);
+    }
+    unsigned char* u = (unsigned char*)I->h_up.get(o_arena + 4 * tab);
+    *(CoderState*)u = CoderState{0, total, 0, 0, 0};
+    memcpy(u + o_seq, seqs.data(), sizeof(SeqInfo) * nseq);
+    uint32_t* ua = (uint32_t*)(u + o_arena);
+    for (uint32_t j = 0; j < nseq; j++) {
+        const EncTable& t = tables[j];
+        memcpy(ua + seqs[j].code_off, t.code.data(), 4ull * t.code.size());
+        memcpy(ua + seqs[j].code_off + seqs[j].smax + 1, t.len.data(), 4ull * t.len.size());
+        memcpy(ua + seqs[j].syms_off, t.symbols.data(), 4ull * t.symbols.size());
+    }
+    CCA_HIP(hipMemcpyAsync(d, u, o_arena + 4 * tab, hipMemcpyHostToDevice, st));
+    uint32_t* dw = I->d_words.as<uint32_t>(std::max<uint64_t>(total, 1));
+    encode_pack(D, job, (SeqInfo*)(d + o_seq), (uint32_t*)(d + o_arena), (CoderState*)d, dw, total, st);
+    uint32_t* hw = I->h_words.as<uint32_t>(std::max<uint64_t>(total, 1));
+    CCA_HIP(hipMemcpyAsync(hw, dw, 4 * total, hipMemcpyDeviceToHost, st));
+    CCA_HIP(hipStreamSynchronize(st));
+
+    // segments that start inside a word: zero bits where the caller's are, the header behind them
+    stage("Encode: Bitstream Layout");
+    for (uint32_t i = 0; i < ns; i++) {
+        const EncodeStream& s = streams[i];
+        if (!s.start_bit) continue;
+        if (s.rl) {
+            hw[I->seg_begin[i]] = 0;
+            continue;
+        }
+        std::vector<uint32_t> head;
+        BitWriter w(head);
+        w.set_pos(s.start_bit);
+        write_table(fmt, tables[first_seq[i]], w);
+        memcpy(hw + I->seg_begin[i], head.data(), 4 * head.size());
+    }
+    I->out_words = hw;
+    I->out_count = total;
 }
 
-void decode_streams(cc_instance* I, bool rl, int symSize, const uint32_t* const* bsWords, const uint64_t* bsBits,
-                    uint64_t* bsPos, uint32_t nbs, const uint32_t* s2b, void* const* outs, uint32_t ns, uint32_t n) {
+void encode_streams(cc_instance* I, bool rl, int symSize, const void* const* streams, uint32_t ns, uint32_t n,
+                    const uint32_t* startBits) {
+    check_symbols(I, symSize);
+    CCA_REQUIRE(ns == 0 || streams != nullptr, CC_ERR_INVALID_ARG, "null stream array");
+    std::vector<EncodeStream> s(ns);
+    for (uint32_t i = 0; i < ns; i++) s[i] = EncodeStream{streams[i], n, rl, 0, startBits ? startBits[i] : 0u};
+    SectionTimer call(I, 1);
+    if (ns) call(rl ? "Encode RLHuff" : "Encode Huff");
+    encode_items(I, symSize, s, 1);
+}
+
+void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, const uint64_t* bsBits,
+                  uint64_t* bsPos, uint32_t nbs, const std::vector<DecodeStream>& streams) {
     DeviceGuard guard(I->device);
     hipStream_t st = I->stream;
-    const bool longSymbols = I->log2 > 16;
-    CCA_REQUIRE(symSize == (longSymbols ? 4 : 2), CC_ERR_INVALID_ARG, "symbol size does not match the instance");
-    CCA_REQUIRE(I->dialect == CC_DIALECT_GPU || symSize == 2, CC_ERR_INVALID_ARG, "the CPU dialect is Symbol16 only");
+    check_symbols(I, symSize);
     CCA_REQUIRE(nbs >= 1 && bsWords && bsBits && bsPos, CC_ERR_INVALID_ARG, "no bitstream");
+    const uint32_t ns = (uint32_t)streams.size();
     if (ns == 0) return;
-    CCA_REQUIRE(outs != nullptr, CC_ERR_INVALID_ARG, "null output array");
     const uint32_t cbs = I->cbs;
     const HeaderFormat fmt = header_format(I->dialect, I->log2);
-    SectionTimer call(I, 1), stage(I, 2);
-    call(rl ? "Decode RLHuff" : "Decode Huff");
+    SectionTimer stage(I, 2);
     stage("Decode: Read Tables + Upload");
 
-    struct Coded {
-        DecTable t;
-        const uint32_t* words;
-        uint32_t nwords;
-        const uint16_t* incs;
-        uint32_t count;
-    };
-    const uint32_t nc = rl ? 2 * ns : ns;
-    std::vector<Coded> coded(nc);
-    std::vector<uint32_t> m(ns, n);
-    auto read_coded = [&](BitReader& r, Coded& c, uint32_t count) {
-        CCA_REQUIRE(read_table(fmt, r, c.t), CC_ERR_CORRUPT_STREAM, "malformed Huffman table header");
+    // ---- the sections' heads ------------------------------------------------------------------
+    // Bit and word positions are kept from the first word of each bitstream that is read.
+    std::vector<uint64_t> w0(nbs, ~0ull), w1(nbs, 0);
+    std::vector<DecSeq> seqs;
+    std::vector<DecItem> items(ns);
+    std::vector<uint32_t> seq_bs;
+    auto read_coded = [&](BitReader& r, uint32_t bs, uint32_t item, uint32_t count) {
+        DecSeq s{};
+        s.hdr_bit = r.pos();
+        s.nlen = r.bits(5);
+        uint64_t codes = 0;
+        for (uint32_t l = 0; l < s.nlen; l++) codes += r.bits(fmt.count_bits);
+        s.nsym = r.bits(fmt.count_bits);
+        s.sb = r.bits(fmt.symbits_bits);
+        // HuffmanTable.cu:138-139: a stored 0 with more than one symbol means 16 (Symbol16 only)
+        if (fmt.dialect == CC_DIALECT_GPU && fmt.symbits_bits == 4 && s.sb == 0 && s.nsym > 1) s.sb = 16;
+        CCA_REQUIRE(s.sb <= 32 && r.ok(), CC_ERR_CORRUPT_STREAM, "malformed Huffman table header");
+        s.sym_bit = r.pos();
+        r.skip_bits((uint64_t)s.sb * s.nsym);
+        CCA_REQUIRE(r.ok() && (s.nsym == 0 || s.nlen == 0 || codes == s.nsym), CC_ERR_CORRUPT_STREAM,
+                    "malformed Huffman table header");
         const uint32_t nbits = r.aligned_u32();
-        c.words = r.word_ptr();
-        c.nwords = (nbits + 31) / 32;
-        r.skip_bits(32ull * c.nwords);
+        s.words_off = r.pos() >> 5;
+        s.nwords_cw = (uint32_t)(((uint64_t)nbits + 31) / 32);
+        r.skip_bits(32ull * s.nwords_cw);
         r.align32();
-        c.incs = (const uint16_t*)r.word_ptr();
-        r.skip_aligned(div_up(count, cbs), 2);
-        c.count = count;
+        s.incs_off = r.pos() >> 5;
+        const uint16_t* incs = (const uint16_t*)r.word_ptr();
+        const uint32_t noff = div_up(count, cbs);
+        r.skip_aligned(noff, 2);
         CCA_REQUIRE(r.ok(), CC_ERR_CORRUPT_STREAM, "bitstream ends inside a coded stream");
-        CCA_REQUIRE(count == 0 || !c.t.symbols.empty(), CC_ERR_CORRUPT_STREAM, "empty table for a non-empty stream");
+        CCA_REQUIRE(count == 0 || s.nsym != 0, CC_ERR_CORRUPT_STREAM, "empty table for a non-empty stream");
+        // the block offsets are running sums (unpackInc16CPU, PackInc.cu:222-229): the last is the largest
+        uint64_t sum = 0;
+        for (uint32_t b = 0; b < noff; b++) sum += incs[b];
+        CCA_REQUIRE(sum <= 32ull * s.nwords_cw, CC_ERR_CORRUPT_STREAM, "coding block offset beyond the codewords");
+        s.count = count;
+        s.item = item;
+        seqs.push_back(s);
+        seq_bs.push_back(bs);
     };
+    uint64_t rl_elems = 0;
+    std::vector<uint64_t> rl_off(ns, 0);
     for (uint32_t i = 0; i < ns; i++) {
-        const uint32_t b = s2b ? s2b[i] : 0u;
+        const DecodeStream& s = streams[i];
+        const uint32_t b = s.bs;
         CCA_REQUIRE(b < nbs && bsWords[b], CC_ERR_INVALID_ARG, "bad bitstream index");
         BitReader r(bsWords[b], bsBits[b], bsPos[b]);
-        if (rl) {
-            m[i] = r.aligned_u32();
-            CCA_REQUIRE(r.ok() && m[i] <= n, CC_ERR_CORRUPT_STREAM, "run-length pair count exceeds the stream length");
-            read_coded(r, coded[2 * i], m[i]);
-            read_coded(r, coded[2 * i + 1], m[i]);
-        } else {
-            read_coded(r, coded[i], n);
+        w0[b] = std::min(w0[b], bsPos[b] >> 5);
+        items[i] = DecItem{s.out, s.n, s.rl ? 1u : 0u, (uint32_t)seqs.size(), 0};
+        uint32_t count = s.n;
+        if (s.rl) {
+            count = r.aligned_u32();
+            CCA_REQUIRE(r.ok() && count <= s.n, CC_ERR_CORRUPT_STREAM, "run-length pair count exceeds the stream length");
+            read_coded(r, b, i, count);
+            rl_off[i] = rl_elems;
+            rl_elems += align_up(std::max<uint32_t>(count, 1), 64);
         }
+        read_coded(r, b, i, count);
         bsPos[b] = r.pos();
+        w1[b] = std::max(w1[b], (r.pos() + 31) >> 5);
+        CCA_REQUIRE(s.out != nullptr || s.n == 0, CC_ERR_INVALID_ARG, "null output stream");
     }
+    const uint32_t nseq = (uint32_t)seqs.size();
 
-    // staging layout
-    Staging s{nullptr, nullptr};
-    std::vector<size_t> o_tab(nc), o_sym(nc), o_off(nc), o_words(nc);
-    uint32_t nwaves = 0;
-    std::vector<uint32_t> wave_base(nc);
-    for (uint32_t j = 0; j < nc; j++) {
-        o_tab[j] = s.push<int32_t>(96);
-        o_sym[j] = s.push<unsigned char>(coded[j].t.symbols.size() * symSize);
-        o_off[j] = s.push<uint32_t>(div_up(coded[j].count, cbs));
-        o_words[j] = s.push<uint32_t>(coded[j].nwords + 2);
-        wave_base[j] = nwaves;
-        nwaves += div_up(div_up(coded[j].count, cbs), 64);
+    // ---- the upload and the arena ----------------------------------------------------------------
+    uint32_t nlong = 0, nshort = 0, nchunks = 0;
+    uint64_t total_syms = 0, arena = 0;
+    for (DecSeq& s : seqs) {
+        const uint32_t nblk = div_up(s.count, cbs);
+        (dec_long(nblk) ? nlong : nshort) += dec_entries(nblk);
+        s.boff_off = arena;
+        s.lut_off = arena + align_up(std::max<uint32_t>(nblk, 1), 16);
+        arena = s.lut_off + align_up((1u << kDecLutBits) + (uint64_t)s.nsym + 1, 16);
     }
-    size_t o_desc = s.push<HuffDecStream>(nc);
-    size_t o_wmap = s.push<uint32_t>(nwaves);
-    uint32_t ntiles = 0;
-    std::vector<uint32_t> tile_base(ns);
-    for (uint32_t i = 0; i < ns && rl; i++) {
-        tile_base[i] = ntiles;
-        ntiles += div_up(m[i], kRleTile);
-    }
-    size_t o_rdesc = s.push<RleDecStream>(rl ? ns : 0);
-    size_t o_tmap = s.push<uint32_t>(ntiles);
+    for (uint32_t i = 0; i < ns; i++) total_syms += items[i].n;
+    Staging s;
+    const size_t o_state = s.push<CoderState>(1), o_seq = s.push<DecSeq>(nseq), o_item = s.push<DecItem>(ns);
+    const size_t o_wseq = s.push<uint32_t>(nlong + nshort), o_wfirst = s.push<uint32_t>(nlong + nshort);
+    const size_t o_ifirst = s.push<uint32_t>(ns + 1);
+    std::vector<size_t> o_words(nbs, 0);
+    for (uint32_t b = 0; b < nbs; b++)
+        if (w1[b] > w0[b]) o_words[b] = s.push<uint32_t>(w1[b] - w0[b]);
     const size_t total = s.off;
-
     const int slot = I->dec_slot;
     I->dec_slot = (I->dec_slot + 1) % kDecodeRing;
     CCA_HIP(hipEventSynchronize(I->dec_event[slot]));  // previous upload from this slot done
     unsigned char* h = (unsigned char*)I->h_dec_stage[slot].get(total);
     unsigned char* d = (unsigned char*)I->d_dec_stage.get(total);
-    const uint64_t cap = align_up(std::max<uint32_t>(n, 1), 64);
-    unsigned char* dsym = rl ? (unsigned char*)I->d_dec_sym.get(cap * ns * symSize) : nullptr;
-    unsigned char* dzc = rl ? (unsigned char*)I->d_dec_zc.get(cap * ns * symSize) : nullptr;
+    unsigned char* dsym = (unsigned char*)I->d_dec_sym.get(std::max<uint64_t>(rl_elems, 1) * symSize);
+    unsigned char* dzc = (unsigned char*)I->d_dec_zc.get(std::max<uint64_t>(rl_elems, 1) * symSize);
 
-    HuffDecStream* hd = (HuffDecStream*)(h + o_desc);
-    uint32_t* hwm = (uint32_t*)(h + o_wmap);
-    for (uint32_t j = 0; j < nc; j++) {
-        const Coded& c = coded[j];
-        int32_t* tab = (int32_t*)(h + o_tab[j]);
-        memcpy(tab, c.t.first, 128);
-        memcpy(tab + 32, c.t.mn, 128);
-        memcpy(tab + 64, c.t.mx, 128);
-        if (symSize == 2) {
-            uint16_t* sy = (uint16_t*)(h + o_sym[j]);
-            for (size_t k = 0; k < c.t.symbols.size(); k++) sy[k] = (uint16_t)c.t.symbols[k];
-        } else {
-            memcpy(h + o_sym[j], c.t.symbols.data(), 4 * c.t.symbols.size());
-        }
-        uint32_t* off = (uint32_t*)(h + o_off[j]);
-        const uint32_t noff = div_up(c.count, cbs);
-        uint32_t acc = 0;
-        for (uint32_t b = 0; b < noff; b++) {  // unpackInc16CPU, PackInc.cu:222-229
-            acc += c.incs[b];
-            off[b] = acc;
-            CCA_REQUIRE(acc <= 32ull * c.nwords, CC_ERR_CORRUPT_STREAM, "coding block offset beyond the codewords");
-        }
-        uint32_t* wd = (uint32_t*)(h + o_words[j]);
-        memcpy(wd, c.words, 4ull * c.nwords);
-        wd[c.nwords] = 0;
-        wd[c.nwords + 1] = 0;
-        void* out;
-        if (rl) out = (j % 2 == 0 ? dsym : dzc) + cap * (j / 2) * symSize;
-        else out = outs[j];
-        CCA_REQUIRE(out != nullptr || c.count == 0, CC_ERR_INVALID_ARG, "null output stream");
-        hd[j] = HuffDecStream{(const uint32_t*)(d + o_words[j]), (const uint32_t*)(d + o_off[j]),
-                              (const int32_t*)(d + o_tab[j]), d + o_sym[j], out, c.count,
-                              (uint32_t)c.t.symbols.size(), wave_base[j], c.nwords};
-        for (uint32_t w = 0; w < div_up(div_up(c.count, cbs), 64); w++) hwm[wave_base[j] + w] = j;
+    *(CoderState*)(h + o_state) = CoderState{};
+    uint32_t* hws = (uint32_t*)(h + o_wseq);
+    uint32_t* hwf = (uint32_t*)(h + o_wfirst);
+    uint32_t* hif = (uint32_t*)(h + o_ifirst);
+    uint32_t wl = 0, ws = nlong;
+    for (uint32_t j = 0; j < nseq; j++) {
+        DecSeq& q = seqs[j];
+        const uint32_t b = seq_bs[j], i = q.item;
+        q.base = (const uint32_t*)(d + o_words[b]);
+        q.nwords = w1[b] - w0[b];
+        q.hdr_bit -= 32 * w0[b];
+        q.sym_bit -= 32 * w0[b];
+        q.words_off -= w0[b];
+        q.incs_off -= w0[b];
+        q.out = !items[i].rl ? items[i].out : (j == items[i].seq ? dsym : dzc) + rl_off[i] * symSize;
+        add_block_entries(j, div_up(q.count, cbs), hws, hwf, wl, ws);
     }
-    if (rl) {
-        RleDecStream* rd = (RleDecStream*)(h + o_rdesc);
-        uint32_t* tm = (uint32_t*)(h + o_tmap);
-        for (uint32_t i = 0; i < ns; i++) {
-            rd[i] = RleDecStream{dsym + cap * i * symSize, dzc + cap * i * symSize, outs[i], m[i], n, tile_base[i], 0};
-            for (uint32_t t = 0; t < div_up(m[i], kRleTile); t++) tm[tile_base[i] + t] = i;
-        }
-        for (uint32_t i = 0; i < ns; i++) CCA_REQUIRE(outs[i] != nullptr || n == 0, CC_ERR_INVALID_ARG, "null output stream");
+    for (uint32_t i = 0; i < ns; i++) {  // an RLE stream without a pair still has its output cleared
+        hif[i] = nchunks;
+        if (items[i].rl && items[i].n) nchunks += std::max(1u, rle_chunks(seqs[items[i].seq].count, true));
     }
+    hif[ns] = nchunks;
+    memcpy(h + o_seq, seqs.data(), sizeof(DecSeq) * nseq);
+    memcpy(h + o_item, items.data(), sizeof(DecItem) * ns);
+    for (uint32_t b = 0; b < nbs; b++)
+        if (w1[b] > w0[b]) memcpy(h + o_words[b], bsWords[b] + w0[b], 4 * (w1[b] - w0[b]));
+    uint32_t* scratch = I->d_dec_arena.as<uint32_t>(arena + std::max<uint32_t>(nchunks, 1));
     CCA_HIP(hipMemcpyAsync(d, h, total, hipMemcpyHostToDevice, st));
     CCA_HIP(hipEventRecord(I->dec_event[slot], st));
-    uint64_t total_syms = 0, total_bits = 0, total_pairs = 0;
-    for (uint32_t j = 0; j < nc; j++) {
-        total_syms += coded[j].count;
-        total_bits += 32ull * coded[j].nwords;
-    }
-    for (uint32_t i = 0; i < ns && rl; i++) total_pairs += m[i];
+
     stage("Decode: Huffman Decode");
-    huffman_decode((const HuffDecStream*)(d + o_desc), nc, (const uint32_t*)(d + o_wmap), nwaves, cbs, symSize,
-                   total_syms, total_bits, st);
-    if (rl) {
+    const RleChunks rc{(const uint32_t*)(d + o_ifirst), nchunks, scratch + arena};
+    const CoderParams p = params_of(I);
+    coder_decode_parsed((DecSeq*)(d + o_seq), nseq, p, symSize, scratch, (CoderState*)(d + o_state),
+                        (const DecItem*)(d + o_item), (const uint32_t*)(d + o_wseq), (const uint32_t*)(d + o_wfirst),
+                        nlong + nshort, nlong, total_syms, rc, st);
+    if (nchunks) {
         stage("Decode: Run Length Decode");
-        uint32_t* sums = I->d_dec_sums.as<uint32_t>(std::max<uint32_t>(ntiles, 1));
-        rle_decode((const RleDecStream*)(d + o_rdesc), ns, sums, ntiles, (const uint32_t*)(d + o_tmap), n, symSize,
-                   total_pairs, (uint64_t)n * ns, st);
+        coder_decode_expand((const DecItem*)(d + o_item), ns, (DecSeq*)(d + o_seq), symSize, rc,
+                            (CoderState*)(d + o_state), total_syms, st);
     }
+}
+
+void decode_streams(cc_instance* I, bool rl, int symSize, const uint32_t* const* bsWords, const uint64_t* bsBits,
+                    uint64_t* bsPos, uint32_t nbs, const uint32_t* s2b, void* const* outs, uint32_t ns, uint32_t n) {
+    check_symbols(I, symSize);
+    CCA_REQUIRE(ns == 0 || outs != nullptr, CC_ERR_INVALID_ARG, "null output array");
+    std::vector<DecodeStream> s(ns);
+    for (uint32_t i = 0; i < ns; i++) s[i] = DecodeStream{outs[i], n, rl, s2b ? s2b[i] : 0u};
+    SectionTimer call(I, 1);
+    if (ns) call(rl ? "Decode RLHuff" : "Decode Huff");
+    decode_items(I, symSize, bsWords, bsBits, bsPos, nbs, s);
 }
 
 }  // namespace cca

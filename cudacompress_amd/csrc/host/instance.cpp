@@ -110,12 +110,10 @@ cc_instance::~cc_instance() {
     cca::profile_owner_forget(this);  // its kernel timing vote and records
     for (auto& e : dec_event)
         if (e) (void)hipEventDestroy(e);
-    cca::DevBuf* devs[] = {&d_rle_sym, &d_rle_zc, &d_desc, &d_tiles, &d_map, &d_map2, &d_results, &d_hist,
-                           &d_tables, &d_words, &d_offsets, &d_block_bits, &d_stream_bits, &d_dec_stage,
-                           &d_dec_sym, &d_dec_zc, &d_dec_sums, &d_dec_desc, &d_vol[0], &d_vol[1], &d_vol[2],
-                           &d_vol[3], &d_vol_ptrs};
+    cca::DevBuf* devs[] = {&d_enc, &d_words, &d_dec_stage, &d_dec_sym, &d_dec_zc, &d_dec_arena,
+                           &d_vol[0], &d_vol[1], &d_vol[2], &d_vol[3], &d_vol_ptrs};
     for (auto* b : devs) b->release();
-    cca::PinBuf* pins[] = {&h_up, &h_down, &h_hist, &h_words, &h_vol_ptrs};
+    cca::PinBuf* pins[] = {&h_up, &h_down, &h_words, &h_vol_ptrs};
     for (auto* b : pins) b->release();
     for (auto& b : h_dec_stage) b.release();
     coder.release();

@@ -86,16 +86,16 @@ struct cc_instance {
     hipStream_t stream = nullptr;
     int dialect = CC_DIALECT_GPU;
 
-    // encode scratch
-    cca::DevBuf d_rle_sym, d_rle_zc;            // compacted streams, [stream][elem capacity]
-    cca::DevBuf d_desc, d_tiles, d_map, d_map2, d_results;
-    cca::DevBuf d_hist, d_tables, d_words, d_offsets, d_block_bits, d_stream_bits;
-    cca::PinBuf h_up, h_down, h_hist, h_words;
-    std::vector<uint32_t> out_words;
+    // encode scratch (host/codec.cpp): state, sequence records and arena; the words
+    cca::DevBuf d_enc, d_words;
+    cca::PinBuf h_up, h_down, h_words;
+    uint64_t enc_arena = 0, enc_down = 0;  // arena words allocated, and brought down with the records
+    const uint32_t* out_words = nullptr;   // the last encode's words (in h_words)
+    uint64_t out_count = 0;
     std::vector<uint64_t> seg_begin, seg_bits;
 
     // decode scratch
-    cca::DevBuf d_dec_stage, d_dec_sym, d_dec_zc, d_dec_sums, d_dec_desc;
+    cca::DevBuf d_dec_stage, d_dec_sym, d_dec_zc, d_dec_arena;
     cca::PinBuf h_dec_stage[cca::kDecodeRing];
     hipEvent_t dec_event[cca::kDecodeRing] = {};
     int dec_slot = 0;
@@ -104,7 +104,6 @@ struct cc_instance {
     cca::DevBuf d_vol[4];
     cca::DevBuf d_vol_ptrs;
     cca::PinBuf h_vol_ptrs;
-    std::vector<uint32_t> vol_bits;
 
     // device-resident coder
     cca::DeviceCoder coder;

@@ -7,6 +7,8 @@
 // layout of src/examples/CompressHeightfield.cpp:116-126.
 //
 // Differences from the reference callers, none of which changes the bitstream:
+//  * the transforms come first and every level's streams are coded in one go (the reference codes
+//    level by level, each with its synchronisations); a 9/7 volume is transformed as a brick of one;
 //  * every kernel runs on the instance stream (the reference quantizes on the default stream);
 //  * decode outputs are not cleared first (decodeRLHuff here writes every element);
 //  * 2D lossless input (sizeZ == 1) uses 3 highpass bands per level -- compressVolumeLossless
@@ -21,16 +23,11 @@
 #include <cstring>
 
 #include "../kernels.hpp"
+#include "bricks.hpp"
 #include "codec.hpp"
 
 namespace cca {
 namespace {
-
-void append_segments(cc_instance* I, std::vector<uint32_t>& bits) {
-    // every encode call here starts on a word boundary, so segments concatenate as words
-    if (I->out_words.empty()) return;
-    bits.insert(bits.end(), I->out_words.begin(), I->out_words.end());
-}
 
 struct Band {
     uint32_t x, y, z;
@@ -40,25 +37,57 @@ Band band_of(uint32_t block, bool is3d) {  // CompressVolume.cpp:375-379, Compre
     return Band{block % 2, block / 2, 0};
 }
 
-}  // namespace
+// Symbol streams of a 3D volume in bitstream order: the lowpass band, then 7 bands a level from the
+// coarsest, stream k from element at[k] of the symbol buffer on.
+struct VolumeStreams {
+    std::vector<uint64_t> at;
+    std::vector<uint32_t> n, call;
+    std::vector<bool> rl;
+    uint64_t elems = 0;
+    VolumeStreams(uint64_t volume, uint32_t levels, bool rle_only_lvl0) {
+        auto add = [&](uint64_t count, bool zero_runs, uint32_t c) {
+            at.push_back(elems);
+            n.push_back((uint32_t)count);
+            rl.push_back(zero_runs);
+            call.push_back(c);
+            elems += align_up(count, 64);
+        };
+        add(volume >> (3 * levels), false, 0);
+        for (uint32_t level = levels; level-- > 0;)
+            for (uint32_t b = 1; b <= 7; b++) add(volume >> (3 * (level + 1)), !(level > 0 && rle_only_lvl0), levels - level);
+    }
+    // stream of band b (1..7) of `level`, and the lowpass one
+    uint32_t band(uint32_t levels, uint32_t level, uint32_t b) const { return 1 + 7 * (levels - 1 - level) + b - 1; }
+};
 
-void compress_volume_float(cc_instance* I, const float* image, uint32_t sx, uint32_t sy, uint32_t sz,
-                           uint32_t levels, float q0, bool rle_only_lvl0, int symSize) {
-    DeviceGuard guard(I->device);
-    hipStream_t st = I->stream;
-    CCA_REQUIRE(levels >= 1, CC_ERR_INVALID_ARG, "numLevels must be >= 1");
-    CCA_REQUIRE(sz > 1, CC_ERR_INVALID_ARG, "compressVolumeFloat is 3D");
+void check_volume(uint32_t sx, uint32_t sy, uint32_t sz, uint32_t levels) {
+    CCA_REQUIRE(levels >= 1 && levels < 32, CC_ERR_INVALID_ARG, "numLevels must be >= 1");
+    CCA_REQUIRE(sz > 1, CC_ERR_INVALID_ARG, "the volume codecs for floats are 3D");
     const uint32_t f_all = 1u << levels;
     CCA_REQUIRE(sx % f_all == 0 && sy % f_all == 0 && sz % f_all == 0, CC_ERR_INVALID_ARG,
                 "sizes must be divisible by 2^numLevels");
-    const uint64_t elems = (uint64_t)sx * sy * sz;
-    const uint32_t nb = 7;
-    float* dwt[2] = {I->d_vol[0].as<float>(elems), I->d_vol[1].as<float>(elems)};
-    const uint64_t per_block_max = elems / 8;
-    unsigned char* sym = (unsigned char*)I->d_vol[2].get(nb * per_block_max * symSize);
-    std::vector<const void*> streams(nb);
-    for (uint32_t i = 0; i < nb; i++) streams[i] = sym + i * per_block_max * symSize;
+}
 
+// The volume as a brick of one: its levels' transforms with the quantizer fused, the streams in
+// bitstream order (of channel `bs` when decoding).
+std::vector<ItemSpec> volume_bricks(cc_instance* I, BrickJob& job, const std::vector<cc_brick>& bricks, uint32_t levels,
+                                    int symSize, bool rle_only_lvl0) {
+    job.bricks = bricks;
+    job.L = levels;
+    job.symSize = symSize;
+    std::vector<ItemSpec> items = bricks_transforms_prepare(I, I->batch, job, I->stream);
+    for (size_t k = 0; k < items.size(); k++)  // streams 1 .. 7 (levels - 1) of a brick: levels above 0
+        if (rle_only_lvl0 && k % (1 + 7 * levels) <= 7 * (levels - 1)) items[k].rl = false;
+    return items;
+}
+
+// Volumes too large for 32-bit element offsets: pitched levels in two buffers.
+void compress_volume_float_large(cc_instance* I, const float* image, uint32_t sx, uint32_t sy, uint32_t sz,
+                                 uint32_t levels, float q0, const VolumeStreams& vs, int symSize) {
+    hipStream_t st = I->stream;
+    const uint64_t elems = (uint64_t)sx * sy * sz;
+    float* dwt[2] = {I->d_vol[0].as<float>(elems), I->d_vol[1].as<float>(elems)};
+    unsigned char* sym = (unsigned char*)I->d_vol[2].get(vs.elems * symSize);
     int d = 0;
     dwt97_forward(dwt[d], dwt[1 - d], dwt[d], image, (int)sx, (int)sy, (int)sz, 1, 0, 0, 0, 0, st);
     uint32_t f = 2;
@@ -68,64 +97,38 @@ void compress_volume_float(cc_instance* I, const float* image, uint32_t sx, uint
         d = 1 - d;
         f *= 2;
     }
-    std::vector<uint32_t>& bits = I->vol_bits;
-    bits.clear();
-    // lowpass band (CompressVolume.cpp:353-362)
-    float q = q0 / float(f / 2);
-    quantize_to_symbols(sym, symSize, dwt[d], false, sx / f, sy / f, sz / f, q, sx, sx * sy, 0, st);
-    encode_streams(I, false, symSize, streams.data(), 1, (uint32_t)(elems / ((uint64_t)f * f * f)), nullptr);
-    append_segments(I, bits);
-    // highpass bands, coarsest level first (CompressVolume.cpp:365-402)
-    for (int level = (int)levels - 1; level >= 0; level--) {
-        q = q0 / float(f / 2);
+    // lowpass band (CompressVolume.cpp:353-362), highpass bands, coarsest level first (:365-402)
+    quantize_to_symbols(sym, symSize, dwt[d], false, sx / f, sy / f, sz / f, q0 / float(f / 2), sx, sx * sy, 0, st);
+    for (uint32_t level = levels; level-- > 0; f /= 2, d = 1 - d) {
         const uint32_t bx = sx / f, by = sy / f, bz = sz / f;
-        for (uint32_t b = 1; b <= nb; b++) {
-            Band bd = band_of(b, true);
-            uint64_t off = bd.x * bx + (uint64_t)bd.y * by * sx + (uint64_t)bd.z * bz * sx * sy;
-            quantize_to_symbols(sym + (b - 1) * per_block_max * symSize, symSize, dwt[d] + off, false, bx, by, bz, q,
-                                sx, sx * sy, 0, st);
+        for (uint32_t b = 1; b <= 7; b++) {
+            const Band bd = band_of(b, true);
+            const uint64_t off = bd.x * bx + (uint64_t)bd.y * by * sx + (uint64_t)bd.z * bz * sx * sy;
+            quantize_to_symbols(sym + vs.at[vs.band(levels, level, b)] * symSize, symSize, dwt[d] + off, false, bx, by,
+                                bz, q0 / float(f / 2), sx, sx * sy, 0, st);
         }
-        d = 1 - d;
-        const uint32_t count = bx * by * bz;
-        encode_streams(I, !(level > 0 && rle_only_lvl0), symSize, streams.data(), nb, count, nullptr);
-        append_segments(I, bits);
-        f /= 2;
     }
+    std::vector<EncodeStream> streams;
+    for (size_t k = 0; k < vs.n.size(); k++)
+        streams.push_back(EncodeStream{sym + vs.at[k] * symSize, vs.n[k], vs.rl[k], vs.call[k], 0});
+    encode_items(I, symSize, streams, levels + 1);
 }
 
-void decompress_volume_float(cc_instance* I, float* image, uint32_t sx, uint32_t sy, uint32_t sz, uint32_t levels,
-                             const uint32_t* words, uint64_t nbits, float q0, bool rle_only_lvl0, int symSize) {
-    DeviceGuard guard(I->device);
+void decompress_volume_float_large(cc_instance* I, float* image, const void* sym, const VolumeStreams& vs, uint32_t sx,
+                                   uint32_t sy, uint32_t sz, uint32_t levels, float q0, int symSize) {
     hipStream_t st = I->stream;
-    CCA_REQUIRE(levels >= 1 && sz > 1, CC_ERR_INVALID_ARG, "bad volume parameters");
-    const uint32_t f_all = 1u << levels;
-    CCA_REQUIRE(sx % f_all == 0 && sy % f_all == 0 && sz % f_all == 0, CC_ERR_INVALID_ARG,
-                "sizes must be divisible by 2^numLevels");
     const uint64_t elems = (uint64_t)sx * sy * sz;
-    const uint32_t nb = 7;
     float* dwt[2] = {I->d_vol[0].as<float>(elems), I->d_vol[1].as<float>(elems)};
-    const uint64_t per_block_max = elems / 8;
-    unsigned char* sym = (unsigned char*)I->d_vol[2].get(nb * per_block_max * symSize);
-    std::vector<void*> streams(nb);
-    for (uint32_t i = 0; i < nb; i++) streams[i] = sym + i * per_block_max * symSize;
-    // device table of the 7 band pointers for the fused dequantize+IDWT
-    void** hptr = I->h_vol_ptrs.as<void*>(nb);
-    for (uint32_t i = 0; i < nb; i++) hptr[i] = streams[i];
-    void** dptr = I->d_vol_ptrs.as<void*>(nb);
-    CCA_HIP(hipMemcpyAsync(dptr, hptr, sizeof(void*) * nb, hipMemcpyHostToDevice, st));
-
-    uint64_t pos = 0;
-    uint32_t f = f_all;
-    // lowpass (CompressVolume.cpp:466-475)
-    const uint32_t nlp = (uint32_t)(elems / ((uint64_t)f * f * f));
-    decode_streams(I, false, symSize, &words, &nbits, &pos, 1, nullptr, streams.data(), 1, nlp);
+    // device table of every level's 7 band pointers for the fused dequantize + IDWT
+    const void** hptr = I->h_vol_ptrs.as<const void*>(7 * levels);
+    for (uint32_t k = 0; k < 7 * levels; k++) hptr[k] = (const unsigned char*)sym + vs.at[1 + k] * symSize;
+    const void** dptr = I->d_vol_ptrs.as<const void*>(7 * levels);
+    CCA_HIP(hipMemcpyAsync(dptr, hptr, sizeof(void*) * 7 * levels, hipMemcpyHostToDevice, st));
+    uint32_t f = 1u << levels;
     unquantize_from_symbols(image, sym, symSize, sx / f, sy / f, sz / f, q0 / float(f / 2), sx, sx * sy, 0, st);
-    for (int level = (int)levels - 1; level >= 0; level--) {
-        const uint32_t count = (sx / f) * (sy / f) * (sz / f);
-        decode_streams(I, !(level > 0 && rle_only_lvl0), symSize, &words, &nbits, &pos, 1, nullptr, streams.data(), nb,
-                       count);
+    for (uint32_t level = levels; level-- > 0;) {
         f /= 2;
-        dwt97_inverse_from_symbols(image, dwt[1], dwt[0], image, (const void* const*)dptr, symSize, q0 / float(f),
+        dwt97_inverse_from_symbols(image, dwt[1], dwt[0], image, dptr + 7 * (levels - 1 - level), symSize, q0 / float(f),
                                    (int)(sx / f), (int)(sy / f), (int)(sz / f), 1, (int)sx, (int)(sx * sy), (int)sx,
                                    (int)(sx * sy), st);
     }
@@ -133,118 +136,136 @@ void decompress_volume_float(cc_instance* I, float* image, uint32_t sx, uint32_t
     CCA_HIP(hipStreamSynchronize(st));
 }
 
-namespace {
-
-void copy3d(int16_t* dst, uint64_t dRow, uint64_t dSlice, const int16_t* src, uint64_t sRow, uint64_t sSlice,
-            uint32_t w, uint32_t h, uint32_t dpt, hipStream_t st) {
-    for (uint32_t z = 0; z < dpt; z++)
-        CCA_HIP(hipMemcpy2DAsync(dst + z * dSlice, dRow * 2, src + z * sSlice, sRow * 2, (size_t)w * 2, h,
-                                 hipMemcpyDeviceToDevice, st));
-}
-
-// compressVolumeLosslessOneLevel, CompressVolume.cpp:84-150 (3D) / compressHeightfieldOneLevel's
-// band layout (2D)
-void lossless_one_level(cc_instance* I, const int16_t* src, uint32_t sx, uint32_t sy, uint32_t sz, int16_t* lowpass,
-                        std::vector<uint32_t>& out) {
-    hipStream_t st = I->stream;
-    const bool is3d = sz > 1;
-    const uint32_t nb = is3d ? 7 : 3;
-    const uint32_t bx = sx / 2, by = sy / 2, bz = is3d ? sz / 2 : 1;
-    const uint64_t elems = (uint64_t)sx * sy * sz;
-    const uint64_t per_block = (uint64_t)bx * by * bz;
-    int16_t* dwt0 = I->d_vol[0].as<int16_t>(elems);
-    int16_t* dwt1 = I->d_vol[1].as<int16_t>(elems);
-    uint16_t* sym = I->d_vol[2].as<uint16_t>(nb * per_block);
-    dwt53_forward(dwt1, dwt0, src, (int)sx, (int)sy, (int)sz, 0, 0, 0, 0, st);
-    copy3d(lowpass, bx, (uint64_t)bx * by, dwt1, sx, (uint64_t)sx * sy, bx, by, bz, st);
-    std::vector<const void*> streams(nb);
-    for (uint32_t b = 1; b <= nb; b++) {
-        Band bd = band_of(b, is3d);
-        uint64_t off = bd.x * bx + (uint64_t)bd.y * by * sx + (uint64_t)bd.z * bz * sx * sy;
-        streams[b - 1] = sym + (b - 1) * per_block;
-        symbolize(sym + (b - 1) * per_block, dwt1 + off, bx, by, bz, sx, sx * sy, st);
-    }
-    encode_streams(I, true, 2, streams.data(), nb, (uint32_t)per_block, nullptr);
-    out.assign(I->out_words.begin(), I->out_words.end());
-}
-
 }  // namespace
 
+void compress_volume_float(cc_instance* I, const float* image, uint32_t sx, uint32_t sy, uint32_t sz,
+                           uint32_t levels, float q0, bool rle_only_lvl0, int symSize) {
+    DeviceGuard guard(I->device);
+    check_volume(sx, sy, sz, levels);
+    CCA_REQUIRE(image, CC_ERR_INVALID_ARG, "null volume");
+    check_symbols(I, symSize);
+    const uint64_t elems = (uint64_t)sx * sy * sz;
+    SectionTimer call(I, 1);
+    if (!bricks_serve(elems, levels)) {
+        call("Encode RLHuff");
+        compress_volume_float_large(I, image, sx, sy, sz, levels, q0, VolumeStreams(elems, levels, rle_only_lvl0), symSize);
+        return;
+    }
+    BrickJob job;
+    const std::vector<ItemSpec> items =
+        volume_bricks(I, job, {cc_brick{image, nullptr, sx, sy, sz, q0}}, levels, symSize, rle_only_lvl0);
+    bricks_forward_launch(job, I->stream);
+    call("Encode RLHuff");
+    std::vector<EncodeStream> streams;
+    for (size_t k = 0; k < items.size(); k++)  // (the lowpass call, then one a level)
+        streams.push_back(EncodeStream{items[k].ptr, items[k].n, items[k].rl, k ? 1 + ((uint32_t)k - 1) / 7 : 0u, 0});
+    encode_items(I, symSize, streams, levels + 1);
+}
+
+void decompress_volume_float(cc_instance* I, float* image, uint32_t sx, uint32_t sy, uint32_t sz, uint32_t levels,
+                             const uint32_t* words, uint64_t nbits, float q0, bool rle_only_lvl0, int symSize) {
+    const VolumeChannelIn ch{image, words, nbits, q0};
+    decompress_volume_float_multichannel(I, &ch, 1, sx, sy, sz, levels, rle_only_lvl0, symSize);
+}
+
+namespace {
+// Streams of a lossless field: the lowpass band, then 3 (2D) or 7 (3D) bands a level from the coarsest;
+// a level's bands lie one after the other, from element at[level] of the symbol buffer on.
+struct LosslessLayout {
+    uint32_t nb, levels;
+    std::vector<uint64_t> at, per_band, low;  // per level: first band, elements of a band, its lowpass in the low buffer
+    uint64_t sym_elems = 0, low_elems = 0;
+    LosslessLayout(uint32_t sx, uint32_t sy, uint32_t sz, uint32_t levels_) : nb(sz > 1 ? 7 : 3), levels(levels_) {
+        at.resize(levels);
+        per_band.resize(levels);
+        low.resize(levels);
+        for (uint32_t l = 0; l < levels; l++) {
+            const uint32_t f = 2u << l;
+            per_band[l] = (uint64_t)(sx / f) * (sy / f) * (sz > 1 ? sz / f : 1);
+            low[l] = low_elems;
+            low_elems += align_up(per_band[l], 64);
+        }
+        sym_elems = align_up(per_band[levels - 1], 64);
+        for (uint32_t l = levels; l-- > 0;) {
+            at[l] = sym_elems;
+            sym_elems += nb * align_up(per_band[l], 64);
+        }
+    }
+    uint64_t stride(uint32_t level) const { return align_up(per_band[level], 64); }
+    // f(symbol offset, count, zero runs, call) for every stream in bitstream order
+    template <class F>
+    void streams(F f) const {
+        f(0, (uint32_t)per_band[levels - 1], false, 0u);
+        for (uint32_t l = levels; l-- > 0;)
+            for (uint32_t b = 0; b < nb; b++) f(at[l] + b * stride(l), (uint32_t)per_band[l], true, levels - l);
+    }
+};
+void check_lossless(cc_instance* I, uint32_t sx, uint32_t sy, uint32_t sz, uint32_t levels) {
+    CCA_REQUIRE(I->log2 <= 16, CC_ERR_INVALID_ARG, "lossless volumes use Symbol16 (log2 <= 16)");
+    CCA_REQUIRE(levels >= 1 && levels < 32, CC_ERR_INVALID_ARG, "numLevels must be >= 1");
+    const uint32_t f_all = 1u << levels;
+    CCA_REQUIRE(sx % f_all == 0 && sy % f_all == 0 && (sz <= 1 || sz % f_all == 0), CC_ERR_INVALID_ARG,
+                "sizes must be divisible by 2^numLevels");
+}
+}  // namespace
+
+// compressVolumeLosslessOneLevel per level, CompressVolume.cpp:84-150 (3D) / compressHeightfieldOneLevel's
+// band layout (2D)
 void compress_volume_lossless(cc_instance* I, const int16_t* image, uint32_t sx, uint32_t sy, uint32_t sz,
                               uint32_t levels) {
     DeviceGuard guard(I->device);
     hipStream_t st = I->stream;
-    CCA_REQUIRE(I->log2 <= 16, CC_ERR_INVALID_ARG, "lossless volumes use Symbol16 (log2 <= 16)");
-    CCA_REQUIRE(levels >= 1, CC_ERR_INVALID_ARG, "numLevels must be >= 1");
+    check_lossless(I, sx, sy, sz, levels);
     const bool is3d = sz > 1;
-    const uint32_t f_all = 1u << levels;
-    CCA_REQUIRE(sx % f_all == 0 && sy % f_all == 0 && (!is3d || sz % f_all == 0), CC_ERR_INVALID_ARG,
-                "sizes must be divisible by 2^numLevels");
     const uint64_t elems = (uint64_t)sx * sy * sz;
-    int16_t* buf0 = I->d_vol[3].as<int16_t>(elems + elems / 4 + 64);
-    int16_t* buf1 = buf0 + align_up(elems, 64);  // lowpass of the current level (<= elems/4)
-    std::vector<std::vector<uint32_t>> level_bits(levels);
-    uint32_t f = 1;
+    const LosslessLayout lay(sx, sy, sz, levels);
+    int16_t* dwt0 = I->d_vol[0].as<int16_t>(elems);
+    int16_t* dwt1 = I->d_vol[1].as<int16_t>(elems);
+    uint16_t* sym = I->d_vol[2].as<uint16_t>(lay.sym_elems);
+    int16_t* low = I->d_vol[3].as<int16_t>(lay.low_elems);
     for (uint32_t level = 0; level < levels; level++) {
-        const int16_t* src = level == 0 ? image : buf0;
-        lossless_one_level(I, src, sx / f, sy / f, is3d ? sz / f : 1, buf1, level_bits[level]);
-        f *= 2;
-        const uint64_t lp = (uint64_t)(sx / f) * (sy / f) * (is3d ? sz / f : 1);
-        CCA_HIP(hipMemcpyAsync(buf0, buf1, lp * 2, hipMemcpyDeviceToDevice, st));
+        const uint32_t cx = sx >> level, cy = sy >> level, cz = is3d ? sz >> level : 1;
+        dwt53_forward(dwt1, dwt0, level == 0 ? image : low + lay.low[level - 1], (int)cx, (int)cy, (int)cz, 0, 0, 0, 0, st);
+        const bool last = level + 1 == levels;
+        symbolize_level(sym + lay.at[level], lay.stride(level), last ? sym : nullptr, last ? nullptr : low + lay.low[level],
+                        dwt1, cx, cy, cz, cx, (uint64_t)cx * cy, st);
     }
-    const uint32_t lx = sx / f, ly = sy / f, lz = is3d ? sz / f : 1;
-    uint16_t* lsym = (uint16_t*)buf1;
-    symbolize(lsym, buf0, lx, ly, lz, lx, lx * ly, st);
-    const void* s0 = lsym;
-    encode_streams(I, false, 2, &s0, 1, lx * ly * lz, nullptr);
-    std::vector<uint32_t>& bits = I->vol_bits;
-    bits.assign(I->out_words.begin(), I->out_words.end());
-    for (int level = (int)levels - 1; level >= 0; level--)
-        bits.insert(bits.end(), level_bits[level].begin(), level_bits[level].end());
+    std::vector<EncodeStream> streams;
+    lay.streams([&](uint64_t off, uint32_t n, bool rl, uint32_t call) {
+        streams.push_back(EncodeStream{sym + off, n, rl, call, 0});
+    });
+    SectionTimer call(I, 1);
+    call("Encode RLHuff");
+    encode_items(I, 2, streams, levels + 1, true);
 }
 
+// decompressVolumeLosslessOneLevel per level, CompressVolume.cpp:152-226
 void decompress_volume_lossless(cc_instance* I, int16_t* image, uint32_t sx, uint32_t sy, uint32_t sz,
                                 uint32_t levels, const uint32_t* words, uint64_t nbits) {
     DeviceGuard guard(I->device);
     hipStream_t st = I->stream;
-    CCA_REQUIRE(I->log2 <= 16, CC_ERR_INVALID_ARG, "lossless volumes use Symbol16 (log2 <= 16)");
-    CCA_REQUIRE(levels >= 1, CC_ERR_INVALID_ARG, "numLevels must be >= 1");
+    check_lossless(I, sx, sy, sz, levels);
     const bool is3d = sz > 1;
-    const uint32_t f_all = 1u << levels;
-    CCA_REQUIRE(sx % f_all == 0 && sy % f_all == 0 && (!is3d || sz % f_all == 0), CC_ERR_INVALID_ARG,
-                "sizes must be divisible by 2^numLevels");
     const uint64_t elems = (uint64_t)sx * sy * sz;
-    int16_t* buf0 = I->d_vol[3].as<int16_t>(elems + elems / 4 + 64);
-    int16_t* buf1 = buf0 + align_up(elems, 64);
-    uint32_t f = f_all;
-    uint32_t lx = sx / f, ly = sy / f, lz = is3d ? sz / f : 1;
+    const LosslessLayout lay(sx, sy, sz, levels);
+    int16_t* dwt0 = I->d_vol[0].as<int16_t>(elems);
+    int16_t* dwt1 = I->d_vol[1].as<int16_t>(elems);
+    uint16_t* sym = I->d_vol[2].as<uint16_t>(lay.sym_elems);
+    int16_t* low = I->d_vol[3].as<int16_t>(lay.low_elems);
+    std::vector<DecodeStream> streams;
+    lay.streams([&](uint64_t off, uint32_t n, bool rl, uint32_t) { streams.push_back(DecodeStream{sym + off, n, rl, 0}); });
     uint64_t pos = 0;
-    void* s0 = buf1;
-    decode_streams(I, false, 2, &words, &nbits, &pos, 1, nullptr, &s0, 1, lx * ly * lz);
-    unsymbolize(buf0, (const uint16_t*)buf1, lx, ly, lz, lx, lx * ly, st);
-    for (int level = (int)levels - 1; level >= 0; level--) {
-        const uint64_t lp = (uint64_t)(sx / f) * (sy / f) * (is3d ? sz / f : 1);
-        CCA_HIP(hipMemcpyAsync(buf1, buf0, lp * 2, hipMemcpyDeviceToDevice, st));
-        f /= 2;
-        int16_t* target = level == 0 ? image : buf0;
-        // decompressVolumeLosslessOneLevel, CompressVolume.cpp:152-226
-        const uint32_t cx = sx / f, cy = sy / f, cz = is3d ? sz / f : 1;
-        const uint32_t nb = is3d ? 7 : 3;
-        const uint32_t bx = cx / 2, by = cy / 2, bz = is3d ? cz / 2 : 1;
-        const uint64_t celems = (uint64_t)cx * cy * cz, per_block = (uint64_t)bx * by * bz;
-        int16_t* dwt0 = I->d_vol[0].as<int16_t>(celems);
-        int16_t* dwt1 = I->d_vol[1].as<int16_t>(celems);
-        uint16_t* sym = I->d_vol[2].as<uint16_t>(nb * per_block);
-        copy3d(dwt1, cx, (uint64_t)cx * cy, buf1, bx, (uint64_t)bx * by, bx, by, bz, st);
-        std::vector<void*> streams(nb);
-        for (uint32_t b = 0; b < nb; b++) streams[b] = sym + b * per_block;
-        decode_streams(I, true, 2, &words, &nbits, &pos, 1, nullptr, streams.data(), nb, (uint32_t)per_block);
-        for (uint32_t b = 1; b <= nb; b++) {
-            Band bd = band_of(b, is3d);
-            uint64_t off = bd.x * bx + (uint64_t)bd.y * by * cx + (uint64_t)bd.z * bz * cx * cy;
-            unsymbolize(dwt1 + off, sym + (b - 1) * per_block, bx, by, bz, cx, cx * cy, st);
-        }
-        dwt53_inverse(target, dwt0, dwt1, (int)cx, (int)cy, (int)cz, 0, 0, 0, 0, st);
+    {
+        SectionTimer call(I, 1);
+        call("Decode RLHuff");
+        decode_items(I, 2, &words, &nbits, &pos, 1, streams);
+    }
+    for (uint32_t level = levels; level-- > 0;) {
+        const uint32_t cx = sx >> level, cy = sy >> level, cz = is3d ? sz >> level : 1;
+        const bool last = level + 1 == levels;
+        unsymbolize_level(dwt1, sym + lay.at[level], lay.stride(level), last ? sym : nullptr,
+                          last ? nullptr : low + lay.low[level], cx, cy, cz, cx, (uint64_t)cx * cy, st);
+        dwt53_inverse(level == 0 ? image : low + lay.low[level - 1], dwt0, dwt1, (int)cx, (int)cy, (int)cz, 0, 0, 0, 0, st);
     }
 }
 
@@ -258,91 +279,35 @@ void compress_volume_float_quant_first(cc_instance* I, const float* image, uint3
     CCA_REQUIRE(sx % f_all == 0 && sy % f_all == 0 && sz % f_all == 0, CC_ERR_INVALID_ARG,
                 "sizes must be divisible by 2^numLevels");
     const uint64_t elems = (uint64_t)sx * sy * sz;
-    const uint32_t nb = 7;
+    const VolumeStreams vs(elems, levels, rle_only_lvl0);
     int16_t* dwt[2] = {I->d_vol[0].as<int16_t>(elems), I->d_vol[1].as<int16_t>(elems)};
-    const uint64_t per_block_max = elems / 8;
-    uint16_t* sym = I->d_vol[2].as<uint16_t>(nb * per_block_max);
-    std::vector<const void*> streams(nb);
-    for (uint32_t i = 0; i < nb; i++) streams[i] = sym + i * per_block_max;
+    uint16_t* sym = I->d_vol[2].as<uint16_t>(vs.elems);
     // uniform quantization of the whole volume (CompressVolume.cpp:685-687)
     quantize_to_short(dwt[0], image, sx, sy, sz, step, sx, sx * sy, 1, st);
-    // every 5/3 level: data path src -> dst -> buf -> dst with src and buf the same buffer, so the
-    // coarsest level's coefficients end in dwt[d], the next finer level's in dwt[1 - d], ...
-    int d = 0;
-    uint32_t f = 1;
+    // every 5/3 level: data path src -> dst -> buf -> dst with src and buf the same buffer, so level l's
+    // coefficients are in dwt[1 - l % 2]; its bands become symbols before the next level but one reuses it
     for (uint32_t level = 0; level < levels; level++) {
+        const uint32_t f = 1u << level;
+        const int d = (int)(level & 1);
         dwt53_forward(dwt[1 - d], dwt[d], dwt[d], (int)(sx / f), (int)(sy / f), (int)(sz / f), (int)sx, (int)(sx * sy),
                       (int)sx, (int)(sx * sy), st);
-        d = 1 - d;
-        f *= 2;
+        symbolize_level(sym + vs.at[vs.band(levels, level, 1)], align_up(vs.n[vs.band(levels, level, 1)], 64),
+                        level + 1 == levels ? sym : nullptr, nullptr, dwt[1 - d], sx / f, sy / f, sz / f, sx,
+                        (uint64_t)sx * sy, st);
     }
-    std::vector<uint32_t>& bits = I->vol_bits;
-    bits.clear();
-    // lowpass band (CompressVolume.cpp:704-712)
-    symbolize(sym, dwt[d], sx / f, sy / f, sz / f, sx, sx * sy, st);
-    encode_streams(I, false, 2, streams.data(), 1, (uint32_t)(elems / ((uint64_t)f * f * f)), nullptr);
-    append_segments(I, bits);
-    // highpass bands, coarsest level first (CompressVolume.cpp:715-749)
-    for (int level = (int)levels - 1; level >= 0; level--) {
-        const uint32_t bx = sx / f, by = sy / f, bz = sz / f;
-        for (uint32_t b = 1; b <= nb; b++) {
-            const Band bd = band_of(b, true);
-            const uint64_t off = bd.x * bx + (uint64_t)bd.y * by * sx + (uint64_t)bd.z * bz * sx * sy;
-            symbolize(sym + (b - 1) * per_block_max, dwt[d] + off, bx, by, bz, sx, sx * sy, st);
-        }
-        d = 1 - d;
-        encode_streams(I, !(level > 0 && rle_only_lvl0), 2, streams.data(), nb, bx * by * bz, nullptr);
-        append_segments(I, bits);
-        f /= 2;
-    }
+    std::vector<EncodeStream> streams;
+    for (size_t k = 0; k < vs.n.size(); k++)
+        streams.push_back(EncodeStream{sym + vs.at[k], vs.n[k], vs.rl[k], vs.call[k], 0});
+    SectionTimer call(I, 1);
+    call("Encode RLHuff");
+    encode_items(I, 2, streams, levels + 1);
 }
 
 void decompress_volume_float_quant_first(cc_instance* I, float* image, uint32_t sx, uint32_t sy, uint32_t sz,
                                          uint32_t levels, const uint32_t* words, uint64_t nbits, float step,
                                          bool rle_only_lvl0) {
-    DeviceGuard guard(I->device);
-    hipStream_t st = I->stream;
-    CCA_REQUIRE(I->log2 <= 16, CC_ERR_INVALID_ARG, "QuantFirst volumes use Symbol16 (log2 <= 16)");
-    CCA_REQUIRE(levels >= 1 && sz > 1, CC_ERR_INVALID_ARG, "QuantFirst volumes are 3D with numLevels >= 1");
-    const uint32_t f_all = 1u << levels;
-    CCA_REQUIRE(sx % f_all == 0 && sy % f_all == 0 && sz % f_all == 0, CC_ERR_INVALID_ARG,
-                "sizes must be divisible by 2^numLevels");
-    const uint64_t elems = (uint64_t)sx * sy * sz;
-    const uint32_t nb = 7;
-    int16_t* dwt[2] = {I->d_vol[0].as<int16_t>(elems), I->d_vol[1].as<int16_t>(elems)};
-    const uint64_t per_block_max = elems / 8;
-    uint16_t* sym = I->d_vol[2].as<uint16_t>(nb * per_block_max);
-    std::vector<void*> streams(nb);
-    for (uint32_t i = 0; i < nb; i++) streams[i] = sym + i * per_block_max;
-    uint64_t pos = 0;
-    uint32_t f = f_all;
-    // lowpass band into dwt[0] (CompressVolume.cpp:794-801)
-    decode_streams(I, false, 2, &words, &nbits, &pos, 1, nullptr, streams.data(), 1,
-                   (uint32_t)(elems / ((uint64_t)f * f * f)));
-    unsymbolize(dwt[0], sym, sx / f, sy / f, sz / f, sx, sx * sy, st);
-    // highpass bands, coarsest level first, alternating buffers from dwt[0] (:804-830)
-    int d = 0;
-    for (int level = (int)levels - 1; level >= 0; level--) {
-        const uint32_t bx = sx / f, by = sy / f, bz = sz / f;
-        decode_streams(I, !(level > 0 && rle_only_lvl0), 2, &words, &nbits, &pos, 1, nullptr, streams.data(), nb,
-                       bx * by * bz);
-        f /= 2;
-        for (uint32_t b = 1; b <= nb; b++) {
-            const Band bd = band_of(b, true);
-            const uint64_t off = bd.x * bx + (uint64_t)bd.y * by * sx + (uint64_t)bd.z * bz * sx * sy;
-            unsymbolize(dwt[d] + off, sym + (b - 1) * per_block_max, bx, by, bz, sx, sx * sy, st);
-        }
-        d = 1 - d;
-    }
-    // inverse levels from the coarsest, whose coefficients are in dwt[0] (:833-838)
-    d = 0;
-    for (int level = (int)levels - 1; level >= 0; level--) {
-        const uint32_t fl = 1u << level;
-        dwt53_inverse(dwt[1 - d], dwt[d], dwt[d], (int)(sx / fl), (int)(sy / fl), (int)(sz / fl), (int)sx,
-                      (int)(sx * sy), (int)sx, (int)(sx * sy), st);
-        d = 1 - d;
-    }
-    unquantize_from_short(image, dwt[d], sx, sy, sz, step, sx, sx * sy, 1, st);
+    const VolumeChannelIn ch{image, words, nbits, step};
+    decompress_volume_float_quant_first_multichannel(I, &ch, 1, sx, sy, sz, levels, rle_only_lvl0);
 }
 
 namespace {
@@ -350,27 +315,23 @@ namespace {
 void check_channels(cc_instance* I, const VolumeChannelIn* ch, uint32_t nch, uint32_t sx, uint32_t sy, uint32_t sz,
                     uint32_t levels) {
     CCA_REQUIRE(nch >= 1 && ch, CC_ERR_INVALID_ARG, "no channels");
-    CCA_REQUIRE(levels >= 1 && sz > 1, CC_ERR_INVALID_ARG, "bad volume parameters");
-    const uint32_t f_all = 1u << levels;
-    CCA_REQUIRE(sx % f_all == 0 && sy % f_all == 0 && sz % f_all == 0, CC_ERR_INVALID_ARG,
-                "sizes must be divisible by 2^numLevels");
+    check_volume(sx, sy, sz, levels);
     for (uint32_t c = 0; c < nch; c++)
         CCA_REQUIRE(ch[c].image && ch[c].words, CC_ERR_INVALID_ARG, "null channel buffer");
 }
 
-// Bitstream cursors of the channels; stream s of a call with `per` streams per channel reads
-// channel s / per.
+// Bitstream cursors of the channels.
 struct ChannelStreams {
     std::vector<const uint32_t*> words;
     std::vector<uint64_t> nbits, pos;
-    std::vector<uint32_t> s2b_lp, s2b_hp;
-    ChannelStreams(const VolumeChannelIn* ch, uint32_t nch, uint32_t per) : nbits(nch), pos(nch, 0) {
+    ChannelStreams(const VolumeChannelIn* ch, uint32_t nch) : nbits(nch), pos(nch, 0) {
         for (uint32_t c = 0; c < nch; c++) {
             words.push_back(ch[c].words);
             nbits[c] = ch[c].nbits;
-            s2b_lp.push_back(c);
-            for (uint32_t b = 0; b < per; b++) s2b_hp.push_back(c);
         }
+    }
+    void decode(cc_instance* I, int symSize, const std::vector<DecodeStream>& streams) {
+        decode_items(I, symSize, words.data(), nbits.data(), pos.data(), (uint32_t)words.size(), streams);
     }
 };
 
@@ -382,38 +343,38 @@ void decompress_volume_float_multichannel(cc_instance* I, const VolumeChannelIn*
     DeviceGuard guard(I->device);
     hipStream_t st = I->stream;
     check_channels(I, ch, nch, sx, sy, sz, levels);
+    check_symbols(I, symSize);
     const uint64_t elems = (uint64_t)sx * sy * sz;
-    const uint32_t nb = 7, ns = nb * nch;
-    float* dwt[2] = {I->d_vol[0].as<float>(elems), I->d_vol[1].as<float>(elems)};
-    const uint64_t per_block_max = elems / 8;
-    unsigned char* sym = (unsigned char*)I->d_vol[2].get((uint64_t)ns * per_block_max * symSize);
-    std::vector<void*> streams(ns);
-    for (uint32_t i = 0; i < ns; i++) streams[i] = sym + i * per_block_max * symSize;
-    // device table of every channel's 7 band pointers for the fused dequantize + IDWT
-    void** hptr = I->h_vol_ptrs.as<void*>(ns);
-    for (uint32_t i = 0; i < ns; i++) hptr[i] = streams[i];
-    void** dptr = I->d_vol_ptrs.as<void*>(ns);
-    CCA_HIP(hipMemcpyAsync(dptr, hptr, sizeof(void*) * ns, hipMemcpyHostToDevice, st));
-    ChannelStreams cs(ch, nch, nb);
-    uint32_t f = 1u << levels;
-    // every channel's lowpass band in one decode (CompressVolume.cpp:588-599)
-    decode_streams(I, false, symSize, cs.words.data(), cs.nbits.data(), cs.pos.data(), nch, cs.s2b_lp.data(),
-                   streams.data(), nch, (uint32_t)(elems / ((uint64_t)f * f * f)));
-    for (uint32_t c = 0; c < nch; c++)
-        unquantize_from_symbols(ch[c].image, streams[c], symSize, sx / f, sy / f, sz / f, ch[c].step / float(f / 2),
-                                sx, sx * sy, 0, st);
-    // per level every channel's 7 bands in one decode, then each channel's IDWT (:602-641)
-    for (int level = (int)levels - 1; level >= 0; level--) {
-        const uint32_t count = (sx / f) * (sy / f) * (sz / f);
-        decode_streams(I, !(level > 0 && rle_only_lvl0), symSize, cs.words.data(), cs.nbits.data(), cs.pos.data(), nch,
-                       cs.s2b_hp.data(), streams.data(), ns, count);
-        f /= 2;
+    SectionTimer call(I, 1);
+    call("Decode RLHuff");
+    ChannelStreams cs(ch, nch);
+    std::vector<DecodeStream> streams;
+    if (!bricks_serve(elems * nch, levels)) {
+        const VolumeStreams vs(elems, levels, rle_only_lvl0);
+        unsigned char* sym = (unsigned char*)I->d_vol[2].get(nch * vs.elems * symSize);
         for (uint32_t c = 0; c < nch; c++)
-            dwt97_inverse_from_symbols(ch[c].image, dwt[1], dwt[0], ch[c].image, (const void* const*)(dptr + nb * c),
-                                       symSize, ch[c].step / float(f), (int)(sx / f), (int)(sy / f), (int)(sz / f), 1,
-                                       (int)sx, (int)(sx * sy), (int)sx, (int)(sx * sy), st);
+            for (size_t k = 0; k < vs.n.size(); k++)
+                streams.push_back(DecodeStream{sym + (c * vs.elems + vs.at[k]) * symSize, vs.n[k], vs.rl[k], c});
+        cs.decode(I, symSize, streams);
+        for (uint32_t c = 0; c < nch; c++)
+            decompress_volume_float_large(I, ch[c].image, sym + c * vs.elems * symSize, vs, sx, sy, sz, levels, ch[c].step,
+                                          symSize);
+        return;
     }
-    // the pointer table upload must finish before the pinned copy is rewritten
+    // every channel is a brick of one batch
+    std::vector<cc_brick> bricks;
+    for (uint32_t c = 0; c < nch; c++) bricks.push_back(cc_brick{nullptr, ch[c].image, sx, sy, sz, ch[c].step});
+    BrickJob job;
+    for (const ItemSpec& it : volume_bricks(I, job, bricks, levels, symSize, rle_only_lvl0))
+        streams.push_back(DecodeStream{it.ptr, it.n, it.rl, it.call});
+    // the level tables' upload must finish before the pinned copy is rewritten
+    try {
+        cs.decode(I, symSize, streams);
+    } catch (...) {
+        (void)hipStreamSynchronize(st);
+        throw;
+    }
+    bricks_inverse_launch(job, st);
     CCA_HIP(hipStreamSynchronize(st));
 }
 
@@ -425,43 +386,30 @@ void decompress_volume_float_quant_first_multichannel(cc_instance* I, const Volu
     CCA_REQUIRE(I->log2 <= 16, CC_ERR_INVALID_ARG, "QuantFirst volumes use Symbol16 (log2 <= 16)");
     check_channels(I, ch, nch, sx, sy, sz, levels);
     const uint64_t elems = (uint64_t)sx * sy * sz;
-    const uint32_t nb = 7, ns = nb * nch;
-    // two coefficient buffers per channel (:880-883)
-    int16_t* b0 = I->d_vol[0].as<int16_t>(elems * nch);
-    int16_t* b1 = I->d_vol[1].as<int16_t>(elems * nch);
-    auto buf = [&](uint32_t c, int k) { return (k == 0 ? b0 : b1) + elems * c; };
-    const uint64_t per_block_max = elems / 8;
-    uint16_t* sym = I->d_vol[2].as<uint16_t>((uint64_t)ns * per_block_max);
-    std::vector<void*> streams(ns);
-    for (uint32_t i = 0; i < ns; i++) streams[i] = sym + i * per_block_max;
-    ChannelStreams cs(ch, nch, nb);
-    uint32_t f = 1u << levels;
-    decode_streams(I, false, 2, cs.words.data(), cs.nbits.data(), cs.pos.data(), nch, cs.s2b_lp.data(), streams.data(),
-                   nch, (uint32_t)(elems / ((uint64_t)f * f * f)));
-    for (uint32_t c = 0; c < nch; c++) unsymbolize(buf(c, 0), (const uint16_t*)streams[c], sx / f, sy / f, sz / f, sx, sx * sy, st);
-    int d = 0;
-    for (int level = (int)levels - 1; level >= 0; level--) {
-        const uint32_t bx = sx / f, by = sy / f, bz = sz / f;
-        decode_streams(I, !(level > 0 && rle_only_lvl0), 2, cs.words.data(), cs.nbits.data(), cs.pos.data(), nch,
-                       cs.s2b_hp.data(), streams.data(), ns, bx * by * bz);
-        f /= 2;
-        for (uint32_t c = 0; c < nch; c++)
-            for (uint32_t b = 1; b <= nb; b++) {
-                const Band bd = band_of(b, true);
-                const uint64_t off = bd.x * bx + (uint64_t)bd.y * by * sx + (uint64_t)bd.z * bz * sx * sy;
-                unsymbolize(buf(c, d) + off, (const uint16_t*)streams[nb * c + b - 1], bx, by, bz, sx, sx * sy, st);
-            }
-        d = 1 - d;
-    }
+    const VolumeStreams vs(elems, levels, rle_only_lvl0);
+    int16_t* dwt[2] = {I->d_vol[0].as<int16_t>(elems), I->d_vol[1].as<int16_t>(elems)};
+    uint16_t* sym = I->d_vol[2].as<uint16_t>(nch * vs.elems);
+    SectionTimer call(I, 1);
+    call("Decode RLHuff");
+    ChannelStreams cs(ch, nch);
+    std::vector<DecodeStream> streams;
+    for (uint32_t c = 0; c < nch; c++)
+        for (size_t k = 0; k < vs.n.size(); k++)
+            streams.push_back(DecodeStream{sym + c * vs.elems + vs.at[k], vs.n[k], vs.rl[k], c});
+    cs.decode(I, 2, streams);
+    // a channel at a time: each level's coefficients from its symbols around the level above's output,
+    // alternating buffers from dwt[0] (CompressVolume.cpp:794-838)
     for (uint32_t c = 0; c < nch; c++) {
-        int dc = 0;  // each channel's coarsest level is in its first buffer
-        for (int level = (int)levels - 1; level >= 0; level--) {
-            const uint32_t fl = 1u << level;
-            dwt53_inverse(buf(c, 1 - dc), buf(c, dc), buf(c, dc), (int)(sx / fl), (int)(sy / fl), (int)(sz / fl),
-                          (int)sx, (int)(sx * sy), (int)sx, (int)(sx * sy), st);
-            dc = 1 - dc;
+        const uint16_t* s = sym + c * vs.elems;
+        int d = 0;
+        for (uint32_t level = levels; level-- > 0; d = 1 - d) {
+            const uint32_t f = 1u << level;
+            unsymbolize_level(dwt[d], s + vs.at[vs.band(levels, level, 1)], align_up(vs.n[vs.band(levels, level, 1)], 64),
+                              level + 1 == levels ? s : nullptr, nullptr, sx / f, sy / f, sz / f, sx, (uint64_t)sx * sy, st);
+            dwt53_inverse(dwt[1 - d], dwt[d], dwt[d], (int)(sx / f), (int)(sy / f), (int)(sz / f), (int)sx,
+                          (int)(sx * sy), (int)sx, (int)(sx * sy), st);
         }
-        unquantize_from_short(ch[c].image, buf(c, dc), sx, sy, sz, ch[c].step, sx, sx * sy, 1, st);
+        unquantize_from_short(ch[c].image, dwt[d], sx, sy, sz, ch[c].step, sx, sx * sy, 1, st);
     }
 }
 

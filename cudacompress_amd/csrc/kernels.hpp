@@ -59,95 +59,19 @@ void quantize_difference_2d(uint16_t* sym, float* data, float step, const uint8_
                             hipStream_t st);
 void unquantize_difference_2d(float* data, const uint16_t* sym, float step, const uint8_t* ref, uint32_t channelCount,
                               uint32_t channel, uint32_t sx, uint32_t sy, uint32_t row, int qtype, hipStream_t st);
+// One level's coefficients (lx x ly x lz from data, row and slice pitches; lz 1: 2D) as symbols: the
+// highpass octants (quadrants) b = bx + 2 by (+ 4 bz) >= 1 to dense bands hp + (b - 1) band_stride, the
+// lowpass one to low_sym as symbols, or to low as values, or (both null) nowhere; and back (with both
+// null the lowpass octant of data stays as it is).
+void symbolize_level(uint16_t* hp, uint64_t band_stride, uint16_t* low_sym, int16_t* low, const int16_t* data,
+                     uint32_t lx, uint32_t ly, uint32_t lz, uint32_t row, uint64_t slice, hipStream_t st);
+void unsymbolize_level(int16_t* data, const uint16_t* hp, uint64_t band_stride, const uint16_t* low_sym,
+                       const int16_t* low, uint32_t lx, uint32_t ly, uint32_t lz, uint32_t row, uint64_t slice,
+                       hipStream_t st);
 void convert_ycocg(uint8_t* out, const uint8_t* in, uint32_t pixels, int channels, bool to_ycocg, hipStream_t st);
 void lsb_get(const int16_t* data, uint32_t* bits, uint32_t n, hipStream_t st);
 void lsb_remove(int16_t* data, uint32_t* bits, uint32_t n, int16_t shift, hipStream_t st);
 void lsb_append(int16_t* data, const uint32_t* bits, uint32_t n, int16_t shift, hipStream_t st);
 void shift_elems(int16_t* data, uint32_t n, int16_t shift, hipStream_t st);
-
-// ---- entropy coder kernels -----------------------------------------------------------------
-// Per-stream descriptors live in device memory; see codec.cpp for how they are filled.
-struct RleStream {
-    const void* in;       // n symbols
-    void* out_sym;        // compacted symbols (capacity n)
-    void* out_zc;         // zero counts (capacity n)
-    uint32_t n;
-    uint32_t tile_base;   // index of this stream's first tile in the tile arrays
-};
-struct RleTile {          // per 2048-symbol tile
-    uint32_t nnz;
-    uint32_t first_pos;   // position of the first nonzero (or 0xFFFFFFFF)
-    uint32_t last_pos;    // position of the last nonzero
-    uint32_t inner_fill;  // filler pairs emitted before nonzeros 2..nnz of this tile
-    uint32_t out_base;    // output index of this tile's first pair (filled by the scan)
-    uint32_t pad[3];
-};
-struct RleResult {        // per stream
-    uint32_t m;           // pair count
-    uint32_t sym_max;     // max compacted symbol (0 when m == 0)
-    uint32_t zc_max;      // max zero count
-    uint32_t pad;
-};
-constexpr int kRleTile = 2048;
-void rle_encode(const RleStream* d_streams, uint32_t nstreams, RleTile* d_tiles, uint32_t ntiles,
-                const uint32_t* d_tile_stream, RleResult* d_results, int symSize, uint64_t in_elems, hipStream_t st);
-
-struct RleDecStream {
-    const void* sym;     // m compacted symbols
-    const void* zc;      // m zero counts
-    void* out;           // n outputs
-    uint32_t m;
-    uint32_t n;
-    uint32_t tile_base;  // first tile (of kRleTile pairs) of this stream
-    uint32_t pad;
-};
-// Zero-fills every output element, then scatters the pairs.
-void rle_decode(const RleDecStream* d_streams, uint32_t nstreams, uint32_t* d_tile_sums, uint32_t ntiles,
-                const uint32_t* d_tile_stream, uint32_t nmax_out, int symSize, uint64_t total_pairs, uint64_t total_out,
-                hipStream_t st);
-// Per-stream max symbol into results[i].sym_max (results[i].m = n) for streams coded without RLE.
-void stream_max(const RleStream* d_streams, uint32_t nstreams, uint32_t nmax, RleResult* d_results, int symSize,
-                hipStream_t st);
-
-struct HistStream {
-    const void* data;
-    uint32_t n;
-    uint32_t nbins;       // stream symbol max + 1
-    uint32_t* hist;       // nbins counters (zeroed by the launcher)
-    uint32_t quirk;       // add the Symbol16 pad word to bin 65535 (see codec.cpp)
-};
-void histogram(const HistStream* d_streams, const HistStream* h_streams, uint32_t nstreams, int symSize,
-               hipStream_t st);
-
-struct HuffEncStream {
-    const void* sym;       // n symbols
-    const uint32_t* code;  // codeword by symbol
-    const uint32_t* len;   // length by symbol
-    uint32_t* words;       // output words (zeroed by the launcher)
-    uint32_t* offsets;     // bit offset of each coding block (ceil(n/cbs))
-    uint32_t n;
-    uint32_t block_base;   // first coding block in the global block numbering
-    uint32_t chunk_base;   // first pack chunk
-    uint32_t pad;
-};
-void huffman_encode(const HuffEncStream* d_streams, const HuffEncStream* h_streams, uint32_t nstreams,
-                    uint32_t cbs, int symSize, uint32_t* d_block_bits, uint32_t nblocks,
-                    const uint32_t* d_block_stream, uint32_t* d_stream_bits, const uint32_t* d_chunk_stream,
-                    uint32_t nchunks, uint64_t total_bits, hipStream_t st);
-
-struct HuffDecStream {
-    const uint32_t* words;     // codeword words (+1 word of padding)
-    const uint32_t* offsets;   // absolute bit offset of each coding block
-    const int32_t* table;      // first[32], min[32], max[32] per codeword length
-    const void* symbols;       // symbol table by codeword index
-    void* out;                 // n decoded symbols
-    uint32_t n;
-    uint32_t nsyms;            // symbol table size
-    uint32_t wave_base;        // first decode wave of this stream
-    uint32_t nwords;           // codeword words (readable: nwords + 2)
-};
-void huffman_decode(const HuffDecStream* d_streams, uint32_t nstreams, const uint32_t* d_wave_stream,
-                    uint32_t nwaves, uint32_t cbs, int symSize, uint64_t total_syms, uint64_t total_bits,
-                    hipStream_t st);
 
 }  // namespace cca
