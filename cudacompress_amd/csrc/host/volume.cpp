@@ -284,12 +284,13 @@ void compress_volume_float_quant_first(cc_instance* I, const float* image, uint3
     uint16_t* sym = I->d_vol[2].as<uint16_t>(vs.elems);
     // uniform quantization of the whole volume (CompressVolume.cpp:685-687)
     quantize_to_short(dwt[0], image, sx, sy, sz, step, sx, sx * sy, 1, st);
-    // every 5/3 level: data path src -> dst -> buf -> dst with src and buf the same buffer, so level l's
-    // coefficients are in dwt[1 - l % 2]; its bands become symbols before the next level but one reuses it
+    // level l's coefficients are in dwt[1 - l % 2]; its bands become symbols before the next level but one
+    // reuses it
+    int16_t* buf = I->d_vol[3].as<int16_t>(elems);
     for (uint32_t level = 0; level < levels; level++) {
         const uint32_t f = 1u << level;
         const int d = (int)(level & 1);
-        dwt53_forward(dwt[1 - d], dwt[d], dwt[d], (int)(sx / f), (int)(sy / f), (int)(sz / f), (int)sx, (int)(sx * sy),
+        dwt53_forward(dwt[1 - d], buf, dwt[d], (int)(sx / f), (int)(sy / f), (int)(sz / f), (int)sx, (int)(sx * sy),
                       (int)sx, (int)(sx * sy), st);
         symbolize_level(sym + vs.at[vs.band(levels, level, 1)], align_up(vs.n[vs.band(levels, level, 1)], 64),
                         level + 1 == levels ? sym : nullptr, nullptr, dwt[1 - d], sx / f, sy / f, sz / f, sx,
@@ -389,6 +390,7 @@ void decompress_volume_float_quant_first_multichannel(cc_instance* I, const Volu
     const VolumeStreams vs(elems, levels, rle_only_lvl0);
     int16_t* dwt[2] = {I->d_vol[0].as<int16_t>(elems), I->d_vol[1].as<int16_t>(elems)};
     uint16_t* sym = I->d_vol[2].as<uint16_t>(nch * vs.elems);
+    int16_t* buf = I->d_vol[3].as<int16_t>(elems);
     SectionTimer call(I, 1);
     call("Decode RLHuff");
     ChannelStreams cs(ch, nch);
@@ -406,7 +408,7 @@ void decompress_volume_float_quant_first_multichannel(cc_instance* I, const Volu
             const uint32_t f = 1u << level;
             unsymbolize_level(dwt[d], s + vs.at[vs.band(levels, level, 1)], align_up(vs.n[vs.band(levels, level, 1)], 64),
                               level + 1 == levels ? s : nullptr, nullptr, sx / f, sy / f, sz / f, sx, (uint64_t)sx * sy, st);
-            dwt53_inverse(dwt[1 - d], dwt[d], dwt[d], (int)(sx / f), (int)(sy / f), (int)(sz / f), (int)sx,
+            dwt53_inverse(dwt[1 - d], buf, dwt[d], (int)(sx / f), (int)(sy / f), (int)(sz / f), (int)sx,
                           (int)(sx * sy), (int)sx, (int)(sx * sy), st);
         }
         unquantize_from_short(ch[c].image, dwt[d], sx, sy, sz, ch[c].step, sx, sx * sy, 1, st);
