@@ -32,6 +32,13 @@ constexpr uint32_t kCoderThreads = 256;
 constexpr uint32_t kPerThread = 8;
 constexpr uint32_t kChunk = kCoderThreads * kPerThread;  // symbols per workgroup step
 
+// A pointer that a kernel reads from a descriptor is generic to the compiler, and every access through
+// it a flat one, which also counts as an LDS access: a wait for either is one for both.  Items,
+// bitstreams and outputs are never LDS or scratch memory, so their pointers are made global ones.
+template <class T>
+using Global = __attribute__((address_space(1))) T*;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), may_alias));
+
 struct CodeItem {
     const void* in;      // symbols
     uint32_t n;          // symbol count

@@ -147,23 +147,46 @@ __device__ uint64_t arena_alloc(CoderState* st, uint64_t words, uint64_t cap, Se
 
 __device__ __forceinline__ uint32_t req_bits(uint32_t v) { return v ? 32u - (uint32_t)__clz(v) : 0u; }
 
+// A thread's 8 consecutive symbols as they lie in memory; unpack8 makes them 8 numbers.  Kept apart, the
+// load of a later chunk is waited for where that chunk is unpacked (2048 mixed bricks: the pack pass
+// 1583 -> 1460 us, the stats pass 1031 -> 989 us, with global in place of flat loads).
 template <class S>
-__device__ __forceinline__ void load8(const S* in, uint64_t p0, uint32_t n, uint32_t (&v)[kPerThread]) {
+struct Syms8 {
+    u32x4 q[sizeof(S) / 2];
+};
+template <class S>
+__device__ __forceinline__ void load8(Global<const S> in, uint64_t p0, uint32_t n, Syms8<S>& r) {
     if (p0 + kPerThread <= n && ((reinterpret_cast<uintptr_t>(in + p0) & 15) == 0)) {
-        if (sizeof(S) == 2) {
-            const uint4 q = *reinterpret_cast<const uint4*>(in + p0);
-            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        const Global<const u32x4> v = (Global<const u32x4>)(in + p0);
 #pragma unroll
-            for (int j = 0; j < 4; j++) { v[2 * j] = w[j] & 0xFFFFu; v[2 * j + 1] = w[j] >> 16; }
-        } else {
-            const uint4 a = *reinterpret_cast<const uint4*>(in + p0);
-            const uint4 b = *reinterpret_cast<const uint4*>(in + p0 + 4);
-            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-        }
+        for (int k = 0; k < (int)sizeof(S) / 2; k++) r.q[k] = v[k];
     } else {
+        constexpr int per = 4 / sizeof(S);  // symbols a word
 #pragma unroll
-        for (int j = 0; j < (int)kPerThread; j++) v[j] = (p0 + j < n) ? (uint32_t)in[p0 + j] : 0u;
+        for (int k = 0; k < (int)sizeof(S) * 2; k++) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int j = 0; j < per; j++) {
+                const uint64_t i = p0 + k * per + j;
+                w |= (i < n ? (uint32_t)in[i] : 0u) << (16 * j);
+            }
+            r.q[k / 4][k % 4] = w;
+        }
     }
+}
+template <class S>
+__device__ __forceinline__ void unpack8(const Syms8<S>& r, uint32_t (&v)[kPerThread]) {
+#pragma unroll
+    for (int j = 0; j < (int)kPerThread; j++) {
+        if (sizeof(S) == 4) v[j] = r.q[j / 4][j % 4];
+        else v[j] = (r.q[j / 8][j / 2 % 4] >> (16 * (j % 2))) & 0xFFFFu;
+    }
+}
+template <class S>
+__device__ __forceinline__ void load8(Global<const S> in, uint64_t p0, uint32_t n, uint32_t (&v)[kPerThread]) {
+    Syms8<S> r;
+    load8(in, p0, n, r);
+    unpack8(r, v);
 }
 
 // Pairs of one thread's 8 positions, computed without branches: a pair is emitted for every
@@ -315,7 +338,7 @@ template <class S>
 __global__ __launch_bounds__(64) void k_seg_last(const CodeItem* items, CodeUnits U) {
     const CodeUnit u = U.units[U.split_list[blockIdx.x]];
     const CodeItem it = items[u.item];
-    const S* in = static_cast<const S*>(it.in);
+    const Global<const S> in = (Global<const S>)it.in;
     const uint64_t lo = (uint64_t)u.chunk0 * kChunk;
     const uint64_t hi = min((uint64_t)it.n, lo + (uint64_t)u.nchunk * kChunk);
     const uint32_t words = U.nsplit * kSplitWords;
@@ -495,7 +518,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* it
     const uint32_t ii = u.item;
     const bool split = Split && u.split != kWholeItem;
     const CodeItem it = items[ii];
-    const S* in = static_cast<const S*>(it.in);
+    const Global<const S> in = (Global<const S>)it.in;
     const bool rl = it.rl != 0;
     const uint32_t n = it.n;
     const uint64_t base0 = split ? (uint64_t)u.chunk0 * kChunk : 0;
@@ -519,13 +542,12 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* it
         }
     };
     const uint32_t t8 = threadIdx.x * kPerThread;
-    uint32_t vn[kPerThread];
+    Syms8<S> vn;
     load8(in, base0 + t8, n, vn);
     uint32_t par = 0;
     for (uint64_t base = base0; base < end; base += kChunk, par ^= 1) {
         uint32_t v[kPerThread];
-#pragma unroll
-        for (int j = 0; j < (int)kPerThread; j++) v[j] = vn[j];
+        unpack8(vn, v);
         if (base + kChunk < end) load8(in, base + kChunk + t8, n, vn);  // next step's symbols in flight
         const uint32_t nvalid = chunk_nvalid(base, n, t8);
         int wl;
@@ -624,7 +646,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats_wide(const CodeIte
     const CodeItem it = items[u.item];
     SeqInfo* ss = &seqs[it.seq];
     if (!ss->wide || ss->err) return;
-    const S* in = static_cast<const S*>(it.in);
+    const Global<const S> in = (Global<const S>)it.in;
     const bool rl = it.rl != 0;
     const uint32_t n = it.n;
     uint32_t* h = scratch + ss->hist_off;
@@ -1248,7 +1270,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_seg_bits(const CodeItem* item
     const SeqInfo& ss = seqs[it.seq];
     const SeqInfo& sz = seqs[it.seq + (rl ? 1 : 0)];
     if (ss.err || sz.err || ss.count == 0) return;
-    const S* in = static_cast<const S*>(it.in);
+    const Global<const S> in = (Global<const S>)it.in;
     const uint32_t n = it.n;
     const bool sglob = ss.smax >= kStatBins;
     const uint32_t* glen = scratch + ss.code_off + ss.smax + 1;
@@ -1261,13 +1283,13 @@ __global__ __launch_bounds__(kCoderThreads) void k_seg_bits(const CodeItem* item
     const long long limit = rl ? (long long)ss.last_nz1 - 1 : (long long)n;
     const uint32_t t8 = threadIdx.x * kPerThread;
     uint64_t bs = 0, bz = 0;
-    uint32_t vn[kPerThread], par = 0;
+    uint32_t par = 0;
+    Syms8<S> vn;
     load8(in, base0 + t8, n, vn);
     __syncthreads();
     for (uint64_t base = base0; base < end; base += kChunk, par ^= 1) {
         uint32_t v[kPerThread];
-#pragma unroll
-        for (int j = 0; j < (int)kPerThread; j++) v[j] = vn[j];
+        unpack8(vn, v);
         if (base + kChunk < end) load8(in, base + kChunk + t8, n, vn);
         const uint32_t nvalid = chunk_nvalid(base, n, t8);
         int wl;
@@ -1410,7 +1432,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
     uint32_t* bz = scratch + sz.boff_off;
     const uint32_t cbs = p.cbs;
     if (M > 0) {
-        const S* in = static_cast<const S*>(it.in);
+        const Global<const S> in = (Global<const S>)it.in;
         const uint32_t n = it.n;
         const bool sglob = ss.smax >= kStatBins;
         const uint32_t* gcode = scratch + ss.code_off;
@@ -1478,7 +1500,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
             long long carry = carry0;  // last nonzero before this chunk
             uint64_t pairs = seg.pairs, cbits_s = seg.bits_s, cbits_z = seg.bits_z;
             for (uint64_t base = base0; base < end && pairs < M; base += kChunk) {
-                uint32_t vnn[kPerThread];
+                Syms8<S> vnn;
                 if (base + 2 * kChunk < end) load8(in, base + 2 * kChunk + t8, n, vnn);
                 const uint32_t nvalid = chunk_nvalid(base, n, t8);
                 // this thread's pairs; code lengths looked up once for both the scan and the packing
@@ -1618,10 +1640,8 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
                 prel = prel_n;
                 ctot = ctot_n;
 #pragma unroll
-                for (int j = 0; j < (int)kPerThread; j++) {
-                    v[j] = vn[j];
-                    vn[j] = vnn[j];
-                }
+                for (int j = 0; j < (int)kPerThread; j++) v[j] = vn[j];
+                unpack8(vnn, vn);
             }
             if (threadIdx.x == 0 && split) {
                 own->last_s = win[0][(uint32_t)(cbits_s >> 5) & WM];

@@ -69,13 +69,13 @@ struct ParseWin {
 __device__ __forceinline__ void parse_load(ParseWin& W, const DecCall& C, uint64_t base) {
     const uint64_t i = base + (uint64_t)threadIdx.x;
     W.base = base;
-    W.v = i < C.nwords ? C.words[i] : 0u;
+    W.v = i < C.nwords ? ((Global<const uint32_t>)C.words)[i] : 0u;
 }
 // stream word i (i < C.nwords): from the window, else from memory
 __device__ __forceinline__ uint32_t parse_word(const ParseWin& W, const DecCall& C, uint64_t i) {
     const uint64_t d = i - W.base;
     if (i >= W.base && d < 64) return (uint32_t)__builtin_amdgcn_readlane((int)W.v, (int)d);
-    return C.words[i];
+    return ((Global<const uint32_t>)C.words)[i];
 }
 // rd_bits over the window
 __device__ __forceinline__ uint32_t parse_bits(const ParseWin& W, const DecCall& C, uint64_t pos, uint32_t n,
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     const uint32_t fb0 = wave_first[wv];
     if (fb0 >= nblk) return;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    S* out = static_cast<S*>(s.out);
+    const Global<S> out = (Global<S>)s.out;
     const bool multi = s.nlen > 0;
     const uint32_t nsym = s.nsym;
     const uint32_t* gsyms = scratch + s.lut_off + (1u << kLut);
@@ -403,7 +403,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     S* run_row = &run_all[wave][lane * RW * 4 / sizeof(S)];
     // the run row and the codeword copy are also accessed as words / 16-byte vectors
     typedef uint32_t __attribute__((may_alias)) u32a;
-    typedef uint32_t u32x4a __attribute__((ext_vector_type(4), may_alias));
     uint32_t* win = &win_all[wave][lane];  // the copy's word k at win[64 k]: a lane's own bank
     const uint32_t b = fb + lane;
     const bool valid = b < nblk;
@@ -412,7 +411,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     // dividing the wave's 64 blocks)
     const DecItem zit = rc.nchunks ? items[s.item] : DecItem{};
     const bool zsum = rc.nchunks != 0 && zit.rl && zit.seq + 1 == sq;
-    const uint32_t* words = s.base + s.words_off;
+    const Global<const uint32_t> words = (Global<const uint32_t>)s.base + s.words_off;
     const uint64_t avail = s.nwords - s.words_off;  // readable words from the codeword start
     auto word = [&](uint32_t i) -> uint32_t { return i < avail ? words[i] : 0u; };
     // window {hi, lo} (the next code: alignbit(hi, lo, q), 32 + q bits unread, q in [0, 31] after a
@@ -436,18 +435,17 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     // words from the 16-byte boundary at or below word nxt into the LDS copy.  The call's buffer
     // holds words [-words_off, avail); a start below it stays in the 16-byte block of the buffer's
     // first word.  Where the copy would reach past the buffer's end, words are read one by one.
-    const uint32_t* cend = s.base + s.nwords;
+    const Global<const uint32_t> cend = (Global<const uint32_t>)s.base + s.nwords;
     auto load_window = [&]() {
-        const uint32_t* gp = reinterpret_cast<const uint32_t*>(reinterpret_cast<uintptr_t>(words + nxt) & ~uintptr_t(15));
+        const auto gp = (Global<const uint32_t>)(reinterpret_cast<uintptr_t>(words + nxt) & ~uintptr_t(15));
         w0 = (int)nxt - (int)(words + nxt - gp);
         const bool fast = !(valid && multi) || gp + kWinWords <= cend;
         if (__all(fast)) {
             if (valid && multi) {
                 // a global-space pointer: the loads cannot alias the LDS stores, so all of them
                 // are issued before the first store waits
-                using G4 = const __attribute__((address_space(1))) u32x4a*;
-                const G4 g4 = (G4)(const void*)gp;
-                u32x4a v[kWinWords / 4];
+                const Global<const u32x4> g4 = (Global<const u32x4>)gp;
+                u32x4 v[kWinWords / 4];
 #pragma unroll
                 for (uint32_t k = 0; k < kWinWords / 4; k++) v[k] = g4[k];
 #pragma unroll
@@ -533,7 +531,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
         if (wide && vlen == kDecRound) {
 #pragma unroll
             for (uint32_t k = 0; k < NW; k += 4)
-                *reinterpret_cast<uint4*>(out + p0 + k * 4 / sizeof(S)) = make_uint4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+                *(Global<u32x4>)(out + p0 + k * 4 / sizeof(S)) = u32x4{v[k], v[k + 1], v[k + 2], v[k + 3]};
         } else {
 #pragma unroll
             for (uint32_t i = 0; i < kDecRound; i++)
@@ -651,31 +649,36 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
 }
 
 // Eight consecutive symbols from a 16-byte aligned address.
-__device__ __forceinline__ void load8_aligned(const uint16_t* p, uint32_t (&o)[8]) {
-    const uint4 w = *reinterpret_cast<const uint4*>(p);
-    const uint32_t a[4] = {w.x, w.y, w.z, w.w};
+template <class S>
+__device__ __forceinline__ void load8_aligned(Global<const S> p, uint32_t (&o)[8]) {
+    const Global<const u32x4> q = (Global<const u32x4>)p;
+    if constexpr (sizeof(S) == 2) {
+        const u32x4 a = q[0];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        o[2 * k] = a[k] & 0xFFFFu;
-        o[2 * k + 1] = a[k] >> 16;
+        for (int k = 0; k < 4; k++) {
+            o[2 * k] = a[k] & 0xFFFFu;
+            o[2 * k + 1] = a[k] >> 16;
+        }
+    } else {
+        const u32x4 a = q[0], b = q[1];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            o[k] = a[k];
+            o[4 + k] = b[k];
+        }
     }
-}
-__device__ __forceinline__ void load8_aligned(const uint32_t* p, uint32_t (&o)[8]) {
-    const uint4 w0 = reinterpret_cast<const uint4*>(p)[0], w1 = reinterpret_cast<const uint4*>(p)[1];
-    o[0] = w0.x; o[1] = w0.y; o[2] = w0.z; o[3] = w0.w;
-    o[4] = w1.x; o[5] = w1.y; o[6] = w1.z; o[7] = w1.w;
 }
 
 template <class S>
-__device__ __forceinline__ void clear_symbols(S* out, uint32_t n) {
+__device__ __forceinline__ void clear_symbols(Global<S> out, uint32_t n) {
     const uintptr_t a = reinterpret_cast<uintptr_t>(out);
     constexpr uint32_t per = 16 / sizeof(S);
     uint32_t head = (uint32_t)(((16 - (a & 15)) & 15) / sizeof(S));
     if ((a % sizeof(S)) != 0 || head > n) head = n;
     for (uint32_t i = threadIdx.x; i < head; i += blockDim.x) out[i] = (S)0;
     const uint32_t nv = (n - head) / per;
-    uint4* v = reinterpret_cast<uint4*>(out + head);
-    for (uint32_t j = threadIdx.x; j < nv; j += blockDim.x) v[j] = make_uint4(0u, 0u, 0u, 0u);
+    const Global<u32x4> v = (Global<u32x4>)(out + head);
+    for (uint32_t j = threadIdx.x; j < nv; j += blockDim.x) v[j] = u32x4{0u, 0u, 0u, 0u};
     for (uint32_t i = head + nv * per + threadIdx.x; i < n; i += blockDim.x) out[i] = (S)0;
 }
 
@@ -721,9 +724,9 @@ __global__ __launch_bounds__(256) void k_dec_rle(const DecItem* items, uint32_t 
     uint64_t before = 0;
     for (uint32_t k = threadIdx.x; k < c; k += 256) before += rc.sums[rc.item_first[ii] + k];
     const uint64_t carry = block_sum_u64<256>(before, shs);
-    const S* sym = static_cast<const S*>(ss.out);
-    const S* zc = static_cast<const S*>(sz.out);
-    S* out = static_cast<S*>(it.out);
+    const Global<const S> sym = (Global<const S>)ss.out;
+    const Global<const S> zc = (Global<const S>)sz.out;
+    const Global<S> out = (Global<S>)it.out;
     // LDS index swizzle: thread t's 8 consecutive entries and the strided reads are both
     // conflict-free across the 64 banks
     auto sw = [](uint32_t i) { return i ^ ((i >> 6) & 7u); };
@@ -734,8 +737,8 @@ __global__ __launch_bounds__(256) void k_dec_rle(const DecItem* items, uint32_t 
     uint32_t z[8], v[8], sum = 0;
     const uint32_t i0 = base + threadIdx.x * 8;
     if (vec && i0 + 8 <= M) {
-        load8_aligned(zc + i0, z);
-        load8_aligned(sym + i0, v);
+        load8_aligned<S>(zc + i0, z);
+        load8_aligned<S>(sym + i0, v);
 #pragma unroll
         for (int k = 0; k < 8; k++) sum += z[k] + 1;
     } else {
@@ -762,7 +765,7 @@ __global__ __launch_bounds__(256) void k_dec_rle(const DecItem* items, uint32_t 
     }
     // the chunk's span of output positions, cleared before its values land
     const uint64_t s1 = last ? (uint64_t)n : min(carry + tot, (uint64_t)n);
-    if (carry < s1) clear_symbols(out + carry, (uint32_t)(s1 - carry));
+    if (carry < s1) clear_symbols<S>(out + carry, (uint32_t)(s1 - carry));
     __syncthreads();  // the clearing stores complete before values land on them
 #pragma unroll
     for (int k = 0; k < 8; k++) {
