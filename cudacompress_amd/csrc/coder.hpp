@@ -71,6 +71,7 @@ struct CodeUnits {
     uint32_t nunits;
     const uint32_t* split_list;
     uint32_t nsplit_units, nsplit;
+    uint32_t unit_chunks;   // most chunks of a segment
     SegState* segs;
     uint32_t* split_state;  // nsplit * kSplitWords
 };

@@ -50,72 +50,6 @@ __device__ uint64_t wg_excl_sum_u64(uint64_t v, uint64_t* sh, uint64_t& total) {
     total = tot;
     return base + x - v;
 }
-__device__ long long wg_excl_max_i64(long long v, long long* sh, long long& total) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const long long x = wave_incl_max_i64(v);
-    const long long ex = wave_shift_up_i64(x, -1);
-    if (lane == 63) sh[w] = x;
-    __syncthreads();
-    long long base = -1, tot = -1;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const long long s = sh[i];
-        if (i < w) base = base > s ? base : s;
-        tot = tot > s ? tot : s;
-    }
-    __syncthreads();
-    total = tot;
-    return base > ex ? base : ex;
-}
-// wg_excl_max_i64 without the closing barrier: sh must not be written again before the next
-// barrier (callers alternate two arrays).
-__device__ __forceinline__ long long wg_excl_max_i64_open(long long v, long long* sh, long long& total) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const long long x = wave_incl_max_i64(v);
-    const long long ex = wave_shift_up_i64(x, -1);
-    if (lane == 63) sh[w] = x;
-    __syncthreads();
-    long long base = -1, tot = -1;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const long long s = sh[i];
-        if (i < w) base = base > s ? base : s;
-        tot = tot > s ? tot : s;
-    }
-    total = tot;
-    return base > ex ? base : ex;
-}
-// Exclusive sum of a and exclusive max of b (identity -1) over a 256-thread workgroup with one
-// barrier: sha and shb (4 entries each) must not be written again before the next barrier.
-__device__ __forceinline__ void wg_excl_sum_max(uint64_t a, long long b, uint64_t* sha, long long* shb,
-                                                uint64_t& ex_a, uint64_t& tot_a, long long& ex_b, long long& tot_b) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint64_t xa = wave_incl_scan_u64(a);
-    const long long xb = wave_incl_max_i64(b);
-    const long long eb = wave_shift_up_i64(xb, -1);
-    if (lane == 63) {
-        sha[w] = xa;
-        shb[w] = xb;
-    }
-    __syncthreads();
-    uint64_t base_a = 0, ta = 0;
-    long long base_b = -1, tb = -1;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint64_t sa = sha[i];
-        const long long sb = shb[i];
-        if (i < w) {
-            base_a += sa;
-            base_b = base_b > sb ? base_b : sb;
-        }
-        ta += sa;
-        tb = tb > sb ? tb : sb;
-    }
-    ex_a = base_a + xa - a;
-    tot_a = ta;
-    ex_b = base_b > eb ? base_b : eb;
-    tot_b = tb;
-}
 __device__ uint32_t wg_sum_u32(uint32_t v, uint32_t* sh) {
     v = wave_sum(v);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
@@ -189,42 +123,6 @@ __device__ __forceinline__ void load8(Global<const S> in, uint64_t p0, uint32_t 
     unpack8(r, v);
 }
 
-// Pairs of one thread's 8 positions, computed without branches: a pair is emitted for every
-// symbol of a plain stream, and in a run-length stream for every nonzero and for every 256th zero
-// of a run (a filler, symbol 0 with zero count 255) at positions < limit; the pair's zero count is
-// the length of the zero run before it modulo 256.  prev: position of the last nonzero before the
-// thread's positions (-1 none); limit: the stream's last nonzero (pass A passes n and removes the
-// trailing run's fillers afterwards).  Returns the emit mask (bit j: position p0 + j) and the zero
-// counts in zc.
-__device__ __forceinline__ uint32_t thread_flags(const uint32_t (&v)[kPerThread], uint64_t p0, uint32_t n, bool rl,
-                                                 long long prev, long long limit, uint32_t (&zc)[kPerThread]) {
-    const uint32_t nvalid = p0 >= n ? 0u : (n - p0 >= kPerThread ? kPerThread : (uint32_t)(n - p0));
-    const long long lim_rel = limit - (long long)p0;
-    uint32_t g = (uint32_t)((long long)p0 - prev - 1);  // only its low 8 bits matter
-    uint32_t emit = 0;
-#pragma unroll
-    for (int j = 0; j < (int)kPerThread; j++) {
-        const bool nz = v[j] != 0u;
-        const uint32_t z = g & 255u;
-        const bool e = (uint32_t)j < nvalid && (!rl || nz || (z == 255u && (long long)j < lim_rel));
-        g = nz ? 0u : g + 1u;
-        zc[j] = rl ? z : 0u;
-        emit |= (uint32_t)e << j;
-    }
-    return emit;
-}
-
-// f(sym, zc) for each pair of thread_flags, in order.
-template <class F>
-__device__ __forceinline__ void thread_pairs(const uint32_t (&v)[kPerThread], uint64_t p0, uint32_t n, bool rl,
-                                             long long prev, long long limit, F f) {
-    uint32_t zc[kPerThread];
-    const uint32_t emit = thread_flags(v, p0, n, rl, prev, limit, zc);
-#pragma unroll
-    for (int j = 0; j < (int)kPerThread; j++)
-        if ((emit >> j) & 1u) f(v[j], zc[j]);
-}
-
 __device__ __forceinline__ long long thread_last_nz(const uint32_t (&v)[kPerThread], uint64_t p0, uint32_t n) {
     const uint32_t nvalid = p0 >= n ? 0u : (n - p0 >= kPerThread ? kPerThread : (uint32_t)(n - p0));
     uint32_t m = 0;
@@ -243,15 +141,25 @@ __device__ __forceinline__ uint32_t chunk_nvalid(uint64_t base, uint32_t n, uint
     const uint32_t r = rem > (uint64_t)kChunk ? kChunk : (uint32_t)rem;
     return r > t8 ? (r - t8 < kPerThread ? r - t8 : kPerThread) : 0u;
 }
-// the thread's last nonzero, chunk-relative (-1: none)
-__device__ __forceinline__ int thread_last_nz_rel(const uint32_t (&v)[kPerThread], uint32_t t8, uint32_t nvalid) {
+// bit j: the thread's symbol j is no zero (load8 gives zeros past the stream's end)
+__device__ __forceinline__ uint32_t nonzeros(const uint32_t (&v)[kPerThread]) {
     uint32_t m = 0;
 #pragma unroll
-    for (int j = 0; j < (int)kPerThread; j++) m |= (uint32_t)(v[j] != 0u && (uint32_t)j < nvalid) << j;
-    return m ? (int)(t8 + 31u - (uint32_t)__clz(m)) : -1;
+    for (int j = 0; j < (int)kPerThread; j++) m |= (uint32_t)(v[j] != 0u) << j;
+    return m;
 }
-// thread_flags with g0 = (first position - last nonzero before it - 1) mod 2^32 and
-// lim = limit - first position (clamped; only lim > j matters)
+// the thread's last nonzero, chunk-relative (-1: none)
+__device__ __forceinline__ int last_nz_rel(uint32_t nz, uint32_t t8) {
+    return nz ? (int)(t8 + 31u - (uint32_t)__clz(nz)) : -1;
+}
+// all ones if bit j of m is set, else 0
+__device__ __forceinline__ uint32_t bit_mask(uint32_t m, int j) { return (uint32_t)__builtin_amdgcn_sbfe((int)m, j, 1); }
+// Pairs of one thread's 8 positions, computed without branches: a pair is emitted for every
+// symbol of a plain stream, and in a run-length stream for every nonzero and for every 256th zero
+// of a run (a filler, symbol 0 with zero count 255) before the stream's last nonzero; the pair's
+// zero count is the length of the zero run before it modulo 256.  g0 = (first position - last
+// nonzero before it - 1) mod 2^32, lim = the last nonzero - first position (clamped; only lim > j
+// matters).  Returns the emit mask (bit j: position j) and the zero counts in zc.
 __device__ __forceinline__ uint32_t thread_flags_rel(const uint32_t (&v)[kPerThread], uint32_t nvalid, bool rl,
                                                      uint32_t g0, int lim, uint32_t (&zc)[kPerThread]) {
     uint32_t g = g0, emit = 0;
@@ -303,6 +211,78 @@ __device__ __forceinline__ void wg_last_combine(int ex, const int* sh, int& excl
     }
     excl = ex >= 0 ? ex : base;
     total = __builtin_amdgcn_readfirstlane(tot);
+}
+
+// Positions [lo, hi) of a stream, of a wave each, for passes to which their order means nothing: a wave
+// takes a run of whole steps of 64 kPerThread positions and keeps the last nonzero before it itself, so
+// there is no barrier.  A wave that does not start the range looks back for the last nonzero before its
+// run (in a run-length stream).  f(e, sym, zc) for each position, by the whole wave at once: e, whether it
+// gives the pair (sym, zc).  Returns the last nonzero up to the end of the wave's run.
+// Where no lane's run can reach 255 zeros (any stream but a sparse one) a position is only compared with
+// zero: the statistics of 2048 mixed bricks took 989 us with a barrier a step and the general rule
+// everywhere.
+constexpr uint32_t kStep = 64 * kPerThread;
+template <bool RL, class S, class F>
+__device__ __forceinline__ long long wave_pairs(Global<const S> in, uint32_t n, uint64_t lo, uint64_t hi, long long carry,
+                                                long long limit, F f) {
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lane = threadIdx.x & 63, l8 = lane * kPerThread;
+    const uint64_t steps = hi > lo ? (hi - lo + kStep - 1) / kStep : 0;
+    const uint64_t per = (steps + 3) / 4, s0 = min(w * per, steps), s1 = min(s0 + per, steps);
+    uint32_t v[kPerThread];
+    // the wave's last nonzero of a step: position from the step's start
+    auto last_nz = [&](uint64_t m, int b) { return __builtin_amdgcn_readlane(b, 63 - __clzll(m)); };
+    auto lane_last = [&]() {
+        int b = -1;
+#pragma unroll
+        for (int j = 0; j < (int)kPerThread; j++) b = v[j] ? (int)l8 + j : b;
+        return b;
+    };
+    Syms8<S> next, prev;
+    const bool back = RL && s0 && s0 < s1;
+    if (back) load8(in, lo + (s0 - 1) * kStep + l8, n, prev);
+    if (s0 < s1) load8(in, lo + s0 * kStep + l8, n, next);
+    if (back)
+        for (uint64_t q = s0 - 1;; q--) {
+            unpack8(prev, v);
+            const int b = lane_last();
+            const uint64_t m = __ballot(b >= 0);
+            if (m) carry = (long long)(lo + q * kStep) + last_nz(m, b);
+            if (m || q == 0) break;
+            load8(in, lo + (q - 1) * kStep + l8, n, prev);
+        }
+    for (uint64_t q = s0; q < s1; q++) {
+        const uint64_t base = lo + q * kStep;
+        unpack8(next, v);
+        if (q + 1 < s1) load8(in, base + kStep + l8, n, next);  // in flight over this step
+        if constexpr (RL) {
+            const int b = lane_last();
+            const uint64_t m = __ballot(b >= 0), below = m & ((1ull << lane) - 1ull);
+            const int before = __shfl(b, below ? 63 - __clzll(below) : 0);
+            uint32_t g = below ? l8 - (uint32_t)before - 1u : chunk_gc(base, carry) + l8;  // zeros before
+            if (__all(g < 256u - kPerThread)) {
+#pragma unroll
+                for (int j = 0; j < (int)kPerThread; j++) {
+                    f(v[j] != 0u, v[j], g);
+                    g = v[j] ? 0u : g + 1u;
+                }
+            } else {
+                const int lim = chunk_lim(base, limit) - (int)l8;
+#pragma unroll
+                for (int j = 0; j < (int)kPerThread; j++) {
+                    const uint32_t z = g & 255u;
+                    f(v[j] != 0u || (z == 255u && j < lim), v[j], z);
+                    g = v[j] ? 0u : g + 1u;
+                }
+            }
+            if (m) carry = (long long)base + last_nz(m, b);
+        } else {
+            const uint32_t nvalid = chunk_nvalid(base, n, l8);
+#pragma unroll
+            for (int j = 0; j < (int)kPerThread; j++) f((uint32_t)j < nvalid, v[j], 0u);
+        }
+    }
+    return carry;
 }
 // a uniform 64-bit value held in vector registers, moved to scalar ones
 __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
@@ -390,16 +370,17 @@ __device__ __forceinline__ SegState seg_before(const SegState* segs, uint32_t lo
     return r;
 }
 
-// Counts this workgroup in at *counter after everything it wrote; true for the last of n, whose
-// reads then see what the others wrote.  Every thread calls.
+// Whether this workgroup is the last of n to arrive; what the others did with device-scope atomics before
+// is done then.  Atomics are performed where every workgroup sees them, so it is enough that a wave waits
+// for its own; a fence would also write the cache back, 0.9 ms for the 16 to 128 workgroups of a 4096^2
+// terrain's lowpass band.  Plain stores are not covered.
 __device__ __forceinline__ bool last_arrival(uint32_t* counter, uint32_t n, uint32_t* sh) {
-    __threadfence();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0) *sh = atomicAdd(counter, 1u);
     __syncthreads();
-    const bool last = *sh == n - 1;
-    if (last) __threadfence();
-    return last;
+    return *sh == n - 1;
 }
 
 // Words of a histogram of nb bins in the arena and, when the table may be designed one per thread
@@ -483,7 +464,7 @@ __device__ __forceinline__ void stats_finish(const CodeItem& it, uint32_t ii, ui
     if (sh_off[0] != ~uint64_t(0)) {
         uint32_t* h = scratch + sh_off[0];
         const uint32_t nb = (M ? smax : 0u) + 1;
-        for (uint32_t i = threadIdx.x; i < nb; i += kCoderThreads) h[i] = wide ? 0u : hs[i];
+        for (uint32_t i = threadIdx.x; i < nb; i += kCoderThreads) h[i] = i < kStatBins ? hs[i] : 0u;
         if (threadIdx.x == 0) ss->hist_off = sh_off[0];
     }
     // the uniform branches below (sh_off is shared) keep every thread at the scans' barriers
@@ -503,14 +484,14 @@ __device__ __forceinline__ void stats_finish(const CodeItem& it, uint32_t ii, ui
 
 // Pass A: pair counts, histograms (LDS), maxima; tables of the LDS class get their histogram
 // copied to the arena (with the leaf list of small tables); streams with symbols >= kStatBins are
-// marked wide and get a zeroed global histogram for k_code_stats_wide.
+// marked wide and get theirs with those bins zero, which k_code_stats_wide counts.
 template <class S, bool Split>  // Split: the job has split items (the checks cost the pack 4 %)
 __global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* items, SeqInfo* seqs, CoderParams p,
                                                               uint32_t* scratch, uint64_t cap, CoderState* st,
                                                               CodeUnits U) {
-    __shared__ uint32_t hs[kStatBins];
+    __shared__ uint32_t hs[kStatBins + 1];  // the last bin: larger symbols
     __shared__ uint32_t hz[256];
-    __shared__ int shl[2][4];  // alternate chunks: one barrier per chunk
+    __shared__ long long shl[4];
     __shared__ uint32_t shu[4];
     __shared__ uint64_t sh_off[2];
     __shared__ uint64_t shq[4];
@@ -523,7 +504,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* it
     const uint32_t n = it.n;
     const uint64_t base0 = split ? (uint64_t)u.chunk0 * kChunk : 0;
     const uint64_t end = split ? min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk) : (uint64_t)n;
-    for (uint32_t i = threadIdx.x; i < kStatBins; i += kCoderThreads) hs[i] = 0;
+    for (uint32_t i = threadIdx.x; i <= kStatBins; i += kCoderThreads) hs[i] = 0;
     for (uint32_t i = threadIdx.x; i < 256; i += kCoderThreads) hz[i] = 0;
     __syncthreads();
     long long carry = -1, limit = (long long)n;
@@ -531,60 +512,35 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats(const CodeItem* it
         carry = (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.seg) - 1;
         limit = (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.nseg) - 1;
     }
-    uint32_t cnt = 0, vmax = 0, wide = 0;
-    // histogram updates are coalesced per thread: runs of one symbol and all zero counts of zero
-    // are counted in registers (zero runs dominate the zero-count histogram)
-    uint32_t run_sym = 0xFFFFFFFFu, run_len = 0, zc0 = 0;
-    auto flush_run = [&]() {
-        if (run_len) {
-            if (run_sym < kStatBins) atomicAdd(&hs[run_sym], run_len);
-            else wide = 1;
-        }
+    uint32_t cnt = 0, vmax = 0;
+    auto count = [&](auto r) {
+        constexpr bool RL = decltype(r)::value;
+        carry = wave_pairs<RL, S>(in, n, base0, end, carry, limit, [&](bool e, uint32_t s, uint32_t z) {
+            cnt += (uint32_t)__popcll(__ballot(e));
+            vmax = max(vmax, s);  // a position that gives no pair holds 0
+            if (e) {
+                atomicAdd(&hs[min(s, kStatBins)], 1u);
+                if (RL && z) atomicAdd(&hz[z], 1u);
+            }
+        });
     };
-    const uint32_t t8 = threadIdx.x * kPerThread;
-    Syms8<S> vn;
-    load8(in, base0 + t8, n, vn);
-    uint32_t par = 0;
-    for (uint64_t base = base0; base < end; base += kChunk, par ^= 1) {
-        uint32_t v[kPerThread];
-        unpack8(vn, v);
-        if (base + kChunk < end) load8(in, base + kChunk + t8, n, vn);  // next step's symbols in flight
-        const uint32_t nvalid = chunk_nvalid(base, n, t8);
-        int wl;
-        const int ex = wave_excl_last(thread_last_nz_rel(v, t8, nvalid), wl);
-        if ((threadIdx.x & 63) == 0) shl[par][threadIdx.x >> 6] = wl;
-        __syncthreads();
-        int prel, ctot;
-        wg_last_combine(ex, shl[par], prel, ctot);
-        uint32_t zc[kPerThread];
-        const uint32_t emit = thread_flags_rel(v, nvalid, rl, thread_g0(prel, t8, chunk_gc(base, carry)),
-                                               chunk_lim(base, limit) - (int)t8, zc);
-#pragma unroll
-        for (int j = 0; j < (int)kPerThread; j++) {
-            if (!((emit >> j) & 1u)) continue;
-            const uint32_t s = v[j], z = zc[j];
-            cnt++;
-            vmax = max(vmax, s);
-            if (s == run_sym) {
-                run_len++;
-            } else {
-                flush_run();
-                run_sym = s;
-                run_len = 1;
-            }
-            if (rl) {
-                if (z == 0) zc0++;
-                else atomicAdd(&hz[z], 1u);
-            }
-        }
-        if (ctot >= 0) carry = (long long)base + ctot;
+    if (rl) count(std::true_type{});
+    else count(std::false_type{});
+    if ((threadIdx.x & 63) == 0) {
+        shl[threadIdx.x >> 6] = carry;
+        shu[threadIdx.x >> 6] = cnt;
     }
-    flush_run();
-    zc0 = wave_sum(zc0);
-    if (rl && (threadIdx.x & 63) == 0 && zc0) atomicAdd(&hz[0], zc0);
-    uint32_t M = wg_sum_u32(cnt, shu);
-    wide = wg_max_u32(wide, shu);
+    __syncthreads();
+    carry = max(max(shl[0], shl[1]), max(shl[2], shl[3]));
+    uint32_t M = shu[0] + shu[1] + shu[2] + shu[3];
+    const uint32_t wide = hs[kStatBins] ? 1u : 0u;
+    __syncthreads();
     vmax = wg_max_u32(vmax, shu);
+    if (rl) {  // zero counts of zero are the rest of the pairs
+        const uint32_t z = wg_sum_u32(hz[threadIdx.x], shu);
+        if (threadIdx.x == 0) hz[0] = M - z;
+        __syncthreads();
+    }
     if (split) {
         // the segments' histograms add up in global memory, k_code_stats_finish goes on with the sums
         uint32_t* sp = U.split_state + (size_t)u.split * kSplitWords;
@@ -634,12 +590,13 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats_finish(const CodeI
     stats_finish(it, u.item, m, sp[2], sp[3], last, hs, hz, seqs, p, scratch, cap, st, shu, sh_off, shq);
 }
 
-// Pass A for streams with symbols >= kStatBins: histogram with global atomics, then the pad
-// quirk (Symbol16, GPU dialect, max symbol 65535, odd count: src/cudaCompress/Histogram.cu:90-105).
+// Pass A for streams with symbols >= kStatBins: those are counted with global atomics (they are no
+// zeros, so each is a pair), then the pad quirk (Symbol16, GPU dialect, max symbol 65535, odd count:
+// src/cudaCompress/Histogram.cu:90-105).  The smaller symbols' counts are there already: counting all of
+// them here, most updates on a few bins, took 3.5 ms for a 4096^2 terrain.
 template <class S>
 __global__ __launch_bounds__(kCoderThreads) void k_code_stats_wide(const CodeItem* items, SeqInfo* seqs,
                                                                    CoderParams p, uint32_t* scratch, CodeUnits U) {
-    __shared__ long long shl[4];
     __shared__ uint32_t shu[4];
     const CodeUnit u = U.units[blockIdx.x];
     const bool split = u.split != kWholeItem;
@@ -647,33 +604,41 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_stats_wide(const CodeIte
     SeqInfo* ss = &seqs[it.seq];
     if (!ss->wide || ss->err) return;
     const Global<const S> in = (Global<const S>)it.in;
-    const bool rl = it.rl != 0;
     const uint32_t n = it.n;
     uint32_t* h = scratch + ss->hist_off;
-    const long long last_nz = (long long)ss->last_nz1 - 1;
-    const uint64_t base0 = (uint64_t)u.chunk0 * kChunk;
-    const uint64_t end = split ? min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk) : (uint64_t)n;
-    long long carry = split ? (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.seg) - 1 : -1;
-    for (uint64_t base = base0; base < end; base += kChunk) {
-        const uint64_t p0 = base + (uint64_t)threadIdx.x * kPerThread;
+    // the workgroups of a segment (blockIdx.y) take its chunks in turn; an item in one unit has one
+    if (!split && blockIdx.y) return;
+    const uint32_t parts = split ? gridDim.y : 1u;
+    const uint64_t base0 = ((uint64_t)u.chunk0 + blockIdx.y) * kChunk;
+    const uint64_t end = split ? min((uint64_t)n, (uint64_t)(u.chunk0 + u.nchunk) * kChunk) : (uint64_t)n;
+    Syms8<S> next;
+    load8(in, base0 + threadIdx.x * kPerThread, n, next);
+    for (uint64_t base = base0; base < end; base += parts * kChunk) {
         uint32_t v[kPerThread];
-        load8(in, p0, n, v);
-        long long chunk_max;
-        long long prev = wg_excl_max_i64(thread_last_nz(v, p0, n), shl, chunk_max);
-        prev = prev > carry ? prev : carry;
-        thread_pairs(v, p0, n, rl, prev, rl ? last_nz : (long long)n,
-                     [&](uint32_t s, uint32_t) { atomicAdd(&h[s], 1u); });
-        carry = chunk_max > carry ? chunk_max : carry;
+        unpack8(next, v);
+        if (base + parts * kChunk < end) load8(in, base + parts * kChunk + threadIdx.x * kPerThread, n, next);
+#pragma unroll
+        for (int j = 0; j < (int)kPerThread; j++)
+            if (v[j] >= kStatBins) atomicAdd(&h[v[j]], 1u);
     }
     __syncthreads();
-    if (split && !last_arrival(U.split_state + (size_t)u.split * kSplitWords + 1, u.nseg, &shu[0])) return;
+    if (split && !last_arrival(U.split_state + (size_t)u.split * kSplitWords + 1, u.nseg * parts, &shu[0])) return;
     const uint32_t nb = ss->smax + 1;
     const uint32_t quirk = (p.dialect == CC_DIALECT_GPU && sizeof(S) == 2 && ss->smax == 65535u && (ss->count & 1u)) ? 1u : 0u;
+    // other workgroups' counts: loads at device scope, several under way at a time (past the end the last
+    // bin is loaded again)
     uint32_t k = 0;
-    for (uint32_t i = threadIdx.x; i < nb; i += kCoderThreads) {
-        uint32_t c = atomicAdd(&h[i], (quirk && i == 65535u) ? 1u : 0u);  // device-coherent read
-        if (quirk && i == 65535u) c++;
-        k += c ? 1u : 0u;
+    constexpr uint32_t kAtOnce = 16;
+    for (uint32_t i = threadIdx.x; i < nb; i += kAtOnce * kCoderThreads) {
+        uint32_t c[kAtOnce];
+#pragma unroll
+        for (uint32_t j = 0; j < kAtOnce; j++)
+            c[j] = __hip_atomic_load(&h[min(i + j * kCoderThreads, nb - 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (uint32_t j = 0; j < kAtOnce; j++) {
+            if (quirk && i + j * kCoderThreads == 65535u) h[65535] = ++c[j];
+            k += i + j * kCoderThreads < nb && c[j] ? 1u : 0u;
+        }
     }
     k = wg_sum_u32(k, shu);
     if (threadIdx.x == 0) {
@@ -1261,7 +1226,6 @@ __global__ __launch_bounds__(kCoderThreads) void k_seg_bits(const CodeItem* item
                                                             uint64_t out_cap, CodeUnits U) {
     __shared__ unsigned char lsh[kStatBins];
     __shared__ unsigned char lz[256];
-    __shared__ int shl[2][4];
     __shared__ uint64_t shq[4];
     if (st->out_base + st->out_words > out_cap) return;
     const CodeUnit u = U.units[U.split_list[blockIdx.x]];
@@ -1281,34 +1245,18 @@ __global__ __launch_bounds__(kCoderThreads) void k_seg_bits(const CodeItem* item
     const uint64_t end = min((uint64_t)n, base0 + (uint64_t)u.nchunk * kChunk);
     long long carry = (long long)seg_max_last(U.segs, u.slot0, u.slot0 + u.seg) - 1;
     const long long limit = rl ? (long long)ss.last_nz1 - 1 : (long long)n;
-    const uint32_t t8 = threadIdx.x * kPerThread;
     uint64_t bs = 0, bz = 0;
-    uint32_t par = 0;
-    Syms8<S> vn;
-    load8(in, base0 + t8, n, vn);
     __syncthreads();
-    for (uint64_t base = base0; base < end; base += kChunk, par ^= 1) {
-        uint32_t v[kPerThread];
-        unpack8(vn, v);
-        if (base + kChunk < end) load8(in, base + kChunk + t8, n, vn);
-        const uint32_t nvalid = chunk_nvalid(base, n, t8);
-        int wl;
-        const int ex = wave_excl_last(thread_last_nz_rel(v, t8, nvalid), wl);
-        if ((threadIdx.x & 63) == 0) shl[par][threadIdx.x >> 6] = wl;
-        __syncthreads();
-        int prel, ctot;
-        wg_last_combine(ex, shl[par], prel, ctot);
-        uint32_t zc[kPerThread];
-        const uint32_t emit = thread_flags_rel(v, nvalid, rl, thread_g0(prel, t8, chunk_gc(base, carry)),
-                                               chunk_lim(base, limit) - (int)t8, zc);
-#pragma unroll
-        for (int j = 0; j < (int)kPerThread; j++) {
-            const bool e = (emit >> j) & 1u;
-            if (e && !single) bs += sglob ? glen[v[j]] : (uint32_t)lsh[v[j]];
-            if (e && !zsingle) bz += lz[zc[j]];
-        }
-        if (ctot >= 0) carry = (long long)base + ctot;
-    }
+    auto add = [&](auto r) {
+        constexpr bool RL = decltype(r)::value;
+        (void)wave_pairs<RL, S>(in, n, base0, end, carry, limit, [&](bool e, uint32_t s, uint32_t z) {
+            const uint32_t l = sglob ? glen[s] : (uint32_t)lsh[s], k = RL ? lz[z] : 0u;  // in the tables, also if not e
+            bs += e && !single ? l : 0u;
+            bz += e && !zsingle ? k : 0u;
+        });
+    };
+    if (rl) add(std::true_type{});
+    else add(std::false_type{});
     bs = block_sum_u64<kCoderThreads>(bs, shq);
     bz = block_sum_u64<kCoderThreads>(bz, shq);
     if (threadIdx.x == 0) {
@@ -1378,13 +1326,60 @@ __global__ __launch_bounds__(kCoderThreads) void k_seg_increments(const CodeItem
     }
 }
 
+// A thread's codewords c (of l bits; none: 0 of 0) into the window from bit o on, one LDS OR per window
+// word touched (ring slot: output word mod kWindowWords).  Codewords are put together in 32-bit registers
+// first, as far as they fit for all lanes: eight as two words, then four words, then one by one.
+template <int N>
+__device__ __forceinline__ void put_words(uint32_t* win, uint32_t o, const uint32_t* c, const uint32_t* l) {
+    constexpr uint32_t WM = kWindowWords - 1;
+    uint32_t wi = o >> 5, nacc = o & 31;
+    uint64_t acc = 0;
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        acc = (acc << l[j]) | c[j];
+        nacc += l[j];
+        if (nacc >= 32) {
+            nacc -= 32;
+            atomicOr(&win[wi & WM], (uint32_t)(acc >> nacc));
+            wi++;
+        }
+    }
+    if (nacc) atomicOr(&win[wi & WM], (uint32_t)(acc << (32 - nacc)));
+}
+__device__ __forceinline__ void put_codes(uint32_t* win, uint32_t o, const uint32_t (&c)[kPerThread],
+                                          const uint32_t (&l)[kPerThread]) {
+    constexpr uint32_t WM = kWindowWords - 1;
+    uint32_t pc[4], pl[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) pl[i] = l[2 * i] + l[2 * i + 1];
+    const uint32_t l0 = pl[0] + pl[1], l1 = pl[2] + pl[3];
+    const bool pairs = max(max(pl[0], pl[1]), max(pl[2], pl[3])) <= 32u;
+    if (!__all(pairs)) {
+        put_words<8>(win, o, c, l);
+        return;
+    }
+    // a part of 32 bits has nothing before it: what a shift by 32 gives does not matter then
+#pragma unroll
+    for (int i = 0; i < 4; i++) pc[i] = (c[2 * i] << (l[2 * i + 1] & 31)) | c[2 * i + 1];
+    if (!__all(max(l0, l1) <= 32u)) {
+        put_words<4>(win, o, pc, pl);
+        return;
+    }
+    const uint32_t c0 = (pc[0] << (pl[1] & 31)) | pc[1], c1 = (pc[2] << (pl[3] & 31)) | pc[3];
+    const uint32_t bits = l0 + l1, sh = o & 31, wi = o >> 5;
+    const uint64_t t = (((uint64_t)c0 << l1) | c1) << ((64 - bits) & 63);  // from the top bit on
+    atomicOr(&win[wi & WM], (uint32_t)(t >> 32) >> sh);
+    if (sh + bits > 32) atomicOr(&win[(wi + 1) & WM], (uint32_t)(t >> sh));
+    if (sh + bits > 64) atomicOr(&win[(wi + 2) & WM], (uint32_t)t << (32 - sh));
+}
+
 // Pass B: pairs recomputed, codewords packed into an LDS window and flushed as whole words
 // straight to their place in the output section (laid out by k_layout_* from the designed bit
 // counts): each workgroup also writes its item's zero-run count, table headers and bit counts, and
 // after the pairs its packInc16 coding-block offsets (src/cudaCompress/PackInc.cu:210-220).  The
 // absolute bit offset of every coding block is kept in the arena for the increments.
 template <class S, bool Split>
-__global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* items, SeqInfo* seqs, CoderParams p,
+__global__ __launch_bounds__(kCoderThreads, 4) void k_code_pack(const CodeItem* items, SeqInfo* seqs, CoderParams p,
                                                              uint32_t* scratch, const CoderState* st, uint32_t* out,
                                                              uint64_t out_cap, CodeUnits U) {
     __shared__ uint32_t cs[kStatBins];
@@ -1485,9 +1480,10 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
         load8(in, base0 + t8, n, v);
         load8(in, base0 + t8 + kChunk, n, vn);
         int prel, ctot;  // this chunk: the exclusive chunk-relative last nonzero, the chunk's last
+        uint32_t nz = nonzeros(v);
         {
             int wl;
-            const int ex = wave_excl_last(thread_last_nz_rel(v, t8, chunk_nvalid(base0, n, t8)), wl);
+            const int ex = wave_excl_last(last_nz_rel(nz, t8), wl);
             if (lane == 0) shl[wv] = wl;
             __syncthreads();
             wg_last_combine(ex, shl, prel, ctot);
@@ -1502,25 +1498,34 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
             for (uint64_t base = base0; base < end && pairs < M; base += kChunk) {
                 Syms8<S> vnn;
                 if (base + 2 * kChunk < end) load8(in, base + 2 * kChunk + t8, n, vnn);
-                const uint32_t nvalid = chunk_nvalid(base, n, t8);
-                // this thread's pairs; code lengths looked up once for both the scan and the packing
+                // this thread's pairs; code lengths looked up once for both the scan and the packing.
+                // Where no lane's zero run can reach 255 (any stream but a sparse one) the nonzeros are
+                // the pairs
                 uint32_t zc[kPerThread], ls[kPerThread], lzs[kPerThread];
-                const uint32_t emit = thread_flags_rel(v, nvalid, rl, thread_g0(prel, t8, chunk_gc(base, carry)),
-                                                       chunk_lim(base, limit) - (int)t8, zc);
+                uint32_t g = thread_g0(prel, t8, chunk_gc(base, carry)), emit = nz;
+                if (rl && __all(g < 256u - kPerThread)) {
+#pragma unroll
+                    for (int j = 0; j < (int)kPerThread; j++) {
+                        zc[j] = g;
+                        g = (g + 1u) & ~bit_mask(nz, j);
+                    }
+                } else {
+                    emit = thread_flags_rel(v, chunk_nvalid(base, n, t8), rl, g, chunk_lim(base, limit) - (int)t8, zc);
+                }
+                const uint32_t emit_s = single ? 0u : emit, emit_z = rl && !zsingle ? emit : 0u;  // pairs with a codeword
                 uint32_t nbs = 0, nbz = 0;
                 // table reads issued together, unconditionally (symbols and zero counts index inside
                 // the tables; a length is then zeroed where no pair is emitted)
 #pragma unroll
                 for (int j = 0; j < (int)kPerThread; j++) {
-                    if (SG) ls[j] = (((emit >> j) & 1u) && !single) ? glen[v[j]] : 0u;
+                    if (SG) ls[j] = ((emit_s >> j) & 1u) ? glen[v[j]] : 0u;
                     else ls[j] = lsh[v[j]];
                     lzs[j] = lz[zc[j]];
                 }
 #pragma unroll
                 for (int j = 0; j < (int)kPerThread; j++) {
-                    const bool e = (emit >> j) & 1u;
-                    ls[j] = (e && !single) ? ls[j] : 0u;
-                    lzs[j] = (e && rl && !zsingle) ? lzs[j] : 0u;
+                    if (!SG) ls[j] &= bit_mask(emit_s, j);
+                    lzs[j] &= bit_mask(emit_z, j);
                     nbs += ls[j];
                     nbz += lzs[j];
                 }
@@ -1528,8 +1533,8 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
                 // pair/bit-count scan, and the next chunk's last nonzeros, over one barrier
                 const bool more = base + kChunk < end;
                 int wl;
-                const int exn =
-                    wave_excl_last(more ? thread_last_nz_rel(vn, t8, chunk_nvalid(base + kChunk, n, t8)) : -1, wl);
+                const uint32_t nzn = more ? nonzeros(vn) : 0u;
+                const int exn = wave_excl_last(last_nz_rel(nzn, t8), wl);
                 const uint64_t a = ((uint64_t)np << 40) | ((uint64_t)nbs << 20) | nbz;
                 const uint64_t xa = wave_incl_scan_u64(a);
                 if (lane == 63) shq[wv] = xa;
@@ -1568,50 +1573,23 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
                         bs[blk] = os;
                         if (rl) bz[blk] = oz;
                     }
-                    // codewords through a 64-bit accumulator, one LDS OR per window word touched
-                    // (ring slot: output word mod kWindowWords)
+                    uint32_t cw[kPerThread];
                     if (!single) {
-                        uint32_t wi = os0 >> 5, nacc = os0 & 31;
-                        uint64_t acc = 0;
-                        uint32_t cw[kPerThread];
 #pragma unroll
                         for (int j = 0; j < (int)kPerThread; j++) {
                             if (SG) cw[j] = ls[j] ? gcode[v[j]] : 0u;
                             else cw[j] = cs[v[j]];
                         }
 #pragma unroll
-                        for (int j = 0; j < (int)kPerThread; j++) {
-                            const uint32_t l = ls[j];
-                            const uint32_t c = l ? cw[j] : 0u;
-                            acc = (acc << l) | c;
-                            nacc += l;
-                            if (nacc >= 32) {
-                                nacc -= 32;
-                                atomicOr(&win[0][wi & WM], (uint32_t)(acc >> nacc));
-                                wi++;
-                            }
-                        }
-                        if (nacc) atomicOr(&win[0][wi & WM], (uint32_t)(acc << (32 - nacc)));
+                        for (int j = 0; j < (int)kPerThread; j++) cw[j] &= bit_mask(emit_s, j);
+                        put_codes(win[0], os0, cw, ls);
                     }
                     if (rl && !zsingle) {
-                        uint32_t wi = oz0 >> 5, nacc = oz0 & 31;
-                        uint64_t acc = 0;
-                        uint32_t cw[kPerThread];
 #pragma unroll
                         for (int j = 0; j < (int)kPerThread; j++) cw[j] = cz[zc[j]];
 #pragma unroll
-                        for (int j = 0; j < (int)kPerThread; j++) {
-                            const uint32_t l = lzs[j];
-                            const uint32_t c = l ? cw[j] : 0u;
-                            acc = (acc << l) | c;
-                            nacc += l;
-                            if (nacc >= 32) {
-                                nacc -= 32;
-                                atomicOr(&win[1][wi & WM], (uint32_t)(acc >> nacc));
-                                wi++;
-                            }
-                        }
-                        if (nacc) atomicOr(&win[1][wi & WM], (uint32_t)(acc << (32 - nacc)));
+                        for (int j = 0; j < (int)kPerThread; j++) cw[j] &= bit_mask(emit_z, j);
+                        put_codes(win[1], oz0, cw, lzs);
                     }
                 }
                 __syncthreads();
@@ -1639,6 +1617,7 @@ __global__ __launch_bounds__(kCoderThreads) void k_code_pack(const CodeItem* ite
                 if (ctot >= 0) carry = (long long)base + ctot;
                 prel = prel_n;
                 ctot = ctot_n;
+                nz = nzn;
 #pragma unroll
                 for (int j = 0; j < (int)kPerThread; j++) v[j] = vn[j];
                 unpack8(vnn, vn);
@@ -1802,7 +1781,9 @@ void coder_stats(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, cons
                        d_items, d_seqs, p, scratch, scratch_cap, d_state, U);
             CCA_LAUNCH_CHECK();
         }
-        CCA_LAUNCH("code_stats_wide", 0, k_code_stats_wide<S>, dim3(U.nunits), dim3(kCoderThreads), 0, st, d_items,
+        // what a workgroup has in global atomics under way bounds it, so a segment's chunks are spread
+        const uint32_t parts = U.nsplit ? std::min(U.unit_chunks, 8u) : 1u;
+        CCA_LAUNCH("code_stats_wide", 0, k_code_stats_wide<S>, dim3(U.nunits, parts), dim3(kCoderThreads), 0, st, d_items,
                    d_seqs, p, scratch, U);
         CCA_LAUNCH_CHECK();
     };

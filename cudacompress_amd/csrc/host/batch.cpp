@@ -75,6 +75,7 @@ void encode_upload(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>& 
     check_symbols(I, symSize);
     const uint32_t nitems = (uint32_t)items.size();
     const uint32_t per_unit = unit_chunks(items);
+    job.unit_chunks = per_unit;
     auto segments = [&](const ItemSpec& it) { return std::max(1u, div_up(div_up(it.n, kChunk), per_unit)); };
     uint32_t nunits = 0, nsplit = 0, nslots = 0;
     for (const ItemSpec& it : items) {
@@ -146,7 +147,7 @@ namespace {
 CodeUnits units_of(const DeviceCoder& D, const EncodeJob& job) {
     const unsigned char* d = (const unsigned char*)D.d_items.p;
     return CodeUnits{(const CodeUnit*)(d + job.o_units), job.nunits, (const uint32_t*)(d + job.o_split),
-                     job.nsplit_units, job.nsplit, (SegState*)D.d_split.p,
+                     job.nsplit_units, job.nsplit, job.unit_chunks, (SegState*)D.d_split.p,
                      (uint32_t*)((unsigned char*)D.d_split.p + sizeof(SegState) * job.nsplit_units)};
 }
 }  // namespace

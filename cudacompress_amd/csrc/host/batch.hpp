@@ -38,6 +38,7 @@ struct EncodeJob {
     // the upload: items, the first item of every call, the units, the list of split ones (byte offsets)
     size_t o_first = 0, o_units = 0, o_split = 0;
     uint32_t nunits = 0, nsplit_units = 0, nsplit = 0;
+    uint32_t unit_chunks = 0;    // most chunks of a segment
     uint32_t design_grid[4] = {4096, 2048, 1536, 768};  // resident workgroups per design class
     uint32_t lane_k = 0;  // tables of at most this many symbols are designed one per thread (0: none)
 };
