@@ -273,13 +273,13 @@ __global__ __launch_bounds__(256) void k_bfwd(const BrickLevel* lv, const uint32
                  [&](int, int, int off, float v) { gst(dst, off, v); });
 }
 
-// Z passes: one thread per column (x, y) of the brick level and per segment of kBrickZP output
+// Z passes: one thread per column (x, y) of the brick level and per segment of zseg output
 // pairs along z.  The 10-sample filter window streams through registers (no LDS, no barrier); a
 // segment reads its z range once plus the filter halo.  A workgroup is one wave of NC columns,
 // numbered band-major (the columns of octant quarter bx + 2 by of the xy plane, then y, then x
 // inside it), so the lanes of a wave read and write consecutive elements of one band (and, for a
 // level whose quarter holds a multiple of NC columns, all serve one quarter: the lowpass quarter's
-// loads and stores differ from the highpass ones).  Tiles (NC columns x kBrickZP pairs) are those
+// loads and stores differ from the highpass ones).  Tiles (NC columns x zseg pairs) are those
 // of brick_tiles along z.  The window and the fmaf order are those of the tiled passes (Fwd97::pair
 // over positions 2q - 4 .. 2q + 5, Inv97::out over interleaved pairs u - 2 .. u + 2), so the
 // results are identical.
@@ -293,11 +293,11 @@ struct ZColumn {
     int q;          // quarter bx + 2 by (-1: past the level's columns)
     uint32_t r;     // (y - by hy) hx + (x - bx hx): offset inside a band plane
     uint32_t xy;    // y lx + x: offset inside a dense plane
-    __device__ ZColumn(const Geo<2>& g, uint32_t local, int hx, int hy) {
+    __device__ ZColumn(const Geo<2>& g, uint32_t local, int hx, int hy, int seg) {
         const int ctiles = (g.ncols + NC - 1) / NC;
         const int c = (int)(local % (uint32_t)ctiles) * NC + (int)threadIdx.x;
-        k0 = (int)(local / (uint32_t)ctiles) * kBrickZP;
-        k1 = min(k0 + kBrickZP, g.m);
+        k0 = (int)(local / (uint32_t)ctiles) * seg;
+        k1 = min(k0 + seg, g.m);
         const int hxy = hx * hy;
         q = c < g.ncols ? c / hxy : -1;
         const int rr = c - q * hxy, yq = rr / hx, xq = rr - yq * hx;
@@ -377,7 +377,7 @@ __global__ __launch_bounds__(NC) void k_bfwd_zq(const BrickLevel* lv, const uint
     const Geo<2> g(L.lx, L.ly, L.lz);
     const int hx = L.lx / 2, hy = L.ly / 2, hxy = hx * hy;
     const uint32_t band = (uint32_t)hxy * (uint32_t)g.m;
-    const ZColumn zc(g, w - tb[i], hx, hy);
+    const ZColumn zc(g, w - tb[i], hx, hy, L.zseg);
     if (zc.q < 0) return;
     S* hp = static_cast<S*>(L.hp);
     const uint32_t ihi = (uint32_t)(zc.q + 3) * band + zc.r;
@@ -458,7 +458,7 @@ __global__ __launch_bounds__(NC) void k_binv_zs(const BrickLevel* lv, const uint
     const Geo<2> g(L.lx, L.ly, L.lz);
     const int hx = L.lx / 2, hy = L.ly / 2, hxy = hx * hy;
     const uint32_t band = (uint32_t)hxy * (uint32_t)g.m;
-    const ZColumn zc(g, w - tb[i], hx, hy);
+    const ZColumn zc(g, w - tb[i], hx, hy, L.zseg);
     if (zc.q < 0) return;
     const S* hp = static_cast<const S*>(L.hp);
     const uint32_t ihi = (uint32_t)(zc.q + 3) * band + zc.r;
@@ -524,8 +524,8 @@ struct XYTile {
         my = ny / 2;
         const int zg = (L.lz + L.zk - 1) / L.zk;
         const int z0 = (int)(local % (uint32_t)zg) * L.zk;
-        k0 = (int)(local / (uint32_t)zg) * kBrickXYSeg;
-        k1 = min(k0 + kBrickXYSeg, my);
+        k0 = (int)(local / (uint32_t)zg) * L.yseg;
+        k1 = min(k0 + L.yseg, my);
         zk = min(L.zk, L.lz - z0);
         s = (int)threadIdx.x / mx;
         k = (int)threadIdx.x - s * mx;

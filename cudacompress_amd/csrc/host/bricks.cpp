@@ -109,6 +109,21 @@ void upload_levels(BrickCtx& ctx, BrickJob& job, float* work, unsigned char* sym
         // keeps them on)
         bool fused = tune.fusedXY != 0;
         for (uint32_t i = 0; i < n; i++) fused = fused && brick_xy_fits((int)(job.bricks[i].sizeX >> l));
+        auto slices = [&](const cc_brick& b) {  // z-slices per workgroup of the fused passes
+            const uint32_t zk = std::min<uint32_t>(b.sizeZ >> l, brick_xy_slices((int)(b.sizeX >> l)));
+            return !fused ? 0u : tune.xySlicesMax ? std::min(zk, tune.xySlicesMax) : zk;
+        };
+        auto level_tiles = [&](auto brick) {
+            uint32_t t = 0;
+            for (const cc_brick& b : job.bricks) t += brick((int)(b.sizeX >> l), (int)(b.sizeY >> l), (int)(b.sizeZ >> l), b);
+            return t;
+        };
+        const int zseg = brick_segment(kBrickZTilesWanted, [&](int s) {
+            return level_tiles([&](int x, int y, int z, const cc_brick&) { return brick_tiles(2, x, y, z, s); });
+        });
+        const int yseg = !fused ? kBrickSegMax : brick_segment(kBrickXYTilesWanted, [&](int s) {
+            return level_tiles([&](int, int y, int z, const cc_brick& b) { return brick_xy_tiles(y, z, (int)slices(b), s); });
+        });
         uint32_t acc[4] = {0, 0, 0, 0};
         for (uint32_t i = 0; i < n; i++) {
             const cc_brick& b = job.bricks[i];
@@ -131,12 +146,12 @@ void upload_levels(BrickCtx& ctx, BrickJob& job, float* work, unsigned char* sym
             e.inv_hp = 1.0f / e.step_hp;      // Quantize.cu:94
             e.step_lp = q0 / float(1u << (L - 1));
             e.inv_lp = 1.0f / e.step_lp;
-            uint32_t zk = fused ? std::min<uint32_t>((uint32_t)e.lz, brick_xy_slices(e.lx)) : 0u;
-            if (fused && tune.xySlicesMax) zk = std::min(zk, tune.xySlicesMax);
-            e.zk = (int)zk;
+            e.zk = (int)slices(b);
+            e.yseg = yseg;
+            e.zseg = zseg;
             for (int ax = 0; ax < 4; ax++) {
                 ht[((size_t)l * 4 + ax) * (n + 1) + i] = acc[ax];
-                acc[ax] += ax < 3 ? brick_tiles(ax, e.lx, e.ly, e.lz) : (fused ? brick_xy_tiles(e.ly, e.lz, e.zk) : 0u);
+                acc[ax] += ax < 3 ? brick_tiles(ax, e.lx, e.ly, e.lz, zseg) : (fused ? brick_xy_tiles(e.ly, e.lz, e.zk, yseg) : 0u);
             }
         }
         for (int ax = 0; ax < 4; ax++) {
