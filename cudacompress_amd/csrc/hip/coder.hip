@@ -14,6 +14,7 @@
 
 #include "../coder.hpp"
 #include "../profile.hpp"
+#include "arrival.hpp"
 #include "huff_design.hpp"
 #include "wave.hpp"
 
@@ -373,14 +374,22 @@ __device__ __forceinline__ SegState seg_before(const SegState* segs, uint32_t lo
 // Whether this workgroup is the last of n to arrive; what the others did with device-scope atomics before
 // is done then.  Atomics are performed where every workgroup sees them, so it is enough that a wave waits
 // for its own; a fence would also write the cache back, 0.9 ms for the 16 to 128 workgroups of a 4096^2
-// terrain's lowpass band.  Plain stores are not covered.
+// terrain's lowpass band.  Plain stores are not covered.  *sh is free again when it returns.
+struct ArrivalEx {
+    uint32_t* counter;
+    uint32_t* sh;
+    __device__ __forceinline__ void arrive() const {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+    }
+    __device__ __forceinline__ void barrier() const { __syncthreads(); }
+    __device__ __forceinline__ bool leader() const { return threadIdx.x == 0; }
+    __device__ __forceinline__ uint32_t count() const { return atomicAdd(counter, 1u); }
+    __device__ __forceinline__ void put(uint32_t v) const { *sh = v; }
+    __device__ __forceinline__ uint32_t get() const { return *sh; }
+};
 __device__ __forceinline__ bool last_arrival(uint32_t* counter, uint32_t n, uint32_t* sh) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0) *sh = atomicAdd(counter, 1u);
-    __syncthreads();
-    return *sh == n - 1;
+    return last_of(ArrivalEx{counter, sh}, n);
 }
 
 // Words of a histogram of nb bins in the arena and, when the table may be designed one per thread
