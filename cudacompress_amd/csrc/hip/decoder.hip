@@ -404,8 +404,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     // the run row and the codeword copy are also accessed as words / 16-byte vectors
     typedef uint32_t __attribute__((may_alias)) u32a;
     uint32_t* win = &win_all[wave][lane];  // the copy's word k at win[64 k]: a lane's own bank
+    // A lane past the sequence's last block decodes that block along and stores nothing: every lane of a
+    // wave then takes every step, so that what the wave votes on or reads by lane number is there.
     const uint32_t b = fb + lane;
     const bool valid = b < nblk;
+    const uint32_t bl = min(b, nblk - 1);
     // the zero counts of an RLE item also give the zero-run expansion its chunk spans: the sum of
     // (count + 1) over each chunk of kRleChunk pairs (kRleChunk / cbs whole blocks, a power of two
     // dividing the wave's 64 blocks)
@@ -419,8 +422,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     // the block's stream
     uint32_t hi = 0, lo = 0, nx = 0, nxt = 0;
     int q = 0, w0 = 0;
-    if (valid && multi) {
-        const uint32_t pos = b == 0 ? 0u : scratch[s.boff_off + b];
+    if (multi) {
+        const uint32_t pos = bl == 0 ? 0u : scratch[s.boff_off + bl];
         const uint32_t wi = pos >> 5, b0 = pos & 31u;
         if (b0 == 0) {
             lo = word(wi);
@@ -439,9 +442,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     auto load_window = [&]() {
         const auto gp = (Global<const uint32_t>)(reinterpret_cast<uintptr_t>(words + nxt) & ~uintptr_t(15));
         w0 = (int)nxt - (int)(words + nxt - gp);
-        const bool fast = !(valid && multi) || gp + kWinWords <= cend;
+        const bool fast = !multi || gp + kWinWords <= cend;
         if (__all(fast)) {
-            if (valid && multi) {
+            if (multi) {
                 // a global-space pointer: the loads cannot alias the LDS stores, so all of them
                 // are issued before the first store waits
                 const Global<const u32x4> g4 = (Global<const u32x4>)gp;
@@ -451,14 +454,14 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
 #pragma unroll
                 for (uint32_t k = 0; k < kWinWords; k++) win[64 * k] = v[k / 4][k % 4];
             }
-        } else if (valid && multi) {
+        } else if (multi) {
 #pragma unroll
             for (uint32_t k = 0; k < kWinWords; k++) {
                 const int i = w0 + (int)k;
                 win[64 * k] = (i >= 0 && (uint64_t)i < avail) ? words[i] : 0u;
             }
         }
-        if (valid && multi) nx = win[64 * (nxt - (uint32_t)w0)];
+        if (multi) nx = win[64 * (nxt - (uint32_t)w0)];
     };
     load_window();
 #pragma unroll
@@ -473,13 +476,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     // words a round may take, at most R (mlen <= 31); the copy serves a round when it holds as many
     // from nxt on and the one read ahead (an entry no code of a broken table reaches takes kLut + 1 bits)
     const uint32_t round_words = min((kDecRound * max(s.nlen, kLut + 1) + 31) / 32 + 1, kDecRound);
-    auto refill = [&]() {
-        const bool need = q < 0;
+    auto refill = [&](bool on) {
+        const bool need = on && q < 0;
         hi = need ? lo : hi;
         lo = need ? nx : lo;
         nxt += need ? 1u : 0u;
         nx = win[64 * (nxt - (uint32_t)w0)];  // on its way beside the code's table lookup
-        q &= 31;
+        q = on ? q & 31 : q;
     };
     const uint32_t sh = 32 - lb;
     const uint32_t mlen = s.nlen;
@@ -487,7 +490,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     // ones to 32 bits, is not below the next 32 bits, and its symbol is number (code - first code +
     // first index) of the symbol table.  Lane l - 1 holds length l's bound (an unused length has the
     // one before it) and the step of the index offset from l to l + 1, read by lane number, so the
-    // lookup is a few vector instructions a length and touches no memory.
+    // lookup is a few vector instructions a length and touches no memory.  All lanes of the wave take it
+    // together, those without such a code with zero bits (never past a bound): a register of a lane that
+    // is masked off need not hold what the lane would have computed.
     const bool used = multi && lane < (int)mlen && lane < 32 && tab[64 + (lane & 31)] >= 0;
     uint32_t len0 = kLut + 1;  // the first used length past the lookup table (the last length if none)
     uint32_t bound = 0;
@@ -561,12 +566,17 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
 #pragma unroll
                 for (uint32_t k = 0; k < NW; k++) reinterpret_cast<u32a*>(run_row)[k] = fill;
                 uint32_t i = 0;
-                while (i < kDecRound) {
-                    refill();
+                // (a lane that is done takes runs of no position until the last one is)
+                while (__any(i < kDecRound)) {
+                    refill(i < kDecRound);
                     const uint32_t pk = __builtin_amdgcn_alignbit(hi, lo, (uint32_t)q);
-                    const bool run = (pk >> 31) == 0u;
+                    const bool run = (pk >> 31) == 0u || i >= kDecRound;
                     uint32_t e = lut[pk >> sh];
-                    if (!run && e == 0u) e = slow(pk);
+                    const bool is_long = !run && e == 0u;
+                    if (__any(is_long)) {
+                        const uint32_t found = slow(is_long ? pk : 0u);
+                        e = is_long ? found : e;
+                    }
                     const uint32_t k = min(pk ? (uint32_t)__clz(pk) : 32u, kDecRound - i);
                     const uint32_t sym = !run && (e & kLong) ? long_symbol(e) : e & 0xFFFFFFu;
                     if (!run) run_row[i] = (S)sym;
@@ -583,10 +593,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
                 uint32_t es[kDecRound], any = 0;
 #pragma unroll
                 for (uint32_t i = 0; i < kDecRound; i++) {
-                    refill();
+                    refill(true);
                     const uint32_t pk = __builtin_amdgcn_alignbit(hi, lo, (uint32_t)q);
                     uint32_t e = lut[pk >> sh];
-                    if (e == 0u) e = slow(pk);
+                    if (__any(e == 0u)) {
+                        const uint32_t found = slow(e ? 0u : pk);
+                        e = e ? e : found;
+                    }
                     q -= (int)((e >> 24) & 31u);
                     es[i] = e;
                     any |= e;
@@ -636,14 +649,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
         }
         return zs;
     };
-    // (lanes without a block stay out: their words are not theirs to read)
     if (zsum) {
-        uint32_t zs = valid ? rounds(std::true_type{}) : 0u;
+        uint32_t zs = rounds(std::true_type{});
         const uint32_t bpc = kRleChunk / cbs;
         for (uint32_t o = 1; o < bpc; o <<= 1) zs += (uint32_t)__shfl_xor((int)zs, (int)o);
         const uint32_t c = b / bpc;
         if ((lane & (bpc - 1)) == 0 && c < (count + kRleChunk - 1) / kRleChunk) rc.sums[rc.item_first[s.item] + c] = zs;
-    } else if (valid) {
+    } else {
         (void)rounds(std::false_type{});
     }
 }

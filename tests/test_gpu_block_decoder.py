@@ -57,3 +57,33 @@ def test_flat_codes(cc, torch_gpu, width):
     torch.cuda.synchronize()
     assert np.array_equal(to_host(out, np.uint16), sym)
     inst.close()
+
+
+@pytest.mark.parametrize("runs", [True, False], ids=["runs", "plain"])
+@pytest.mark.parametrize("depth,blocks", [(11, 2), (12, 3), (14, 7), (18, 43), (19, 70)])
+def test_long_codes_in_a_wave_of_few_blocks(cc, torch_gpu, depth, blocks, runs):
+    """Codes of up to `depth` bits (the lookup table holds 10) in blocks of 256 symbols, so that most lanes of
+    the last wave have no block of their own: Fibonacci counts, whose codes have every length from one bit on
+    (runs of that code are taken at once), or with the commonest symbol as two, which has no such code."""
+    torch = torch_gpu
+    counts = [1, 1]
+    while len(counts) < depth + 1:
+        counts.append(counts[-1] + counts[-2])
+    if not runs:
+        counts[-1:] = [counts[-1] // 2, counts[-1] - counts[-1] // 2]
+    rng = np.random.default_rng(depth)
+    sym = np.repeat(np.arange(1, len(counts) + 1, dtype=np.uint16) * 37, counts)
+    n = sym.size
+    assert -(-n // 256) == blocks
+    print("block decoder, few blocks", n, depth, runs, flush=True)
+    rng.shuffle(sym)
+    inst = cc.createInstance(0, 1, n, 256, 14)
+    for rl in (False, True):
+        words, _ = o.encode([sym], rl=rl, log2=14, cbs=256)
+        lengths = words[0 if not rl else 1] >> 27  # a table's header starts with its longest code's length
+        assert lengths == depth - (not runs)
+        out = torch.full((n,), -1, dtype=torch.int16, device="cuda")
+        cc.decodeDevice(inst, rl, to_dev(torch, words.astype(np.uint32)), [out], n)
+        torch.cuda.synchronize()
+        assert np.array_equal(to_host(out, np.uint16), sym)
+    inst.close()
