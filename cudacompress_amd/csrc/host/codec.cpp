@@ -279,6 +279,9 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
         s.sb = r.bits(fmt.symbits_bits);
         // HuffmanTable.cu:138-139: a stored 0 with more than one symbol means 16 (Symbol16 only)
         if (fmt.dialect == CC_DIALECT_GPU && fmt.symbits_bits == 4 && s.sb == 0 && s.nsym > 1) s.sb = 16;
+        // lengths without a symbol code nothing: an empty table (the device refuses lengths and symbols that
+        // do not fit, and would leave the output of a stream without a pair as it is)
+        if (s.nsym == 0) s.nlen = 0;
         CCA_REQUIRE(s.sb <= 32 && r.ok(), CC_ERR_CORRUPT_STREAM, "malformed Huffman table header");
         s.sym_bit = r.pos();
         r.skip_bits((uint64_t)s.sb * s.nsym);

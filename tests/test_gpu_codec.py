@@ -195,3 +195,27 @@ def test_cpu_dialect_matches_reference_cpu_coder(cc, torch_gpu):
         for a, b in zip(dec, streams):
             assert np.array_equal(a, b)
     inst.close()
+
+
+@pytest.mark.parametrize("rl", [True, False], ids=["rlhuff", "huff"])
+def test_table_of_lengths_without_symbols(cc, torch_gpu, rl):
+    """A table that states code lengths and no symbol is as good as an empty one where nothing is coded by it:
+    a run-length stream without a pair still has its output written."""
+    log("table of lengths without symbols, rl", rl)
+    n = 1000 if rl else 0
+    bits = cc.BitStream()
+    if rl:
+        bits.writeAligned(np.zeros(1, np.uint32))  # no pair
+    for _ in range(2 if rl else 1):
+        for value, width in ((2, 5), (1, 14), (2, 14), (0, 14), (3, 4)):  # two lengths, their counts, no symbol
+            bits.writeBits(value, width)
+        bits.writeAligned(np.zeros(1, np.uint32))  # no codeword
+    bits.setBitPosition(0)
+    inst = cc.createInstance(0, 1, 1000, 128, 14)
+    out = torch_gpu.full((1000,), -1, dtype=torch_gpu.int16, device="cuda")
+    ok = (cc.decodeRLHuff if rl else cc.decodeHuff)(inst, bits, [out], n)
+    torch_gpu.cuda.synchronize()
+    assert ok is not False and bits.getBitPosition() == bits.getBitSize()
+    got = out.cpu().numpy()
+    assert np.all(got[:n] == 0) and np.all(got[n:] == -1)
+    inst.close()
