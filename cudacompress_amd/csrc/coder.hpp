@@ -252,12 +252,19 @@ void coder_decode(const DecCall* d_calls, uint32_t ncalls, const DecItem* d_item
                   CoderState* d_state, DecCallOut* d_out, const uint32_t* d_wave_seq, const uint32_t* d_wave_first,
                   uint32_t nwaves, uint32_t nlong, uint64_t total_symbols, const RleChunks& rc,
                   hipStream_t st);
+// Work of one workgroup of the table build for sequences parsed on the host: symbols
+// [2^kDecLutBits + part kPartSymbols, + kPartSymbols) and block offsets from part kPartBlocks on, which start
+// at carry; part 0 has the tables too.
+struct DecPart {
+    uint32_t seq, part, carry, pad;
+};
+constexpr uint32_t kPartSymbols = 2048, kPartBlocks = 4096;
 // The same stages for sequences parsed on the host (records with the positions, counts, outputs and
 // arena ranges filled in): tables and block decode, then the zero-run expansion.
 void coder_decode_parsed(DecSeq* d_seqs, uint32_t nseq, const CoderParams& p, int symSize, uint32_t* scratch,
                          CoderState* d_state, const DecItem* d_items, const uint32_t* d_wave_seq,
-                         const uint32_t* d_wave_first, uint32_t nwaves, uint32_t nlong, uint64_t total_symbols,
-                         const RleChunks& rc, hipStream_t st);
+                         const uint32_t* d_wave_first, uint32_t nwaves, uint32_t nlong, const DecPart* d_parts,
+                         uint32_t nparts, uint64_t total_symbols, const RleChunks& rc, hipStream_t st);
 void coder_decode_expand(const DecItem* d_items, uint32_t nitems, DecSeq* d_seqs, int symSize, const RleChunks& rc,
                          CoderState* d_state, uint64_t total_symbols, hipStream_t st);
 // Resident decode index: parse + tables of every call once (RLE sequences get no decode buffer),

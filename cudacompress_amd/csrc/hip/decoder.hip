@@ -209,21 +209,33 @@ __global__ __launch_bounds__(64) void k_dec_parse(const DecCall* calls, uint32_t
 }
 
 // One workgroup per coded sequence: first/min/max codeword per length (closed form of the
-// canonical assignment) and absolute coding-block offsets.
-__global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, CoderParams p, uint32_t* scratch,
-                                                    CoderState* st) {
+// canonical assignment), symbol table and absolute coding-block offsets.  Parts: the host has walked the
+// heads, and a sequence of many symbols or blocks comes as several workgroups, part 0 with the tables;
+// each takes its symbols past the lookup table's and its block offsets, which start at a sum that the
+// host gives.  One workgroup a sequence took 3.7 us for every 256 symbols of a table and 1.6 us for every
+// 1024 blocks, each waited for.  On the plain calls' decode, before and now: one stream of 10^6 symbols of
+// 65,000 values 235 and 20 us, of 971,000 values 3,538 and 24 us, 3 * 10^6 symbols of 8,000 values 77 and
+// 21 us, few values and as many symbols 36 and 16 us.
+template <bool Parts>
+__global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, const DecPart* parts, CoderParams p,
+                                                    uint32_t* scratch, CoderState* st) {
     constexpr uint32_t kSymPer = (1u << kLut) / 256;  // symbols per thread read up front
     __shared__ uint32_t cpl[32];
     __shared__ uint32_t sh[4];
     __shared__ uint32_t bad;
     __shared__ int tab_sh[96];
     __shared__ uint32_t sym_lo[1 << kLut];
-    DecSeq& s = seqs[blockIdx.x];
+    const DecPart part = Parts ? parts[blockIdx.x] : DecPart{blockIdx.x, 0, 0, 0};
+    DecSeq& s = seqs[part.seq];
     if (s.err) return;
+    const uint32_t nblk = (s.count + p.cbs - 1) / p.cbs;
+    const uint32_t b0 = part.part * kPartBlocks, b1 = Parts ? min(b0 + kPartBlocks, nblk) : nblk;
+    const uint32_t tail0 = (1u << kLut) + part.part * kPartSymbols, tail1 = Parts ? min(tail0 + kPartSymbols, s.nsym) : s.nsym;
     // every independent header read is issued before the first barrier: the code-length counts,
     // the first 2^kLut symbols and the first 1024 block-offset increments
     bool ok = true;
-    const uint32_t cplv = threadIdx.x < s.nlen
+    const bool head = part.part == 0;
+    const uint32_t cplv = head && threadIdx.x < s.nlen
                               ? rd_bits(s.base, s.nwords, s.hdr_bit + 5 + (uint64_t)p.count_bits * threadIdx.x,
                                         p.count_bits, ok)
                               : 0u;
@@ -231,21 +243,20 @@ __global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, CoderParams p,
 #pragma unroll
     for (uint32_t j = 0; j < kSymPer; j++) {
         const uint32_t k = threadIdx.x + 256 * j;
-        symv[j] = k < s.nsym ? rd_bits(s.base, s.nwords, s.sym_bit + (uint64_t)s.sb * k, s.sb, ok) : 0u;
+        symv[j] = head && k < s.nsym ? rd_bits(s.base, s.nwords, s.sym_bit + (uint64_t)s.sb * k, s.sb, ok) : 0u;
     }
-    const uint32_t nblk = (s.count + p.cbs - 1) / p.cbs;
     const uint32_t* inc = s.base + s.incs_off;
     uint32_t incv[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const uint32_t b = threadIdx.x * 4 + k;
-        incv[k] = b < nblk ? (inc[b >> 1] >> (16 * (b & 1))) & 0xFFFFu : 0u;
+        const uint32_t b = b0 + threadIdx.x * 4 + k;
+        incv[k] = b < b1 ? (inc[b >> 1] >> (16 * (b & 1))) & 0xFFFFu : 0u;
     }
     if (threadIdx.x == 0) bad = 0;
     if (threadIdx.x < 32) cpl[threadIdx.x] = cplv;
     __syncthreads();
     if (!ok) atomicOr(&bad, 1u);
-    if (threadIdx.x == 0) {
+    if (head && threadIdx.x == 0) {
         uint32_t fc[32], fi[32];
         design::first_codes(cpl, (int)s.nlen, fc, fi);
         uint64_t total = 0;
@@ -265,21 +276,29 @@ __global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, CoderParams p,
 #pragma unroll
     for (uint32_t j = 0; j < kSymPer; j++) {
         const uint32_t k = threadIdx.x + 256 * j;
-        if (k < s.nsym) {
+        if (head && k < s.nsym) {
             gsyms[k] = symv[j];
             sym_lo[k] = symv[j];
         }
     }
-    for (uint32_t k = threadIdx.x + (1u << kLut); k < s.nsym; k += 256) {
+    constexpr uint32_t kTail = kPartSymbols / 256;  // symbols of a thread under way at a time
+    for (uint32_t k0 = tail0 + threadIdx.x; k0 < tail1; k0 += kPartSymbols) {
         bool ok2 = true;
-        gsyms[k] = rd_bits(s.base, s.nwords, s.sym_bit + (uint64_t)s.sb * k, s.sb, ok2);
+        uint32_t v[kTail];
+#pragma unroll
+        for (uint32_t j = 0; j < kTail; j++)
+            v[j] = k0 + 256 * j < tail1
+                       ? rd_bits(s.base, s.nwords, s.sym_bit + (uint64_t)s.sb * (k0 + 256 * j), s.sb, ok2) : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < kTail; j++)
+            if (k0 + 256 * j < tail1) gsyms[k0 + 256 * j] = v[j];
         if (!ok2) atomicOr(&bad, 1u);
     }
     __syncthreads();
-    if (threadIdx.x < 96) s.tab[threadIdx.x] = tab_sh[threadIdx.x];
+    if (head && threadIdx.x < 96) s.tab[threadIdx.x] = tab_sh[threadIdx.x];
     // the table is indexed by the next lb = min(longest code, kLut) bits: 2^lb entries
     const uint32_t lb = s.nlen < kLut ? s.nlen : kLut;
-    for (uint32_t e = threadIdx.x; e < (1u << lb); e += 256) {
+    for (uint32_t e = threadIdx.x; head && e < (1u << lb); e += 256) {
         uint32_t entry = 0;
         for (int l = 1; l <= (int)lb; l++) {
             const int cw = (int)(e >> (lb - l));
@@ -295,12 +314,12 @@ __global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, CoderParams p,
     // absolute block offsets: running sum of the u16 increments
     uint32_t* boff = scratch + s.boff_off;
     const uint64_t limit = 32ull * s.nwords_cw;
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < nblk; base += 256 * 4) {
+    uint32_t carry = part.carry;
+    for (uint32_t base = b0; base < b1; base += 256 * 4) {
         uint32_t v[4], sum = 0;
         for (int k = 0; k < 4; k++) {
             const uint32_t b = base + threadIdx.x * 4 + k;
-            v[k] = base == 0 ? incv[k] : (b < nblk ? (inc[b >> 1] >> (16 * (b & 1))) & 0xFFFFu : 0u);
+            v[k] = base == b0 ? incv[k] : (b < b1 ? (inc[b >> 1] >> (16 * (b & 1))) & 0xFFFFu : 0u);
             sum += v[k];
         }
         uint32_t tot;
@@ -309,7 +328,7 @@ __global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, CoderParams p,
         for (int k = 0; k < 4; k++) {
             const uint32_t b = base + threadIdx.x * 4 + k;
             acc += v[k];
-            if (b < nblk) {
+            if (b < b1) {
                 boff[b] = acc;
                 if (acc > limit) atomicOr(&bad, 1u);
             }
@@ -915,7 +934,8 @@ void coder_decode(const DecCall* d_calls, uint32_t ncalls, const DecItem* d_item
                p, symSize, scratch, scratch_cap, d_state, d_out, 0);
     CCA_LAUNCH_CHECK();
     if (nseq == 0) return;
-    CCA_LAUNCH("dec_tables", 0, k_dec_tables, dim3(nseq), dim3(256), 0, st, d_seqs, p, scratch, d_state);
+    CCA_LAUNCH("dec_tables", 0, k_dec_tables<false>, dim3(nseq), dim3(256), 0, st, d_seqs, nullptr, p, scratch,
+               d_state);
     CCA_LAUNCH_CHECK();
     const uint64_t outb = total_symbols * symSize;
     if (symSize == 2)
@@ -944,10 +964,11 @@ void launch_blocks_rle(const DecItem* d_items, uint32_t nitems, DecSeq* d_seqs, 
 
 void coder_decode_parsed(DecSeq* d_seqs, uint32_t nseq, const CoderParams& p, int symSize, uint32_t* scratch,
                          CoderState* d_state, const DecItem* d_items, const uint32_t* d_wave_seq,
-                         const uint32_t* d_wave_first, uint32_t nwaves, uint32_t nlong, uint64_t total_symbols,
-                         const RleChunks& rc, hipStream_t st) {
+                         const uint32_t* d_wave_first, uint32_t nwaves, uint32_t nlong, const DecPart* d_parts,
+                         uint32_t nparts, uint64_t total_symbols, const RleChunks& rc, hipStream_t st) {
     if (nseq == 0) return;
-    CCA_LAUNCH("dec_tables", 0, k_dec_tables, dim3(nseq), dim3(256), 0, st, d_seqs, p, scratch, d_state);
+    CCA_LAUNCH("dec_tables", 0, k_dec_tables<true>, dim3(nparts), dim3(256), 0, st, d_seqs, d_parts, p, scratch,
+               d_state);
     CCA_LAUNCH_CHECK();
     const uint64_t outb = total_symbols * symSize;
     if (symSize == 2)
@@ -973,7 +994,8 @@ void coder_decode_index(const DecCall* d_calls, uint32_t ncalls, const DecItem* 
                p, symSize, scratch, scratch_cap, d_state, d_out, 1);
     CCA_LAUNCH_CHECK();
     if (nseq == 0) return;
-    CCA_LAUNCH("dec_tables", 0, k_dec_tables, dim3(nseq), dim3(256), 0, st, d_seqs, p, scratch, d_state);
+    CCA_LAUNCH("dec_tables", 0, k_dec_tables<false>, dim3(nseq), dim3(256), 0, st, d_seqs, nullptr, p, scratch,
+               d_state);
     CCA_LAUNCH_CHECK();
     if (ncalls) {
         CCA_LAUNCH("dec_finish", 0, k_dec_finish, dim3(ncalls), dim3(64), 0, st, d_calls, ncalls, d_items, d_seqs,

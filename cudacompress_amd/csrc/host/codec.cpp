@@ -269,6 +269,7 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
     std::vector<DecSeq> seqs;
     std::vector<DecItem> items(ns);
     std::vector<uint32_t> seq_bs;
+    std::vector<DecPart> parts;
     auto read_coded = [&](BitReader& r, uint32_t bs, uint32_t item, uint32_t count) {
         DecSeq s{};
         s.hdr_bit = r.pos();
@@ -299,8 +300,14 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
         CCA_REQUIRE(r.ok(), CC_ERR_CORRUPT_STREAM, "bitstream ends inside a coded stream");
         CCA_REQUIRE(count == 0 || s.nsym != 0, CC_ERR_CORRUPT_STREAM, "empty table for a non-empty stream");
         // the block offsets are running sums (unpackInc16CPU, PackInc.cu:222-229): the last is the largest
+        const uint32_t tail = s.nsym > (1u << kDecLutBits) ? s.nsym - (1u << kDecLutBits) : 0u;
+        const uint32_t np = std::max({1u, div_up(noff, kPartBlocks), div_up(tail, kPartSymbols)});
         uint64_t sum = 0;
-        for (uint32_t b = 0; b < noff; b++) sum += incs[b];
+        for (uint32_t k = 0; k < np; k++) {
+            parts.push_back(DecPart{(uint32_t)seqs.size(), k, (uint32_t)sum, 0});
+            const uint64_t end = std::min<uint64_t>(noff, (uint64_t)(k + 1) * kPartBlocks);
+            for (uint64_t b = (uint64_t)k * kPartBlocks; b < end; b++) sum += incs[b];
+        }
         CCA_REQUIRE(sum <= 32ull * s.nwords_cw, CC_ERR_CORRUPT_STREAM, "coding block offset beyond the codewords");
         s.count = count;
         s.item = item;
@@ -345,7 +352,7 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
     Staging s;
     const size_t o_state = s.push<CoderState>(1), o_seq = s.push<DecSeq>(nseq), o_item = s.push<DecItem>(ns);
     const size_t o_wseq = s.push<uint32_t>(nlong + nshort), o_wfirst = s.push<uint32_t>(nlong + nshort);
-    const size_t o_ifirst = s.push<uint32_t>(ns + 1);
+    const size_t o_ifirst = s.push<uint32_t>(ns + 1), o_part = s.push<DecPart>(parts.size());
     std::vector<size_t> o_words(nbs, 0);
     for (uint32_t b = 0; b < nbs; b++)
         if (w1[b] > w0[b]) o_words[b] = s.push<uint32_t>(w1[b] - w0[b]);
@@ -382,6 +389,7 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
     hif[ns] = nchunks;
     memcpy(h + o_seq, seqs.data(), sizeof(DecSeq) * nseq);
     memcpy(h + o_item, items.data(), sizeof(DecItem) * ns);
+    memcpy(h + o_part, parts.data(), sizeof(DecPart) * parts.size());
     for (uint32_t b = 0; b < nbs; b++)
         if (w1[b] > w0[b]) memcpy(h + o_words[b], bsWords[b] + w0[b], 4 * (w1[b] - w0[b]));
     uint32_t* scratch = I->d_dec_arena.as<uint32_t>(arena + std::max<uint32_t>(nchunks, 1));
@@ -393,7 +401,7 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
     const CoderParams p = params_of(I);
     coder_decode_parsed((DecSeq*)(d + o_seq), nseq, p, symSize, scratch, (CoderState*)(d + o_state),
                         (const DecItem*)(d + o_item), (const uint32_t*)(d + o_wseq), (const uint32_t*)(d + o_wfirst),
-                        nlong + nshort, nlong, total_syms, rc, st);
+                        nlong + nshort, nlong, (const DecPart*)(d + o_part), (uint32_t)parts.size(), total_syms, rc, st);
     if (nchunks) {
         stage("Decode: Run Length Decode");
         coder_decode_expand((const DecItem*)(d + o_item), ns, (DecSeq*)(d + o_seq), symSize, rc,
