@@ -224,6 +224,9 @@ void coder_concat(const ConcatGroup* d_groups, uint32_t ngroups, uint32_t* dst, 
 void coder_stats(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, const CoderParams& p, int symSize,
                  uint32_t* scratch, uint64_t scratch_cap, CoderState* d_state, uint32_t* d_classes,
                  uint64_t total_symbols, const CodeUnits& units, hipStream_t st);
+// The code tables (codes and lengths by symbol at code_off) of sequences whose symbols in codeword order,
+// counts per length and offsets are in place, most_syms symbols at most.
+void coder_code_tables(const SeqInfo* d_seqs, uint32_t nseq, uint32_t most_syms, uint32_t* scratch, hipStream_t st);
 void coder_pack(const CodeItem* d_items, SeqInfo* d_seqs, const CoderParams& p, int symSize, uint32_t* scratch,
                 const CoderState* d_state, uint32_t* d_out, uint64_t out_cap, uint64_t total_symbols,
                 const CodeUnits& units, hipStream_t st);

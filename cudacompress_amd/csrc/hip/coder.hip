@@ -1383,6 +1383,30 @@ __device__ __forceinline__ void put_codes(uint32_t* win, uint32_t o, const uint3
     if (sh + bits > 64) atomicOr(&win[(wi + 2) & WM], (uint32_t)t << (32 - sh));
 }
 
+// Canonical codes and their lengths, by symbol, of tables that were designed on the host: workgroups
+// (x, y) write a share of sequence x's.  Only the symbols come up and not tables of the whole alphabet (a
+// 4096^2 terrain's largest: 0.26 of 0.79 MB each); entries of unused symbols are left as they are, nothing
+// that is coded reads them.
+constexpr uint32_t kTableShare = 4 * kCoderThreads;
+__global__ __launch_bounds__(kCoderThreads) void k_code_tables(const SeqInfo* seqs, uint32_t* scratch) {
+    __shared__ uint32_t fc[32], fi[32];
+    const SeqInfo& s = seqs[blockIdx.x];
+    const uint32_t nlen = s.nlen, nsym = s.nsym, k0 = blockIdx.y * kTableShare;
+    if (nlen == 0 || k0 >= nsym) return;
+    if (threadIdx.x == 0) design::first_codes(s.cpl, (int)nlen, fc, fi);
+    __syncthreads();
+    const uint32_t* syms = scratch + s.syms_off;
+    uint32_t* code = scratch + s.code_off;
+    uint32_t* len = code + s.smax + 1;
+    for (uint32_t k = k0 + threadIdx.x; k < min(k0 + kTableShare, nsym); k += kCoderThreads) {
+        const uint32_t sym = syms[k];
+        uint32_t l = 0;  // the last length that starts at or before k (unused ones start where the next does)
+        for (uint32_t i = 1; i < nlen; i++) l = fi[i] <= k ? i : l;
+        code[sym] = fc[l] + (k - fi[l]);
+        len[sym] = l + 1;
+    }
+}
+
 // Pass B: pairs recomputed, codewords packed into an LDS window and flushed as whole words
 // straight to their place in the output section (laid out by k_layout_* from the designed bit
 // counts): each workgroup also writes its item's zero-run count, table headers and bit counts, and
@@ -1799,6 +1823,13 @@ void coder_stats(const CodeItem* d_items, uint32_t nitems, SeqInfo* d_seqs, cons
     };
     if (symSize == 2) stats(uint16_t{});
     else stats(uint32_t{});
+}
+
+void coder_code_tables(const SeqInfo* d_seqs, uint32_t nseq, uint32_t most_syms, uint32_t* scratch, hipStream_t st) {
+    if (nseq == 0 || most_syms == 0) return;
+    CCA_LAUNCH("code_tables", 0, k_code_tables, dim3(nseq, div_up(most_syms, kTableShare)), dim3(kCoderThreads), 0, st,
+               d_seqs, scratch);
+    CCA_LAUNCH_CHECK();
 }
 
 void coder_pack(const CodeItem* d_items, SeqInfo* d_seqs, const CoderParams& p, int symSize, uint32_t* scratch,

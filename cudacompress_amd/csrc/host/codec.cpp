@@ -7,7 +7,8 @@
 //   1. upload of the stream list; the stats pass (zero-run pairs, histograms)     -> sync #1: histograms
 //   2. table design on the host (libstdc++ heap/sort, as the reference), exact bit counts from
 //      histogram x length, the layout of every section (Encode.cpp:402-463 rl, :751-782 huff)
-//   3. one upload (tables and sequence records); the pack writes the sections in place -> sync #2: words
+//   3. one upload (sequence records, symbols in codeword order), from which the device makes the code
+//      tables; the pack writes the sections in place -> sync #2: words
 // The reference does >= streams + 6 host synchronisations per encodeRLHuff, per level of a volume.
 //
 // Decode walks the sections' heads on the host (counts, sizes, as Encode.cpp:522-621; the symbol
@@ -59,6 +60,8 @@ struct Staging {
     }
 };
 
+constexpr uint64_t kArenaGuess = 1u << 24;  // words (64 MB)
+
 }  // namespace
 
 void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& streams, uint32_t ncalls,
@@ -91,14 +94,18 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
     const uint32_t nseq = job.nseq;
     // one device buffer: the coder's state, the sequence records, the arena
     const size_t o_seq = align_up(sizeof(CoderState), 64), o_arena = align_up(o_seq + sizeof(SeqInfo) * nseq, 256);
-    uint64_t cap = std::max<uint64_t>(I->enc_arena, 1024 + (uint64_t)nseq * (kStatBins + 2 * design_leaf_words()));
+    // room for a histogram of the whole alphabet per stream, so that wide symbols do not have the statistics
+    // run twice; above kArenaGuess a guess, with a second run where it was too small
+    const uint64_t alphabet = I->dialect == CC_DIALECT_CPU ? 65536u : std::min<uint64_t>(1ull << I->log2, 65536u);
+    const uint64_t least = 1024 + (uint64_t)nseq * (kStatBins + 2 * design_leaf_words());
+    uint64_t cap = std::max({I->enc_arena, least, std::min(least + ns * alphabet, kArenaGuess)});
     unsigned char *d, *h;
     for (int attempt = 0;; attempt++) {
         d = (unsigned char*)I->d_enc.get(o_arena + 4 * cap);
         encode_stats(D, job, (SeqInfo*)(d + o_seq), (uint32_t*)(d + o_arena), cap, (CoderState*)d, st);
         // the state, the records and as much of the arena as the last call used come down together
         const uint64_t first = std::min(cap, std::max<uint64_t>(I->enc_down, 4096));
-        h = (unsigned char*)I->h_down.get(o_arena + 4 * cap);
+        h = (unsigned char*)I->h_down.get(o_arena + 4 * first);
         CCA_HIP(hipMemcpyAsync(h, d, o_arena + 4 * first, hipMemcpyDeviceToHost, st));
         CCA_HIP(hipStreamSynchronize(st));
         const CoderState s = *(const CoderState*)h;
@@ -109,8 +116,10 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
         CCA_REQUIRE(s.err == kErrNone, CC_ERR_OUT_OF_MEMORY, "coder arena exhausted");
         const uint64_t used = std::min<uint64_t>(s.scratch_used, cap);
         if (used > first) {
-            CCA_HIP(hipMemcpyAsync(h + o_arena + 4 * first, d + o_arena + 4 * first, 4 * (used - first),
-                                   hipMemcpyDeviceToHost, st));
+            // pinned for what comes down, not for the arena: fresh pinned pages cost 0.4 ms a megabyte to touch
+            const uint64_t have = I->h_down.cap < o_arena + 4 * used ? 0 : o_arena + 4 * first;
+            h = (unsigned char*)I->h_down.get(o_arena + 4 * used);
+            CCA_HIP(hipMemcpyAsync(h + have, d + have, o_arena + 4 * used - have, hipMemcpyDeviceToHost, st));
             CCA_HIP(hipStreamSynchronize(st));
         }
         I->enc_arena = cap;
@@ -134,8 +143,12 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
         rcs[j] = design_table(fmt.dialect, hist, s.smax, tables[j]);
         if (rcs[j] != CC_OK) return;
         uint64_t b = 0;
-        for (uint32_t k : tables[j].symbols) b += (uint64_t)hist[k] * tables[j].len[k];
-        if (s.quirk) b -= tables[j].len[65535];  // the counted pad is not encoded
+        const EncTable& t = tables[j];
+        for (size_t l = 0, k = 0; l < t.count_per_length.size(); l++)
+            for (uint32_t c = t.count_per_length[l]; c > 0; c--, k++) {
+                const uint32_t sym = t.symbols[k];
+                b += (uint64_t)(hist[sym] - (s.quirk && sym == 65535u ? 1u : 0u)) * (l + 1);  // the counted pad is not encoded
+            }
         bits[j] = b;
     });
     // first sequence of every stream, and of every call (streams come grouped by call)
@@ -163,9 +176,11 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
             CCA_REQUIRE(bits[j] < (1ull << 32), CC_ERR_INVALID_ARG, "coded stream exceeds 2^32 bits");
         }
     }
-    // sections in stream order; the arena: every table (code, len by symbol, symbols in codeword order),
-    // then the coding-block offsets, which the pack fills
-    uint64_t pos = 0, tab = 0;
+    // sections in stream order; the arena: every table's symbols in codeword order, which go up, then its
+    // codes and lengths by symbol, which the device makes of them, and the coding-block offsets, which the
+    // pack fills
+    uint64_t pos = 0, up = 0;
+    uint32_t most_syms = 0;
     for (uint32_t i = 0; i < ns; i++) {
         const EncodeStream& s = streams[i];
         I->seg_begin[i] = pos;
@@ -184,36 +199,32 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
             r.nsym = (uint32_t)t.symbols.size();
             r.bits = bits[j];
             for (uint32_t l = 0; l < 32; l++) r.cpl[l] = l < r.nlen ? t.count_per_length[l] : 0u;
-            r.code_off = tab;
-            r.syms_off = tab + 2ull * (r.smax + 1);
-            tab = align_up(r.syms_off + std::max<uint32_t>(r.nsym, 1), 16);
+            r.syms_off = up;
+            up = align_up(up + std::max<uint32_t>(r.nsym, 1), 16);
+            most_syms = std::max(most_syms, r.nsym);
         }
         I->seg_bits[i] = (pos - I->seg_begin[i]) * 32;
     }
     const uint64_t total = pos;
-    uint64_t arena_words = tab;
+    uint64_t arena_words = up;
     for (SeqInfo& r : seqs) {
+        r.code_off = arena_words;
+        arena_words = align_up(arena_words + 2ull * (r.smax + 1), 16);
         r.boff_off = arena_words;
         arena_words += align_up(std::max<uint32_t>(div_up(r.count, cbs), 1), 16);
     }
 
     // ---- 3. codewords ----------------------------------------------------------------------------
     stage("Encode: Huffman Encode");
-    if (arena_words > cap) {  // (nothing in the arena is needed any more)
-        I->enc_arena = arena_words;
-        d = (unsigned char*)I->d_enc.get(o_arena + 4 * arena_words);
-    }
-    unsigned char* u = (unsigned char*)I->h_up.get(o_arena + 4 * tab);
+    d = (unsigned char*)I->d_enc.get(o_arena + 4 * std::max(arena_words, cap));  // (what is there is not needed any more)
+    unsigned char* u = (unsigned char*)I->h_up.get(o_arena + 4 * up);
     *(CoderState*)u = CoderState{0, total, 0, 0, 0};
     memcpy(u + o_seq, seqs.data(), sizeof(SeqInfo) * nseq);
     uint32_t* ua = (uint32_t*)(u + o_arena);
-    for (uint32_t j = 0; j < nseq; j++) {
-        const EncTable& t = tables[j];
-        memcpy(ua + seqs[j].code_off, t.code.data(), 4ull * t.code.size());
-        memcpy(ua + seqs[j].code_off + seqs[j].smax + 1, t.len.data(), 4ull * t.len.size());
-        memcpy(ua + seqs[j].syms_off, t.symbols.data(), 4ull * t.symbols.size());
-    }
-    CCA_HIP(hipMemcpyAsync(d, u, o_arena + 4 * tab, hipMemcpyHostToDevice, st));
+    for (uint32_t j = 0; j < nseq; j++)
+        memcpy(ua + seqs[j].syms_off, tables[j].symbols.data(), 4ull * tables[j].symbols.size());
+    CCA_HIP(hipMemcpyAsync(d, u, o_arena + 4 * up, hipMemcpyHostToDevice, st));
+    coder_code_tables((const SeqInfo*)(d + o_seq), nseq, most_syms, (uint32_t*)(d + o_arena), st);
     uint32_t* dw = I->d_words.as<uint32_t>(std::max<uint64_t>(total, 1));
     encode_pack(D, job, (SeqInfo*)(d + o_seq), (uint32_t*)(d + o_arena), (CoderState*)d, dw, total, st);
     uint32_t* hw = I->h_words.as<uint32_t>(std::max<uint64_t>(total, 1));

@@ -65,8 +65,6 @@ cc_status design_table(int dialect, const uint32_t* hist, uint32_t symbol_max, E
     t.symbols.clear();
     t.symbol_max = symbol_max;
     const uint32_t nsym_space = symbol_max + 1;
-    t.code.assign(nsym_space, 0u);
-    t.len.assign(nsym_space, 0xFFFFFFFFu);
 
     std::vector<uint64_t> leaves;  // (count, leaf), leaf k being symbol t.symbols[k]
     for (uint32_t s = 0; s < nsym_space; s++) {
@@ -110,15 +108,6 @@ cc_status design_table(int dialect, const uint32_t* hist, uint32_t symbol_max, E
         const uint32_t l = (uint32_t)(leaves[i] >> 32);
         if (l > 0) t.count_per_length[l - 1]++;
         t.symbols[i] = (uint32_t)leaves[i];
-    }
-    // canonical codes in codeword-index order (HuffmanTable.cu:553-580)
-    uint32_t code = 0, prev_len = (uint32_t)(leaves[0] >> 32);
-    for (uint32_t i = 0; i < k; i++) {
-        const uint32_t l = (uint32_t)(leaves[i] >> 32);
-        if (i > 0) code = (code + 1) << (l - prev_len);
-        t.code[t.symbols[i]] = code;
-        t.len[t.symbols[i]] = l;
-        prev_len = l;
     }
     return CC_OK;
 }

@@ -22,7 +22,6 @@ struct EncTable {
     std::vector<uint32_t> count_per_length;  // [length-1]
     std::vector<uint32_t> symbols;           // in codeword-index order
     uint32_t symbol_max = 0;                 // stream max symbol (source of symbolBits)
-    std::vector<uint32_t> code, len;         // by symbol, size symbol_max+1 (len 0xFFFFFFFF: unused)
 };
 
 // Designs the table of one stream from its histogram (symbol_max+1 bins).
