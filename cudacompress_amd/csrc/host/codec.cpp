@@ -368,9 +368,17 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
     for (uint32_t b = 0; b < nbs; b++)
         if (w1[b] > w0[b]) o_words[b] = s.push<uint32_t>(w1[b] - w0[b]);
     const size_t total = s.off;
-    const int slot = I->dec_slot;
-    I->dec_slot = (I->dec_slot + 1) % kDecodeRing;
-    CCA_HIP(hipEventSynchronize(I->dec_event[slot]));  // previous upload from this slot done
+    // the first staging slot whose upload is done, or the next one in turn after a wait: a caller that waits
+    // for its decodes uses one (a volume is one decode, and four slots of its size are four times its words
+    // pinned, each megabyte 0.4 ms to touch for the first time)
+    int slot = 0;
+    while (slot < kDecodeRing && hipEventQuery(I->dec_event[slot]) != hipSuccess) slot++;
+    if (slot > 0) (void)hipGetLastError();  // "not ready" is no error of this call
+    if (slot == kDecodeRing) {
+        slot = I->dec_slot;
+        CCA_HIP(hipEventSynchronize(I->dec_event[slot]));
+    }
+    I->dec_slot = (slot + 1) % kDecodeRing;
     unsigned char* h = (unsigned char*)I->h_dec_stage[slot].get(total);
     unsigned char* d = (unsigned char*)I->d_dec_stage.get(total);
     unsigned char* dsym = (unsigned char*)I->d_dec_sym.get(std::max<uint64_t>(rl_elems, 1) * symSize);

@@ -219,3 +219,35 @@ def test_table_of_lengths_without_symbols(cc, torch_gpu, rl):
     got = out.cpu().numpy()
     assert np.all(got[:n] == 0) and np.all(got[n:] == -1)
     inst.close()
+
+
+def test_decodes_one_after_the_other_share_their_staging(cc, torch_gpu):
+    """Decodes that a caller waits for use one pinned staging buffer between them: after the first call the
+    process does not grow by another one with each of the next."""
+    torch = torch_gpu
+    n = 6000000
+    inst = cc.createInstance(0, 1, n, 128, 14)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    sym = torch.randint(0, 16000, (n,), generator=g, device="cuda", dtype=torch.int32).to(torch.int16)
+    bits = cc.BitStream()
+    assert cc.encodeHuff(inst, bits, [sym], n)
+    out = torch.empty_like(sym)
+    staged = bits.getBitSize() // 8
+    assert staged > 10 << 20
+
+    def size():
+        with open("/proc/self/statm") as f:
+            return int(f.read().split()[0]) * 4096
+
+    sizes = []
+    for _ in range(5):
+        out.fill_(-1)
+        bits.setBitPosition(0)
+        cc.decodeHuff(inst, bits, [out], n)
+        torch.cuda.synchronize()
+        assert torch.equal(out, sym)
+        sizes.append(size())
+    log("process size after each decode, MB", [s >> 20 for s in sizes], "staged", staged >> 20)
+    assert sizes[-1] - sizes[0] < staged
+    inst.close()
