@@ -18,35 +18,15 @@
 #include "codec.hpp"
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
-#include <thread>
 
 #include "batch.hpp"
 #include "bitio.hpp"
 #include "huffman_table.hpp"
+#include "parallel.hpp"
 
 namespace cca {
 namespace {
-
-// f(i) for i < n, on up to 16 threads when the work (in microseconds) repays starting them.
-template <class F>
-void parallel_for(size_t n, double work_us, F f) {
-    const size_t hw = std::max(1u, std::thread::hardware_concurrency());
-    const size_t nt = std::min<size_t>({hw, n, (size_t)16, (size_t)(work_us / 75.0) + 1});
-    if (nt <= 1) {
-        for (size_t i = 0; i < n; i++) f(i);
-        return;
-    }
-    std::vector<std::thread> th;
-    std::atomic<size_t> next{0};
-    auto work = [&]() {
-        for (size_t i = next++; i < n; i = next++) f(i);
-    };
-    for (size_t t = 1; t < nt; t++) th.emplace_back(work);
-    work();
-    for (auto& x : th) x.join();
-}
 
 // Bump allocator over a pinned host buffer mirrored by a device buffer.
 struct Staging {
