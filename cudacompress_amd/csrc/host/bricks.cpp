@@ -56,7 +56,7 @@ void make_layout(BrickJob& job) {
     job.sym.resize(n);
     job.lp.assign(L, std::vector<uint64_t>(n, 0));
     job.level_elems.assign(L, 0);
-    uint64_t w = 0, s = 0;
+    uint64_t w = 0, s = job.sym_base;
     for (uint32_t i = 0; i < n; i++) {
         const uint64_t N = elems(job.bricks[i]);
         job.a[i] = w;
@@ -174,13 +174,21 @@ cc_status status_of_encode(uint32_t e) {
 
 }  // namespace
 
-std::vector<ItemSpec> bricks_transforms_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, hipStream_t st) {
+std::vector<ItemSpec> bricks_transforms_layout(BrickCtx& ctx, BrickJob& job) {
     check_bricks(job.bricks.data(), (uint32_t)job.bricks.size(), job.L);
     make_layout(job);
-    float* work = ctx.d_bwork.as<float>(std::max<uint64_t>(job.work_floats, 64));
-    unsigned char* sym = (unsigned char*)ctx.d_bsym.get(std::max<uint64_t>(job.sym_elems, 64) * job.symSize);
-    upload_levels(ctx, job, work, sym, I->tuning, st);
-    return brick_items(job, sym);
+    ctx.d_bwork.as<float>(std::max<uint64_t>(job.work_floats, 64));
+    return brick_items(job, (unsigned char*)ctx.d_bsym.get(std::max<uint64_t>(job.sym_elems, 64) * job.symSize));
+}
+
+void bricks_transforms_upload(cc_instance* I, BrickCtx& ctx, BrickJob& job, hipStream_t st) {
+    upload_levels(ctx, job, (float*)ctx.d_bwork.p, (unsigned char*)ctx.d_bsym.p, I->tuning, st);
+}
+
+uint64_t brick_work_bytes(uint64_t volume_elems, uint32_t levels) {
+    uint64_t floats = 2 * align_up(volume_elems, 64);
+    for (uint32_t l = 1; l < levels; l++) floats += align_up(volume_elems >> (3 * l), 64);
+    return 4 * floats;
 }
 
 bool bricks_serve(uint64_t volume_elems, uint32_t levels) { return volume_elems < (1ull << 31) && levels <= 10; }
@@ -193,7 +201,8 @@ void bricks_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, bool enc, bool
         CCA_REQUIRE(!enc || job.bricks[i].src, CC_ERR_INVALID_ARG, "null brick source");
         CCA_REQUIRE(!dec || job.bricks[i].dst, CC_ERR_INVALID_ARG, "null brick destination");
     }
-    const std::vector<ItemSpec> items = bricks_transforms_prepare(I, ctx, job, st);
+    const std::vector<ItemSpec> items = bricks_transforms_layout(ctx, job);
+    bricks_transforms_upload(I, ctx, job, st);
     if (enc) encode_prepare(I, ctx.coder, items, n, job.symSize, job.ej, st);
     if (dec) {
         if (calls) {
@@ -213,8 +222,9 @@ void bricks_prepare_bound(cc_instance* I, BrickCtx& ctx, BrickJob& job, const De
     check_bricks(job.bricks.data(), n, job.L);
     for (uint32_t i = 0; i < n; i++)
         CCA_REQUIRE(job.bricks[i].dst, CC_ERR_INVALID_ARG, "null brick destination");
-    decode_prepare_bound(I, ctx.coder, X, bricks_transforms_prepare(I, ctx, job, st), index_calls, job.symSize, job.bj,
-                         st);
+    const std::vector<ItemSpec> items = bricks_transforms_layout(ctx, job);
+    bricks_transforms_upload(I, ctx, job, st);
+    decode_prepare_bound(I, ctx.coder, X, items, index_calls, job.symSize, job.bj, st);
     job.index = &X;
 }
 

@@ -20,6 +20,7 @@ struct BrickJob {
     std::vector<std::vector<uint64_t>> lp;
     std::vector<uint64_t> level_elems;
     uint64_t work_floats = 0, sym_elems = 0;
+    uint64_t sym_base = 0;  // where its symbols start in the context's symbol buffer
     // device tables
     const BrickLevel* d_levels = nullptr;  // [L][n]
     const uint32_t* d_tiles = nullptr;     // [L][4][n+1]
@@ -32,9 +33,15 @@ struct BrickJob {
     uint64_t out_cap = 0;
 };
 
-// The transforms of a job alone: layout, buffers and level tables; returns the bricks' symbol streams
-// in bitstream order (lowpass, then 7 bands a level from the coarsest), one call per brick.
-std::vector<ItemSpec> bricks_transforms_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, hipStream_t st);
+// The transforms of a job alone: layout and buffers; returns the bricks' symbol streams in bitstream order
+// (lowpass, then 7 bands a level from the coarsest), one call per brick.  Jobs that share a context's work
+// buffers and take turns have their layouts made first (with the symbol buffer sized for all of them), then
+// each its level tables and its launches.
+std::vector<ItemSpec> bricks_transforms_layout(BrickCtx& ctx, BrickJob& job);
+// The level tables: a pinned copy of the context's, which has to be up before the next job's is written.
+void bricks_transforms_upload(cc_instance* I, BrickCtx& ctx, BrickJob& job, hipStream_t st);
+// bytes of work buffers of a brick's transforms
+uint64_t brick_work_bytes(uint64_t volume_elems, uint32_t levels);
 // whether a volume of so many elements and levels can be a brick
 bool bricks_serve(uint64_t volume_elems, uint32_t levels);
 // decode calls: one bitstream per brick, or when `calls` is null the device results of the

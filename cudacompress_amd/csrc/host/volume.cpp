@@ -20,6 +20,7 @@
 //  * the multi-channel decoders give each channel exactly its single-channel decode.
 #include "volume.hpp"
 
+#include <algorithm>
 #include <cstring>
 
 #include "../kernels.hpp"
@@ -68,14 +69,11 @@ void check_volume(uint32_t sx, uint32_t sy, uint32_t sz, uint32_t levels) {
                 "sizes must be divisible by 2^numLevels");
 }
 
-// The volume as a brick of one: its levels' transforms with the quantizer fused, the streams in
-// bitstream order (of channel `bs` when decoding).
-std::vector<ItemSpec> volume_bricks(cc_instance* I, BrickJob& job, const std::vector<cc_brick>& bricks, uint32_t levels,
-                                    int symSize, bool rle_only_lvl0) {
-    job.bricks = bricks;
+// Volumes as bricks: their levels' transforms with the quantizer fused, the streams in bitstream order.
+std::vector<ItemSpec> volume_bricks(cc_instance* I, BrickJob& job, uint32_t levels, int symSize, bool rle_only_lvl0) {
     job.L = levels;
     job.symSize = symSize;
-    std::vector<ItemSpec> items = bricks_transforms_prepare(I, I->batch, job, I->stream);
+    std::vector<ItemSpec> items = bricks_transforms_layout(I->batch, job);
     for (size_t k = 0; k < items.size(); k++)  // streams 1 .. 7 (levels - 1) of a brick: levels above 0
         if (rle_only_lvl0 && k % (1 + 7 * levels) <= 7 * (levels - 1)) items[k].rl = false;
     return items;
@@ -152,8 +150,9 @@ void compress_volume_float(cc_instance* I, const float* image, uint32_t sx, uint
         return;
     }
     BrickJob job;
-    const std::vector<ItemSpec> items =
-        volume_bricks(I, job, {cc_brick{image, nullptr, sx, sy, sz, q0}}, levels, symSize, rle_only_lvl0);
+    job.bricks = {cc_brick{image, nullptr, sx, sy, sz, q0}};
+    const std::vector<ItemSpec> items = volume_bricks(I, job, levels, symSize, rle_only_lvl0);
+    bricks_transforms_upload(I, I->batch, job, I->stream);
     bricks_forward_launch(job, I->stream);
     call("Encode RLHuff");
     std::vector<EncodeStream> streams;
@@ -336,6 +335,11 @@ struct ChannelStreams {
     }
 };
 
+// Most work buffers (bytes) that the channels of a float decode have between them, one channel's at least:
+// 8.6 bytes a voxel for each that is transformed at a time.  A channel that needs a good part of this keeps
+// the chip busy by itself, and three of 512^3 would hold 3.4 GB.
+constexpr uint64_t kChannelWork = 1u << 27;
+
 }  // namespace
 
 void decompress_volume_float_multichannel(cc_instance* I, const VolumeChannelIn* ch, uint32_t nch, uint32_t sx,
@@ -362,12 +366,20 @@ void decompress_volume_float_multichannel(cc_instance* I, const VolumeChannelIn*
                                           symSize);
         return;
     }
-    // every channel is a brick of one batch
-    std::vector<cc_brick> bricks;
-    for (uint32_t c = 0; c < nch; c++) bricks.push_back(cc_brick{nullptr, ch[c].image, sx, sy, sz, ch[c].step});
-    BrickJob job;
-    for (const ItemSpec& it : volume_bricks(I, job, bricks, levels, symSize, rle_only_lvl0))
-        streams.push_back(DecodeStream{it.ptr, it.n, it.rl, it.call});
+    // the channels are bricks of one batch, or of several that take turns with the work buffers
+    const uint32_t at_once = (uint32_t)std::max<uint64_t>(1, kChannelWork / brick_work_bytes(elems, levels));
+    std::vector<BrickJob> jobs;
+    I->batch.d_bsym.get(nch * align_up(elems, 64) * symSize);
+    for (uint32_t c = 0; c < nch; c += at_once) {
+        BrickJob job;
+        job.sym_base = c * align_up(elems, 64);
+        for (uint32_t k = c; k < std::min(nch, c + at_once); k++)
+            job.bricks.push_back(cc_brick{nullptr, ch[k].image, sx, sy, sz, ch[k].step});
+        for (const ItemSpec& it : volume_bricks(I, job, levels, symSize, rle_only_lvl0))
+            streams.push_back(DecodeStream{it.ptr, it.n, it.rl, c + it.call});
+        jobs.push_back(std::move(job));
+    }
+    bricks_transforms_upload(I, I->batch, jobs[0], st);
     // the level tables' upload must finish before the pinned copy is rewritten
     try {
         cs.decode(I, symSize, streams);
@@ -375,8 +387,11 @@ void decompress_volume_float_multichannel(cc_instance* I, const VolumeChannelIn*
         (void)hipStreamSynchronize(st);
         throw;
     }
-    bricks_inverse_launch(job, st);
-    CCA_HIP(hipStreamSynchronize(st));
+    for (size_t j = 0; j < jobs.size(); j++) {
+        if (j) bricks_transforms_upload(I, I->batch, jobs[j], st);
+        bricks_inverse_launch(jobs[j], st);
+        CCA_HIP(hipStreamSynchronize(st));
+    }
 }
 
 void decompress_volume_float_quant_first_multichannel(cc_instance* I, const VolumeChannelIn* ch, uint32_t nch,
