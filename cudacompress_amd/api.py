@@ -166,6 +166,11 @@ class Instance:
         """Concurrent groups of a brick batch (0: chosen from the batch size)."""
         _check(_capi.load().cc_set_instance_brick_groups(self._h, groups), "setBrickGroups")
 
+    def setBrickVolumeLimit(self, voxels):
+        """Float volumes of at least this many voxels, over all channels, take the single-volume transforms
+        (cc_set_instance_brick_volume_limit; 0: 2^31)."""
+        _check(_capi.load().cc_set_instance_brick_volume_limit(self._h, voxels), "setBrickVolumeLimit")
+
 
 def createInstance(cudaDevice=-1, streamCountMax=1, elemCountPerStreamMax=1, codingBlockSize=0,
                    log2HuffmanDistinctSymbolCountMax=0):

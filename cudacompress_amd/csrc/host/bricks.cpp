@@ -191,7 +191,9 @@ uint64_t brick_work_bytes(uint64_t volume_elems, uint32_t levels) {
     return 4 * floats;
 }
 
-bool bricks_serve(uint64_t volume_elems, uint32_t levels) { return volume_elems < (1ull << 31) && levels <= 10; }
+bool bricks_serve(const cc_instance* I, uint64_t volume_elems, uint32_t levels) {
+    return volume_elems < I->brick_voxels && levels <= 10;
+}
 
 void bricks_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, bool enc, bool dec,
                     const std::vector<CallWords>* calls, hipStream_t st) {

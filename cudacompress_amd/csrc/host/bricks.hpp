@@ -42,8 +42,8 @@ std::vector<ItemSpec> bricks_transforms_layout(BrickCtx& ctx, BrickJob& job);
 void bricks_transforms_upload(cc_instance* I, BrickCtx& ctx, BrickJob& job, hipStream_t st);
 // bytes of work buffers of a brick's transforms
 uint64_t brick_work_bytes(uint64_t volume_elems, uint32_t levels);
-// whether a volume of so many elements and levels can be a brick
-bool bricks_serve(uint64_t volume_elems, uint32_t levels);
+// whether volumes of so many elements in all and levels go through the brick passes
+bool bricks_serve(const cc_instance* I, uint64_t volume_elems, uint32_t levels);
 // decode calls: one bitstream per brick, or when `calls` is null the device results of the
 // encode staged in the same context
 void bricks_prepare(cc_instance* I, BrickCtx& ctx, BrickJob& job, bool enc, bool dec,

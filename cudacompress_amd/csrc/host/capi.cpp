@@ -157,6 +157,12 @@ cc_status cc_set_instance_dialect(cc_instance* inst, int dialect) {
         inst->dialect = dialect;
     });
 }
+cc_status cc_set_instance_brick_volume_limit(cc_instance* inst, uint64_t voxels) {
+    return guarded([&] {
+        CCA_REQUIRE(inst && voxels <= (1ull << 31), CC_ERR_INVALID_ARG, "null instance or more than 2^31 voxels");
+        inst->brick_voxels = voxels ? voxels : 1ull << 31;
+    });
+}
 cc_status cc_set_instance_brick_groups(cc_instance* inst, uint32_t groups) {
     return guarded_for(inst, [&] {
         CCA_REQUIRE(inst && groups <= 64, CC_ERR_INVALID_ARG, "brick groups must be in [0, 64]");

@@ -113,6 +113,7 @@ struct cc_instance {
     std::vector<std::unique_ptr<cca::BrickCtx>> groups;
     hipEvent_t group_fork = nullptr;
     uint32_t brick_groups = 0;  // groups per brick batch, 0: chosen from the batch size
+    uint64_t brick_voxels = 1ull << 31;  // float volumes of fewer voxels go through the brick passes
     cc_tuning tuning{};         // kernel shapes of brick batches and the device coder (cc_set_instance_tuning)
 
     // section timing (cc_set_timing_detail)

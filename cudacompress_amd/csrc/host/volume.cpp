@@ -144,7 +144,7 @@ void compress_volume_float(cc_instance* I, const float* image, uint32_t sx, uint
     check_symbols(I, symSize);
     const uint64_t elems = (uint64_t)sx * sy * sz;
     SectionTimer call(I, 1);
-    if (!bricks_serve(elems, levels)) {
+    if (!bricks_serve(I, elems, levels)) {
         call("Encode RLHuff");
         compress_volume_float_large(I, image, sx, sy, sz, levels, q0, VolumeStreams(elems, levels, rle_only_lvl0), symSize);
         return;
@@ -354,7 +354,7 @@ void decompress_volume_float_multichannel(cc_instance* I, const VolumeChannelIn*
     call("Decode RLHuff");
     ChannelStreams cs(ch, nch);
     std::vector<DecodeStream> streams;
-    if (!bricks_serve(elems * nch, levels)) {
+    if (!bricks_serve(I, elems * nch, levels)) {
         const VolumeStreams vs(elems, levels, rle_only_lvl0);
         unsigned char* sym = (unsigned char*)I->d_vol[2].get(nch * vs.elems * symSize);
         for (uint32_t c = 0; c < nch; c++)

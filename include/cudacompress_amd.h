@@ -70,6 +70,10 @@ CC_API cc_status cc_set_instance_dialect(cc_instance* inst, int dialect);
  * run as concurrent pipelines on their own streams, their bitstreams still back to back in brick
  * order.  0 or 1 (default): one pipeline.  Plans always capture one.  No reference counterpart. */
 CC_API cc_status cc_set_instance_brick_groups(cc_instance* inst, uint32_t groups);
+/* Float volumes (all channels together) of at least this many voxels go through the single-volume
+ * transforms, level by level, and smaller ones through the brick passes, whose offsets are 32 bits.
+ * The values and bitstreams are the same.  0: 2^31, which is also the most.  No reference counterpart. */
+CC_API cc_status cc_set_instance_brick_volume_limit(cc_instance* inst, uint64_t voxels);
 
 /* ---- Entropy coding: include/cudaCompress/Encode.h:28-57 ---------------------------------- */
 
