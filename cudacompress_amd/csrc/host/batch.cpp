@@ -137,9 +137,12 @@ void encode_upload(cc_instance* I, DeviceCoder& D, const std::vector<ItemSpec>& 
     job.symSize = symSize;
     job.p = params_of(I);
     for (int c = 0; c < 4; c++) job.design_grid[c] = I->tuning.designGrid[c];
-    // one table a thread pays when there are more tables than waves to give them; up to a table a compute
-    // unit, a wave each is faster (6 tables: whole call 387 us, 445 us with small ones one a thread)
-    job.lane_k = job.nseq <= kWaveTablesMax ? 0u : I->tuning.laneDesignK;
+    // One table a thread pays when there are far more tables than waves to give them (2048 bricks, 59,392
+    // tables: 12.79 ms with 32 symbols at most, 12.94 with none).  Up to a table a compute unit a wave each is
+    // faster: 2 to 256 tables of the device coder 267-314 us against 324-525 with 64 symbols at most, 29 to 232
+    // of bricks 0.72-2.15 against 0.85-2.30 ms.  (It still is by 5 % at 696; where the lines cross is not known.)
+    // A tuning that the caller set is taken as it is.
+    job.lane_k = !I->tuning_set && job.nseq <= kWaveTablesMax ? 0u : I->tuning.laneDesignK;
     D.d_items.get(stage_bytes);
     D.d_split.get(sizeof(SegState) * nslots + 4ull * kSplitWords * nsplit);
     D.d_classes.as<uint32_t>(kDesignListBase + (uint64_t)kDesignLists * std::max<uint32_t>(job.nseq, 1));

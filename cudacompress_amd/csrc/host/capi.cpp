@@ -420,6 +420,7 @@ cc_status cc_set_instance_tuning(cc_instance* inst, const cc_tuning* tuning) {
         CCA_REQUIRE(inst, CC_ERR_INVALID_ARG, "null instance");
         if (tuning) cca::validate_tuning(*tuning);
         inst->tuning = tuning ? *tuning : cca::library_tuning();
+        inst->tuning_set = tuning != nullptr;
     });
 }
 cc_status cc_get_instance_tuning(const cc_instance* inst, cc_tuning* out) {

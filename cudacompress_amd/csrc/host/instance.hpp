@@ -115,6 +115,7 @@ struct cc_instance {
     uint32_t brick_groups = 0;  // groups per brick batch, 0: chosen from the batch size
     uint64_t brick_voxels = 1ull << 31;  // float volumes of fewer voxels go through the brick passes
     cc_tuning tuning{};         // kernel shapes of brick batches and the device coder (cc_set_instance_tuning)
+    bool tuning_set = false;    // by the caller: used as it is for jobs of any size
 
     // section timing (cc_set_timing_detail)
     int timing_detail = 0;

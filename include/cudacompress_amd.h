@@ -469,7 +469,9 @@ typedef struct cc_tuning {
                                  threads cover, one thread per x pair) */
     uint32_t codingBlockSize; /* recommended coding block size (32..256) */
     uint32_t laneDesignK;     /* tables of at most this many distinct symbols (0, 32, 64, 128 or 256;
-                                 0: none) are designed one per thread, the others one per wave */
+                                 0: none) are designed one per thread, the others one per wave.  The
+                                 library's table applies it to jobs of more than 256 tables, a tuning
+                                 that the caller set to every job */
 } cc_tuning;
 /* The built-in defaults. */
 CC_API cc_status cc_default_tuning(cc_tuning* out);

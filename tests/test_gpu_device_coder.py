@@ -224,3 +224,22 @@ def test_device_encode_decode_chain(cc, torch_gpu, inst14):
     assert used == nw
     for a, b in zip(outs, s):
         assert np.array_equal(a.cpu().numpy().view(np.uint16), b)
+
+
+def test_per_thread_tables_are_designed_where_they_are_asked_for(cc, torch_gpu, inst_lanes):
+    """A tuning the caller set holds for jobs of any size; the library's own leaves jobs of at most 256 tables
+    to the waves."""
+    rng = np.random.default_rng(5)
+    own = cc.createInstance(0, 300, 1 << 12, 128, 14)
+    own.setTuning(None)
+    lanes = cc.loadTuning()["laneDesignK"] > 0
+    for inst, count, want in ((inst_lanes, 1, True), (own, 1, False), (own, 256, False), (own, 257, lanes)):
+        streams = [laplace_symbols(rng, 200) for _ in range(count)]
+        cc.setTimingDetail(inst, cc.TIMING_DETAIL_HIGH)
+        check(cc, torch_gpu, inst, streams, False, 14, 128)
+        names, _ = cc.getTimings(inst)
+        cc.resetTimings(inst)
+        cc.setTimingDetail(inst, cc.TIMING_DETAIL_NONE)
+        log("per-thread designs", count, want)
+        assert any("huff_design_lanes" in x for x in names) == want, names
+    own.close()
