@@ -15,6 +15,7 @@
 #include "../coder.hpp"
 #include "../profile.hpp"
 #include "arrival.hpp"
+#include "choice_heap.hpp"
 #include "huff_design.hpp"
 #include "wave.hpp"
 
@@ -825,144 +826,26 @@ struct WaveEx {
     }
 };
 
-// The merge loop's heap operations with the descent known beforehand: every node with two children has
-// a choice bit (1: the pop's hole goes on to the right child, i.e. the left one is not strictly rarer;
-// the other nodes' bits mean nothing), kept up to date by each pop and push, so a pop reads the heap
-// once, along its path, instead of once per six levels and once more along the path.  `top`: the choices
-// of the top six levels, bit j local node j; lane b's lo and hi: those of the six levels below node
-// 64 + b (12 levels, heaps of up to 4095 entries).  Lane i finds out whether a walk over such a mask
-// ends at leaf i: its six ancestors' bits (all) then spell i (want).
-// A merge is one wave's serial chain of instructions and sets the length of the design phase, so the
-// forms below are the short ones: a lane decides by its own entry whether it moves (counts do not fall
-// along a path), masks are combined on the scalar unit, and no branch depends on a lane.  Measured on MI355X:
-// 64 mixed bricks (largest table about 1,900 symbols) 2.6 -> 1.75 ms in the design phase, 2048 bricks
-// 5.2 -> 4.2 ms; a form with the bits as one mask a subtree but the old, longer selections took 2.15 ms.
-struct ChoiceEx : WaveEx {
-    uint64_t top;
-    uint32_t lo, hi;
-    uint32_t all_lo, all_hi, want_lo, want_hi;
-    uint32_t sd_up, sd_bit;  // 6 - depth of this lane's local node (lane 63: none), 1 << depth
-    uint32_t up, turn;       // shift to this lane's node of a 12-level path (lane: depth), bit of its choice
-
+// The lanes of a wave, for the merge loop's heap operations.
+struct WaveLanes {
+    static __device__ __forceinline__ int lane() { return (int)threadIdx.x; }
     static __device__ __forceinline__ uint64_t vote(bool b) { return __builtin_amdgcn_ballot_w64(b); }
-    static __device__ __forceinline__ uint32_t rdl(uint32_t v, uint32_t l) {
+    static __device__ __forceinline__ uint32_t read(uint32_t v, uint32_t l) {
         return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
     }
-    __device__ __forceinline__ uint64_t subtree(uint32_t b) const { return ((uint64_t)rdl(hi, b) << 32) | rdl(lo, b); }
-    __device__ __forceinline__ void set_subtree(uint32_t b, uint64_t m) {
-        lo = (uint32_t)lane() == b ? (uint32_t)m : lo;
-        hi = (uint32_t)lane() == b ? (uint32_t)(m >> 32) : hi;
+    static __device__ __forceinline__ uint32_t next(uint32_t v, uint32_t last) {
+        return dpp::mov<0x101>(last, v);  // row_shl:1
     }
-    __device__ void heap_begin(const HeapEntry* h, int K) {
-        const int ln = lane();
-        const int sd = ln < 63 ? 31 - __builtin_clz(ln + 1) : 0;
-        sd_up = 6 - sd;
-        sd_bit = 1u << sd;
-        up = ln < 12 ? 12 - ln : 0;
-        turn = ln < 12 ? 1u << (11 - ln) : 0u;
-        uint64_t mall = 0, mwant = 0;
-        for (int d = 0; d < 6; d++) {
-            const int a = ((64 | ln) >> (6 - d)) - 1;
-            mall |= 1ull << a;
-            mwant |= (uint64_t)(((64 | ln) >> (5 - d)) & 1) << a;
-        }
-        all_lo = (uint32_t)mall;
-        all_hi = (uint32_t)(mall >> 32);
-        want_lo = (uint32_t)mwant;
-        want_hi = (uint32_t)(mwant >> 32);
-        auto choices = [&](int root) {  // of the six levels below 1-based node `root`
-            const int c = (root << sd) + (ln + 1) - (1 << sd);
-            return vote(ln < 63 && 2 * c < K && !(h[2 * c - 1].count < h[2 * c].count));
-        };
-        top = choices(1);
-        lo = hi = 0;
-        for (int b = 0; b < 64 && 2 * (64 + b) < K; b++) set_subtree(b, choices(64 + b));
-    }
-    // the leaf at which the walk over a subtree's choices ends
-    __device__ __forceinline__ uint32_t walk(uint64_t m) const {
-        return (uint32_t)__builtin_ctzll(vote(((uint32_t)m & all_lo) == want_lo) &
-                                         vote(((uint32_t)(m >> 32) & all_hi) == want_hi));
-    }
-    // the choices m of a subtree after those on the way to its leaf e (64 + leaf) became bits of nb
-    __device__ __forceinline__ uint64_t changed(uint64_t m, uint32_t e, uint32_t nb) const {
-        const uint64_t on = vote((e >> sd_up) == (uint32_t)lane() + 1u);
-        return (m & ~on) | (on & vote((nb & sd_bit) != 0u));
-    }
-    static __device__ __forceinline__ HeapEntry& node(HeapEntry* h, uint32_t c) {  // 1-based
+    static __device__ __forceinline__ HeapEntry& entry(HeapEntry* h, uint32_t c) {
         return *reinterpret_cast<HeapEntry*>(reinterpret_cast<char*>(h - 1) + 8u * c);
     }
-
-    // The heap's n entries left after its last one, v, was taken out.  Deep: n >= 128, so the path
-    // runs through the top six levels.
-    template <bool Deep>
-    __device__ __forceinline__ HeapEntry pop(HeapEntry* h, uint32_t n, HeapEntry v) {
-        const uint32_t ln = (uint32_t)lane();
-        const uint32_t e1 = 64u | walk(top);
-        uint64_t sub = 0;
-        uint32_t E = e1 << 6;  // the path's node at depth k is E >> (12 - k), 1-based
-        if (Deep) {
-            sub = subtree(e1 - 64u);
-            E |= walk(sub);
-        }
-        // the parent of a lone left child n may still point right, to n + 1
-        const uint32_t below_d = (uint32_t)__builtin_clz(n) - 19u;  // 12 - depth of n
-        const uint32_t gone = (n & 1u) ? 0u : n + 1u;
-        E -= (E >> below_d) == gone ? 1u << below_d : 0u;
-        const uint32_t pk = E >> up, parents = n >> 1;  // (nodes up to n / 2 have a child)
-        const uint32_t last = parents > 1u ? parents : 1u;
-        const HeapEntry* ch = &node(h, 2u * (pk < last ? pk : last));
-        const HeapEntry l = ch[0], r = ch[1];
-        const uint64_t act = vote(pk <= parents);
-        const bool right = (E & turn) != 0u;
-        const HeapEntry pn{right ? r.count : l.count, right ? r.node : l.node};
-        const uint32_t sib = right ? l.count : r.count;
-        // the path's entries move up until one is larger than v, which takes its place
-        const uint64_t rise = vote(pn.count <= v.count) & act;
-        const uint32_t is = (uint32_t)__builtin_popcountll(rise);
-        const bool mv = ln < is;
-        const HeapEntry moved{mv ? pn.count : v.count, mv ? pn.node : v.node};
-        if (ln <= is) node(h, pk) = moved;
-        // the new count one level down the path: what moved there, or what was there below v
-        const uint32_t below = dpp::mov<0x101>(0u, moved.count);  // row_shl:1 (paths are shorter than a row)
-        const uint32_t now = mv ? below : pn.count;
-        const uint32_t nb = (uint32_t)vote((right ? sib : now) >= (right ? now : sib));
-        top = changed(top, e1, nb);
-        if (Deep) set_subtree(e1 - 64u, changed(sub, 64u | (E & 63u), nb >> 6));
-        return HeapEntry{rdl(moved.count, 0), rdl(moved.node, 0)};
-    }
-    __device__ __forceinline__ HeapEntry heap_pop(HeapEntry* h, int len) {
-        const HeapEntry v = h[len - 1];
-        if (len <= 1) return v;
-        return len > 128 ? pop<true>(h, (uint32_t)len - 1u, v) : pop<false>(h, (uint32_t)len - 1u, v);
-    }
-    // v at the new 1-based position Q; lane d holds the ancestor at depth d.  Deep: Q >= 128.
-    template <bool Deep>
-    __device__ __forceinline__ HeapEntry push(HeapEntry* h, uint32_t Q, HeapEntry v, HeapEntry top_entry) {
-        const uint32_t ln = (uint32_t)lane(), T = 31u - (uint32_t)__builtin_clz(Q);
-        const uint64_t act = (1ull << T) - 1ull;
-        const uint32_t cq = Q >> ((T - ln - 1u) & 31u);  // the chain's node one level down
-        const uint32_t c = cq > 2u ? cq : 2u;            // (any node in range for the lanes past the chain)
-        const HeapEntry e = node(h, c >> 1);
-        const uint32_t sib = node(h, c ^ 1u).count;
-        const uint64_t sink = vote(v.count < e.count) & act;  // the ancestors that move down
-        const uint32_t at = (uint32_t)__builtin_ctzll(sink | (1ull << T));  // v's depth
-        const bool mv = ln >= at;
-        if (mv & (ln < T)) node(h, c) = e;
-        node(h, Q >> (T - at)) = v;
-        // the new count one level down the chain: an ancestor that moved, v, or what was there above v
-        const uint32_t ec = ln < T ? e.count : 0xFFFFFFFFu;
-        const uint32_t below = dpp::mov<0x101>(0xFFFFFFFFu, ec);
-        const uint32_t now = mv ? ec : (v.count < below ? v.count : below);
-        const bool odd = (c & 1u) != 0u;
-        const uint32_t nb = (uint32_t)vote((odd ? sib : now) >= (odd ? now : sib)), E = Q << (12 - T), e1 = E >> 6;
-        // nodes below depth T - 1 on E's leftmost way down have no two children
-        top = changed(top, e1, nb);
-        if (Deep) set_subtree(e1 - 64u, changed(subtree(e1 - 64u), 64u | (E & 63u), nb >> 6));
-        return at == 0 ? v : top_entry;
-    }
-    __device__ __forceinline__ HeapEntry heap_push(HeapEntry* h, int pos, HeapEntry v, HeapEntry top_entry) {
-        const uint32_t Q = (uint32_t)pos + 1u;
-        return Q >= 128u ? push<true>(h, Q, v, top_entry) : push<false>(h, Q, v, top_entry);
+};
+struct ChoiceEx : WaveEx {
+    design::ChoiceHeap<WaveLanes> choices;
+    __device__ __forceinline__ void heap_begin(HeapEntry* h, int K) { choices.begin(h, K); }
+    __device__ __forceinline__ HeapEntry heap_pop(HeapEntry* h, int len) { return choices.pop(h, len); }
+    __device__ __forceinline__ HeapEntry heap_push(HeapEntry* h, int pos, HeapEntry v, HeapEntry top) {
+        return choices.push(h, pos, v, top);
     }
 };
 
