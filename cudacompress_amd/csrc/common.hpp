@@ -44,7 +44,6 @@ struct Error {
     } while (0)
 
 __host__ __device__ inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
-__host__ __device__ inline uint32_t div_up_dev(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 inline uint64_t align_up(uint64_t a, uint64_t b) { return (a + b - 1) / b * b; }
 
 // Number of bits needed to store maxValue, src/cudaCompress/util.h:23-32.

@@ -33,17 +33,6 @@ __device__ __forceinline__ uint32_t rd_bits(const uint32_t* w, uint64_t nwords, 
     return (uint32_t)((win << o) >> (64 - n));
 }
 
-__device__ uint64_t arena_take(CoderState* st, uint64_t words, uint64_t cap, bool& ok) {
-    words = (words + 15) & ~uint64_t(15);
-    const uint64_t off = atomicAdd(&st->scratch_used, (unsigned long long)words);
-    if (off + words > cap) {
-        ok = false;
-        atomicCAS(&st->err, 0u, (uint32_t)kDecScratch);
-        return 0;
-    }
-    return off;
-}
-
 __global__ void k_dec_init(CoderState* st) {
     if (threadIdx.x == 0) {
         st->scratch_used = 0;

@@ -63,10 +63,6 @@ __device__ __forceinline__ uint64_t wave_incl_scan_u64(uint64_t v) {
 __device__ __forceinline__ long long wave_incl_max_i64(long long v) {
     return dpp::incl_scan<long long>(v, -1ll, [](long long a, long long b) { return a > b ? a : b; });
 }
-// the previous lane's value (lane 0: identity)
-__device__ __forceinline__ long long wave_shift_up_i64(long long v, long long identity) {
-    return (long long)dpp::mov64<dpp::kWaveShr1>((uint64_t)identity, (uint64_t)v);
-}
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) { return dpp::last_lane(wave_incl_scan(v)); }
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) { return dpp::last_lane64(wave_incl_scan_u64(v)); }
 __device__ __forceinline__ uint32_t wave_max(uint32_t v) {

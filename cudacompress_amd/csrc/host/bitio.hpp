@@ -1,10 +1,9 @@
 // Host bit writer/reader with the semantics of include/cudaCompress/BitStream.h: bits are
-// written MSB-first into 32-bit words (writeBits, BitStream.h:377-416); aligned writes pad to
-// the next 32-bit word and store little-endian bytes (writeAligned, :421-456).
+// written MSB-first into 32-bit words (writeBits, BitStream.h:377-416); what is read aligned starts
+// on the next 32-bit word and is little-endian (:421-456).
 #pragma once
 
 #include <cstdint>
-#include <cstring>
 #include <vector>
 
 namespace cca {
@@ -37,25 +36,6 @@ public:
             w_[wi + 1] = (w_[wi + 1] & ~mask2) | (v << sh);
         }
         pos_ += n;
-    }
-    void align32() {
-        pos_ = (pos_ + 31) & ~uint64_t(31);
-        grow(pos_);
-    }
-    void aligned_u32(const uint32_t* v, uint64_t count) {
-        align32();
-        if (count == 0) return;
-        grow(pos_ + 32 * count);
-        memcpy(&w_[pos_ >> 5], v, 4 * count);
-        pos_ += 32 * count;
-    }
-    void aligned_u16(const uint16_t* v, uint64_t count) {
-        align32();
-        if (count == 0) return;
-        grow(pos_ + 16 * count);
-        memcpy(reinterpret_cast<unsigned char*>(w_.data()) + (pos_ >> 3), v, 2 * count);
-        pos_ += 16 * count;
-        align32();
     }
 
 private:

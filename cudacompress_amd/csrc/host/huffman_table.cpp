@@ -134,38 +134,4 @@ uint64_t table_bits(const HeaderFormat& f, const EncTable& t) {
            (uint64_t)sb * t.symbols.size();
 }
 
-bool read_table(const HeaderFormat& f, BitReader& r, DecTable& d) {
-    for (int i = 0; i < 32; i++) d.first[i] = d.mn[i] = d.mx[i] = -1;
-    const uint32_t nlen = r.bits(5);
-    uint32_t counts[32] = {0};
-    for (uint32_t i = 0; i < nlen; i++) counts[i] = r.bits(f.count_bits);
-    const uint32_t nsym = r.bits(f.count_bits);
-    uint32_t sb = r.bits(f.symbits_bits);
-    // HuffmanTable.cu:138-139: a stored 0 with more than one symbol means 16 (Symbol16 only).
-    // A single-symbol table whose symbol needs 16 bits is read with 0 bits, as the reference does.
-    if (f.dialect == CC_DIALECT_GPU && f.symbits_bits == 4 && sb == 0 && nsym > 1) sb = 16;
-    if (sb > 32 || !r.ok()) return false;
-    d.symbols.resize(nsym);
-    for (uint32_t i = 0; i < nsym; i++) d.symbols[i] = r.bits(sb);
-    if (!r.ok()) return false;
-    if (nsym == 0 || nlen == 0) return true;
-    uint64_t total = 0;
-    for (uint32_t i = 0; i < nlen; i++) total += counts[i];
-    if (total != nsym) return false;
-    // canonical codes; first/min/max per length (HuffmanTable.cu:205-266)
-    int32_t code = 0;
-    uint32_t prev_len = 0, e = 0;
-    for (uint32_t l = 1; l <= nlen; l++) {
-        if (counts[l - 1] == 0) continue;
-        for (uint32_t k = 0; k < counts[l - 1]; k++, e++) {
-            if (e > 0) code = (code + 1) << (l - prev_len);
-            else code = 0;
-            prev_len = l;
-            if (k == 0) { d.first[l - 1] = (int32_t)e; d.mn[l - 1] = code; }
-            d.mx[l - 1] = code;
-        }
-    }
-    return true;
-}
-
 }  // namespace cca

@@ -1,4 +1,4 @@
-// Huffman table design, header serialisation and decode-table construction (host).
+// Huffman table design and header serialisation (host).
 #pragma once
 
 #include <cstdint>
@@ -30,13 +30,5 @@ cc_status design_table(int dialect, const uint32_t* hist, uint32_t symbol_max, E
 void write_table(const HeaderFormat& f, const EncTable& t, BitWriter& w);
 // exact number of header bits write_table produces
 uint64_t table_bits(const HeaderFormat& f, const EncTable& t);
-
-struct DecTable {
-    int32_t first[32], mn[32], mx[32];  // device layout: first[32] | min[32] | max[32]
-    std::vector<uint32_t> symbols;
-};
-// Parses a header and builds first/min/max per length (HuffmanTable.cu:117-151, :205-266).
-// Returns false on a malformed header.
-bool read_table(const HeaderFormat& f, BitReader& r, DecTable& d);
 
 }  // namespace cca
