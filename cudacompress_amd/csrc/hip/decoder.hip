@@ -484,13 +484,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     // words a round may take, at most R (mlen <= 31); the copy serves a round when it holds as many
     // from nxt on and the one read ahead (an entry no code of a broken table reaches takes kLut + 1 bits)
     const uint32_t round_words = min((kDecRound * max(s.nlen, kLut + 1) + 31) / 32 + 1, kDecRound);
-    auto refill = [&](bool on) {
-        const bool need = on && q < 0;
+    auto refill = [&]() {
+        const bool need = q < 0;
         hi = need ? lo : hi;
         lo = need ? nx : lo;
         nxt += need ? 1u : 0u;
         nx = win[64 * (nxt - (uint32_t)w0)];  // on its way beside the code's table lookup
-        q = on ? q & 31 : q;
+        q &= 31;
     };
     const uint32_t sh = 32 - lb;
     const uint32_t mlen = s.nlen;
@@ -523,10 +523,18 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
         for (uint32_t l = len0; l < mlen; l++) {
             const bool past = pk > (uint32_t)__builtin_amdgcn_readlane((int)bound, (int)l - 1);
             if (!__any(past)) break;  // (bounds do not fall, so no lane passes a later one)
+            const int step = __builtin_amdgcn_readlane(off_step, (int)l - 1);
             len += past ? 1u : 0u;
-            idx += past ? __builtin_amdgcn_readlane(off_step, (int)l - 1) : 0;
+            idx += past ? step : 0;
         }
         idx += (int)(pk >> (32 - len));
+        return kLong | (len << 24) | (((uint32_t)idx < nsym ? (uint32_t)idx : 0xFFFFFFu) & 0xFFFFFFu);
+    };
+    // The same by one lane, from the table in LDS: where the lanes of a wave take their own ways.
+    auto walk = [&](uint32_t pk) -> uint32_t {
+        uint32_t len = kLut + 1;
+        while (len < mlen && (int)(pk >> (32 - len)) > tab[64 + len - 1]) len++;
+        const int idx = tab[len - 1] + (int)(pk >> (32 - len)) - tab[32 + len - 1];
         return kLong | (len << 24) | (((uint32_t)idx < nsym ? (uint32_t)idx : 0xFFFFFFu) & 0xFFFFFFu);
     };
     auto long_symbol = [&](uint32_t e) { return symbol_at((int)(e & 0xFFFFFFu)); };
@@ -574,17 +582,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
 #pragma unroll
                 for (uint32_t k = 0; k < NW; k++) reinterpret_cast<u32a*>(run_row)[k] = fill;
                 uint32_t i = 0;
-                // (a lane that is done takes runs of no position until the last one is)
-                while (__any(i < kDecRound)) {
-                    refill(i < kDecRound);
+                // (a lane that is done takes steps of no position and no bit until the last one is)
+                while (i < kDecRound) {
+                    refill();
                     const uint32_t pk = __builtin_amdgcn_alignbit(hi, lo, (uint32_t)q);
-                    const bool run = (pk >> 31) == 0u || i >= kDecRound;
+                    const bool run = (pk >> 31) == 0u;
                     uint32_t e = lut[pk >> sh];
-                    const bool is_long = !run && e == 0u;
-                    if (__any(is_long)) {
-                        const uint32_t found = slow(is_long ? pk : 0u);
-                        e = is_long ? found : e;
-                    }
+                    if (!run && e == 0u) e = walk(pk);
                     const uint32_t k = min(pk ? (uint32_t)__clz(pk) : 32u, kDecRound - i);
                     const uint32_t sym = !run && (e & kLong) ? long_symbol(e) : e & 0xFFFFFFu;
                     if (!run) run_row[i] = (S)sym;
@@ -601,7 +605,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
                 uint32_t es[kDecRound], any = 0;
 #pragma unroll
                 for (uint32_t i = 0; i < kDecRound; i++) {
-                    refill(true);
+                    refill();
                     const uint32_t pk = __builtin_amdgcn_alignbit(hi, lo, (uint32_t)q);
                     uint32_t e = lut[pk >> sh];
                     if (__any(e == 0u)) {
