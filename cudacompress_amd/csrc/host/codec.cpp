@@ -7,8 +7,9 @@
 //   1. upload of the stream list; the stats pass (zero-run pairs, histograms)     -> sync #1: histograms
 //   2. table design on the host (libstdc++ heap/sort, as the reference), exact bit counts from
 //      histogram x length, the layout of every section (Encode.cpp:402-463 rl, :751-782 huff)
-//   3. one upload (sequence records, symbols in codeword order), from which the device makes the code
-//      tables; the pack writes the sections in place -> sync #2: words
+//   3. one upload (sequence records, symbols in codeword order and, for small alphabets, the code tables,
+//      which the device makes of the symbols otherwise); the pack writes the sections in place -> sync #2:
+//      words
 // The reference does >= streams + 6 host synchronisations per encodeRLHuff, per level of a volume.
 //
 // Decode walks the sections' heads on the host (counts, sizes, as Encode.cpp:522-621; the symbol
@@ -20,6 +21,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "../hip/huff_design.hpp"
 #include "batch.hpp"
 #include "bitio.hpp"
 #include "huffman_table.hpp"
@@ -40,7 +42,18 @@ struct Staging {
     }
 };
 
-constexpr uint64_t kArenaGuess = 1u << 24;  // words (64 MB)
+// Most arena words (64 MB) that are taken on the chance that every stream uses its whole alphabet, and the
+// guess up to which none are: below a megabyte an allocation costs next to nothing and above 0.35 ms, more
+// than to run the statistics again (first call of an instance on 32^3 floats 355 us with 0.7 MB and 1063 with
+// 1.2; on a 64^3 lossless field, which needs 5.8 MB, the second run is 70 us).
+constexpr uint64_t kArenaGuess = 1u << 24, kArenaSmall = 200000;
+// Words that come down with the records at most, and that are pinned for it from the start (a megabyte; an
+// allocation of pinned memory takes 0.02 or 0.35 ms, whatever its size, and each megabyte 0.4 ms to touch).
+constexpr uint64_t kDownMost = 1u << 18;
+// Bins of a call's alphabets up to which the code tables go up whole: 128 KB take about as long as the launch
+// that makes them of the symbols (32^3 floats: 325 us with the tables, 335 with the launch; a 4096^2 terrain's
+// alphabets are 4 MB).
+constexpr uint64_t kDenseBins = 16384;
 
 }  // namespace
 
@@ -74,18 +87,18 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
     const uint32_t nseq = job.nseq;
     // one device buffer: the coder's state, the sequence records, the arena
     const size_t o_seq = align_up(sizeof(CoderState), 64), o_arena = align_up(o_seq + sizeof(SeqInfo) * nseq, 256);
-    // room for a histogram of the whole alphabet per stream, so that wide symbols do not have the statistics
-    // run twice; above kArenaGuess a guess, with a second run where it was too small
+    // a guess, with a second run of the statistics where it was too small
     const uint64_t alphabet = I->dialect == CC_DIALECT_CPU ? 65536u : std::min<uint64_t>(1ull << I->log2, 65536u);
-    const uint64_t least = 1024 + (uint64_t)nseq * (kStatBins + 2 * design_leaf_words());
-    uint64_t cap = std::max({I->enc_arena, least, std::min(least + ns * alphabet, kArenaGuess)});
+    uint64_t cap = 1024 + (uint64_t)nseq * (kStatBins + 2 * design_leaf_words());
+    if (cap > kArenaSmall) cap = std::max(cap, std::min(cap + ns * alphabet, kArenaGuess));
+    cap = std::max(cap, I->enc_arena);
     unsigned char *d, *h;
     for (int attempt = 0;; attempt++) {
         d = (unsigned char*)I->d_enc.get(o_arena + 4 * cap);
         encode_stats(D, job, (SeqInfo*)(d + o_seq), (uint32_t*)(d + o_arena), cap, (CoderState*)d, st);
         // the state, the records and as much of the arena as the last call used come down together
         const uint64_t first = std::min(cap, std::max<uint64_t>(I->enc_down, 4096));
-        h = (unsigned char*)I->h_down.get(o_arena + 4 * first);
+        h = (unsigned char*)I->h_down.get(o_arena + 4 * std::min<uint64_t>(cap, kDownMost));
         CCA_HIP(hipMemcpyAsync(h, d, o_arena + 4 * first, hipMemcpyDeviceToHost, st));
         CCA_HIP(hipStreamSynchronize(st));
         const CoderState s = *(const CoderState*)h;
@@ -96,14 +109,14 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
         CCA_REQUIRE(s.err == kErrNone, CC_ERR_OUT_OF_MEMORY, "coder arena exhausted");
         const uint64_t used = std::min<uint64_t>(s.scratch_used, cap);
         if (used > first) {
-            // pinned for what comes down, not for the arena: fresh pinned pages cost 0.4 ms a megabyte to touch
+            // (past kDownMost pinned for what comes down, not for the arena)
             const uint64_t have = I->h_down.cap < o_arena + 4 * used ? 0 : o_arena + 4 * first;
             h = (unsigned char*)I->h_down.get(o_arena + 4 * used);
             CCA_HIP(hipMemcpyAsync(h + have, d + have, o_arena + 4 * used - have, hipMemcpyDeviceToHost, st));
             CCA_HIP(hipStreamSynchronize(st));
         }
         I->enc_arena = cap;
-        I->enc_down = std::min<uint64_t>(align_up(used, 4096), 1u << 18);
+        I->enc_down = std::min<uint64_t>(align_up(used, 4096), kDownMost);
         break;
     }
     std::vector<SeqInfo> seqs((const SeqInfo*)(h + o_seq), (const SeqInfo*)(h + o_seq) + nseq);
@@ -156,10 +169,9 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
             CCA_REQUIRE(bits[j] < (1ull << 32), CC_ERR_INVALID_ARG, "coded stream exceeds 2^32 bits");
         }
     }
-    // sections in stream order; the arena: every table's symbols in codeword order, which go up, then its
-    // codes and lengths by symbol, which the device makes of them, and the coding-block offsets, which the
-    // pack fills
-    uint64_t pos = 0, up = 0;
+    // sections in stream order; the arena: every table's symbols in codeword order, then its codes and lengths
+    // by symbol, which go up too or which the device makes, and the coding-block offsets, which the pack fills
+    uint64_t pos = 0, up = 0, bins = 0;
     uint32_t most_syms = 0;
     for (uint32_t i = 0; i < ns; i++) {
         const EncodeStream& s = streams[i];
@@ -182,6 +194,7 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
             r.syms_off = up;
             up = align_up(up + std::max<uint32_t>(r.nsym, 1), 16);
             most_syms = std::max(most_syms, r.nsym);
+            bins += r.smax + 1;
         }
         I->seg_bits[i] = (pos - I->seg_begin[i]) * 32;
     }
@@ -190,6 +203,10 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
     for (SeqInfo& r : seqs) {
         r.code_off = arena_words;
         arena_words = align_up(arena_words + 2ull * (r.smax + 1), 16);
+    }
+    const bool dense = bins <= kDenseBins;
+    if (dense) up = arena_words;
+    for (SeqInfo& r : seqs) {
         r.boff_off = arena_words;
         arena_words += align_up(std::max<uint32_t>(div_up(r.count, cbs), 1), 16);
     }
@@ -201,10 +218,21 @@ void encode_items(cc_instance* I, int symSize, const std::vector<EncodeStream>& 
     *(CoderState*)u = CoderState{0, total, 0, 0, 0};
     memcpy(u + o_seq, seqs.data(), sizeof(SeqInfo) * nseq);
     uint32_t* ua = (uint32_t*)(u + o_arena);
-    for (uint32_t j = 0; j < nseq; j++)
-        memcpy(ua + seqs[j].syms_off, tables[j].symbols.data(), 4ull * tables[j].symbols.size());
+    for (uint32_t j = 0; j < nseq; j++) {
+        const SeqInfo& r = seqs[j];
+        const std::vector<uint32_t>& syms = tables[j].symbols;
+        memcpy(ua + r.syms_off, syms.data(), 4ull * syms.size());
+        if (!dense) continue;
+        uint32_t fc[32], fi[32], *code = ua + r.code_off, *len = code + r.smax + 1;
+        design::first_codes(r.cpl, (int)r.nlen, fc, fi);
+        for (uint32_t l = 0; l < r.nlen; l++)
+            for (uint32_t c = 0; c < r.cpl[l]; c++) {
+                code[syms[fi[l] + c]] = fc[l] + c;
+                len[syms[fi[l] + c]] = l + 1;
+            }
+    }
     CCA_HIP(hipMemcpyAsync(d, u, o_arena + 4 * up, hipMemcpyHostToDevice, st));
-    coder_code_tables((const SeqInfo*)(d + o_seq), nseq, most_syms, (uint32_t*)(d + o_arena), st);
+    if (!dense) coder_code_tables((const SeqInfo*)(d + o_seq), nseq, most_syms, (uint32_t*)(d + o_arena), st);
     uint32_t* dw = I->d_words.as<uint32_t>(std::max<uint64_t>(total, 1));
     encode_pack(D, job, (SeqInfo*)(d + o_seq), (uint32_t*)(d + o_arena), (CoderState*)d, dw, total, st);
     uint32_t* hw = I->h_words.as<uint32_t>(std::max<uint64_t>(total, 1));

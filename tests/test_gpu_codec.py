@@ -251,3 +251,19 @@ def test_decodes_one_after_the_other_share_their_staging(cc, torch_gpu):
     log("process size after each decode, MB", [s >> 20 for s in sizes], "staged", staged >> 20)
     assert sizes[-1] - sizes[0] < staged
     inst.close()
+
+
+@pytest.mark.parametrize("bins", [4096, 4097, 16383, 16384, 16385, 65000])
+def test_code_tables_from_the_host_and_from_the_device(cc, torch_gpu, bins):
+    """Alphabets around the sizes at which a stream's statistics and a call's code tables change their way."""
+    rng = np.random.default_rng(bins)
+    inst = cc.createInstance(0, 2, 20000, 64, 16)
+    for rl in (True, False):
+        stream = laplace_symbols(rng, 20000, scale=bins / 12, density=0.6, maxsym=bins - 1)
+        stream[777] = bins - 1
+        others = [] if rl or bins % 2 else [np.zeros(20000, np.uint16)]
+        bits = cc.BitStream()
+        assert (cc.encodeRLHuff if rl else cc.encodeHuff)(inst, bits, [to_dev(torch_gpu, s) for s in [stream] + others], 20000)
+        want, nbits = o.encode([stream] + others, rl=rl, log2=16, cbs=64)
+        assert bits.getBitSize() == nbits and np.array_equal(bits.words(), want)
+    inst.close()
