@@ -263,7 +263,8 @@ struct DecPart {
 };
 constexpr uint32_t kPartSymbols = 2048, kPartBlocks = 4096;
 // The same stages for sequences parsed on the host (records with the positions, counts, outputs and
-// arena ranges filled in): tables and block decode, then the zero-run expansion.
+// arena ranges filled in): tables (no parts: they are in the records and the arena) and block decode, then
+// the zero-run expansion.
 void coder_decode_parsed(DecSeq* d_seqs, uint32_t nseq, const CoderParams& p, int symSize, uint32_t* scratch,
                          CoderState* d_state, const DecItem* d_items, const uint32_t* d_wave_seq,
                          const uint32_t* d_wave_first, uint32_t nwaves, uint32_t nlong, const DecPart* d_parts,

@@ -960,9 +960,11 @@ void coder_decode_parsed(DecSeq* d_seqs, uint32_t nseq, const CoderParams& p, in
                          const uint32_t* d_wave_first, uint32_t nwaves, uint32_t nlong, const DecPart* d_parts,
                          uint32_t nparts, uint64_t total_symbols, const RleChunks& rc, hipStream_t st) {
     if (nseq == 0) return;
-    CCA_LAUNCH("dec_tables", 0, k_dec_tables<true>, dim3(nparts), dim3(256), 0, st, d_seqs, d_parts, p, scratch,
-               d_state);
-    CCA_LAUNCH_CHECK();
+    if (nparts) {
+        CCA_LAUNCH("dec_tables", 0, k_dec_tables<true>, dim3(nparts), dim3(256), 0, st, d_seqs, d_parts, p, scratch,
+                   d_state);
+        CCA_LAUNCH_CHECK();
+    }
     const uint64_t outb = total_symbols * symSize;
     if (symSize == 2)
         launch_blocks<uint16_t>(d_seqs, d_wave_seq, d_wave_first, nwaves, nlong, p, scratch, d_items, rc, outb, st);

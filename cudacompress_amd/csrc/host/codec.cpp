@@ -13,9 +13,9 @@
 // The reference does >= streams + 6 host synchronisations per encodeRLHuff, per level of a volume.
 //
 // Decode walks the sections' heads on the host (counts, sizes, as Encode.cpp:522-621; the symbol
-// lists and codewords are left to the device), stages the sequence records and the bitstream in one
-// pinned buffer, uploads it with a single copy and enqueues the table build, the block decode and the
-// zero-run expansion.
+// lists, unless they are few and short, and the codewords are left to the device), stages the sequence
+// records and the bitstream in one pinned buffer, uploads it with a single copy and enqueues the table build,
+// the block decode and the zero-run expansion.
 #include "codec.hpp"
 
 #include <algorithm>
@@ -54,6 +54,41 @@ constexpr uint64_t kDownMost = 1u << 18;
 // that makes them of the symbols (32^3 floats: 325 us with the tables, 335 with the launch; a 4096^2 terrain's
 // alphabets are 4 MB).
 constexpr uint64_t kDenseBins = 16384;
+
+// A decode of at most so many sequences, symbols and blocks in all has its tables made here: the launch that
+// makes them takes 7 us of the 45 to 70 that such a call has, two sequences 1 to 2 us (one stream of 1000
+// symbols, zero runs: 71 us with the launch, 63 without).
+constexpr uint32_t kHostTables = 4, kHostSymbols = 1024, kHostBlocks = 1024;
+
+// Code table, lookup table, symbols and block offsets of a sequence, as k_dec_tables makes them.
+void host_tables(const HeaderFormat& fmt, const uint32_t* words, uint64_t nbits, uint32_t nblk, DecSeq& s,
+                 uint32_t* arena) {
+    uint32_t cpl[32] = {0}, fc[32], fi[32];
+    BitReader counts(words, nbits, s.hdr_bit + 5), symbols(words, nbits, s.sym_bit);
+    for (uint32_t l = 0; l < s.nlen; l++) cpl[l] = counts.bits(fmt.count_bits);
+    design::first_codes(cpl, (int)s.nlen, fc, fi);
+    for (uint32_t l = 0; l < 32; l++) {
+        const bool used = l < s.nlen && cpl[l] > 0;
+        s.tab[l] = used ? (int32_t)fi[l] : -1;
+        s.tab[32 + l] = used ? (int32_t)fc[l] : -1;
+        s.tab[64 + l] = used ? (int32_t)(fc[l] + cpl[l] - 1) : -1;
+    }
+    uint32_t* lut = arena + s.lut_off;
+    uint32_t* syms = lut + (1u << kDecLutBits);
+    for (uint32_t k = 0; k < s.nsym; k++) syms[k] = symbols.bits(s.sb);
+    // (length << 24) | symbol by the next lb bits; of the codes of a broken table the shorter one counts
+    const uint32_t lb = std::min(s.nlen, kDecLutBits);
+    std::fill(lut, lut + (1u << lb), 0u);
+    for (uint32_t l = lb; l-- > 0;)
+        for (uint64_t c = 0; c < cpl[l]; c++) {
+            const uint64_t first = ((uint64_t)fc[l] + c) << (lb - l - 1), last = first + (1ull << (lb - l - 1));
+            if (last > (1ull << lb)) break;
+            const uint32_t sym = fi[l] + c < s.nsym ? syms[fi[l] + c] & 0xFFFFFFu : 0u;
+            std::fill(lut + first, lut + last, (l + 1) << 24 | sym);
+        }
+    const uint16_t* incs = (const uint16_t*)(words + s.incs_off);
+    for (uint32_t b = 0, at = 0; b < nblk; b++) arena[s.boff_off + b] = at += incs[b];
+}
 
 }  // namespace
 
@@ -359,19 +394,26 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
 
     // ---- the upload and the arena ----------------------------------------------------------------
     uint32_t nlong = 0, nshort = 0, nchunks = 0;
-    uint64_t total_syms = 0, arena = 0;
+    uint64_t total_syms = 0, arena = 0, total_nsym = 0, total_blk = 0;
     for (DecSeq& s : seqs) {
         const uint32_t nblk = div_up(s.count, cbs);
+        total_nsym += s.nsym;
+        total_blk += nblk;
         (dec_long(nblk) ? nlong : nshort) += dec_entries(nblk);
         s.boff_off = arena;
         s.lut_off = arena + align_up(std::max<uint32_t>(nblk, 1), 16);
         arena = s.lut_off + align_up((1u << kDecLutBits) + (uint64_t)s.nsym + 1, 16);
     }
     for (uint32_t i = 0; i < ns; i++) total_syms += items[i].n;
+    for (uint32_t i = 0; i < ns; i++)  // an RLE stream without a pair still has its output cleared
+        if (items[i].rl && items[i].n) nchunks += std::max(1u, rle_chunks(seqs[items[i].seq].count, true));
+    const bool made_here = nseq <= kHostTables && total_nsym <= kHostSymbols && total_blk <= kHostBlocks;
+    if (made_here) parts.clear();
     Staging s;
     const size_t o_state = s.push<CoderState>(1), o_seq = s.push<DecSeq>(nseq), o_item = s.push<DecItem>(ns);
     const size_t o_wseq = s.push<uint32_t>(nlong + nshort), o_wfirst = s.push<uint32_t>(nlong + nshort);
     const size_t o_ifirst = s.push<uint32_t>(ns + 1), o_part = s.push<DecPart>(parts.size());
+    const size_t o_arena = s.push<uint32_t>(made_here ? arena + nchunks : 0);
     std::vector<size_t> o_words(nbs, 0);
     for (uint32_t b = 0; b < nbs; b++)
         if (w1[b] > w0[b]) o_words[b] = s.push<uint32_t>(w1[b] - w0[b]);
@@ -400,6 +442,7 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
     for (uint32_t j = 0; j < nseq; j++) {
         DecSeq& q = seqs[j];
         const uint32_t b = seq_bs[j], i = q.item;
+        if (made_here) host_tables(fmt, bsWords[b], bsBits[b], div_up(q.count, cbs), q, (uint32_t*)(h + o_arena));
         q.base = (const uint32_t*)(d + o_words[b]);
         q.nwords = w1[b] - w0[b];
         q.hdr_bit -= 32 * w0[b];
@@ -409,17 +452,16 @@ void decode_items(cc_instance* I, int symSize, const uint32_t* const* bsWords, c
         q.out = !items[i].rl ? items[i].out : (j == items[i].seq ? dsym : dzc) + rl_off[i] * symSize;
         add_block_entries(j, div_up(q.count, cbs), hws, hwf, wl, ws);
     }
-    for (uint32_t i = 0; i < ns; i++) {  // an RLE stream without a pair still has its output cleared
-        hif[i] = nchunks;
-        if (items[i].rl && items[i].n) nchunks += std::max(1u, rle_chunks(seqs[items[i].seq].count, true));
-    }
-    hif[ns] = nchunks;
+    hif[0] = 0;
+    for (uint32_t i = 0; i < ns; i++)
+        hif[i + 1] = hif[i] + (items[i].rl && items[i].n ? std::max(1u, rle_chunks(seqs[items[i].seq].count, true)) : 0u);
     memcpy(h + o_seq, seqs.data(), sizeof(DecSeq) * nseq);
     memcpy(h + o_item, items.data(), sizeof(DecItem) * ns);
     memcpy(h + o_part, parts.data(), sizeof(DecPart) * parts.size());
     for (uint32_t b = 0; b < nbs; b++)
         if (w1[b] > w0[b]) memcpy(h + o_words[b], bsWords[b] + w0[b], 4 * (w1[b] - w0[b]));
-    uint32_t* scratch = I->d_dec_arena.as<uint32_t>(arena + std::max<uint32_t>(nchunks, 1));
+    uint32_t* scratch =
+        made_here ? (uint32_t*)(d + o_arena) : I->d_dec_arena.as<uint32_t>(arena + std::max<uint32_t>(nchunks, 1));
     CCA_HIP(hipMemcpyAsync(d, h, total, hipMemcpyHostToDevice, st));
     CCA_HIP(hipEventRecord(I->dec_event[slot], st));
 
