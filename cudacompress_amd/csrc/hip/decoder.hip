@@ -341,7 +341,7 @@ __global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, const DecPart*
 // The kernel is bound by instruction issue and latency, so a code costs a handful of vector
 // instructions: the bit window is two words {hi, lo} read with one funnel shift (`alignbit`, the
 // next code starting q bits above lo's lowest bit); codewords reach a lane through an LDS copy of
-// WW words from the 16-byte boundary at or below its next word, so refilling the bit window is a
+// win_words<R>() words from the 16-byte boundary at or below its next word, so refilling the bit window is a
 // branch-free select; the round is unrolled, its symbols collect in registers at fixed positions;
 // and the zero-count sums run only in the instance for the zero counts of RLE items.
 // A round of R codes of at most l bits takes at most (R l + 31) / 32 + 1 words, so the copy
@@ -352,8 +352,8 @@ __global__ __launch_bounds__(256) void k_dec_tables(DecSeq* seqs, const DecPart*
 // lane stays in its own bank.
 // A code longer than the lookup table used to cost a wave a walk over the lengths in LDS and a
 // load of its symbol, each waited for (some lane of a wave meets one at most steps).
-// Measured on MI355X, the two launches (long + short): 2048 mixed bricks 1.33 + 0.17 -> 1.22 + 0.14
-// ms, one 128^3 brick 32 + 27 -> 27 + 21 us.  A copy of R + 8 words (fewer loads) took 1.30 ms, of
+// Measured on MI355X, the two launches (long + short): 2048 mixed bricks 1.33 + 0.17 -> 1.18 + 0.14
+// ms, one 128^3 brick 32 + 27 -> 25 + 20 us.  A copy of R + 8 words (fewer loads) took 1.30 ms, of
 // R + 12 1.37 ms: the LDS costs more waves than the loads cost time.
 template <uint32_t R>
 constexpr uint32_t win_words() { return R + 4; }
@@ -375,6 +375,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     constexpr uint32_t NW = kDecRound * sizeof(S) / 4;  // words of a round's symbols
     __shared__ uint32_t lut[1 << kLut];
     __shared__ int tab[96];
+    __shared__ uint32_t bounds_all[W][32];
     __shared__ S run_all[W][64 * RW * 4 / sizeof(S)];
     __shared__ uint32_t win_all[W][64 * kWinWords];
     // the workgroups of one sequence (consecutive in the list) on one XCD: its tables leave HBM once
@@ -411,6 +412,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     S* run_row = &run_all[wave][lane * RW * 4 / sizeof(S)];
     // the run row and the codeword copy are also accessed as words / 16-byte vectors
     typedef uint32_t __attribute__((may_alias)) u32a;
+    uint32_t* bounds = bounds_all[wave];
     uint32_t* win = &win_all[wave][lane];  // the copy's word k at win[64 k]: a lane's own bank
     // A lane past the sequence's last block decodes that block along and stores nothing: every lane of a
     // wave then takes every step, so that what the wave votes on or reads by lane number is there.
@@ -496,38 +498,33 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(7))) voi
     const uint32_t mlen = s.nlen;
     // A code longer than the lookup table: its length is the first l whose last code, extended with
     // ones to 32 bits, is not below the next 32 bits, and its symbol is number (code - first code +
-    // first index) of the symbol table.  Lane l - 1 holds length l's bound (an unused length has the
-    // one before it) and the step of the index offset from l to l + 1, read by lane number, so the
-    // lookup is a few vector instructions a length and touches no memory.  All lanes of the wave take it
-    // together, those without such a code with zero bits (never past a bound): a register of a lane that
-    // is masked off need not hold what the lane would have computed.
+    // first index) of the symbol table.  The bounds (an unused length has the one before it) lie in LDS,
+    // made by each wave for itself: one read a length that all lanes share, and no register of another
+    // lane, which need not hold anything where that lane is masked off.  All lanes of the wave take the
+    // lookup together, those without such a code with zero bits (never past a bound).  With the bounds and
+    // offsets in registers, read by lane number, the kernel did not fit its 72 registers: 2048 mixed bricks
+    // 1.23 ms in the long workgroups, now 1.18, a burst of 32 requests of 1 to 64 bricks 9.29 ms, now 9.05.
     const bool used = multi && lane < (int)mlen && lane < 32 && tab[64 + (lane & 31)] >= 0;
     uint32_t len0 = kLut + 1;  // the first used length past the lookup table (the last length if none)
-    uint32_t bound = 0;
-    int off = 0, off_step = 0;
     if (multi && mlen > kLut) {
         const uint64_t m = __ballot(used) >> kLut;
         len0 = m ? min(kLut + (uint32_t)__ffsll((unsigned long long)m), mlen) : mlen;
         const uint64_t end = used ? (uint64_t)((uint32_t)tab[64 + (lane & 31)] + 1u) << (31 - (lane & 31)) : 1ull;
-        bound = lane + 1 >= (int)len0 ? (uint32_t)min(end - 1, (uint64_t)0xFFFFFFFFu) : 0u;
+        uint32_t bound = lane + 1 >= (int)len0 ? (uint32_t)min(end - 1, (uint64_t)0xFFFFFFFFu) : 0u;
         bound = dpp::incl_scan<uint32_t>(bound, 0u, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
-        const int o = lane < 32 ? tab[lane] - tab[32 + lane] : 0;
-        off_step = __shfl_down(o, 1) - o;
-        off = __builtin_amdgcn_readlane(o, (int)len0 - 1);
+        if (lane < 32) bounds[lane] = bound;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // written and read by one wave
     }
     // kLong | (length << 24) | index into the symbol table (all ones: none)
     constexpr uint32_t kLong = 0x80000000u;
     auto slow = [&](uint32_t pk) -> uint32_t {
         uint32_t len = len0;
-        int idx = off;
         for (uint32_t l = len0; l < mlen; l++) {
-            const bool past = pk > (uint32_t)__builtin_amdgcn_readlane((int)bound, (int)l - 1);
+            const bool past = pk > bounds[l - 1];
             if (!__any(past)) break;  // (bounds do not fall, so no lane passes a later one)
-            const int step = __builtin_amdgcn_readlane(off_step, (int)l - 1);
             len += past ? 1u : 0u;
-            idx += past ? step : 0;
         }
-        idx += (int)(pk >> (32 - len));
+        const int idx = tab[len - 1] + (int)(pk >> (32 - len)) - tab[32 + len - 1];
         return kLong | (len << 24) | (((uint32_t)idx < nsym ? (uint32_t)idx : 0xFFFFFFu) & 0xFFFFFFu);
     };
     // The same by one lane, from the table in LDS: where the lanes of a wave take their own ways.
