@@ -7,11 +7,11 @@
 // symbol streams to the final bitstream stays in device memory:
 //   stats   one workgroup per item (or segment of a long one): zero-run RLE computed on the fly,
 //           histograms in LDS
-//   design  one wave per coded sequence: the table design of huff_design.hpp
+//   design  one wave per coded sequence, or one thread: the table design of huff_design.hpp
+//   layout  word offset of every section (sizes from the tables and bit counts)
 //   pack    one workgroup per item or segment: RLE recomputed, codewords packed through an LDS window
-//   layout  one workgroup: word offset of every section (sizes from the tables and bit counts)
-//   gather  one workgroup per coded sequence: table header, bit count, codewords, offsets
-// Intermediate data (histograms, tables, codewords, block offsets) live in a scratch arena
+//           into their section, beside its table header, bit count and block offsets
+// Intermediate data (histograms, tables, block offsets) live in a scratch arena
 // carved by an atomic bump allocator; the final layout does not depend on allocation order.
 #pragma once
 

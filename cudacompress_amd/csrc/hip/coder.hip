@@ -1,4 +1,4 @@
-// Device-resident entropy coder for gfx950: stats -> design -> pack -> layout -> gather.
+// Device-resident entropy coder for gfx950: stats -> design -> layout -> pack.
 // The bitstream it writes is word for word the layout of src/cudaCompress/Encode.cpp:402-463
 // (encodeRLHuff) and :751-782 (encodeHuff) with the table headers of
 // src/cudaCompress/HuffmanTable.cu:470-485; see coder.hpp for the pipeline.

@@ -117,8 +117,9 @@ cc_status cc_create_instance(int device, uint32_t streamCountMax, uint32_t elemC
                 CCA_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
                 CCA_HIP(hipEventRecord(e, nullptr));
             }
-            // reserve the per-stream buffers up front, as the reference sizes its arena
-            // (InstanceImpl.cpp:85-96), so running out of memory shows up here
+            // reserve the buffers of decoded pairs up front, as the reference sizes its arena
+            // (InstanceImpl.cpp:85-96), so running out of memory for them shows up here; an encode keeps no
+            // pairs, and its buffers are sized by its first call
             const uint64_t symSize = I->log2 > 16 ? 4 : 2;
             const uint64_t per = (uint64_t)streamCountMax * cca::align_up(std::max<uint32_t>(elemCountPerStreamMax, 1), 64) * symSize;
             if (per > 0) {

@@ -108,7 +108,8 @@ struct cc_instance {
     // device-resident coder
     cca::DeviceCoder coder;
 
-    // brick batches of the eager API (host/bricks.cpp): one context per group of a grouped batch
+    // the volume codecs' bricks (host/volume.cpp), and the brick batches of the eager API
+    // (host/bricks.cpp): one context per group of a grouped batch
     cca::BrickCtx batch;
     std::vector<std::unique_ptr<cca::BrickCtx>> groups;
     hipEvent_t group_fork = nullptr;

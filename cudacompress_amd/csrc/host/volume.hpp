@@ -1,4 +1,4 @@
-// Volume codecs (caller layouts of src/examples/CompressVolume.cpp); output in inst->vol_bits.
+// Volume codecs (caller layouts of src/examples/CompressVolume.cpp); output in inst->out_words.
 #pragma once
 
 #include "instance.hpp"
