@@ -68,7 +68,7 @@ CC_API void* cc_get_instance_stream(const cc_instance* inst);
 CC_API cc_status cc_set_instance_dialect(cc_instance* inst, int dialect);
 /* Groups of an eager brick batch (cc_compress/decompress_bricks_float): contiguous brick ranges
  * run as concurrent pipelines on their own streams, their bitstreams still back to back in brick
- * order.  0 or 1 (default): one pipeline.  Plans always capture one.  No reference counterpart. */
+ * order.  0 or 1 (default): one pipeline.  A plan captures as many.  No reference counterpart. */
 CC_API cc_status cc_set_instance_brick_groups(cc_instance* inst, uint32_t groups);
 /* Float volumes (all channels together) of at least this many voxels go through the single-volume
  * transforms, level by level, and smaller ones through the brick passes, whose offsets are 32 bits.
